@@ -1,13 +1,17 @@
-"""Loader for the in-tree HIP library ``csrc/libofq_hip.so`` (the C ABI of ``include/ofq.h``).
+"""Loader for the in-tree HIP library ``csrc/libofq_hip.so`` (the C ABI of ``include/ofq.h``) and
+for ``csrc/ofq_torch.so``, the extension module that calls it with torch tensors.
 
-There is no CPU fallback: if the library is missing the import fails, and every call checks the
+There is no CPU fallback: if a library is missing the first call fails, and every call checks the
 returned status and raises.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libofq_hip.so")
+TORCH_LIB_PATH = os.path.join(_HERE, "csrc", "ofq_torch.so")
 
 # mirror of the enums in include/ofq.h
 OK = 0
@@ -77,14 +81,18 @@ class OfqError(RuntimeError):
 _lib = None
 
 
+def _require(path):
+    if not os.path.exists(path):
+        raise RuntimeError(
+            f"{path} is missing: build it with `make -C {os.path.dirname(path)}` "
+            "(or __graft_entry__.build()); there is no CPU fallback")
+
+
 def lib():
     """The loaded library with prototypes set.  Raises if it has not been built."""
     global _lib
     if _lib is None:
-        if not os.path.exists(LIB_PATH):
-            raise RuntimeError(
-                f"{LIB_PATH} is missing: build it with `make -C {os.path.dirname(LIB_PATH)}` "
-                "(or __graft_entry__.build()); there is no CPU fallback")
+        _require(LIB_PATH)
         handle = ctypes.CDLL(LIB_PATH)
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(handle, name)
@@ -94,6 +102,27 @@ def lib():
     return _lib
 
 
-def check(fn_name, status):
-    if status != OK:
-        raise OfqError(fn_name, status, lib().ofq_status_string(status).decode())
+class CheckFailedError(RuntimeError):
+    """Raised where the reference functor's CHECK_OR_RETURN would fail."""
+
+
+class _Native:
+    """The functions of ``csrc/ofq_torch.cpp``.  The module is loaded when the first of them is
+    looked up; from then on each is a plain attribute of this object."""
+
+    def __getattr__(self, name):
+        _require(LIB_PATH)
+        _require(TORCH_LIB_PATH)
+        loader = importlib.machinery.ExtensionFileLoader("ofq_torch", TORCH_LIB_PATH)
+        module = importlib.util.module_from_spec(
+            importlib.util.spec_from_loader("ofq_torch", loader))
+        loader.exec_module(module)
+        module.set_errors(CheckFailedError, OfqError)
+        self.__dict__.update({k: v for k, v in vars(module).items() if not k.startswith("_")})
+        try:
+            return self.__dict__[name]
+        except KeyError:
+            raise AttributeError(name) from None
+
+
+native = _Native()

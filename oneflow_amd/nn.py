@@ -6,6 +6,7 @@ import torch
 
 from . import functional as _C
 from ._lib import OfqError
+from ._lib import native as _native
 
 
 class MinMaxObserver(torch.nn.Module):
@@ -69,11 +70,12 @@ class MovingAverageMinMaxObserver(torch.nn.Module):
         self.moving_min.fill_(0)
 
     def forward(self, input, current_train_step):
-        if self.moving_max.dtype != input.dtype:
-            self.moving_max = self.moving_max.to(input.dtype)
+        moving_max = self.moving_max
+        if moving_max.dtype != input.dtype:
+            self.moving_max = moving_max = moving_max.to(input.dtype)
             self.moving_min = self.moving_min.to(input.dtype)
         return _C.moving_average_min_max_observer(
-            input, current_train_step, self.moving_max, self.moving_min, self.training,
+            input, current_train_step, moving_max, self.moving_min, self.training,
             self.stop_update_after_iters, self.quantization_formula, self.quantization_bit,
             self.quantization_scheme, self.momentum)
 
@@ -165,23 +167,30 @@ class QuantizedLinear(torch.nn.Module):
         super()._load_from_state_dict(*args, **kwargs)
         self.weight_tiled, self._tiled_from = None, None
 
+    def _packed(self):
+        """(weight, weight_scale, weight_zero, bias).  Read from the buffer dict: a look-up through
+        ``Module.__getattr__`` costs 0.4 us, four of them a third of a decode call's host time."""
+        b = self._buffers
+        try:
+            return b["weight"], b["weight_scale"], b["weight_zero"], b["bias"]
+        except KeyError:  # registered as something other than a buffer since
+            return self.weight, self.weight_scale, self.weight_zero, self.bias
+
     def forward(self, x):
-        tiled = self._decode_copy()
-        if tiled is not None and x.dtype == torch.float16 and self.group_size % 128 == 0:
-            m = x.numel() // x.shape[-1]
-            if 2 <= m <= 16:
-                try:
-                    return _C.fused_linear_with_tiled_groupwise_quantized_weight(
-                        x, tiled, self.weight_scale, w_zero=self.weight_zero, b=self.bias,
-                        num_bits=self.num_bits, symmetric=self.symmetric, group_dim=1,
-                        group_size=self.group_size)
-                except OfqError as e:  # e.g. m * k beyond what the kernel stages in LDS
-                    if e.status != 5:  # OFQ_ERR_UNSUPPORTED
-                        raise
-        return _C.fused_linear_with_groupwise_quantized_weight(
-            x, self.weight, self.weight_scale, w_zero=self.weight_zero, b=self.bias,
-            num_bits=self.num_bits, symmetric=self.symmetric, group_dim=1,
-            group_size=self.group_size)
+        w, scale, zero, bias = self._packed()
+        if self._tiled_from is not None:
+            tiled = self._decode_copy()
+            if tiled is not None and x.dtype == torch.float16 and self.group_size % 128 == 0:
+                m = x.numel() // x.shape[-1]
+                if 2 <= m <= 16:
+                    try:
+                        return _native.fused_linear_tiled(x, tiled, scale, zero, bias, self.num_bits,
+                                                          self.symmetric, 1, self.group_size)
+                    except OfqError as e:  # e.g. m * k beyond what the kernel stages in LDS
+                        if e.status != 5:  # OFQ_ERR_UNSUPPORTED
+                            raise
+        return _native.fused_linear(x, w, scale, zero, bias, self.num_bits, self.symmetric, 1,
+                                    self.group_size)
 
     def extra_repr(self):
         return (f"in_features={self.in_features}, out_features={self.out_features}, "
@@ -208,11 +217,12 @@ class QuantizedGLU(torch.nn.Module):
                    QuantizedLinear.from_float(gate_linear, **quant_args), activation)
 
     def forward(self, x):
-        h, g = self.hidden, self.gate
-        return _C.fused_glu_with_groupwise_quantized_weight(
-            x, h.weight, h.weight_scale, w_zero=h.weight_zero, b=h.bias, v=g.weight,
-            v_scale=g.weight_scale, v_zero=g.weight_zero, c=g.bias, activation=self.activation,
-            num_bits=h.num_bits, symmetric=h.symmetric, group_dim=1, group_size=h.group_size)
+        modules = self._modules
+        h, g = modules["hidden"], modules["gate"]
+        w, w_scale, w_zero, b = h._packed()
+        v, v_scale, v_zero, c = g._packed()
+        return _native.fused_glu(x, w, w_scale, w_zero, b, v, v_scale, v_zero, c, self.activation,
+                                 h.num_bits, h.symmetric, 1, h.group_size)
 
 
 class GroupedQuantizedLinear(torch.nn.Module):
@@ -229,14 +239,13 @@ class GroupedQuantizedLinear(torch.nn.Module):
         self.linears = torch.nn.ModuleList(linears)
 
     def forward(self, x):
-        ls = list(self.linears)
-        biases = [m.bias for m in ls]
+        ls = list(self._modules["linears"]._modules.values())
+        ws, scales, zeros, biases = zip(*[m._packed() for m in ls])
         if any(b is None for b in biases):
             if not all(b is None for b in biases):
                 raise ValueError("either every linear has a bias or none")
             biases = None
-        return tuple(_C.grouped_linear_with_groupwise_quantized_weight(
-            [x] * len(ls), [m.weight for m in ls], [m.weight_scale for m in ls],
-            w_zeros=None if ls[0].symmetric else [m.weight_zero for m in ls], bs=biases,
-            num_bits=ls[0].num_bits, symmetric=ls[0].symmetric, group_dim=1,
-            group_size=ls[0].group_size))
+        first = ls[0]
+        return tuple(_native.grouped_linear(
+            [x] * len(ls), ws, scales, None if first.symmetric else zeros, biases, first.num_bits,
+            first.symmetric, 1, first.group_size))
