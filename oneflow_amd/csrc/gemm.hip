@@ -43,7 +43,7 @@ int pick_tile_width(int64_t m, int64_t n, bool allow_wide) {
 namespace {
 
 // x[m,k] * wt[n,k]^T with both operands in T (the dequantised weight of the two-pass path)
-template<typename T, class MF>
+template<bool RG, typename T, class MF>
 int launch_plain(hipStream_t st, const LinearArgs& a, const void* wt) {
   typedef typename TT<T>::storage S;
   typedef EpBias<T> EP;
@@ -59,22 +59,22 @@ int launch_plain(hipStream_t st, const LinearArgs& a, const void* wt) {
   const int64_t b256 = ((a.m + 255) / 256) * ((a.n + 127) / 128);
   const int64_t b128 = ((a.m + 127) / 128) * ((a.n + 127) / 128);
   if (b256 < 192 && b128 >= 192 && b128 <= 512) {
-    return launch_core2<MF, B2Copy<128, 512>, EP, 128, 128, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                  a.n, a.k / 64);
+    return launch_core2<MF, B2Copy<RG, 128, 512>, EP, 128, 128, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
+                                                                  a.n, (a.k + 63) / 64);
   }
   switch (pick_tile_width(a.m, a.n, true)) {
     case 384:
-      return launch_core2<MF, B2Copy<384, 512>, EP, 256, 384, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                    a.n, a.k / 64);
+      return launch_core2<MF, B2Copy<RG, 384, 512>, EP, 256, 384, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
+                                                                    a.n, (a.k + 63) / 64);
     case 256:
-      return launch_core2<MF, B2Copy<256, 512>, EP, 256, 256, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                    a.n, a.k / 64);
+      return launch_core2<MF, B2Copy<RG, 256, 512>, EP, 256, 256, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
+                                                                    a.n, (a.k + 63) / 64);
     case 192:
-      return launch_core2<MF, B2Copy<192, 512>, EP, 256, 192, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                    a.n, a.k / 64);
+      return launch_core2<MF, B2Copy<RG, 192, 512>, EP, 256, 192, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
+                                                                    a.n, (a.k + 63) / 64);
     default:
-      return launch_core2<MF, B2Copy<128, 512>, EP, 256, 128, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                    a.n, a.k / 64);
+      return launch_core2<MF, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
+                                                                    a.n, (a.k + 63) / 64);
   }
 }
 
@@ -125,7 +125,7 @@ int wq_splits(const LinearArgs& a) {
   const int64_t slots = a.m > 128 ? 256 : 512;
   const int64_t blocks = ((a.m + bm - 1) / bm) * ((a.n + 127) / 128);
   int64_t s = slots / blocks;
-  const int64_t kt = a.k / 64;
+  const int64_t kt = (a.k + 63) / 64;
   if (s > 8) s = 8;
   if (s > kt / 4) s = kt / 4;
   if (s < 1) s = 1;
@@ -134,7 +134,7 @@ int wq_splits(const LinearArgs& a) {
   return (int)s;
 }
 
-template<typename T, class MF, int BITS, bool SIGNED, int ZMODE>
+template<bool RG, typename T, class MF, int BITS, bool SIGNED, int ZMODE>
 int launch_wq_variant(hipStream_t st, const LinearArgs& a, float* partials, int splits) {
   typedef typename TT<T>::storage S;
   typedef EpBias<T> EP;
@@ -154,13 +154,13 @@ int launch_wq_variant(hipStream_t st, const LinearArgs& a, float* partials, int 
     pp.out = partials;
     int rc;
     if (a.m > 128) {
-      rc = launch_core2<MF, B2Dequant<T, BITS, SIGNED, ZMODE, 128, 512>, EpPartial, 256, 128, 4,
-                        2>(st, a.x, a.k * 2, bp, pp, a.m, a.n, a.k / 64, splits);
+      rc = launch_core2<MF, B2Dequant<RG, T, BITS, SIGNED, ZMODE, 128, 512>, EpPartial, 256, 128, 4,
+                        2>(st, a.x, a.k * 2, bp, pp, a.m, a.n, (a.k + 63) / 64, splits);
     } else {
       // 8 waves on the 128x128 tile (32x64 per wave): more waves to hide the slice's short
       // k loop behind (28 us against 33 us on 4 waves at m = 128, 11008x4096)
-      rc = launch_core2<MF, B2Dequant<T, BITS, SIGNED, ZMODE, 128, 512>, EpPartial, 128, 128, 4,
-                        2>(st, a.x, a.k * 2, bp, pp, a.m, a.n, a.k / 64, splits);
+      rc = launch_core2<MF, B2Dequant<RG, T, BITS, SIGNED, ZMODE, 128, 512>, EpPartial, 128, 128, 4,
+                        2>(st, a.x, a.k * 2, bp, pp, a.m, a.n, (a.k + 63) / 64, splits);
     }
     if (rc != OFQ_OK) return rc;
     const int64_t mn = a.m * a.n;
@@ -176,29 +176,30 @@ int launch_wq_variant(hipStream_t st, const LinearArgs& a, float* partials, int 
   // 256x128 tiles on 8 waves when there are enough rows of x to fill them, else 128x128 on 4
   if (a.m > 128) {
     if (pick_tile_width(a.m, a.n, false) == 192) {
-      return launch_core2<MF, B2Dequant<T, BITS, SIGNED, ZMODE, 192, 512>, EP, 256, 192, 4, 2>(
-          st, a.x, a.k * 2, bp, ep, a.m, a.n, a.k / 64);
+      return launch_core2<MF, B2Dequant<RG, T, BITS, SIGNED, ZMODE, 192, 512>, EP, 256, 192, 4, 2>(
+          st, a.x, a.k * 2, bp, ep, a.m, a.n, (a.k + 63) / 64);
     }
-    return launch_core2<MF, B2Dequant<T, BITS, SIGNED, ZMODE, 128, 512>, EP, 256, 128, 4, 2>(
-        st, a.x, a.k * 2, bp, ep, a.m, a.n, a.k / 64);
+    return launch_core2<MF, B2Dequant<RG, T, BITS, SIGNED, ZMODE, 128, 512>, EP, 256, 128, 4, 2>(
+        st, a.x, a.k * 2, bp, ep, a.m, a.n, (a.k + 63) / 64);
   }
   // few rows of x: 128-wide weight tiles would leave most CUs without a block (86 tiles for
   // n = 11008), so the weight tile shrinks until the grid covers the chip
   const int64_t n_tiles128 = (a.n + 127) / 128;
   if (n_tiles128 < 192) {
-    return launch_core2<MF, B2Dequant<T, BITS, SIGNED, ZMODE, 32, 256>, EP, 128, 32, 4, 1>(
-        st, a.x, a.k * 2, bp, ep, a.m, a.n, a.k / 64);
+    return launch_core2<MF, B2Dequant<RG, T, BITS, SIGNED, ZMODE, 32, 256>, EP, 128, 32, 4, 1>(
+        st, a.x, a.k * 2, bp, ep, a.m, a.n, (a.k + 63) / 64);
   }
-  return launch_core2<MF, B2Dequant<T, BITS, SIGNED, ZMODE, 128, 256>, EP, 128, 128, 2, 2>(
-      st, a.x, a.k * 2, bp, ep, a.m, a.n, a.k / 64);
+  return launch_core2<MF, B2Dequant<RG, T, BITS, SIGNED, ZMODE, 128, 256>, EP, 128, 128, 2, 2>(
+      st, a.x, a.k * 2, bp, ep, a.m, a.n, (a.k + 63) / 64);
 }
 
 template<typename T, class MF>
 int launch_wq_t(hipStream_t st, const LinearArgs& a, float* partials, int splits) {
   const int zmode = !a.symmetric ? 2 : (a.w_signed ? 0 : 1);
-#define OFQ_V(B, SG, ZM)                                       \
-  if (a.bits == B && a.w_signed == SG && zmode == ZM)          \
-    return launch_wq_variant<T, MF, B, SG, ZM>(st, a, partials, splits);
+#define OFQ_V(B, SG, ZM)                                                                       \
+  if (a.bits == B && a.w_signed == SG && zmode == ZM)                                          \
+    return a.k % 64 == 0 ? launch_wq_variant<false, T, MF, B, SG, ZM>(st, a, partials, splits) \
+                         : launch_wq_variant<true, T, MF, B, SG, ZM>(st, a, partials, splits);
   OFQ_V(4, true, 0)
   OFQ_V(4, false, 1)
   OFQ_V(4, false, 2)
@@ -215,7 +216,9 @@ bool gemm_wq_supported(const LinearArgs& a) {
   if (a.t_dtype != OFQ_F16 && a.t_dtype != OFQ_BF16) return false;
   if (a.group_dim != 1 || a.m < 1) return false;
   const int elems_per_chunk = a.bits == 4 ? 32 : 16;
-  if (a.k % 64 != 0 || a.group_size % elems_per_chunk != 0) return false;
+  // whole chunks of codes (and whole 16-byte pieces of x) per row; a last k-tile that is not full
+  // is padded with zeros in LDS
+  if (a.k % elems_per_chunk != 0 || a.group_size % elems_per_chunk != 0) return false;
   return true;
 }
 
@@ -246,8 +249,12 @@ int launch_gemm_wq(hipStream_t st, const LinearArgs& a, void* workspace, size_t 
                                             a.symmetric ? 1 : 0, a.n * (a.k / a.group_size),
                                             a.group_size, 1);
     if (rc != OFQ_OK) return rc;
-    if (a.t_dtype == OFQ_F16) return launch_plain<f16, MfmaF16>(st, a, workspace);
-    return launch_plain<bf16, MfmaBF16>(st, a, workspace);
+    if (a.k % 64 != 0) {
+      return a.t_dtype == OFQ_F16 ? launch_plain<true, f16, MfmaF16>(st, a, workspace)
+                                  : launch_plain<true, bf16, MfmaBF16>(st, a, workspace);
+    }
+    if (a.t_dtype == OFQ_F16) return launch_plain<false, f16, MfmaF16>(st, a, workspace);
+    return launch_plain<false, bf16, MfmaBF16>(st, a, workspace);
   }
   if (a.t_dtype == OFQ_F16) return launch_wq_t<f16, MfmaF16>(st, a, nullptr, 1);
   return launch_wq_t<bf16, MfmaBF16>(st, a, nullptr, 1);
@@ -264,7 +271,7 @@ namespace {
 int gn_splits(const LinearArgs& a) {
   const int64_t blocks = ((a.m + 255) / 256) * ((a.n + 127) / 128);
   int64_t s = 256 / blocks;
-  const int64_t kt = a.k / 64;
+  const int64_t kt = (a.k + 63) / 64;
   if (s > 8) s = 8;
   if (s > kt / 4) s = kt / 4;
   if (s < 1) s = 1;
@@ -275,6 +282,7 @@ int gn_splits(const LinearArgs& a) {
 template<typename T, class MF>
 int launch_plain_split(hipStream_t st, const LinearArgs& a, const void* wt, float* partials,
                        int splits) {
+  constexpr bool RG = false;  // whole k-tiles (gemm_gn_workspace_bytes)
   typedef typename TT<T>::storage S;
   BCopyParams bp;
   bp.b = static_cast<const uint8_t*>(wt);
@@ -282,8 +290,8 @@ int launch_plain_split(hipStream_t st, const LinearArgs& a, const void* wt, floa
   bp.N = (int)a.n;
   EpPartial::Params pp;
   pp.out = partials;
-  const int rc = launch_core2<MF, B2Copy<128, 512>, EpPartial, 256, 128, 4, 2>(
-      st, a.x, a.k * 2, bp, pp, a.m, a.n, a.k / 64, splits);
+  const int rc = launch_core2<MF, B2Copy<RG, 128, 512>, EpPartial, 256, 128, 4, 2>(
+      st, a.x, a.k * 2, bp, pp, a.m, a.n, (a.k + 63) / 64, splits);
   if (rc != OFQ_OK) return rc;
   const int64_t mn = a.m * a.n;
   const S* bias = static_cast<const S*>(a.bias);
@@ -326,8 +334,8 @@ int launch_gemm_gn(hipStream_t st, const LinearArgs& a, void* workspace) {
     }
     return launch_plain_split<bf16, MfmaBF16>(st, a, workspace, partials, splits);
   }
-  if (a.t_dtype == OFQ_F16) return launch_plain<f16, MfmaF16>(st, a, workspace);
-  return launch_plain<bf16, MfmaBF16>(st, a, workspace);
+  if (a.t_dtype == OFQ_F16) return launch_plain<false, f16, MfmaF16>(st, a, workspace);
+  return launch_plain<false, bf16, MfmaBF16>(st, a, workspace);
 }
 
 }  // namespace ofq
@@ -355,7 +363,7 @@ namespace {
 //    512 x 11008 x 4096: 40.5 against 48.3 us).
 enum MqTile { kMqTileDefault = 0, kMqTile64 = 64, kMqTile128 = 128 };
 MqTile mq_tile(int64_t m, int64_t n, int64_t k) {
-  if (m <= kMatmulQuantRowsMaxM || k % 128 != 0 || k > 6144) return kMqTileDefault;
+  if (m <= kMatmulQuantRowsMaxM || k > 6144) return kMqTileDefault;
   const int64_t t64 = ((m + 63) / 64) * ((n + 63) / 64);
   if (m <= 768 && t64 >= 128 && t64 <= 768) return kMqTile64;
   const int64_t b256 = ((m + 255) / 256) * ((n + 127) / 128);
@@ -368,7 +376,7 @@ int mq_splits(int64_t m, int64_t n, int64_t k) {
   if (mq_tile(m, n, k) != kMqTileDefault) return 1;
   // long rows (k >= 8192) already pay for slices from 33 rows of a on: 4096 x 11008 at m = 64
   // streams in 33 us and runs in 22 us as slices
-  if (m <= (k >= 8192 ? kMatmulQuantRowsMaxM / 2 : kMatmulQuantRowsMaxM) || k % 128 != 0) return 1;
+  if (m <= (k >= 8192 ? kMatmulQuantRowsMaxM / 2 : kMatmulQuantRowsMaxM)) return 1;
   int64_t bm = m > 128 ? 256 : 128;
   int64_t slots = m > 128 ? 256 : 512;
   // up to 512 rows on a weight with few column tiles: 128-row tiles and fewer, longer slices
@@ -380,7 +388,7 @@ int mq_splits(int64_t m, int64_t n, int64_t k) {
   }
   const int64_t blocks = ((m + bm - 1) / bm) * ((n + 127) / 128);
   int64_t s = slots / blocks;
-  const int64_t kt = k / 128;
+  const int64_t kt = (k + 127) / 128;
   if (s > 8) s = 8;
   if (s > kt / 4) s = kt / 4;
   if (s < 1) s = 1;
@@ -422,7 +430,7 @@ splitk_finalize_i32(const int* __restrict__ part, const float* __restrict__ a_sc
   }
 }
 
-template<typename T>
+template<bool RG, typename T>
 int launch_mq_split(hipStream_t st, const void* a, const BCopyParams& bp, const float* a_scale,
                     const float* b_scale, const void* bias, void* out, int64_t m, int64_t n,
                     int64_t k, float* partials, int splits) {
@@ -432,11 +440,11 @@ int launch_mq_split(hipStream_t st, const void* a, const BCopyParams& bp, const 
   int rc;
   const bool few_tiles = m <= 512 && ((m + 127) / 128) * ((n + 127) / 128) <= 128;  // as mq_splits
   if (m > 128 && !few_tiles) {
-    rc = launch_core2<MfmaI8, B2Copy<128, 512>, EpPartialI32, 256, 128, 4, 2>(st, a, k, bp, pp, m,
-                                                                             n, k / 128, splits);
+    rc = launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EpPartialI32, 256, 128, 4, 2>(st, a, k, bp, pp, m,
+                                                                             n, (k + 127) / 128, splits);
   } else {
-    rc = launch_core2<MfmaI8, B2Copy<128, 512>, EpPartialI32, 128, 128, 4, 2>(st, a, k, bp, pp, m,
-                                                                             n, k / 128, splits);
+    rc = launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EpPartialI32, 128, 128, 4, 2>(st, a, k, bp, pp, m,
+                                                                             n, (k + 127) / 128, splits);
   }
   if (rc != OFQ_OK) return rc;
   const int64_t mn = m * n;
@@ -449,6 +457,39 @@ int launch_mq_split(hipStream_t st, const void* a, const BCopyParams& bp, const 
         pi, a_scale, b_scale, static_cast<const S*>(bias), static_cast<S*>(out), mn, (int)n, splits);
   }
   return ofq_check_launch();
+}
+
+// one launch, no K slices
+template<bool RG, typename T>
+int launch_mq(hipStream_t st, const void* a, const BCopyParams& bp, const float* a_scale,
+              const float* b_scale, const void* bias, void* out, int64_t m, int64_t n, int64_t k) {
+  typedef EpScale<T> EP;
+  typename EP::Params ep;
+  ep.a_scale = a_scale;
+  ep.b_scale = b_scale;
+  ep.bias = static_cast<const typename TT<T>::storage*>(bias);
+  ep.out = static_cast<typename TT<T>::storage*>(out);
+  const int64_t kt = (k + 127) / 128;
+  const MqTile tile = mq_tile(m, n, k);
+  if (tile == kMqTile64) {
+    return launch_core2<MfmaI8, B2Copy<RG, 64, 256>, EP, 64, 64, 2, 2>(st, a, k, bp, ep, m, n, kt);
+  }
+  if (tile == kMqTile128) {
+    return launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EP, 128, 128, 4, 2>(st, a, k, bp, ep, m, n, kt);
+  }
+  if (m <= 128) {
+    return launch_core2<MfmaI8, B2Copy<RG, 128, 256>, EP, 128, 128, 2, 2>(st, a, k, bp, ep, m, n, kt);
+  }
+  switch (pick_tile_width(m, n, true)) {
+    case 384:
+      return launch_core2<MfmaI8, B2Copy<RG, 384, 512>, EP, 256, 384, 4, 2>(st, a, k, bp, ep, m, n, kt);
+    case 256:
+      return launch_core2<MfmaI8, B2Copy<RG, 256, 512>, EP, 256, 256, 4, 2>(st, a, k, bp, ep, m, n, kt);
+    case 192:
+      return launch_core2<MfmaI8, B2Copy<RG, 192, 512>, EP, 256, 192, 4, 2>(st, a, k, bp, ep, m, n, kt);
+    default:
+      return launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a, k, bp, ep, m, n, kt);
+  }
 }
 
 }  // namespace
@@ -482,7 +523,8 @@ extern "C" int ofq_matmul_quant_ws(void* stream, const void* a, const void* b, c
   if (m == 0 || n == 0) return OFQ_OK;
   const int64_t i32max = 0x7FFFFFFF;
   OFQ_RETURN_IF(m * k > i32max || n * k > i32max || m * n > i32max, OFQ_ERR_UNSUPPORTED);
-  // rows are consumed in 64-byte chunks of K (streaming kernel) or 128-byte tiles (GEMM)
+  // rows are consumed in 64-byte chunks of K (streaming kernel) or 128-byte tiles (GEMM, the last
+  // one padded with zeros)
   OFQ_RETURN_IF(k % 64 != 0, OFQ_ERR_UNSUPPORTED);
   OFQ_RETURN_IF(a == nullptr || b == nullptr || a_scale == nullptr || b_scale == nullptr
                     || out == nullptr,
@@ -498,64 +540,37 @@ extern "C" int ofq_matmul_quant_ws(void* stream, const void* a, const void* b, c
     const size_t need = (size_t)splits * (size_t)m * (size_t)n * 4;
     if (splits > 1 && workspace != nullptr && workspace_bytes >= need && ofq_aligned16(workspace)) {
       float* part = static_cast<float*>(workspace);
-      switch (out_dtype) {
-        case OFQ_F16:
-          return launch_mq_split<f16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, part, splits);
-        case OFQ_BF16:
-          return launch_mq_split<bf16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, part,
-                                       splits);
-        default:
-          return launch_mq_split<float>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, part,
-                                        splits);
+#define OFQ_MQS(RG, T)                                                                           \
+  return launch_mq_split<RG, T>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, part, splits)
+      if (k % 128 != 0) {
+        switch (out_dtype) {
+          case OFQ_F16: OFQ_MQS(true, f16);
+          case OFQ_BF16: OFQ_MQS(true, bf16);
+          default: OFQ_MQS(true, float);
+        }
       }
+      switch (out_dtype) {
+        case OFQ_F16: OFQ_MQS(false, f16);
+        case OFQ_BF16: OFQ_MQS(false, bf16);
+        default: OFQ_MQS(false, float);
+      }
+#undef OFQ_MQS
     }
   }
-  // few rows of a, or a K the GEMM's tiles do not divide: the weights stream once per 64 rows
-  if ((m <= kMatmulQuantRowsMaxM || k % 128 != 0) && matmul_quant_rows_supported(m, n, k)) {
+  // few rows of a: the weights stream once
+  if (m <= kMatmulQuantRowsMaxM && matmul_quant_rows_supported(m, n, k)) {
     return launch_matmul_quant_rows(st, a, b, a_scale, b_scale, bias, out, out_dtype, m, n, k);
   }
-  OFQ_RETURN_IF(k % 128 != 0, OFQ_ERR_UNSUPPORTED);
-#define OFQ_MQ(T)                                                                              \
-  {                                                                                            \
-    typedef EpScale<T> EP;                                                                     \
-    EP::Params ep;                                                                             \
-    ep.a_scale = a_scale;                                                                      \
-    ep.b_scale = b_scale;                                                                      \
-    ep.bias = static_cast<const TT<T>::storage*>(bias);                                        \
-    ep.out = static_cast<TT<T>::storage*>(out);                                                \
-    const MqTile tile = mq_tile(m, n, k);                                                      \
-    if (tile == kMqTile64) {                                                                   \
-      return launch_core2<MfmaI8, B2Copy<64, 256>, EP, 64, 64, 2, 2>(st, a, k, bp, ep, m, n,   \
-                                                                    k / 128);                  \
-    }                                                                                          \
-    if (tile == kMqTile128) {                                                                  \
-      return launch_core2<MfmaI8, B2Copy<128, 512>, EP, 128, 128, 4, 2>(st, a, k, bp, ep, m,   \
-                                                                       n, k / 128);            \
-    }                                                                                          \
-    const int bn = m > 128 ? pick_tile_width(m, n, true) : 128;                                \
-    if (bn == 256) {                                                                           \
-      return launch_core2<MfmaI8, B2Copy<256, 512>, EP, 256, 256, 4, 2>(st, a, k, bp, ep, m,   \
-                                                                        n, k / 128);           \
-    }                                                                                          \
-    if (bn == 384) {                                                                           \
-      return launch_core2<MfmaI8, B2Copy<384, 512>, EP, 256, 384, 4, 2>(st, a, k, bp, ep, m,   \
-                                                                        n, k / 128);           \
-    }                                                                                          \
-    if (bn == 192) {                                                                           \
-      return launch_core2<MfmaI8, B2Copy<192, 512>, EP, 256, 192, 4, 2>(st, a, k, bp, ep, m,   \
-                                                                        n, k / 128);           \
-    }                                                                                          \
-    if (m > 128) {                                                                             \
-      return launch_core2<MfmaI8, B2Copy<128, 512>, EP, 256, 128, 4, 2>(st, a, k, bp, ep, m,   \
-                                                                        n, k / 128);           \
-    }                                                                                          \
-    return launch_core2<MfmaI8, B2Copy<128, 256>, EP, 128, 128, 2, 2>(st, a, k, bp, ep, m, n,  \
-                                                                      k / 128);                \
+  if (k % 128 != 0) {
+    switch (out_dtype) {
+      case OFQ_F16: return launch_mq<true, f16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k);
+      case OFQ_BF16: return launch_mq<true, bf16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k);
+      default: return launch_mq<true, float>(st, a, bp, a_scale, b_scale, bias, out, m, n, k);
+    }
   }
   switch (out_dtype) {
-    case OFQ_F16: OFQ_MQ(f16)
-    case OFQ_BF16: OFQ_MQ(bf16)
-    default: OFQ_MQ(float)
+    case OFQ_F16: return launch_mq<false, f16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k);
+    case OFQ_BF16: return launch_mq<false, bf16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k);
+    default: return launch_mq<false, float>(st, a, bp, a_scale, b_scale, bias, out, m, n, k);
   }
-#undef OFQ_MQ
 }

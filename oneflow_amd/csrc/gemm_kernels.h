@@ -229,8 +229,12 @@ __device__ __forceinline__ void wait_vmem_le() {
 }
 __device__ __forceinline__ void wait_vmem_all() { wait_vmem_le<0>(); }
 
-// rows [0, ROWS) x 128 bytes of tile kt of a row-major byte matrix -> swizzled LDS tile
-template<int ROWS, int NWAVES>
+// rows [0, ROWS) x 128 bytes of tile kt of a row-major byte matrix -> swizzled LDS tile.  Rows are
+// `ld` bytes, a multiple of 16 but not of 128: of the last tile of such a ragged matrix the pieces
+// past the end of a row are not requested, their lanes write zeros to LDS instead (both operands
+// do so, or one does and the other is finite there: the products add 0).  RAGGED is a flag of the
+// kernel: the same test made at run time cost 8 % of 2048 x 11008 x 4096 (registers).
+template<bool RAGGED, int ROWS, int NWAVES>
 __device__ __forceinline__ void async_tile(const uint8_t* __restrict__ g, int64_t ld, int row0,
                                            int row_limit, int kt, uint8_t* lds_tile, int wave,
                                            int lane) {
@@ -251,26 +255,32 @@ __device__ __forceinline__ void async_tile(const uint8_t* __restrict__ g, int64_
     int rel = grp * 8 + sub;  // row within the tile; rows past the matrix repeat its last row
     rel = row0 + rel < row_limit ? rel : row_limit - 1 - row0;
     const uint32_t off = (uint32_t)rel * (uint32_t)ld + (uint32_t)(piece * 16);
-    async_copy16_at(gk, off, lds0 + grp * 1024);
+    if (!RAGGED || kt * kStageRow + piece * 16 < (int)ld) {
+      async_copy16_at(gk, off, lds0 + grp * 1024);
+    } else {
+      *reinterpret_cast<u32x4*>(lds_tile + grp * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+    }
   }
 }
 
-template<int BN, int NT>
+template<bool RAGGED, int BN, int NT>
 struct B2Copy {
+  static constexpr bool kRaggedK = RAGGED;
   typedef BCopyParams Params;
   static constexpr bool kDirect = true;
   struct Regs {};
   static __device__ __forceinline__ void load(const Params& p, int n0, int kt, int wave, int lane,
                                               int, Regs&, uint8_t* lds_b) {
-    async_tile<BN, NT / 64>(p.b, p.ldb, n0, p.N, kt, lds_b, wave, lane);
+    async_tile<RAGGED, BN, NT / 64>(p.b, p.ldb, n0, p.N, kt, lds_b, wave, lane);
   }
   static __device__ __forceinline__ void store_part(const Params&, const Regs&, uint8_t*, int, int) {}
 };
 
 // Groupwise-quantised weights: codes are loaded as stored
 // ([N, K*bits/8] bytes) two k-tiles ahead, and turned into T when written to the swizzled LDS tile.
-template<typename T, int BITS, bool SIGNED, int ZMODE, int BN, int NT>
+template<bool RAGGED, typename T, int BITS, bool SIGNED, int ZMODE, int BN, int NT>
 struct B2Dequant {
+  static constexpr bool kRaggedK = RAGGED;
   typedef WqParams<T> Params;
   static constexpr bool kDirect = false;
   static constexpr int kCodeBytesPerRow = 64 * BITS / 8;
@@ -298,9 +308,11 @@ struct B2Dequant {
       int row = n0 + q / kChunksPerRow;
       row = row < p.N ? row : p.N - 1;
       const int c = q % kChunksPerRow;
-      r.v[i] = *reinterpret_cast<const u32x4*>(p.w + (int64_t)row * p.ldw
-                                               + (int64_t)kt * kCodeBytesPerRow + c * 16);
-      const int k = kt * 64 + c * kElemsPerChunk;
+      // past the end of a ragged row: its first chunk again (finite, and x is zero there)
+      const int byte = kt * kCodeBytesPerRow + c * 16;
+      const bool in_row = !RAGGED || byte < (int)p.ldw;
+      r.v[i] = *reinterpret_cast<const u32x4*>(p.w + (int64_t)row * p.ldw + (in_row ? byte : 0));
+      const int k = in_row ? kt * 64 + c * kElemsPerChunk : 0;
       const int64_t si = (int64_t)row * p.G + k / p.group_size;
       r.s[i] = reinterpret_cast<const uint16_t*>(p.scale)[si];
       if (ZMODE == 2) r.z[i] = reinterpret_cast<const uint16_t*>(p.zero)[si];
@@ -390,7 +402,7 @@ gemm_core2(const uint8_t* __restrict__ A, int64_t lda, typename BP::Params bp,
   constexpr int kCopyOps = BM / (8 * NWAVES) + (BP::kDirect ? BN / (8 * NWAVES) : 0);
   auto stage_of = [&](int t) { return lds + (t % NSTAGE) * kStage; };
   auto issue_copies = [&](int t, typename BP::Regs& regs) {
-    async_tile<BM, NWAVES>(A, lda, m0, M, kt_base + t, stage_of(t), wave, lane);
+    async_tile<BP::kRaggedK, BM, NWAVES>(A, lda, m0, M, kt_base + t, stage_of(t), wave, lane);
     if (BP::kDirect) BP::load(bp, n0, kt_base + t, wave, lane, tid, regs, stage_of(t) + kABytes);
   };
 

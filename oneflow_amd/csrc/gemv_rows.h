@@ -10,6 +10,12 @@
 // so bf16 (whose products have to be rounded in fp32 arithmetic: there is no packed bf16 math)
 // and 8-bit codes get the same treatment as the fp16 4-bit case.  Groups may be as short as one
 // lane's 16 bytes of codes (32 4-bit or 16 8-bit elements).
+//
+// K is any multiple of a lane's share of a chunk (LK = 32 4-bit or 16 8-bit elements), so a lane's
+// share lies inside or outside the row as a whole.  In the last chunk of a ragged row (a K shard
+// of 43 groups of 64, say) the lanes beyond K re-read the row's first bytes and meet zeros of x:
+// nothing out of bounds is read and their products add 0.  Before, such rows went to the
+// one-wave-per-row fallback (2 layers of 4352 / 14624 columns, groups of 32, 3 rows of x: 836 us).
 #pragma once
 
 #include "dequant_regs.h"
@@ -68,9 +74,9 @@ gemv_rows_body(int block, const uint16_t* __restrict__ x, const uint8_t* __restr
   constexpr int CK = BITS == 4 ? 128 : 64;  // elements per chunk: 64 bytes of codes per row
   constexpr int LK = CK / 4;                // elements per lane and chunk
   constexpr int XV = LK / 8;                // 16-byte pieces of x per lane and chunk
-  const int nchunks = K / CK;
+  const int nchunks = (K + CK - 1) / CK;
   const int npairs = (nchunks + 1) >> 1;
-  const int row_bytes = nchunks * 64;
+  const int row_bytes = K / LK * 16;
   const int G = K / group_size;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -128,7 +134,7 @@ gemv_rows_body(int block, const uint16_t* __restrict__ x, const uint8_t* __restr
   }
 
   // ---- codes of (tile, pair): one 16-byte load per lane and chunk ------------------------------
-  const uint8_t* wbase = w + (int64_t)row0 * row_bytes + kb * 16;
+  const uint8_t* wbase = w + (int64_t)row0 * row_bytes;
   // Straight-line on purpose: a load under a branch makes the compiler wait for everything in
   // flight at the first LDS fill.  A slot without an item reads one and the same 16 bytes in
   // every lane; lanes past the block's rows re-read its first row (never stored).
@@ -138,8 +144,8 @@ gemv_rows_body(int block, const uint16_t* __restrict__ x, const uint8_t* __restr
     const uint8_t* p = wbase + (int64_t)(ok ? row_l : 0) * row_bytes;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const int c = 2 * pair + u;
-      const uint8_t* q = p + (c < nchunks ? c : 0) * 64;
+      const int off = (2 * pair + u) * 64 + kb * 16;
+      const uint8_t* q = p + (off < row_bytes ? off : 0);
       dst[u] = __builtin_nontemporal_load(
           reinterpret_cast<const u32x4*>(live ? q : w + (int64_t)row0 * row_bytes));
     }
@@ -208,9 +214,21 @@ gemv_rows_body(int block, const uint16_t* __restrict__ x, const uint8_t* __restr
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int c = 2 * pair + u;
-      const u32x4* xp = reinterpret_cast<const u32x4*>(xlane + (size_t)(c < nchunks ? c : 0) * xstride);
+      const bool in_row = c * CK + kb * LK < K;
+      if (STAGED) {
+        const u32x4* xp = reinterpret_cast<const u32x4*>(in_row ? xlane + (size_t)c * xstride : zrec);
 #pragma unroll
-      for (int j = 0; j < XV; ++j) xa[u][j] = xp[j];
+        for (int j = 0; j < XV; ++j) xa[u][j] = xp[j];
+      } else {
+        const u32x4* xp = reinterpret_cast<const u32x4*>(xlane + (size_t)(in_row ? c : 0) * xstride
+                                                         - (in_row ? 0 : kb * LK * 2));
+#pragma unroll
+        for (int j = 0; j < XV; ++j) xa[u][j] = xp[j];
+        if ((c + 1) * CK > K) {  // (the same for every lane: the last chunk of a ragged row)
+#pragma unroll
+          for (int j = 0; j < XV; ++j) xa[u][j] = in_row ? xa[u][j] : u32x4{0u, 0u, 0u, 0u};
+        }
+      }
     }
 #pragma unroll
     for (int t = 0; t < kRowsMaxTiles; ++t) {
@@ -220,7 +238,8 @@ gemv_rows_body(int block, const uint16_t* __restrict__ x, const uint8_t* __restr
         for (int u = 0; u < 2; ++u) {
           const int c = 2 * pair + u;
           if (c < nchunks) {
-            const int k0 = c * CK + kb * LK;
+            int k0 = c * CK + kb * LK;
+            k0 = k0 < K ? k0 : 0;
             const int grp = gs_shift >= 0 ? (k0 >> gs_shift) : (k0 / group_size);
             const float s = TT<T>::load(reinterpret_cast<const S*>(sl) + srow + grp);
             float z = 0.f;
@@ -350,8 +369,8 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
   constexpr int CK = BITS == 4 ? 128 : 64;
   constexpr int LK = CK / 4;
   constexpr int XV = LK / 8;
-  const int nchunks = K / CK;
-  const int row_bytes = nchunks * 64;
+  const int nchunks = (K + CK - 1) / CK;
+  const int row_bytes = K / LK * 16;
   const int G = K / group_size;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -376,11 +395,12 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
   uint16_t* zl = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(sl) + tile_bytes);
   uint8_t* xbuf = smem + (size_t)wave * XB::kWaveBytes;
 
-  const uint8_t* wbase = w + (int64_t)row0 * row_bytes + kb * 16;
+  const uint8_t* wbase = w + (int64_t)row0 * row_bytes;
   auto issue = [&](int tile, int c, bool live) {
     const int row_l = tile * 16 + r;
     const bool ok = row_l < rows_blk;
-    const uint8_t* q = wbase + (int64_t)(ok ? row_l : 0) * row_bytes + (int64_t)c * 64;
+    const int off = c * 64 + kb * 16;  // (past the end of a ragged row: its first bytes again)
+    const uint8_t* q = wbase + (int64_t)(ok ? row_l : 0) * row_bytes + (off < row_bytes ? off : 0);
     return __builtin_nontemporal_load(
         reinterpret_cast<const u32x4*>(live ? q : w + (int64_t)row0 * row_bytes));
   };
@@ -415,11 +435,12 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
                 + (lane % XB::kLanesPerRow) * 16;
     }
   }
+  const int xpiece = (lane % XB::kLanesPerRow) * 16;  // of this lane in a row's chunk
   auto request_x = [&](int chunk) {  // (a chunk past the end re-reads chunk 0)
+    const int off = chunk * XB::kRowBytes;
+    const int at = off + xpiece < K * 2 ? off : -xpiece;  // past a ragged row: its first piece
 #pragma unroll
-    for (int i = 0; i < XB::kReqs; ++i) {
-      xg[i] = *reinterpret_cast<const u32x4*>(xreq[i] + (size_t)chunk * XB::kRowBytes);
-    }
+    for (int i = 0; i < XB::kReqs; ++i) xg[i] = *reinterpret_cast<const u32x4*>(xreq[i] + at);
   };
   if (XLDS) request_x(c < nchunks ? c : 0);
   f32x4 acc[kRowsMaxTiles][MT];
@@ -430,7 +451,17 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
 
   while (c < nchunks) {
     u32x4 xa[MT][XV];
+    int k0 = c * CK + kb * LK;
+    const bool in_row = k0 < K;
+    k0 = in_row ? k0 : 0;
+    const bool ragged = (c + 1) * CK > K;  // (the same for every lane)
     if (XLDS) {
+      if (ragged) {
+#pragma unroll
+        for (int i = 0; i < XB::kReqs; ++i) {
+          xg[i] = c * XB::kRowBytes + xpiece < K * 2 ? xg[i] : u32x4{0u, 0u, 0u, 0u};
+        }
+      }
       // the wave's own buffer: its LDS operations retire in order, so these stores cannot pass
       // the operand reads of the chunk before
 #pragma unroll
@@ -450,12 +481,18 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
     } else {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        const u32x4* xp = reinterpret_cast<const u32x4*>(xrow[mt] + (size_t)c * (CK * 2));
+        const u32x4* xp = reinterpret_cast<const u32x4*>(
+            in_row ? xrow[mt] + (size_t)c * (CK * 2) : xrow[mt] - kb * LK * 2);
 #pragma unroll
         for (int j = 0; j < XV; ++j) xa[mt][j] = xp[j];
       }
+      if (ragged) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int j = 0; j < XV; ++j) xa[mt][j] = in_row ? xa[mt][j] : u32x4{0u, 0u, 0u, 0u};
+      }
     }
-    const int k0 = c * CK + kb * LK;
     const int grp = gs_shift >= 0 ? (k0 >> gs_shift) : (k0 / group_size);
 #pragma unroll
     for (int t = 0; t < kRowsMaxTiles; ++t) {

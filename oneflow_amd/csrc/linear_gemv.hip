@@ -310,9 +310,9 @@ int launch_rows_inst(hipStream_t st, const LinearArgs& a, int grid, int rows_per
 bool rows_supported(const LinearArgs& a) {
   if (a.t_dtype != OFQ_F16 && a.t_dtype != OFQ_BF16) return false;
   if (a.bits != 4 && a.bits != 8) return false;
-  const int ck = a.bits == 4 ? 128 : 64;
-  return a.group_dim == 1 && a.m >= 1 && a.m <= 16 && a.k % ck == 0
-         && a.group_size % (ck / 4) == 0 && a.k <= (1 << 20) && a.n <= 0x7FFFFFFF - 16
+  const int lk = a.bits == 4 ? 32 : 16;  // elements behind a lane's 16 bytes of codes
+  return a.group_dim == 1 && a.m >= 1 && a.m <= 16 && a.k % lk == 0
+         && a.group_size % lk == 0 && a.k <= (1 << 20) && a.n <= 0x7FFFFFFF - 16
          && (a.symmetric || !a.w_signed);
 }
 

@@ -292,29 +292,21 @@ int launch_part(hipStream_t st, const uint8_t* a, const uint8_t* b, const float*
 }  // namespace
 
 bool matmul_quant_rows_supported(int64_t m, int64_t n, int64_t k) {
-  return m >= 1 && n >= 1 && k % 64 == 0 && k <= (1 << 24) && n <= 0x7FFFFFFF - 64;
+  return m >= 1 && m <= 64 && n >= 1 && k % 64 == 0 && k <= (1 << 24) && n <= 0x7FFFFFFF - 64;
 }
 
-// a [m,k], b [n,k] int8; any m, 64 rows of a per pass over b
+// a [m,k], b [n,k] int8, m <= 64
 int launch_matmul_quant_rows(hipStream_t st, const void* a, const void* b, const float* a_scale,
                              const float* b_scale, const void* bias, void* out, int out_dtype,
                              int64_t m, int64_t n, int64_t k) {
-  const size_t esz = out_dtype == OFQ_F32 ? 4 : 2;
-  for (int64_t m0 = 0; m0 < m; m0 += 64) {
-    const int mp = (int)(m - m0 < 64 ? m - m0 : 64);
-    const uint8_t* ap = static_cast<const uint8_t*>(a) + (size_t)m0 * k;
-    void* op = static_cast<char*>(out) + (size_t)m0 * n * esz;
-    const uint8_t* bp = static_cast<const uint8_t*>(b);
-    int rc;
-    switch (out_dtype) {
-      case OFQ_F16: rc = launch_part<f16>(st, ap, bp, a_scale, b_scale, bias, op, mp, n, k); break;
-      case OFQ_BF16: rc = launch_part<bf16>(st, ap, bp, a_scale, b_scale, bias, op, mp, n, k); break;
-      case OFQ_F32: rc = launch_part<float>(st, ap, bp, a_scale, b_scale, bias, op, mp, n, k); break;
-      default: return OFQ_ERR_BAD_DTYPE;
-    }
-    if (rc != OFQ_OK) return rc;
+  const uint8_t* ap = static_cast<const uint8_t*>(a);
+  const uint8_t* bp = static_cast<const uint8_t*>(b);
+  switch (out_dtype) {
+    case OFQ_F16: return launch_part<f16>(st, ap, bp, a_scale, b_scale, bias, out, (int)m, n, k);
+    case OFQ_BF16: return launch_part<bf16>(st, ap, bp, a_scale, b_scale, bias, out, (int)m, n, k);
+    case OFQ_F32: return launch_part<float>(st, ap, bp, a_scale, b_scale, bias, out, (int)m, n, k);
+    default: return OFQ_ERR_BAD_DTYPE;
   }
-  return OFQ_OK;
 }
 
 }  // namespace ofq
