@@ -117,13 +117,14 @@ int ofq_groupwise_dequantize(void* stream, const void* in, const void* scale, co
  *   otherwise) forms w~ with the two roundings of groupwise_dequantize.  The same weights in the two containers can therefore
  *   differ in the last bits of the output.
  * Any m is accepted (the reference kernel has no m limit either, :473,590).
- * workspace: optional.  ofq_fused_linear_gq_workspace_bytes() is non-zero only for large m on the
- *   GEMM path (n*k*sizeof(T)): with it the weight is dequantised once into the workspace and a
- *   copy-fed MFMA GEMM runs on the result (the functor's own m > 8 decomposition); with NULL or
- *   a smaller buffer the weight tiles are dequantised inside the GEMM instead (same results up to
- *   fp32 summation order, slower at large m).  With group_dim 0 it is n*k*sizeof(T) for m > 64
- *   (same decomposition; plus fp32 partial sums of K slices when there are few output tiles);
- *   without it the streaming kernel takes x 64 rows at a time.
+ * workspace: optional.  With a buffer of ofq_fused_linear_gq_workspace_bytes() (0 for m <= 16) the
+ *   problem may be cut along K into blocks that leave fp32 partial sums there (16 < m < 1024), or,
+ *   for m >= 1024 (n*k*sizeof(T)), the weight is dequantised once into it and a copy-fed MFMA GEMM
+ *   runs on the result (the functor's own m > 8 decomposition); with NULL or a smaller buffer the
+ *   weights are expanded inside the GEMM and a block walks all of K (same results up to fp32
+ *   summation order, slower).  With group_dim 0 it is n*k*sizeof(T) for m > 64 (same decomposition;
+ *   plus fp32 partial sums of K slices when there are few output tiles); without it the streaming
+ *   kernel takes x 64 rows at a time.
  */
 size_t ofq_fused_linear_gq_workspace_bytes(int w_dtype, int t_dtype, int num_bits, int symmetric,
                                            int group_dim, int64_t group_size, int64_t m,

@@ -23,21 +23,21 @@ __device__ __forceinline__ uint32_t add_bf16_pair(uint32_t r, float z) {
                    __builtin_bit_cast(float, r & 0xFFFF0000u) + z);
 }
 
-// 16 values of T (two 128-bit pieces) from 16 byte codes.
+// 8 values of T (fp16 or bf16, one 128-bit piece) from 8 byte codes (two words).
 // bf16: v_cvt_f32_ubyteN, v_mul_f32 (v_fma_f32 for a signed container: the codes are read as
 // offset binary and the offset is taken out inside the fused multiply-add, which is exact),
 // v_cvt_pk_bf16_f32, and for a zero term re-widen, v_add_f32, v_cvt_pk_bf16_f32.
 // fp16: the 0x6400 trick with packed fp16 math (2 instructions per element).
 template<typename T, bool SIGNED, int ZMODE>
-__device__ __forceinline__ void dequant16_b8(const u32x4 codes, float s, float z, u32x4& o0,
-                                             u32x4& o1) {
-  uint32_t r[8];
-  if constexpr (TT<T>::dtype == OFQ_BF16) {
-    const float off = SIGNED ? -128.0f * s : 0.f;
+__device__ __forceinline__ u32x4 dequant8_b8(uint32_t word0, uint32_t word1, float s, float z) {
+  static_assert(TT<T>::dtype == OFQ_BF16 || TT<T>::dtype == OFQ_F16, "16-bit T only");
+  u32x4 o;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      uint32_t x = codes[w];
-      if (SIGNED) x ^= 0x80808080u;
+  for (int w = 0; w < 2; ++w) {
+    uint32_t x = w == 0 ? word0 : word1;
+    if (SIGNED) x ^= 0x80808080u;
+    if constexpr (TT<T>::dtype == OFQ_BF16) {
+      const float off = SIGNED ? -128.0f * s : 0.f;
       float p[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -50,44 +50,34 @@ __device__ __forceinline__ void dequant16_b8(const u32x4 codes, float s, float z
         r01 = add_bf16_pair(r01, z);
         r23 = add_bf16_pair(r23, z);
       }
-      r[2 * w] = r01;
-      r[2 * w + 1] = r23;
-    }
-  } else if constexpr (TT<T>::dtype == OFQ_F16) {
-    const f16 sh = (f16)s, zh = (f16)z;  // s and z were widened from fp16: exact
-    const f16x2 s2 = {sh, sh}, z2 = {zh, zh};
-    const f16 off = SIGNED ? (f16)(-1152.0f) : (f16)(-1024.0f);
-    const f16x2 off2 = {off, off};
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      uint32_t word = codes[w];
-      if (SIGNED) word ^= 0x80808080u;
-      f16x2 a = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(word, 0x64646464u, 0x00050004u)) + off2;
-      f16x2 b = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(word, 0x64646464u, 0x00070006u)) + off2;
+      o[2 * w] = r01;
+      o[2 * w + 1] = r23;
+    } else {
+      const f16 sh = (f16)s, zh = (f16)z;  // s and z were widened from fp16: exact
+      const f16x2 s2 = {sh, sh}, z2 = {zh, zh};
+      const f16 off = SIGNED ? (f16)(-1152.0f) : (f16)(-1024.0f);
+      const f16x2 off2 = {off, off};
+      f16x2 a = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(x, 0x64646464u, 0x00050004u)) + off2;
+      f16x2 b = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(x, 0x64646464u, 0x00070006u)) + off2;
       a = a * s2;
       b = b * s2;
       if (ZMODE != 0) {
         a = a + z2;
         b = b + z2;
       }
-      r[2 * w] = __builtin_bit_cast(uint32_t, a);
-      r[2 * w + 1] = __builtin_bit_cast(uint32_t, b);
+      o[2 * w] = __builtin_bit_cast(uint32_t, a);
+      o[2 * w + 1] = __builtin_bit_cast(uint32_t, b);
     }
-  } else {
-    typename TT<T>::storage vals[16];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const uint32_t b = (codes[e >> 2] >> ((e & 3) * 8)) & 0xFFu;
-      const int code = SIGNED ? (int)(int8_t)b : (int)b;
-      float v = TT<T>::round((float)code * s);
-      if (ZMODE != 0) v = v + z;
-      TT<T>::store(&vals[e], v);
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) r[i] = reinterpret_cast<const uint32_t*>(vals)[i];
   }
-  o0 = u32x4{r[0], r[1], r[2], r[3]};
-  o1 = u32x4{r[4], r[5], r[6], r[7]};
+  return o;
+}
+
+// 16 values of T (two 128-bit pieces) from 16 byte codes
+template<typename T, bool SIGNED, int ZMODE>
+__device__ __forceinline__ void dequant16_b8(const u32x4 codes, float s, float z, u32x4& o0,
+                                             u32x4& o1) {
+  o0 = dequant8_b8<T, SIGNED, ZMODE>(codes[0], codes[1], s, z);
+  o1 = dequant8_b8<T, SIGNED, ZMODE>(codes[2], codes[3], s, z);
 }
 
 // 8 values of T (fp16 or bf16, one 128-bit piece) from one word of 4-bit codes.  Element 2b is

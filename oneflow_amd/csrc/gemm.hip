@@ -12,6 +12,8 @@
 // of K (64 fp16/bf16 or 128 int8 elements), a k-step of the 32x32 MFMA consumes 32 of those bytes
 // per row (16 bytes per lane), so the same LDS layout and fragment addressing serve every type.
 // This file only picks tile shapes and fills parameter blocks.
+#include <cmath>
+
 #include "gemm_kernels.h"
 #include "ofq_device.h"
 #include "ofq_internal.h"
@@ -222,6 +224,98 @@ bool gemm_wq_supported(const LinearArgs& a) {
   return true;
 }
 
+namespace {
+
+double slices_us(const LinearArgs& a, int64_t s) {
+  return s > 1 ? 4 + 8e-6 * s * a.m * a.n / 6.5 : 0.0;
+}
+
+// Tile and K slices of gemm_wr for 16 < m < 1024 (fewer rows stream, more are worth a converted copy of
+// the weight), by the time a plan is expected to take in us: 4 to the first step, the steps of a block,
+// and for slices 4 (second launch, end of the first) plus their fp32 sums out and back at 6.5 TB/s.
+// A step was timed per tile on symmetric fp16 4-bit codes (m = 32..384, n = 4096, one slice); what it
+// converts in the shadow of the matrix instructions no longer hides where the type and the zero point
+// make that longer: 1.65 times the step for bf16 with a zero point, 1.3 for fp16, 1.2 for bf16 without.
+double wr_plan_us(const LinearArgs& a, WrPlan* plan) {
+  double best = 1e30;
+  if (a.m <= 16 || a.m >= 1024) return best;
+  if (a.group_size % 32 != 0 || a.k % 32 != 0) return best;
+  // k / group_size as a multiply-high by ceil(2^32 / group_size) is exact up to here
+  if ((a.group_size & (a.group_size - 1)) != 0 && a.k * a.group_size >= ((int64_t)1 << 32)) return best;
+  struct Tile {
+    WrTile tile;
+    int bm, bn, step_k;
+    double step_us;
+    bool any_bits;
+  };
+  static const Tile tiles[] = {{kWr32x128, 32, 128, 128, 0.54, true},
+                               {kWr64x128, 64, 128, 128, 0.68, true},
+                               {kWr96x128, 96, 128, 128, 0.77, false},
+                               {kWr128x256, 128, 256, 64, 0.72, true},
+                               {kWr192x256, 192, 256, 64, 0.88, false}};
+  const bool zero = !a.symmetric || !a.w_signed;
+  const bool bf = a.t_dtype == OFQ_BF16;
+  const double convert = zero ? (bf ? 1.65 : 1.3) : (bf ? 1.2 : 1.0);
+  for (const Tile& t : tiles) {
+    if (!t.any_bits && a.bits != 4) continue;
+    const int blocks = (int)(((a.m + t.bm - 1) / t.bm) * ((a.n + t.bn - 1) / t.bn));
+    const int steps = (int)((a.k + t.step_k - 1) / t.step_k);
+    const double step_us = t.step_us * convert;
+    auto consider = [&](int s) {
+      const int per = (steps + s - 1) / s;
+      s = (steps + per - 1) / per;  // no empty last slice
+      const double us = 4 + (blocks * s + 255) / 256 * per * step_us + slices_us(a, s);
+      if (us < best) {
+        best = us;
+        plan->tile = t.tile;
+        plan->splits = s;
+      }
+    };
+    consider(1);
+    // steps / s falls, the sums grow with s: least where the two are equal, or where the chip is full
+    int most = 256 / blocks < steps / 2 ? 256 / blocks : steps / 2;
+    most = most < 16 ? most : 16;
+    if (most < 2) continue;
+    const int s = (int)std::sqrt(steps * step_us / (8e-6 * a.m * a.n / 6.5));
+    consider(s < 2 ? 2 : (s > most ? most : s));
+    if (s >= 2 && s < most) consider(s + 1);
+  }
+  return best;
+}
+
+// gemm_wr or gemm_core2 on its tile of 256 x 128, whose k-tile of 64 takes about 1.12 us: that one
+// converts a code once per block where gemm_wr does once per wave, so with bf16 zero points and several
+// tiles of rows it keeps up (m = 900, n = k = 4096: 53 us against 58).
+bool wr_plan(const LinearArgs& a, WrPlan* plan) {
+  const double us = wr_plan_us(a, plan);
+  if (us >= 1e30) return false;
+  if (a.m > 128) {
+    const int64_t s = wq_splits(a);
+    const int64_t blocks = ((a.m + 255) / 256) * ((a.n + 127) / 128) * s;
+    const double rounds = (double)((blocks + 255) / 256);
+    if (4 + rounds * ((a.k + 63) / 64 / s) * 1.12 + slices_us(a, s) < us) return false;
+  }
+  return true;
+}
+
+size_t wq_partial_bytes(const LinearArgs& a) {
+  const int splits = wq_splits(a);
+  return splits > 1 ? (size_t)splits * (size_t)a.m * (size_t)a.n * 4 : 0;
+}
+
+// fp32 sums of the slices in whole 32 x 32 tiles, rounded up to whole [m, n] matrices of them; never
+// less than what gemm_core2's slices take, so that a problem that has few tiles has a workspace
+size_t wr_partial_bytes(const LinearArgs& a, const WrPlan& plan) {
+  const size_t mn = (size_t)a.m * (size_t)a.n * 4;
+  const size_t least = a.m > 64 ? wq_partial_bytes(a) : 0;
+  if (plan.splits == 1) return least;
+  const size_t tiles = (size_t)plan.splits * ((a.m + 31) / 32) * ((a.n + 31) / 32) * 4096;
+  const size_t need = (tiles + mn - 1) / mn * mn;
+  return need > least ? need : least;
+}
+
+}  // namespace
+
 // Two passes pay once m is large: the in-tile path converts every weight tile once per 256 rows
 // of x (8 times at m = 2048) and that conversion, not the MFMAs, bounds it; converting the weight
 // once into the workspace and running the copy-fed GEMM on it is what the reference functor does
@@ -229,14 +323,31 @@ bool gemm_wq_supported(const LinearArgs& a) {
 size_t gemm_wq_workspace_bytes(const LinearArgs& a) {
   if (!gemm_wq_supported(a)) return 0;
   if (a.m >= 1024) return (size_t)a.n * (size_t)a.k * 2;
-  const int splits = wq_splits(a);
-  return splits > 1 ? (size_t)splits * (size_t)a.m * (size_t)a.n * 4 : 0;  // fp32 partial sums
+  WrPlan plan;
+  if (wr_plan(a, &plan)) return wr_partial_bytes(a, plan);
+  return wq_partial_bytes(a);
+}
+
+// The streaming kernel's rival for 16 < m <= 64: what gemm_wr is expected to take with a workspace.
+double gemm_wr_us(const LinearArgs& a, bool have_workspace) {
+  WrPlan plan{kWr32x128, 1};
+  const double us = wr_plan_us(a, &plan);
+  return plan.splits > 1 && !have_workspace ? 1e30 : us;
 }
 
 int launch_gemm_wq(hipStream_t st, const LinearArgs& a, void* workspace, size_t workspace_bytes) {
   const size_t need = gemm_wq_workspace_bytes(a);
   const bool have_ws =
       need != 0 && workspace != nullptr && workspace_bytes >= need && ofq_aligned16(workspace);
+  {
+    WrPlan plan;
+    if (wr_plan(a, &plan)) {
+      if (!have_ws) plan.splits = 1;
+      float* partials = static_cast<float*>(workspace);
+      return a.t_dtype == OFQ_F16 ? launch_gemm_wr_f16(st, a, plan, partials)
+                                  : launch_gemm_wr_bf16(st, a, plan, partials);
+    }
+  }
   if (have_ws && a.m < 1024) {
     float* partials = static_cast<float*>(workspace);
     const int splits = wq_splits(a);

@@ -219,6 +219,16 @@ __device__ __forceinline__ void async_copy16_at(const uint8_t* base_uniform, uin
                : "v"(lane_off), "s"(base_uniform), "s"(lds_addr_uniform)
                : "memory", "m0");
 }
+// The same for a caller whose LDS reads around the copy touch other stages: without the memory
+// clobber the compiler may move them across it (the barrier that opens the stage has one).
+__device__ __forceinline__ void async_copy16_unordered(const uint8_t* base_uniform,
+                                                       uint32_t lane_off,
+                                                       uint32_t lds_addr_uniform) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :
+               : "v"(lane_off), "s"(base_uniform), "s"(lds_addr_uniform)
+               : "m0");
+}
 #pragma clang diagnostic pop
 // wait until at most N of this wave's vector-memory operations (incl. global->LDS copies) are
 // still outstanding; they complete in issue order, so this retires everything but the N newest

@@ -21,6 +21,7 @@
 #include "dequant_regs.h"
 #include "gemv_kernels.h"
 #include "ofq_device.h"
+#include "scale_panel.h"
 
 namespace ofq {
 namespace {
@@ -329,22 +330,30 @@ gemv_rows_grouped(GemvGroup g, int M, int K, int group_size, int gs_shift, int r
 }
 
 // ---------------------------------------------------------------------------------------------
-// 16 < m <= 64: the same row split with MT = 2 or 4 sixteen-row tiles of x per MFMA group.  A
+// 16 < m <= 64: the same row split with MT = 2, 3 or 4 sixteen-row tiles of x per MFMA group.  A
 // weight tile is expanded once per chunk and meets all MT tiles of x, which come from L2 chunk
 // by chunk (x is far too large for LDS here: m * k * 2 bytes per block); a wave walks chunks
-// c = wave, wave + NWAVES, ... and, per chunk, every 16-row weight tile of the block, with the
-// codes of the next (tile, chunk) requested before the current ones are used.  Sums stay in
-// registers (kRowsMaxTiles * MT accumulators) and are folded through LDS one weight tile at a
-// time.  No barrier inside the k loop, unlike the tiled GEMM, whose per-k-tile cost does not
-// shrink with m.
+// c = wave, wave + NWAVES, ... and, per chunk, every 16-row weight tile of the block.  Sums stay in
+// registers and are folded through LDS one weight tile at a time.  No barrier inside the k loop.
+//
+// What bounds it: every block reads all of x from L2, 256 * m * k * 2 bytes at about 11 TB/s, so the
+// time follows the chunks per wave (64 x 4096 x 11008 fp16: 27.6 us for 23 MB of weights); the dispatch
+// leaves long rows of weights to gemm_wr for that.  Everything a chunk needs, its MT * 16 rows x 2 CK
+// bytes of x and its NTL weight tiles, is requested while the chunk before is worked on (one weight tile
+// in flight took 20.3 us at 64 x 11008 x 4096 where this takes 19.0, and 26.1 against 21.2 at 48 rows
+// of 8-bit codes).  The requests are unconditional and straight line (a tile past the block's rows
+// re-reads its first row in every lane: one cached line), which keeps the compiler's wait counts exact.
+//
+// x.  A lane's operand of x is 16 bytes out of a 64-byte run of one of 16 rows, so a wave-level
+// request straight from global memory would touch 64 cache lines for 1 KB of data and the vector
+// cache's tag rate would bound the kernel.  A wave requests x with neighbouring lanes on
+// neighbouring bytes (8 cache lines per request), parks the chunk in a buffer of its own in LDS
+// (rows padded by 16 bytes) and reads its operands from there.  The buffers share their memory with
+// the reduction area, which is used only after the k loop.
+//
+// Scales.  The scales (and zeros) of the block's rows are copied to LDS for panel_chunks chunks at a
+// time: all of K unless long rows of short groups leave no room for it.
 // ---------------------------------------------------------------------------------------------
-// XLDS: a lane's operand of x is 16 bytes out of a 64-byte run of one of 16 rows, so a
-// wave-level request straight from global memory touches 64 cache lines for 1 KB of data and the
-// vector cache's tag rate bounds the kernel (4096 x 11008 at 64 rows of x: 6 us per chunk and
-// wave).  With XLDS a wave requests the chunk's MT * 16 rows x 2 CK bytes of x with neighbouring
-// lanes on neighbouring bytes (8 cache lines per request), one chunk ahead, parks them in a
-// buffer of its own in LDS (rows padded by 16 bytes) and reads its operands from there.  The
-// buffers share their memory with the reduction area, which is used only after the k loop.
 template<int BITS, int MT>
 struct RowsMtX {
   static constexpr int CK = BITS == 4 ? 128 : 64;
@@ -356,19 +365,18 @@ struct RowsMtX {
   static constexpr int kWaveBytes = MT * 16 * kPitch;
 };
 
-template<typename T, int BITS, bool SIGNED, int ZMODE, int NWAVES, int MT, bool XLDS = false>
+template<typename T, int BITS, bool SIGNED, int ZMODE, int NWAVES, int MT, int NTL>
 __global__ void __launch_bounds__(NWAVES * 64)
 gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
              const uint16_t* __restrict__ scale, const uint16_t* __restrict__ zero,
              const uint16_t* __restrict__ bias, uint16_t* __restrict__ out, int M, int N, int K,
-             int group_size, int gs_shift, int rows_per_block) {
+             int group_size, int gs_shift, int rows_per_block, int panel_chunks, int panel_groups) {
   typedef typename TT<T>::storage S;
   static_assert(sizeof(S) == 2, "16-bit element types");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   constexpr int NT = NWAVES * 64;
   constexpr int CK = BITS == 4 ? 128 : 64;
   constexpr int LK = CK / 4;
-  constexpr int XV = LK / 8;
   const int nchunks = (K + CK - 1) / CK;
   const int row_bytes = K / LK * 16;
   const int G = K / group_size;
@@ -383,157 +391,159 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
   if (rows_blk <= 0) return;
   const int ntiles = (rows_blk + 15) >> 4;
 
-  // LDS: [red NWAVES*MT*256 f32 | the waves' x buffers (XLDS)][scales rows_per_block*G, padded
+  // LDS: [the waves' x buffers | red NWAVES*MT*256 f32][scales rows_per_block*panel_groups, padded
   //      to 16 B][zeros (asymmetric)]
   typedef RowsMtX<BITS, MT> XB;
   float* red = reinterpret_cast<float*>(smem);
-  const int tile_bytes = (rows_per_block * G * 2 + 15) & ~15;
+  const int panel_bytes = (rows_per_block * panel_groups * 2 + 15) & ~15;
   constexpr size_t kRedBytes = (size_t)NWAVES * MT * 256 * 4;
-  constexpr size_t kFront = XLDS && (size_t)NWAVES * XB::kWaveBytes > kRedBytes
+  constexpr size_t kFront = (size_t)NWAVES * XB::kWaveBytes > kRedBytes
                                 ? (size_t)NWAVES * XB::kWaveBytes : kRedBytes;
   uint16_t* sl = reinterpret_cast<uint16_t*>(smem + kFront);
-  uint16_t* zl = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(sl) + tile_bytes);
+  uint16_t* zl = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(sl) + panel_bytes);
   uint8_t* xbuf = smem + (size_t)wave * XB::kWaveBytes;
 
-  const uint8_t* wbase = w + (int64_t)row0 * row_bytes;
-  auto issue = [&](int tile, int c, bool live) {
-    const int row_l = tile * 16 + r;
-    const bool ok = row_l < rows_blk;
-    const int off = c * 64 + kb * 16;  // (past the end of a ragged row: its first bytes again)
-    const uint8_t* q = wbase + (int64_t)(ok ? row_l : 0) * row_bytes + (off < row_bytes ? off : 0);
-    return __builtin_nontemporal_load(
-        reinterpret_cast<const u32x4*>(live ? q : w + (int64_t)row0 * row_bytes));
-  };
-  int c = wave;
-  u32x4 cur = issue(0, c < nchunks ? c : 0, c < nchunks);
-
-  const int tile_halves = rows_blk * G;
-  const uint16_t* stile = scale + (int64_t)row0 * G;
-  const uint16_t* ztile = ZMODE == kZeroAsym ? zero + (int64_t)row0 * G : stile;
-  for (int e = tid; e < tile_halves; e += NT) {
-    sl[e] = stile[e];
-    if (ZMODE == kZeroAsym) zl[e] = ztile[e];
-  }
-  __syncthreads();
-
-  // this lane's rows of x: row mt*16 + r of every tile (rows >= M feed outputs never stored and
-  // re-read row 0), k-slot kb
-  const uint8_t* xrow[MT];
+  const uint8_t* wblk = w + (int64_t)row0 * row_bytes;
+  uint32_t roff[NTL];  // of this lane's row of every tile
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int row = mt * 16 + r;
-    xrow[mt] = reinterpret_cast<const uint8_t*>(x) + ((size_t)(row < M ? row : 0) * K + kb * LK) * 2;
+  for (int t = 0; t < NTL; ++t) {
+    const int row_l = t * 16 + r;
+    roff[t] = row_l < rows_blk ? (uint32_t)row_l * (uint32_t)row_bytes : 0u;
   }
-  // XLDS: request i of a chunk covers rows kRowsPerReq * i + lane / kLanesPerRow, 16 bytes per lane
-  const uint8_t* xreq[XLDS ? XB::kReqs : 1];
-  u32x4 xg[XLDS ? XB::kReqs : 1];
-  if (XLDS) {
+  auto request_codes = [&](int c, u32x4 (&dst)[NTL]) {  // (a chunk past the end re-reads chunk 0)
+    int off = c * 64 + kb * 16;
+    off = off < row_bytes ? off : 0;
+#pragma unroll
+    for (int t = 0; t < NTL; ++t) {
+      dst[t] = __builtin_nontemporal_load(
+          reinterpret_cast<const u32x4*>(wblk + roff[t] + (uint32_t)off));
+    }
+  };
+  // request i of a chunk covers rows kRowsPerReq * i + lane / kLanesPerRow, 16 bytes per lane; rows
+  // >= M feed outputs never stored and re-read row 0
+  const int xpiece = (lane % XB::kLanesPerRow) * 16;
+  uint32_t xoff[XB::kReqs];
+#pragma unroll
+  for (int i = 0; i < XB::kReqs; ++i) {
+    const int row = i * XB::kRowsPerReq + lane / XB::kLanesPerRow;
+    xoff[i] = (uint32_t)(row < M ? row : 0) * (uint32_t)(K * 2);
+  }
+  u32x4 xg[XB::kReqs];
+  auto request_x = [&](int c) {
+    int off = c * XB::kRowBytes + xpiece;
+    off = off < K * 2 ? off : 0;
 #pragma unroll
     for (int i = 0; i < XB::kReqs; ++i) {
-      const int row = i * XB::kRowsPerReq + lane / XB::kLanesPerRow;
-      xreq[i] = reinterpret_cast<const uint8_t*>(x) + (size_t)(row < M ? row : 0) * K * 2
-                + (lane % XB::kLanesPerRow) * 16;
+      xg[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(x) + xoff[i]
+                                              + (uint32_t)off);
     }
-  }
-  const int xpiece = (lane % XB::kLanesPerRow) * 16;  // of this lane in a row's chunk
-  auto request_x = [&](int chunk) {  // (a chunk past the end re-reads chunk 0)
-    const int off = chunk * XB::kRowBytes;
-    const int at = off + xpiece < K * 2 ? off : -xpiece;  // past a ragged row: its first piece
-#pragma unroll
-    for (int i = 0; i < XB::kReqs; ++i) xg[i] = *reinterpret_cast<const u32x4*>(xreq[i] + at);
   };
-  if (XLDS) request_x(c < nchunks ? c : 0);
-  f32x4 acc[kRowsMaxTiles][MT];
+  f32x4 acc[NTL][MT];
 #pragma unroll
-  for (int t = 0; t < kRowsMaxTiles; ++t)
+  for (int t = 0; t < NTL; ++t)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  while (c < nchunks) {
-    u32x4 xa[MT][XV];
+  int c = wave;
+  u32x4 code_a[NTL], code_b[NTL];
+  request_x(c);
+  request_codes(c, code_a);
+
+  const uint16_t* sblk = scale + (int64_t)row0 * G;
+  const uint16_t* zblk = ZMODE == kZeroAsym ? zero + (int64_t)row0 * G : sblk;
+  int g0 = 0;  // first group of the panel
+  auto fill_panel = [&](int first_chunk) {
+    g0 = gs_shift >= 0 ? (first_chunk * CK) >> gs_shift : (first_chunk * CK) / group_size;
+    const int ng = G - g0 < panel_groups ? G - g0 : panel_groups;
+    copy_scale_panel<NT, ZMODE == kZeroAsym, false>(sblk + g0, zblk + g0, G, rows_blk, rows_blk, ng,
+                                                    panel_groups, sl, zl, tid);
+    __syncthreads();
+  };
+
+  auto work = [&](const u32x4 (&cur)[NTL], u32x4 (&nxt)[NTL]) {
     int k0 = c * CK + kb * LK;
-    const bool in_row = k0 < K;
-    k0 = in_row ? k0 : 0;
-    const bool ragged = (c + 1) * CK > K;  // (the same for every lane)
-    if (XLDS) {
-      if (ragged) {
-#pragma unroll
-        for (int i = 0; i < XB::kReqs; ++i) {
-          xg[i] = c * XB::kRowBytes + xpiece < K * 2 ? xg[i] : u32x4{0u, 0u, 0u, 0u};
-        }
-      }
-      // the wave's own buffer: its LDS operations retire in order, so these stores cannot pass
-      // the operand reads of the chunk before
+    k0 = k0 < K ? k0 : 0;
+    if ((c + 1) * CK > K) {  // (the same for every lane: the last chunk of a ragged row)
 #pragma unroll
       for (int i = 0; i < XB::kReqs; ++i) {
-        const int row = i * XB::kRowsPerReq + lane / XB::kLanesPerRow;
-        *reinterpret_cast<u32x4*>(xbuf + row * XB::kPitch + (lane % XB::kLanesPerRow) * 16) = xg[i];
+        xg[i] = c * XB::kRowBytes + xpiece < K * 2 ? xg[i] : u32x4{0u, 0u, 0u, 0u};
       }
-      request_x(c + NWAVES < nchunks ? c + NWAVES : 0);
+    }
+    // the wave's own buffer: its LDS operations retire in order, so these stores cannot pass the
+    // operand reads of the chunk before
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
+    for (int i = 0; i < XB::kReqs; ++i) {
+      const int row = i * XB::kRowsPerReq + lane / XB::kLanesPerRow;
+      *reinterpret_cast<u32x4*>(xbuf + row * XB::kPitch + xpiece) = xg[i];
+    }
+    request_x(c + NWAVES);
+    request_codes(c + NWAVES, nxt);
+    int grp = (gs_shift >= 0 ? (k0 >> gs_shift) : (k0 / group_size)) - g0;
+    grp = grp < 0 ? 0 : grp;  // (a lane past the end of a row: any scale, its x is zero)
+    float s[NTL], z[NTL];
 #pragma unroll
-        for (int j = 0; j < XV; ++j) {
-          xa[mt][j] = *reinterpret_cast<const u32x4*>(xbuf + (mt * 16 + r) * XB::kPitch
-                                                      + kb * (LK * 2) + j * 16);
+    for (int t = 0; t < NTL; ++t) {
+      const int at = (t * 16 + r) * panel_groups + grp;
+      s[t] = TT<T>::load(reinterpret_cast<const S*>(sl) + at);
+      z[t] = 0.f;
+      if (ZMODE == kZeroAsym) z[t] = TT<T>::load(reinterpret_cast<const S*>(zl) + at);
+      if (ZMODE == kZeroSymU) z[t] = TT<T>::round(-(float)((1 << (BITS - 1)) - 1) * s[t]);
+    }
+    const uint8_t* xl = xbuf + r * XB::kPitch + kb * (LK * 2);
+    if constexpr (BITS == 4) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        u32x4 xa[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          xa[mt] = *reinterpret_cast<const u32x4*>(xl + mt * 16 * XB::kPitch + j * 16);
+        }
+#pragma unroll
+        for (int t = 0; t < NTL; ++t) {
+          if (t < ntiles) {
+            const u32x4 b = dequant8_b4<T, SIGNED, ZMODE>(cur[t][j], s[t], z[t]);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) acc[t][mt] = MfmaK32<T>::mma(xa[mt], b, acc[t][mt]);
+          }
         }
       }
     } else {
+      u32x4 xa[MT][2];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        const u32x4* xp = reinterpret_cast<const u32x4*>(
-            in_row ? xrow[mt] + (size_t)c * (CK * 2) : xrow[mt] - kb * LK * 2);
-#pragma unroll
-        for (int j = 0; j < XV; ++j) xa[mt][j] = xp[j];
+        xa[mt][0] = *reinterpret_cast<const u32x4*>(xl + mt * 16 * XB::kPitch);
+        xa[mt][1] = *reinterpret_cast<const u32x4*>(xl + mt * 16 * XB::kPitch + 16);
       }
-      if (ragged) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-          for (int j = 0; j < XV; ++j) xa[mt][j] = in_row ? xa[mt][j] : u32x4{0u, 0u, 0u, 0u};
-      }
-    }
-    const int grp = gs_shift >= 0 ? (k0 >> gs_shift) : (k0 / group_size);
-#pragma unroll
-    for (int t = 0; t < kRowsMaxTiles; ++t) {
-      if (t < ntiles) {
-        // codes of the next item first: the next tile of this chunk, else tile 0 of the wave's
-        // next chunk
-        const bool last_t = t + 1 >= ntiles;
-        const int nc = last_t ? c + NWAVES : c;
-        const bool live = nc < nchunks;
-        const u32x4 nxt = issue(last_t ? 0 : t + 1, live ? nc : 0, live);
-        const int srow = (t * 16 + r) * G;
-        const float s = TT<T>::load(reinterpret_cast<const S*>(sl) + srow + grp);
-        float z = 0.f;
-        if (ZMODE == kZeroAsym) z = TT<T>::load(reinterpret_cast<const S*>(zl) + srow + grp);
-        if (ZMODE == kZeroSymU) z = TT<T>::round(-(float)((1 << (BITS - 1)) - 1) * s);
-        if constexpr (BITS == 4) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const u32x4 b = dequant8_b4<T, SIGNED, ZMODE>(cur[j], s, z);
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) acc[t][mt] = MfmaK32<T>::mma(xa[mt][j], b, acc[t][mt]);
-          }
-        } else {
+      for (int t = 0; t < NTL; ++t) {
+        if (t < ntiles) {
           u32x4 b0, b1;
-          dequant16_b8<T, SIGNED, ZMODE>(cur, s, z, b0, b1);
+          dequant16_b8<T, SIGNED, ZMODE>(cur[t], s[t], z[t], b0, b1);
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) {
-            acc[t][mt] = MfmaK32<T>::mma(xa[mt][0], b0, acc[t][mt]);
-            acc[t][mt] = MfmaK32<T>::mma(xa[mt][1], b1, acc[t][mt]);
-          }
+          for (int mt = 0; mt < MT; ++mt) acc[t][mt] = MfmaK32<T>::mma(xa[mt][0], b0, acc[t][mt]);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) acc[t][mt] = MfmaK32<T>::mma(xa[mt][1], b1, acc[t][mt]);
         }
-        cur = nxt;
       }
     }
     c += NWAVES;
+  };
+  for (int first = 0; first < nchunks; first += panel_chunks) {
+    if (first > 0) __syncthreads();  // every wave is done with the panel before
+    fill_panel(first);
+    const int last = nchunks - first < panel_chunks ? nchunks : first + panel_chunks;
+    // (panel_chunks is a multiple of 2 * NWAVES: every wave enters a panel with its codes in code_a)
+    while (c < last) {
+      work(code_a, code_b);
+      if (c >= last) break;
+      work(code_b, code_a);
+    }
   }
 
   // fold, one weight tile at a time: red[wave][m (MT*16)][n (16)]
-  if (XLDS) __syncthreads();  // the reduction area overlays the x buffers of other waves
+  __syncthreads();  // the reduction area overlays the x buffers of other waves
 #pragma unroll
-  for (int t = 0; t < kRowsMaxTiles; ++t) {
+  for (int t = 0; t < NTL; ++t) {
     if (t < ntiles) {
       if (t > 0) __syncthreads();  // the previous tile's sums have been read
 #pragma unroll
@@ -564,7 +574,7 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
 // groupwise_quantization_kernels.cu:844-851): the same row split on v_mfma_f32_16x16x4_f32, one
 // fp32 value of x and one of w~ per lane and MFMA.  w~ = (float(q) * s) + z, both operations
 // rounded to fp32 as in the reference; products and sums are fp32 inside the matrix core.
-// x (m <= 16 rows) comes from L2.  Structure of gemv_rows_mt with a single tile of x.
+// x (m <= 16 rows) comes from L2.
 // ---------------------------------------------------------------------------------------------
 template<int BITS, bool SIGNED, int ZMODE, int NWAVES>
 __global__ void __launch_bounds__(NWAVES * 64)
@@ -710,14 +720,12 @@ inline size_t gemv_rows_f32_lds_bytes(int nwaves, int K, int group_size, int row
   return (size_t)nwaves * 256 * 4 + (size_t)(asym ? 2 : 1) * rows_per_block * G * 4;
 }
 
-inline size_t gemv_rows_mt_lds_bytes(int nwaves, int mt, int K, int group_size,
-                                     int rows_per_block, bool asym, int bits = 4,
-                                     bool xlds = false) {
-  const int G = K / group_size;
-  size_t front = (size_t)nwaves * mt * 256 * 4;
+inline size_t gemv_rows_mt_lds_bytes(int nwaves, int mt, int bits, int rows_per_block,
+                                     int panel_groups, bool asym) {
+  const size_t red = (size_t)nwaves * mt * 256 * 4;
   const size_t xb = (size_t)nwaves * mt * 16 * ((bits == 4 ? 256 : 128) + 16);
-  if (xlds && xb > front) front = xb;
-  return front + (size_t)(asym ? 2 : 1) * ((rows_per_block * G * 2 + 15) & ~15);
+  return (xb > red ? xb : red)
+         + (size_t)(asym ? 2 : 1) * ((rows_per_block * panel_groups * 2 + 15) & ~15);
 }
 
 inline size_t gemv_rows_lds_bytes(int nwaves, int M, int K, int group_size, int rows_per_block,

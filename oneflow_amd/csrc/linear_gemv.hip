@@ -439,28 +439,34 @@ int launch_gemv_variant(hipStream_t st, const LinearArgs& a) {
   return ofq_check_launch();
 }
 
-// ---- 16 < m <= 128: several tiles of x per weight tile ----------------------------------------
-template<typename T, int BITS, bool SIGNED, int ZMODE, int NW, int MT, bool XLDS>
-int launch_rows_mt_inst(hipStream_t st, const LinearArgs& a, const void* x, void* out, int m,
-                        int grid, int rows_per_block, size_t lds) {
-  auto kern = gemv_rows_mt<T, BITS, SIGNED, ZMODE, NW, MT, XLDS>;
+// ---- 16 < m <= 64: several tiles of x per weight tile -----------------------------------------
+struct RowsMtPlan {
+  int grid, rows_per_block, panel_chunks, panel_groups;
+  size_t lds;
+};
+
+template<typename T, int BITS, bool SIGNED, int ZMODE, int NW, int MT, int NTL>
+int launch_rows_mt_inst(hipStream_t st, const LinearArgs& a, const RowsMtPlan& p) {
+  auto kern = gemv_rows_mt<T, BITS, SIGNED, ZMODE, NW, MT, NTL>;
   static std::atomic<uint64_t> lds_allowed{0};  // devices on which the kernel's LDS limit is raised
   if (!ofq_allow_dynamic_lds(reinterpret_cast<const void*>(kern), 160 * 1024, lds_allowed)) return OFQ_ERR_LAUNCH;
-  kern<<<grid, NW * 64, lds, st>>>(
-      static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(a.w),
+  kern<<<p.grid, NW * 64, p.lds, st>>>(
+      static_cast<const uint16_t*>(a.x), static_cast<const uint8_t*>(a.w),
       static_cast<const uint16_t*>(a.scale), static_cast<const uint16_t*>(a.zero),
-      static_cast<const uint16_t*>(a.bias), static_cast<uint16_t*>(out), m, (int)a.n, (int)a.k,
-      (int)a.group_size, ilog2_exact(a.group_size), rows_per_block);
+      static_cast<const uint16_t*>(a.bias), static_cast<uint16_t*>(a.out), (int)a.m, (int)a.n,
+      (int)a.k, (int)a.group_size, ilog2_exact(a.group_size), p.rows_per_block, p.panel_chunks,
+      p.panel_groups);
   return ofq_check_launch();
 }
 
-template<typename T, int NW, int MT, bool XLDS>
-int launch_rows_mt_t(hipStream_t st, const LinearArgs& a, const void* x, void* out, int m,
-                     int grid, int rpb, size_t lds) {
+template<typename T, int NW, int MT>
+int launch_rows_mt_t(hipStream_t st, const LinearArgs& a, const RowsMtPlan& p) {
   const int zmode = !a.symmetric ? kZeroAsym : (a.w_signed ? kZeroNone : kZeroSymU);
-#define OFQ_R(B, SG, ZM)                                              \
-  if (a.bits == B && a.w_signed == SG && zmode == ZM)                 \
-    return launch_rows_mt_inst<T, B, SG, ZM, NW, MT, XLDS>(st, a, x, out, m, grid, rpb, lds);
+#define OFQ_R(B, SG, ZM)                                                                     \
+  if (a.bits == B && a.w_signed == SG && zmode == ZM)                                        \
+    return p.rows_per_block <= 16   ? launch_rows_mt_inst<T, B, SG, ZM, NW, MT, 1>(st, a, p) \
+           : p.rows_per_block <= 32 ? launch_rows_mt_inst<T, B, SG, ZM, NW, MT, 2>(st, a, p) \
+                                    : launch_rows_mt_inst<T, B, SG, ZM, NW, MT, 4>(st, a, p);
   OFQ_R(4, true, kZeroNone)
   OFQ_R(4, false, kZeroSymU)
   OFQ_R(4, false, kZeroAsym)
@@ -471,52 +477,38 @@ int launch_rows_mt_t(hipStream_t st, const LinearArgs& a, const void* x, void* o
   return OFQ_ERR_UNSUPPORTED;
 }
 
-// rows [m0, m0 + m) of x, m <= 64
-int launch_rows_mt_part(hipStream_t st, const LinearArgs& a, int64_t m0, int m) {
+template<typename T>
+int launch_rows_mt(hipStream_t st, const LinearArgs& a) {
   constexpr int kCUs = 256;
   const int64_t max_rows = 16 * kRowsMaxTiles;
   int64_t grid = kCUs;
   if ((a.n + grid - 1) / grid > max_rows) grid = (a.n + max_rows - 1) / max_rows;
-  int rpb = (int)((a.n + grid - 1) / grid);
-  if (rpb < 16) rpb = 16;
-  grid = (a.n + rpb - 1) / rpb;
-  const int mt = (m + 15) / 16;  // 2, 3 or 4 tiles of x
-  const size_t esz = 2;
-  const void* x = static_cast<const char*>(a.x) + (size_t)m0 * a.k * esz;
-  void* out = static_cast<char*>(a.out) + (size_t)m0 * a.n * esz;
-  // x through per-wave buffers in LDS (coalesced requests, one chunk ahead): 12 waves for two
-  // tiles of x, 8 for three and four (the buffers and the registers of the chunk in flight)
-  {
-    const int nw = mt == 2 ? 12 : 8;
-    const size_t lds = gemv_rows_mt_lds_bytes(nw, mt, (int)a.k, (int)a.group_size, rpb,
-                                              !a.symmetric, a.bits, true);
-    if (lds <= 160u * 1024u) {
-#define OFQ_MTX(TT_)                                                                            \
-  switch (mt) {                                                                                 \
-    case 2: return launch_rows_mt_t<TT_, 12, 2, true>(st, a, x, out, m, (int)grid, rpb, lds);   \
-    case 3: return launch_rows_mt_t<TT_, 8, 3, true>(st, a, x, out, m, (int)grid, rpb, lds);    \
-    default: return launch_rows_mt_t<TT_, 8, 4, true>(st, a, x, out, m, (int)grid, rpb, lds);   \
+  RowsMtPlan p;
+  p.rows_per_block = (int)((a.n + grid - 1) / grid);
+  if (p.rows_per_block < 16) p.rows_per_block = 16;
+  p.grid = (int)((a.n + p.rows_per_block - 1) / p.rows_per_block);
+  // 12 waves for two tiles of x, 8 for three and four (the x buffers and the registers of the
+  // requests in flight)
+  const int mt = (int)((a.m + 15) / 16);
+  const int nw = mt == 2 ? 12 : 8;
+  // the longest panel of scales that fits beside the x buffers, in whole turns of the waves
+  const int ck = a.bits == 4 ? 128 : 64;
+  const int turn = 2 * nw;
+  int turns = (int)(((a.k + ck - 1) / ck + turn - 1) / turn);
+  for (;; --turns) {
+    if (turns < 1) return OFQ_ERR_UNSUPPORTED;
+    p.panel_chunks = turns * turn;
+    const int64_t groups = ((int64_t)p.panel_chunks * ck) / a.group_size + 2;
+    const int64_t all = a.k / a.group_size;
+    p.panel_groups = (int)(groups < all ? groups : all);
+    p.lds = gemv_rows_mt_lds_bytes(nw, mt, a.bits, p.rows_per_block, p.panel_groups, !a.symmetric);
+    if (p.lds <= 160u * 1024u) break;
   }
-      if (a.t_dtype == OFQ_BF16) { OFQ_MTX(bf16) }
-      OFQ_MTX(f16)
-#undef OFQ_MTX
-    }
+  switch (mt) {
+    case 2: return launch_rows_mt_t<T, 12, 2>(st, a, p);
+    case 3: return launch_rows_mt_t<T, 8, 3>(st, a, p);
+    default: return launch_rows_mt_t<T, 8, 4>(st, a, p);
   }
-  // x straight from L2 (the scales of a long-rowed block leave no room for the buffers):
-  // 16 waves while the registers allow four waves per SIMD, 12 beyond
-  const int nw = mt == 2 ? 16 : 12;
-  const size_t lds =
-      gemv_rows_mt_lds_bytes(nw, mt, (int)a.k, (int)a.group_size, rpb, !a.symmetric);
-  if (lds > 160u * 1024u) return OFQ_ERR_UNSUPPORTED;
-#define OFQ_MT(TT_)                                                                               \
-  switch (mt) {                                                                                   \
-    case 2: return launch_rows_mt_t<TT_, 16, 2, false>(st, a, x, out, m, (int)grid, rpb, lds);    \
-    case 3: return launch_rows_mt_t<TT_, 12, 3, false>(st, a, x, out, m, (int)grid, rpb, lds);    \
-    default: return launch_rows_mt_t<TT_, 12, 4, false>(st, a, x, out, m, (int)grid, rpb, lds);   \
-  }
-  if (a.t_dtype == OFQ_BF16) { OFQ_MT(bf16) }
-  OFQ_MT(f16)
-#undef OFQ_MT
 }
 
 // ---- fp32 activations -------------------------------------------------------------------------
@@ -829,6 +821,8 @@ int launch_gemv_grouped(hipStream_t st, const LinearArgs* pr, int count) {
 #undef OFQ_RG
 }
 
+namespace {
+
 bool gemv_mt_supported(const LinearArgs& a) {
   // beyond 64 rows the weights would be walked twice and the tiled GEMM with K slices is faster
   if (a.m <= 16 || a.m > 64) return false;
@@ -837,13 +831,30 @@ bool gemv_mt_supported(const LinearArgs& a) {
   return rows_supported(b) && a.n * a.k <= 0x7FFFFFFFLL * 8;
 }
 
+}  // namespace
+
+// Every block of gemv_rows_mt reads all of x, from L2: that, with a part per weight tile, is the time
+// of a turn of its waves over their chunks (us, measured for n = 4096, 11008 and 32000 at m = 32 and
+// 64, within 15 %).  gemm_wr reads x once per 128 rows of weights but starts a second kernel where
+// it slices K; it has to win by 2.5 us, what its second launch costs the host and cold weights its
+// slices.  So long rows of weights leave the streaming kernel (64 x 4096 x 11008: 27.6 us here, 18 there) and
+// n = 11008 of k = 4096 stays (19.0 us here, 19.4 there).
+bool gemv_mt_preferred(const LinearArgs& a, bool have_workspace) {
+  if (!gemv_mt_supported(a)) return false;
+  const int nw = a.m <= 32 ? 12 : 8;
+  const int ck = a.bits == 4 ? 128 : 64;
+  int64_t rows = (a.n + 255) / 256;
+  rows = rows < 16 ? 16 : (rows > 16 * kRowsMaxTiles ? 16 * kRowsMaxTiles : rows);
+  const int64_t grid = (a.n + rows - 1) / rows, tiles = (rows + 15) / 16;
+  const int64_t rounds = (grid + 255) / 256;
+  const int64_t turns = ((a.k + ck - 1) / ck + nw - 1) / nw;
+  double turn_us = a.bits == 4 ? 1.2 + 0.95 * tiles : 0.6 + 0.75 * tiles;
+  if (a.bits == 4 && a.t_dtype == OFQ_BF16 && !a.symmetric) turn_us *= 1.15;  // the longest conversion
+  return 2 + rounds * turns * turn_us < gemm_wr_us(a, have_workspace) + 2.5;
+}
+
 int launch_gemv_mt(hipStream_t st, const LinearArgs& a) {
-  for (int64_t m0 = 0; m0 < a.m; m0 += 64) {
-    const int m = (int)(a.m - m0 < 64 ? a.m - m0 : 64);
-    const int rc = launch_rows_mt_part(st, a, m0, m);
-    if (rc != OFQ_OK) return rc;  // OFQ_ERR_UNSUPPORTED can only come from the first part
-  }
-  return OFQ_OK;
+  return a.t_dtype == OFQ_BF16 ? launch_rows_mt<bf16>(st, a) : launch_rows_mt<f16>(st, a);
 }
 
 bool gemv_wq_supported(const LinearArgs& a) {
@@ -928,7 +939,7 @@ extern "C" size_t ofq_fused_linear_gq_workspace_bytes(int w_dtype, int t_dtype, 
   a.m = m;
   a.n = n;
   a.k = k;
-  if (gemv_wq_supported(a) || gemv_m1_any_supported(a) || gemv_mt_supported(a)) return 0;
+  if (gemv_wq_supported(a) || gemv_m1_any_supported(a) || gemv_mt_preferred(a, true)) return 0;
   if (group_dim == 0) return gemm_gn_workspace_bytes(a);
   return gemm_wq_workspace_bytes(a);  // 0 for every path but the two-pass GEMM at large m
 }
@@ -985,7 +996,7 @@ extern "C" int ofq_fused_linear_gq(void* stream, const void* x, const void* w,
     const int rc = launch_gemv_wq(st, a);
     if (rc != OFQ_ERR_UNSUPPORTED) return rc;  // e.g. bf16 with an x too large to stage
   }
-  if (gemv_mt_supported(a)) {
+  if (a.m > 16 && gemv_mt_preferred(a, workspace != nullptr && workspace_bytes >= gemm_wq_workspace_bytes(a))) {
     const int rc = launch_gemv_mt(st, a);
     if (rc != OFQ_ERR_UNSUPPORTED) return rc;
   }

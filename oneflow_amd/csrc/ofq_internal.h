@@ -31,6 +31,18 @@ bool gemm_wq_supported(const LinearArgs& a);
 size_t gemm_wq_workspace_bytes(const LinearArgs& a);
 int launch_gemm_wq(hipStream_t st, const LinearArgs& a, void* workspace, size_t workspace_bytes);
 
+// The GEMM whose weights stay packed until they are in registers (gemm_wr.h): a tile of rows of x by
+// columns of the output and a number of K slices.
+enum WrTile { kWr32x128, kWr64x128, kWr96x128, kWr128x256, kWr192x256 };
+struct WrPlan {
+  WrTile tile;
+  int splits;
+};
+// expected time (us; 1e30: not this kernel's problem) of a problem of 16 < m <= 64 on it
+double gemm_wr_us(const LinearArgs& a, bool have_workspace);
+int launch_gemm_wr_f16(hipStream_t st, const LinearArgs& a, const WrPlan& plan, float* partials);
+int launch_gemm_wr_bf16(hipStream_t st, const LinearArgs& a, const WrPlan& plan, float* partials);
+
 // m = 1, fp16, 4-bit symmetric codes in an int8 container, groups along K: a wave owns whole
 // weight rows (contiguous requests, packed dot products, no cross-wave fold).
 bool gemv_m1_supported(const LinearArgs& a);
@@ -52,8 +64,8 @@ bool gemv_wq_supported(const LinearArgs& a);
 int launch_gemv_wq(hipStream_t st, const LinearArgs& a);
 
 // 16 < m <= 64 without a workspace: the decode kernel's row split with several 16-row tiles of x
-// per weight tile.
-bool gemv_mt_supported(const LinearArgs& a);
+// per weight tile.  Not where gemm_wr is expected to take clearly less.
+bool gemv_mt_preferred(const LinearArgs& a, bool have_workspace);
 int launch_gemv_mt(hipStream_t st, const LinearArgs& a);
 
 // Groups along N (group_dim = 0), fp16 / bf16: the streaming kernel with one scale per k (any m,
