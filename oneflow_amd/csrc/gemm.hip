@@ -64,20 +64,10 @@ int launch_plain(hipStream_t st, const LinearArgs& a, const void* wt) {
     return launch_core2<MF, B2Copy<RG, 128, 512>, EP, 128, 128, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
                                                                   a.n, (a.k + 63) / 64);
   }
-  switch (pick_tile_width(a.m, a.n, true)) {
-    case 384:
-      return launch_core2<MF, B2Copy<RG, 384, 512>, EP, 256, 384, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                    a.n, (a.k + 63) / 64);
-    case 256:
-      return launch_core2<MF, B2Copy<RG, 256, 512>, EP, 256, 256, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                    a.n, (a.k + 63) / 64);
-    case 192:
-      return launch_core2<MF, B2Copy<RG, 192, 512>, EP, 256, 192, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                    a.n, (a.k + 63) / 64);
-    default:
-      return launch_core2<MF, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                    a.n, (a.k + 63) / 64);
-  }
+  const int width = pick_tile_width(a.m, a.n, true);
+  return std::is_same<T, f16>::value
+             ? launch_gemm_pp_f16(st, a.x, wt, a.bias, a.out, a.m, a.n, a.k, width)
+             : launch_gemm_pp_bf16(st, a.x, wt, a.bias, a.out, a.m, a.n, a.k, width);
 }
 
 // Few blocks (m small against the tile height, or few weight tiles): K is cut into `splits`
@@ -591,16 +581,9 @@ int launch_mq(hipStream_t st, const void* a, const BCopyParams& bp, const float*
   if (m <= 128) {
     return launch_core2<MfmaI8, B2Copy<RG, 128, 256>, EP, 128, 128, 2, 2>(st, a, k, bp, ep, m, n, kt);
   }
-  switch (pick_tile_width(m, n, true)) {
-    case 384:
-      return launch_core2<MfmaI8, B2Copy<RG, 384, 512>, EP, 256, 384, 4, 2>(st, a, k, bp, ep, m, n, kt);
-    case 256:
-      return launch_core2<MfmaI8, B2Copy<RG, 256, 512>, EP, 256, 256, 4, 2>(st, a, k, bp, ep, m, n, kt);
-    case 192:
-      return launch_core2<MfmaI8, B2Copy<RG, 192, 512>, EP, 256, 192, 4, 2>(st, a, k, bp, ep, m, n, kt);
-    default:
-      return launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a, k, bp, ep, m, n, kt);
-  }
+  const int out_dtype = TT<T>::dtype;
+  return launch_gemm_pp_i8(st, a, bp.b, a_scale, b_scale, bias, out, out_dtype, m, n, k,
+                           pick_tile_width(m, n, true));
 }
 
 }  // namespace

@@ -359,6 +359,92 @@ struct B2Dequant {
   }
 };
 
+// ---- epilogue: registers -> (wave-private, padded) LDS tile -> 128-bit row-contiguous stores --
+// Each lane holds, per 32x32 tile and register quad g, the 4 consecutive outputs
+// out[m = .. + lane%32][n = .. + 8g + 4*(lane/32) + 0..3]; they are converted (bias / scales,
+// one rounding to T), packed to 8 bytes and written to LDS; rows are then read back 16 bytes
+// per lane so that every global store instruction writes whole row segments.
+// (n0w, m0w): the wave's first column and row of the output; lds: LDS_BYTES that nobody reads any more.
+template<class MF, class EP, int TM, int TN, int NWAVES, int LDS_BYTES>
+__device__ __forceinline__ void store_wave_tile(const typename EP::Params& ep,
+                                                typename MF::Acc (&acc)[TM][TN], uint8_t* lds,
+                                                int m0w, int n0w, int M, int N, int wave, int lane) {
+  typedef typename EP::elem_t OT;
+  typedef typename TT<OT>::storage OS;
+  static_assert(sizeof(OS) == 2 || sizeof(OS) == 4, "output element size");
+  // The wave tile is written in panels of JP 32-column MFMA tiles so that the staging area of all
+  // waves fits in the stage memory.
+  constexpr int WTM = TM * 32;
+  constexpr int JP0 = (LDS_BYTES / (NWAVES * WTM) - 8) / (32 * (int)sizeof(OS));
+  constexpr int JP = JP0 >= TN ? TN : (JP0 >= 4 ? (JP0 / 2) * 2 : JP0);  // whole 128-byte pieces
+  static_assert(JP >= 1, "no room for the epilogue staging area");
+  constexpr int kRowBytesOut = JP * 32 * (int)sizeof(OS) + 8;  // +8: conflict-free 8-byte writes
+  uint8_t* ep_tile = lds + wave * (WTM * kRowBytesOut);  // all waves passed the last barrier
+#pragma unroll
+  for (int jp = 0; jp < TN; jp += JP) {
+    const int panel_cols = (TN - jp < JP ? TN - jp : JP) * 32;
+    const int ncol0 = n0w + jp * 32;  // first column of the panel
+    const bool vec_ok = (N % 8 == 0) && (ncol0 + panel_cols <= N);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int jj = 0; jj < JP; ++jj) {
+        const int j = jp + jj;
+        if (j >= TN) break;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int nl = jj * 32 + 8 * g + 4 * (lane >> 5);  // column of the quad in the panel
+          const int n = ncol0 + nl;
+          OS q[4];
+          typename MF::Acc& a = acc[i][j];
+          if (n + 3 < N) {
+            const typename MF::Scalar quad[4] = {a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+            EP::convert4(ep, quad, n, q);
+          } else {
+            // quad straddles or lies beyond N: element-wise, out-of-range slots are never stored
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              q[e] = OS();
+              if (n + e < N) q[e] = EP::convert1(ep, a[4 * g + e], n + e);
+            }
+          }
+          uint8_t* dst = ep_tile + (i * 32 + (lane & 31)) * kRowBytesOut + nl * (int)sizeof(OS);
+          if (sizeof(OS) == 2) {
+            *reinterpret_cast<u32x2*>(dst) = *reinterpret_cast<const u32x2*>(q);
+          } else {
+            *reinterpret_cast<u32x2*>(dst) = reinterpret_cast<const u32x2*>(q)[0];
+            *reinterpret_cast<u32x2*>(dst + 8) = reinterpret_cast<const u32x2*>(q)[1];
+          }
+        }
+      }
+    }
+    // a wave only reads what it wrote itself; LDS operations of one wave complete in order.
+    // 16 bytes per lane: piece p of row r, pieces_per_row = panel bytes / 16.
+    const int pieces_per_row = panel_cols * (int)sizeof(OS) / 16;
+    const int total_pieces = WTM * pieces_per_row;
+    for (int t = lane; t < total_pieces; t += 64) {
+      const int ml = t / pieces_per_row;
+      const int cpiece = t - ml * pieces_per_row;
+      const int m = m0w + ml;
+      if (m >= M) continue;
+      const uint8_t* src = ep_tile + ml * kRowBytesOut + cpiece * 16;
+      const u32x2 lo = *reinterpret_cast<const u32x2*>(src);
+      const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8);
+      const int ncol = ncol0 + cpiece * (16 / (int)sizeof(OS));
+      OS* gdst = ep.out + (int64_t)m * N + ncol;
+      const u32x4 v = {lo[0], lo[1], hi[0], hi[1]};
+      if (vec_ok) {
+        *reinterpret_cast<u32x4*>(gdst) = v;
+      } else {
+        const OS* e = reinterpret_cast<const OS*>(&v);
+#pragma unroll
+        for (int t2 = 0; t2 < 16 / (int)sizeof(OS); ++t2)
+          if (ncol + t2 < N) gdst[t2] = e[t2];
+      }
+    }
+  }
+}
+
 // NSTAGE LDS stages; the copies of tile t are issued at the top of iteration t-(NSTAGE-1).
 template<class MF, class BP, class EP, int BM, int BN, int WM, int WN, int NSTAGE = 2>
 __global__ void __launch_bounds__(WM * WN * 64)
@@ -502,85 +588,9 @@ gemm_core2(const uint8_t* __restrict__ A, int64_t lda, typename BP::Params bp,
     if (kt + 1 < KT) iteration(kt + 1, breg0, breg1);
   }
 
-  // ---- epilogue: registers -> (wave-private, padded) LDS tile -> 128-bit row-contiguous stores --
-  // Each lane holds, per 32x32 tile and register quad g, the 4 consecutive outputs
-  // out[m = .. + lane%32][n = .. + 8g + 4*(lane/32) + 0..3]; they are converted (bias / scales,
-  // one rounding to T), packed to 8 bytes and written to LDS; rows are then read back 16 bytes
-  // per lane so that every global store instruction writes whole row segments.
-  typedef typename EP::elem_t OT;
-  typedef typename TT<OT>::storage OS;
-  static_assert(sizeof(OS) == 2 || sizeof(OS) == 4, "output element size");
-  // The wave tile is written in panels of JP 32-column MFMA tiles so that the staging area of all
-  // waves fits in the stage memory.
-  constexpr int kLdsBudget = NSTAGE * kStage;
-  constexpr int JP0 = (kLdsBudget / (NWAVES * WTM) - 8) / (32 * (int)sizeof(OS));
-  constexpr int JP = JP0 >= TN ? TN : (JP0 >= 4 ? (JP0 / 2) * 2 : JP0);  // whole 128-byte pieces
-  static_assert(JP >= 1, "no room for the epilogue staging area");
-  constexpr int kRowBytesOut = JP * 32 * (int)sizeof(OS) + 8;  // +8: conflict-free 8-byte writes
-  uint8_t* ep_tile = lds + wave * (WTM * kRowBytesOut);  // all waves passed the last barrier
-#pragma unroll
-  for (int jp = 0; jp < TN; jp += JP) {
-    const int panel_cols = (TN - jp < JP ? TN - jp : JP) * 32;
-    const int ncol0 = n0 + wn0 + jp * 32;  // first column of the panel
-    const bool vec_ok = (N % 8 == 0) && (ncol0 + panel_cols <= N);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-      for (int jj = 0; jj < JP; ++jj) {
-        const int j = jp + jj;
-        if (j >= TN) break;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int nl = jj * 32 + 8 * g + 4 * (lane >> 5);  // column of the quad in the panel
-          const int n = ncol0 + nl;
-          OS q[4];
-          typename MF::Acc& a = acc[i][j];
-          if (n + 3 < N) {
-            const typename MF::Scalar quad[4] = {a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
-            EP::convert4(ep, quad, n, q);
-          } else {
-            // quad straddles or lies beyond N: element-wise, out-of-range slots are never stored
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              q[e] = OS();
-              if (n + e < N) q[e] = EP::convert1(ep, a[4 * g + e], n + e);
-            }
-          }
-          uint8_t* dst = ep_tile + (i * 32 + (lane & 31)) * kRowBytesOut + nl * (int)sizeof(OS);
-          if (sizeof(OS) == 2) {
-            *reinterpret_cast<u32x2*>(dst) = *reinterpret_cast<const u32x2*>(q);
-          } else {
-            *reinterpret_cast<u32x2*>(dst) = reinterpret_cast<const u32x2*>(q)[0];
-            *reinterpret_cast<u32x2*>(dst + 8) = reinterpret_cast<const u32x2*>(q)[1];
-          }
-        }
-      }
-    }
-    // a wave only reads what it wrote itself; LDS operations of one wave complete in order.
-    // 16 bytes per lane: piece p of row r, pieces_per_row = panel bytes / 16.
-    const int pieces_per_row = panel_cols * (int)sizeof(OS) / 16;
-    const int total_pieces = WTM * pieces_per_row;
-    for (int t = lane; t < total_pieces; t += 64) {
-      const int ml = t / pieces_per_row;
-      const int cpiece = t - ml * pieces_per_row;
-      const int m = m0 + wm0 + ml;
-      if (m >= M) continue;
-      const uint8_t* src = ep_tile + ml * kRowBytesOut + cpiece * 16;
-      const u32x2 lo = *reinterpret_cast<const u32x2*>(src);
-      const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8);
-      const int ncol = ncol0 + cpiece * (16 / (int)sizeof(OS));
-      OS* gdst = ep.out + (int64_t)m * N + ncol;
-      const u32x4 v = {lo[0], lo[1], hi[0], hi[1]};
-      if (vec_ok) {
-        *reinterpret_cast<u32x4*>(gdst) = v;
-      } else {
-        const OS* e = reinterpret_cast<const OS*>(&v);
-#pragma unroll
-        for (int t2 = 0; t2 < 16 / (int)sizeof(OS); ++t2)
-          if (ncol + t2 < N) gdst[t2] = e[t2];
-      }
-    }
-  }
+  // all waves passed the last barrier
+  store_wave_tile<MF, EP, TM, TN, NWAVES, NSTAGE * kStage>(ep, acc, lds, m0 + wm0, n0 + wn0, M, N,
+                                                           wave, lane);
 }
 
 template<class MF, class BP, class EP, int BM, int BN, int WM, int WN, int NSTAGE = 2>

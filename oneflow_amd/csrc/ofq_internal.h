@@ -43,6 +43,16 @@ double gemm_wr_us(const LinearArgs& a, bool have_workspace);
 int launch_gemm_wr_f16(hipStream_t st, const LinearArgs& a, const WrPlan& plan, float* partials);
 int launch_gemm_wr_bf16(hipStream_t st, const LinearArgs& a, const WrPlan& plan, float* partials);
 
+// Copy-fed GEMMs for more than 128 rows (gemm_pp.h) on tiles of 256 x width; the linear's with the
+// weight already in the dtype of x.
+int launch_gemm_pp_f16(hipStream_t st, const void* x, const void* w, const void* bias, void* out,
+                       int64_t m, int64_t n, int64_t k, int width);
+int launch_gemm_pp_bf16(hipStream_t st, const void* x, const void* w, const void* bias, void* out,
+                        int64_t m, int64_t n, int64_t k, int width);
+int launch_gemm_pp_i8(hipStream_t st, const void* a, const void* b, const float* a_scale,
+                      const float* b_scale, const void* bias, void* out, int out_dtype, int64_t m,
+                      int64_t n, int64_t k, int width);
+
 // m = 1, fp16, 4-bit symmetric codes in an int8 container, groups along K: a wave owns whole
 // weight rows (contiguous requests, packed dot products, no cross-wave fold).
 bool gemv_m1_supported(const LinearArgs& a);
