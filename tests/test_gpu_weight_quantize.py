@@ -154,3 +154,24 @@ def test_quantized_linear_module(num_bits, symmetric, dtype_name):
     clone.load_state_dict(ql.state_dict())
     x = torch.randn((4, 1024), device="cuda", dtype=dtype)
     assert torch.equal(clone(x), ql(x))
+
+
+@pytest.mark.parametrize("group", [8, 16, 32, 64, 128, 256, 512])
+@pytest.mark.parametrize("bits,signed", [(4, True), (4, False), (8, True), (8, False)])
+def test_symmetric_bf16_groups_of_arbitrary_bit_patterns(bits, signed, group):
+    """bf16 groups of every exponent: largest magnitudes inside [2^-50, 2^60], where the division is a
+    corrected product, at its edges and beyond, with elements of any smaller exponent, and an all-zero
+    group; every number of lanes that share a group."""
+    rng = np.random.default_rng(bits * 2 + signed + group)
+    x = rng.integers(0, 65536, size=(1200, group)).astype(np.uint16)
+    top = rng.integers(20, 250, size=(1200, 1)).astype(np.int64)
+    top[:300, 0] = rng.integers(75, 80, 300)    # 2^-52 .. 2^-47
+    top[300:600, 0] = rng.integers(184, 190, 300)  # 2^57 .. 2^62
+    spread = np.where(rng.random((1200, 1)) < 0.8, 6, 120)
+    exponent = np.maximum(top - rng.integers(0, 1 << 20, size=x.shape) % spread, 0)
+    x = (x & np.uint16(0x807F)) | (exponent.astype(np.uint16) << np.uint16(7))
+    x[7] = 0
+    qr, sr, _ = O.groupwise_quantize(x, bits, True, 1, group, signed)
+    q, s, _ = _run(x, bits, True, 1, group, signed)
+    assert np.array_equal(q.view(np.uint8), qr.view(np.uint8))
+    assert np.array_equal(s.view(np.uint16), sr.view(np.uint16))
