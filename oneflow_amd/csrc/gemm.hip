@@ -65,6 +65,10 @@ int launch_plain(hipStream_t st, const LinearArgs& a, const void* wt) {
                                                                   a.n, (a.k + 63) / 64);
   }
   const int width = pick_tile_width(a.m, a.n, true);
+  if (width == 128) {
+    return launch_core2<MF, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
+                                                                  a.n, (a.k + 63) / 64);
+  }
   return std::is_same<T, f16>::value
              ? launch_gemm_pp_f16(st, a.x, wt, a.bias, a.out, a.m, a.n, a.k, width)
              : launch_gemm_pp_bf16(st, a.x, wt, a.bias, a.out, a.m, a.n, a.k, width);
@@ -581,9 +585,11 @@ int launch_mq(hipStream_t st, const void* a, const BCopyParams& bp, const float*
   if (m <= 128) {
     return launch_core2<MfmaI8, B2Copy<RG, 128, 256>, EP, 128, 128, 2, 2>(st, a, k, bp, ep, m, n, kt);
   }
-  const int out_dtype = TT<T>::dtype;
-  return launch_gemm_pp_i8(st, a, bp.b, a_scale, b_scale, bias, out, out_dtype, m, n, k,
-                           pick_tile_width(m, n, true));
+  const int width = pick_tile_width(m, n, true);
+  if (width == 128) {
+    return launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a, k, bp, ep, m, n, kt);
+  }
+  return launch_gemm_pp_i8(st, a, bp.b, a_scale, b_scale, bias, out, TT<T>::dtype, m, n, k, width);
 }
 
 }  // namespace

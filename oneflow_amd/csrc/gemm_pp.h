@@ -36,11 +36,11 @@ __device__ __forceinline__ void copy_pieces(const uint8_t* __restrict__ a_kt,
 
 // gemm_core2 keeps its eight waves in step: after the barrier of a k-tile both waves of a SIMD fetch
 // fragments while the matrix cores idle.  Here waves 0-3 and 4-7 (one of each on every SIMD) are one
-// slot apart: in a slot one group fetches the fragments of KS k-steps and requests copies while the
+// slot apart: in a slot one group fetches the fragments of a k-step and requests copies while the
 // other multiplies, and a barrier swaps the roles.
 //
-// Slots of group 0 in a k-tile: fetch 0, multiply 0, fetch 1, ... (2P of them, P = 4 / KS); group 1
-// does the same one slot later.  The other stage is free once group 1 has fetched the last k-steps of
+// Slots of group 0 in a k-tile: fetch 0, multiply 0, fetch 1, ... multiply 3; group 1 does the same one
+// slot later.  The other stage is free once group 1 has fetched the last k-steps of
 // the tile before, i.e. in the slot in which group 0 fetches first; copies are requested in the fetch
 // slots from there on, and each wave waits for its own before the barrier that opens the next tile
 // (group 0 in its last multiplying slot, group 1 in its last fetching one).
@@ -52,7 +52,7 @@ __device__ __forceinline__ void copy_pieces(const uint8_t* __restrict__ a_kt,
 // taken: waves of 128 x 96 (fewer LDS reads: 314 / 563 us), copies spread over more slots (312 / 558) or
 // requested before the fetches (320 / 564), rows of 64 bytes in a ring of four stages (three in flight:
 // 355 / 621, half lines cost more than the distance gives), non-temporal stores (within 1.5 %).
-template<class MF, bool RAGGED, class EP, int BN, int KS>
+template<class MF, bool RAGGED, class EP, int BN>
 __global__ void __launch_bounds__(512)
 gemm_pp(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int64_t ld,
         typename EP::Params ep, int M, int N, int KT, int m_tiles, int n_tiles) {
@@ -61,7 +61,6 @@ gemm_pp(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int64_t ld
   constexpr int kABytes = BM * kStageRow;
   constexpr int kStage = (BM + BN) * kStageRow;
   constexpr int kPieces = (BM + BN) / 64;
-  constexpr int P = 4 / KS;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
   // an XCD takes consecutive tiles; within them 8 row tiles share a column of b, so that the 32
@@ -124,28 +123,21 @@ gemm_pp(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int64_t ld
     const uint8_t* cur = lds + (kt & 1) * kStage;
     const bool more = kt + 1 < KT;
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
+    for (int p = 0; p < 4; ++p) {
       // ---- fetch --------------------------------------------------------------------------------
-      u32x4 af[KS][TM], bf[KS][TN];
+      u32x4 af[TM], bf[TN];
+      const int off = ((2 * p + half) ^ key) << 4;
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const int off = ((2 * (p * KS + s) + half) ^ key) << 4;
+      for (int i = 0; i < TM; ++i)
+        af[i] = *reinterpret_cast<const u32x4*>(cur + a_base + i * 32 * kStageRow + off);
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-          af[s][i] = *reinterpret_cast<const u32x4*>(cur + a_base + i * 32 * kStageRow + off);
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          bf[s][j] = *reinterpret_cast<const u32x4*>(cur + b_base + j * 32 * kStageRow + off);
-      }
+      for (int j = 0; j < TN; ++j)
+        bf[j] = *reinterpret_cast<const u32x4*>(cur + b_base + j * 32 * kStageRow + off);
       if (more) {
-        if constexpr (P == 4) {
-          if (p == 0) OFQ_PP_COPY(0, kPieces / 2, kt + 1);
-          if (p == 1) OFQ_PP_COPY(kPieces / 2, kPieces, kt + 1);
-        } else {
-          if (p == 0) OFQ_PP_COPY(0, kPieces, kt + 1);
-        }
+        if (p == 0) OFQ_PP_COPY(0, kPieces / 2, kt + 1);
+        if (p == 1) OFQ_PP_COPY(kPieces / 2, kPieces, kt + 1);
       }
-      if (p == P - 1 && late) wait_vmem_all();
+      if (p == 3 && late) wait_vmem_all();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_barrier();
@@ -153,17 +145,15 @@ gemm_pp(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int64_t ld
       // ---- multiply -----------------------------------------------------------------------------
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int s = 0; s < KS; ++s)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = MF::mma(bf[s][j], af[s][i], acc[i][j]);
+        for (int j = 0; j < TN; ++j) acc[i][j] = MF::mma(bf[j], af[i], acc[i][j]);
       __builtin_amdgcn_s_setprio(0);
-      if (p == P - 1 && !late) wait_vmem_all();
+      if (p == 3 && !late) wait_vmem_all();
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
       // (the last barrier of the late group would have no partner: both groups pass as many)
-      if (p < P - 1 || more || !late) __builtin_amdgcn_s_barrier();
+      if (p < 3 || more || !late) __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -173,17 +163,17 @@ gemm_pp(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int64_t ld
   store_wave_tile<MF, EP, TM, TN, 8, 2 * kStage>(ep, acc, lds, m0 + wm0, n0 + wn0, M, N, wave, lane);
 }
 
-template<class MF, bool RAGGED, class EP, int BN, int KS>
+template<class MF, bool RAGGED, class EP, int BN>
 int launch_pp_tile(hipStream_t st, const void* a, const void* b, int64_t row_bytes,
                    const typename EP::Params& ep, int64_t M, int64_t N) {
   const int m_tiles = (int)((M + 255) / 256);
   const int n_tiles = (int)((N + BN - 1) / BN);
   constexpr int kLds = 2 * (256 + BN) * kStageRow;
-  auto kern = gemm_pp<MF, RAGGED, EP, BN, KS>;
+  auto kern = gemm_pp<MF, RAGGED, EP, BN>;
   static std::atomic<uint64_t> lds_allowed{0};  // devices on which the kernel's LDS limit is raised
   if (!ofq_allow_dynamic_lds(reinterpret_cast<const void*>(kern), kLds, lds_allowed)) return OFQ_ERR_LAUNCH;
-  // the copies address a tile's rows with 32-bit offsets from its first row, one step of 64 rows past it
-  if (row_bytes * (int64_t)(BN > 256 ? BN + 64 : 320) >= ((int64_t)1 << 32)) return OFQ_ERR_UNSUPPORTED;
+  // the copies address a tile's rows with 32-bit offsets from its first row
+  if (row_bytes * (int64_t)(BN > 256 ? BN : 256) >= ((int64_t)1 << 32)) return OFQ_ERR_UNSUPPORTED;
   const int64_t KT = (row_bytes + kStageRow - 1) / kStageRow;
   if (KT < 1 || row_bytes > 0x7FFFFFFF - kStageRow) return OFQ_ERR_UNSUPPORTED;
   kern<<<m_tiles * n_tiles, 512, kLds, st>>>(static_cast<const uint8_t*>(a),
@@ -192,20 +182,23 @@ int launch_pp_tile(hipStream_t st, const void* a, const void* b, int64_t row_byt
   return ofq_check_launch();
 }
 
-// width: what pick_tile_width says.  One k-step a slot for the wide tiles (256: 330 us, two 336; 384 has
-// no registers for two), two for the narrow ones, whose slots would be too short to hide a fetch.
+// width: what pick_tile_width says, 192 or more.  Tiles of 128 columns stay with gemm_core2: a slot
+// of four matrix instructions here is too short for the fetch beside it (1100 x 4096 x 4096: int8 33.3 us
+// there, 35.2 here, bf16 57.3 and 60.9; two k-steps a slot here, which at 192 and 256 columns is slower
+// than one: bf16 1024 x 11008 x 4096 82.0 against 78.2).  gemm_core2 against this kernel in bf16:
+// 192 columns 1024 x 11008 x 4096 80.4 -> 78.2, 256 columns 4096 x 4096 x 4096 107.8 -> 105.0,
+// 384 columns 4096 x 5000 x 4096 140.2 -> 134.9.
 template<class MF, class EP>
 int launch_pp(hipStream_t st, const void* a, const void* b, int64_t row_bytes,
               const typename EP::Params& ep, int64_t M, int64_t N, int width) {
-#define OFQ_PP(BN, KS)                                                                          \
-  return row_bytes % kStageRow != 0                                                             \
-             ? launch_pp_tile<MF, true, EP, BN, KS>(st, a, b, row_bytes, ep, M, N)              \
-             : launch_pp_tile<MF, false, EP, BN, KS>(st, a, b, row_bytes, ep, M, N)
+#define OFQ_PP(BN)                                                                     \
+  return row_bytes % kStageRow != 0                                                    \
+             ? launch_pp_tile<MF, true, EP, BN>(st, a, b, row_bytes, ep, M, N)         \
+             : launch_pp_tile<MF, false, EP, BN>(st, a, b, row_bytes, ep, M, N)
   switch (width) {
-    case 384: OFQ_PP(384, 1);
-    case 256: OFQ_PP(256, 1);
-    case 192: OFQ_PP(192, 2);
-    default: OFQ_PP(128, 2);
+    case 384: OFQ_PP(384);
+    case 256: OFQ_PP(256);
+    default: OFQ_PP(192);
   }
 #undef OFQ_PP
 }

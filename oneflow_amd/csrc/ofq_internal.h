@@ -43,7 +43,7 @@ double gemm_wr_us(const LinearArgs& a, bool have_workspace);
 int launch_gemm_wr_f16(hipStream_t st, const LinearArgs& a, const WrPlan& plan, float* partials);
 int launch_gemm_wr_bf16(hipStream_t st, const LinearArgs& a, const WrPlan& plan, float* partials);
 
-// Copy-fed GEMMs for more than 128 rows (gemm_pp.h) on tiles of 256 x width; the linear's with the
+// Copy-fed GEMMs for more than 128 rows (gemm_pp.h) on tiles of 256 x width (192, 256 or 384); the linear's with the
 // weight already in the dtype of x.
 int launch_gemm_pp_f16(hipStream_t st, const void* x, const void* w, const void* bias, void* out,
                        int64_t m, int64_t n, int64_t k, int width);

@@ -93,8 +93,8 @@ __device__ __forceinline__ void quant_codes8(u32x4 raw, float sc, uint32_t (&w)[
 
 // groups along K, g = 8 * L with L a power of two <= 64, rows 16-byte aligned.  Bound by its vector
 // instructions until symmetric 16-bit groups took their largest magnitude as an integer maximum of bit
-// patterns (11008 x 4096 fp16 to 4 bit, groups of 128:
-// 27.7 -> 20.1 us, 5.6 TB/s; four packs per thread, all requested first: slower, 31.5 us before this).
+// patterns and the codes from quant_codes8: 11008 x 4096 fp16 to 4 bit, groups of 128, 27.7 -> 20.1 us
+// (5.6 TB/s).  Four packs a thread, all requested first, had made it 31.5 us: it was not short of requests.
 template<typename T, bool SYM, bool SIGNED, int BITS>
 __global__ void __launch_bounds__(256)
 quantize_pack_rows(const typename TT<T>::storage* __restrict__ x, uint8_t* __restrict__ q,

@@ -7,8 +7,9 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# (m, n): tiles of 256 x 128, 192, 256, 384; 12 and 17 tiles of rows
-SHAPES = [(1300, 1001), (2305, 4000), (1025, 11005), (2047, 11005), (2900, 2100), (4100, 3900)]
+# (m, n): tiles of 256 x 192, 256, 384, 384 with 10, 5, 8 and 17 tiles of rows; 256 x 128 (the kernel
+# whose waves stay in step) with 6 and 12
+SHAPES = [(2305, 4000), (1025, 11005), (2047, 11005), (4100, 3900), (1300, 1001), (2900, 2100)]
 
 
 @pytest.mark.parametrize("k", [64, 128, 192, 384, 448])
