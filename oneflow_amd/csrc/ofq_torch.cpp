@@ -767,6 +767,7 @@ PyObject* quantization(PyObject* const* args) {
 
 // The reference's gradient of fake_quantization: the output gradient passes to `in` unchanged,
 // scale and zero_point get none (oneflow/core/autograd/gradient_funcs/fake_quantization.cpp:36-42).
+// Forward mode is the same rule: the tangent of `in` is the tangent of the result.
 struct FakeQuantizationBackward : public torch::autograd::Node {
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
     return std::move(grads);
@@ -802,6 +803,10 @@ PyObject* fake_quantization(PyObject* const* args) {
                                                           torch::autograd::deleteNode);
     node->set_next_edges(torch::autograd::collect_next_edges(in));
     torch::autograd::set_history(out, node);
+  }
+  const Tensor& tangent = in._fw_grad(/*level=*/0);  // undefined where forward mode is off
+  if (tangent.defined()) {
+    out._set_fw_grad(tangent.clone(), /*level=*/0, /*is_inplace_op=*/false);
   }
   return wrap(std::move(out));
 }

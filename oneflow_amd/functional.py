@@ -122,7 +122,8 @@ def quantization(in_, scale, zero_point, quantization_formula="google", quantiza
 def fake_quantization(in_, scale, zero_point, quantization_formula="google", quantization_bit=8,
                       quantization_scheme="symmetric", *, zp_mode="float"):
     """Differentiable in ``in_``: the output gradient passes to it unchanged, scale and zero_point
-    get none (oneflow/core/autograd/gradient_funcs/fake_quantization.cpp:36-42)."""
+    get none (oneflow/core/autograd/gradient_funcs/fake_quantization.cpp:36-42).  In forward mode
+    the tangent of ``in_`` becomes the tangent of the result."""
     return _native.fake_quantization(in_, scale, zero_point, quantization_formula, quantization_bit,
                                      quantization_scheme, zp_mode)
 
