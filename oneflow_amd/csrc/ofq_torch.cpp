@@ -164,14 +164,23 @@ inline void* stream_of(const Tensor& t) {
   return c10::hip::getCurrentHIPStream(t.get_device()).stream();
 }
 
-// a call into the library; the interpreter lock is released, since a launch waits when the
-// stream's queue is full
-template<typename F>
-int unlocked(F f) {
-  PyThreadState* save = PyEval_SaveThread();
-  const int st = f();
-  PyEval_RestoreThread(save);
-  return st;
+// A call into the library.  The interpreter lock is released, since a launch waits when the stream's
+// queue is full.  The arguments are evaluated before that: taking a tensor's pointer can throw (a
+// tensor of a function transform has no storage), and the error has to be set under the lock.
+class Unlocked {
+ public:
+  Unlocked() : save_(PyEval_SaveThread()) {}
+  ~Unlocked() { PyEval_RestoreThread(save_); }
+  Unlocked(const Unlocked&) = delete;
+
+ private:
+  PyThreadState* save_;
+};
+
+template<typename... Params, typename... Args>
+int unlocked(int (*fn)(Params...), Args... args) {
+  const Unlocked released;
+  return fn(args...);
 }
 
 void check_status(const char* fn, int st) {
@@ -284,10 +293,9 @@ PyObject* groupwise_dequantize(PyObject* const* args) {
   for (int64_t d = 0; d < gd; ++d) outer *= shape[d];
   for (int64_t d = gd + 1; d < nd; ++d) inner *= shape[d];
   void* st = stream_of(in);
-  check_status("ofq_groupwise_dequantize", unlocked([&] {
-    return ofq_groupwise_dequantize(st, ptr(i_), ptr(s_), ptr(z_), ptr(out), code_of(i_),
-                                    code_of(s_), (int)num_bits, symmetric, outer, gs, inner);
-  }));
+  check_status("ofq_groupwise_dequantize", unlocked(
+      ofq_groupwise_dequantize, st, ptr(i_), ptr(s_), ptr(z_), ptr(out), code_of(i_), code_of(s_),
+      (int)num_bits, symmetric, outer, gs, inner));
   return wrap(std::move(out));
 }
 
@@ -395,10 +403,9 @@ PyObject* fused_linear(PyObject* const* args) {
   Tensor ws;
   if (ws_bytes != 0) ws = workspace(ws_bytes, x);
   void* st = stream_of(x);
-  check_status("ofq_fused_linear_gq", unlocked([&] {
-    return ofq_fused_linear_gq(st, ptr(x_), ptr(w_), ptr(s_), ptr(z_), ptr(b_), ptr(out), wd, td,
-                               num_bits, symmetric, gd, d.gs, d.m, d.n, d.k, ptr(ws), ws_bytes);
-  }));
+  check_status("ofq_fused_linear_gq", unlocked(
+      ofq_fused_linear_gq, st, ptr(x_), ptr(w_), ptr(s_), ptr(z_), ptr(b_), ptr(out), wd, td,
+      num_bits, symmetric, gd, d.gs, d.m, d.n, d.k, ptr(ws), ws_bytes));
   return wrap(std::move(out));
 }
 
@@ -417,9 +424,8 @@ PyObject* groupwise_repack(PyObject* const* args) {
         + " (k should be a multiple of 128)");
   Tensor tiled = empty({(int64_t)nbytes}, w.scalar_type(), w);
   void* st = stream_of(w);
-  check_status("ofq_groupwise_repack", unlocked([&] {
-    return ofq_groupwise_repack(st, ptr(w_), ptr(tiled), (int)num_bits, n, k);
-  }));
+  check_status("ofq_groupwise_repack", unlocked(
+      ofq_groupwise_repack, st, ptr(w_), ptr(tiled), (int)num_bits, n, k));
   return wrap(std::move(tiled));
 }
 
@@ -455,10 +461,9 @@ PyObject* fused_linear_tiled(PyObject* const* args) {
   Tensor out = empty(linear_shape(x, n), x.scalar_type(), x);
   const int wd = code_of(w_tiled), td = code_of(x);
   void* st = stream_of(x);
-  check_status("ofq_fused_linear_gq_tiled", unlocked([&] {
-    return ofq_fused_linear_gq_tiled(st, ptr(x_), ptr(w_tiled), ptr(s_), ptr(z_), ptr(b_), ptr(out),
-                                     wd, td, num_bits, symmetric, 1, gs, m, n, k);
-  }));
+  check_status("ofq_fused_linear_gq_tiled", unlocked(
+      ofq_fused_linear_gq_tiled, st, ptr(x_), ptr(w_tiled), ptr(s_), ptr(z_), ptr(b_), ptr(out),
+      wd, td, num_bits, symmetric, 1, gs, m, n, k));
   return wrap(std::move(out));
 }
 
@@ -543,10 +548,9 @@ PyObject* grouped_linear(PyObject* const* args) {
   }
   const int wd = code_of(w0), td = code_of(x0);
   void* st = stream_of(x0);
-  check_status("ofq_grouped_linear_gq", unlocked([&] {
-    return ofq_grouped_linear_gq(st, (int)count, px, pw, ps, symmetric ? nullptr : pz, pb, po, ms,
-                                 ns, ks, wd, td, num_bits, symmetric, (int)dims[0].gd, dims[0].gs);
-  }));
+  check_status("ofq_grouped_linear_gq", unlocked(
+      ofq_grouped_linear_gq, st, (int)count, px, pw, ps, symmetric ? nullptr : pz, pb, po, ms, ns,
+      ks, wd, td, num_bits, symmetric, (int)dims[0].gd, dims[0].gs));
   PyObject* list = PyList_New(count);
   for (int64_t i = 0; i < count; ++i) PyList_SET_ITEM(list, i, wrap(std::move(outs[i])));
   return list;
@@ -620,11 +624,10 @@ PyObject* fused_glu(PyObject* const* args) {
   void* vx = split ? wx + wx_bytes : nullptr;
   const int wd = code_of(w), td = code_of(x);
   void* st = stream_of(x);
-  check_status("ofq_fused_glu_gq", unlocked([&] {
-    return ofq_fused_glu_gq(st, ptr(x_), ptr(w_), ptr(ws_), ptr(wz_), ptr(b_), ptr(v_), ptr(vs_),
-                            ptr(vz_), ptr(c_), ptr(y), wx, vx, act, wd, td, num_bits, symmetric,
-                            (int)d.gd, d.gs, d.m, n, d.k);
-  }));
+  check_status("ofq_fused_glu_gq", unlocked(
+      ofq_fused_glu_gq, st, ptr(x_), ptr(w_), ptr(ws_), ptr(wz_), ptr(b_), ptr(v_), ptr(vs_),
+      ptr(vz_), ptr(c_), ptr(y), wx, vx, act, wd, td, num_bits, symmetric, (int)d.gd, d.gs, d.m, n,
+      d.k));
   return wrap(std::move(y));
 }
 
@@ -668,10 +671,9 @@ PyObject* min_max_observer(PyObject* const* args) {
   const size_t ws_bytes = ofq_min_max_observer_workspace_bytes(code_of(t), in.numel(), channels);
   const Tensor ws = workspace(ws_bytes, in);
   void* st = stream_of(in);
-  check_status("ofq_min_max_observer", unlocked([&] {
-    return ofq_min_max_observer(st, ptr(i_), ptr(scale), ptr(zero_point), code_of(t), i_.numel(),
-                                channels, q.bit, q.scheme, q.formula, ptr(ws), ws_bytes);
-  }));
+  check_status("ofq_min_max_observer", unlocked(
+      ofq_min_max_observer, st, ptr(i_), ptr(scale), ptr(zero_point), code_of(t), i_.numel(),
+      channels, q.bit, q.scheme, q.formula, ptr(ws), ws_bytes));
   return tuple_of(wrap(std::move(scale)), wrap(std::move(zero_point)));
 }
 
@@ -707,12 +709,10 @@ PyObject* moving_average_min_max_observer(PyObject* const* args) {
   const size_t ws_bytes = ofq_moving_average_min_max_observer_workspace_bytes(code_of(t), in.numel());
   const Tensor ws = workspace(ws_bytes, in);
   void* st = stream_of(in);
-  check_status("ofq_moving_average_min_max_observer", unlocked([&] {
-    return ofq_moving_average_min_max_observer(
-        st, ptr(i_), static_cast<const int64_t*>(ptr(step)), ptr(moving_max), ptr(moving_min),
-        ptr(scale), ptr(zero_point), code_of(t), i_.numel(), q.bit, q.scheme, q.formula,
-        (float)momentum, stop, training, ptr(ws), ws_bytes);
-  }));
+  check_status("ofq_moving_average_min_max_observer", unlocked(
+      ofq_moving_average_min_max_observer, st, ptr(i_), static_cast<const int64_t*>(ptr(step)),
+      ptr(moving_max), ptr(moving_min), ptr(scale), ptr(zero_point), code_of(t), i_.numel(), q.bit,
+      q.scheme, q.formula, (float)momentum, stop, training, ptr(ws), ws_bytes));
   return tuple_of(wrap(std::move(scale)), wrap(std::move(zero_point)));
 }
 
@@ -758,10 +758,9 @@ PyObject* quantization(PyObject* const* args) {
   Tensor out = empty(in.sizes(), to, in);
   const int id = code_of(in), od = code_of(to);
   void* st = stream_of(in);
-  check_status("ofq_quantization", unlocked([&] {
-    return ofq_quantization(st, ptr(i_), ptr(s_), ptr(z_), ptr(out), id, od, i_.numel(), s_.numel(),
-                            q.bit, q.scheme, q.formula, zp_mode);
-  }));
+  check_status("ofq_quantization", unlocked(
+      ofq_quantization, st, ptr(i_), ptr(s_), ptr(z_), ptr(out), id, od, i_.numel(), s_.numel(),
+      q.bit, q.scheme, q.formula, zp_mode));
   return wrap(std::move(out));
 }
 
@@ -793,10 +792,9 @@ PyObject* fake_quantization(PyObject* const* args) {
     out = empty(in.sizes(), in.scalar_type(), in);
     const int id = code_of(in);
     void* st = stream_of(in);
-    check_status("ofq_fake_quantization", unlocked([&] {
-      return ofq_fake_quantization(st, ptr(i_), ptr(s_), ptr(z_), ptr(out), id, i_.numel(),
-                                   s_.numel(), q.bit, q.scheme, q.formula, zp_mode);
-    }));
+    check_status("ofq_fake_quantization", unlocked(
+        ofq_fake_quantization, st, ptr(i_), ptr(s_), ptr(z_), ptr(out), id, i_.numel(), s_.numel(),
+        q.bit, q.scheme, q.formula, zp_mode));
   }
   if (in.requires_grad() && at::GradMode::is_enabled()) {
     auto node = std::shared_ptr<FakeQuantizationBackward>(new FakeQuantizationBackward(),
@@ -852,11 +850,10 @@ PyObject* layer_norm_observer(PyObject* const* args) {
   void* st = stream_of(x);
   float* ps = static_cast<float*>(ptr(scale));
   float* pz = static_cast<float*>(ptr(zero_point));
-  check_status("ofq_fused_layer_norm_min_max_observer", unlocked([&] {
-    return ofq_fused_layer_norm_min_max_observer_stats(
-        st, ptr(x_), nullptr, nullptr, 0.0, 0, ptr(g_), ptr(b_), ptr(y), ps, pz, td, rows, cols,
-        epsilon, (int)bit, exact ? OFQ_LN_STATS_FP64 : OFQ_LN_STATS_FP32, ptr(ws), ws_bytes);
-  }));
+  check_status("ofq_fused_layer_norm_min_max_observer", unlocked(
+      ofq_fused_layer_norm_min_max_observer_stats, st, ptr(x_), nullptr, nullptr, 0.0, 0, ptr(g_),
+      ptr(b_), ptr(y), ps, pz, td, rows, cols, epsilon, (int)bit,
+      exact ? OFQ_LN_STATS_FP64 : OFQ_LN_STATS_FP32, ptr(ws), ws_bytes));
   return tuple_of(wrap(std::move(y)), wrap(std::move(scale)), wrap(std::move(zero_point)));
 }
 
@@ -899,11 +896,10 @@ PyObject* skip_layer_norm_observer(PyObject* const* args) {
   void* st = stream_of(x);
   float* ps = static_cast<float*>(ptr(scale));
   float* pz = static_cast<float*>(ptr(zero_point));
-  check_status("ofq_fused_skip_layer_norm_min_max_observer", unlocked([&] {
-    return ofq_fused_layer_norm_min_max_observer_stats(
-        st, ptr(x_), ptr(p_), ptr(s_), alpha, 1, ptr(g_), ptr(b_), ptr(y), ps, pz, td, rows, cols,
-        epsilon, (int)bit, exact ? OFQ_LN_STATS_FP64 : OFQ_LN_STATS_FP32, ptr(ws), ws_bytes);
-  }));
+  check_status("ofq_fused_skip_layer_norm_min_max_observer", unlocked(
+      ofq_fused_layer_norm_min_max_observer_stats, st, ptr(x_), ptr(p_), ptr(s_), alpha, 1,
+      ptr(g_), ptr(b_), ptr(y), ps, pz, td, rows, cols, epsilon, (int)bit,
+      exact ? OFQ_LN_STATS_FP64 : OFQ_LN_STATS_FP32, ptr(ws), ws_bytes));
   return tuple_of(wrap(std::move(y)), wrap(std::move(scale)), wrap(std::move(zero_point)));
 }
 
@@ -936,26 +932,22 @@ PyObject* layer_norm_quantization(PyObject* const* args) {
   int rc;
   {
     const Tensor ws = workspace(ws_bytes, x);
-    rc = unlocked([&] {
-      return ofq_fused_layer_norm_quantization(st, ptr(x_), ptr(g_), ptr(b_), ptr(codes), ps, pz,
-                                               td, rows, cols, epsilon, (int)bit, stats, ptr(ws),
-                                               ws_bytes);
-    });
+    rc = unlocked(
+        ofq_fused_layer_norm_quantization, st, ptr(x_), ptr(g_), ptr(b_), ptr(codes), ps, pz, td,
+        rows, cols, epsilon, (int)bit, stats, ptr(ws), ws_bytes);
   }
   if (rc == OFQ_ERR_UNSUPPORTED) {
     // the two ops in a row
     const Tensor y = empty(x.sizes(), x.scalar_type(), x);
     const size_t ws2_bytes = ofq_fused_layer_norm_min_max_observer_workspace_bytes(td, rows, cols);
     const Tensor ws2 = workspace(ws2_bytes, x);
-    check_status("ofq_fused_layer_norm_min_max_observer", unlocked([&] {
-      return ofq_fused_layer_norm_min_max_observer_stats(
-          st, ptr(x_), nullptr, nullptr, 0.0, 0, ptr(g_), ptr(b_), ptr(y), ps, pz, td, rows, cols,
-          epsilon, (int)bit, stats, ptr(ws2), ws2_bytes);
-    }));
-    check_status("ofq_quantization", unlocked([&] {
-      return ofq_quantization(st, ptr(y), ps, pz, ptr(codes), td, OFQ_I8, y.numel(), 1, (int)bit,
-                              OFQ_SCHEME_SYMMETRIC, OFQ_FORMULA_GOOGLE, OFQ_ZP_FLOAT);
-    }));
+    check_status("ofq_fused_layer_norm_min_max_observer", unlocked(
+        ofq_fused_layer_norm_min_max_observer_stats, st, ptr(x_), nullptr, nullptr, 0.0, 0,
+        ptr(g_), ptr(b_), ptr(y), ps, pz, td, rows, cols, epsilon, (int)bit, stats, ptr(ws2),
+        ws2_bytes));
+    check_status("ofq_quantization", unlocked(
+        ofq_quantization, st, ptr(y), ps, pz, ptr(codes), td, OFQ_I8, y.numel(), 1, (int)bit,
+        OFQ_SCHEME_SYMMETRIC, OFQ_FORMULA_GOOGLE, OFQ_ZP_FLOAT));
   } else {
     check_status("ofq_fused_layer_norm_quantization", rc);
   }
@@ -992,11 +984,9 @@ PyObject* matmul_quant(PyObject* const* args) {
   Tensor ws;
   if (ws_bytes != 0) ws = workspace(ws_bytes, a);
   void* st = stream_of(a);
-  check_status("ofq_matmul_quant_ws", unlocked([&] {
-    return ofq_matmul_quant_ws(st, ptr(a_), ptr(b_), static_cast<const float*>(ptr(as_)),
-                               static_cast<const float*>(ptr(bs_)), ptr(bias_), ptr(out), od, m, n,
-                               k, ptr(ws), ws_bytes);
-  }));
+  check_status("ofq_matmul_quant_ws", unlocked(
+      ofq_matmul_quant_ws, st, ptr(a_), ptr(b_), static_cast<const float*>(ptr(as_)),
+      static_cast<const float*>(ptr(bs_)), ptr(bias_), ptr(out), od, m, n, k, ptr(ws), ws_bytes));
   return wrap(std::move(out));
 }
 
@@ -1030,10 +1020,9 @@ PyObject* groupwise_quantize(PyObject* const* args) {
   Tensor scale = empty({sn, sk}, t, x), zero;
   if (!symmetric) zero = empty({sn, sk}, t, x);
   void* st = stream_of(x);
-  check_status("ofq_groupwise_quantize", unlocked([&] {
-    return ofq_groupwise_quantize(st, ptr(x_), ptr(q), ptr(scale), ptr(zero), code_of(t),
-                                  code_of(qt), (int)num_bits, symmetric, (int)gd, gs, n, k);
-  }));
+  check_status("ofq_groupwise_quantize", unlocked(
+      ofq_groupwise_quantize, st, ptr(x_), ptr(q), ptr(scale), ptr(zero), code_of(t), code_of(qt),
+      (int)num_bits, symmetric, (int)gd, gs, n, k));
   return tuple_of(wrap(std::move(q)), wrap(std::move(scale)),
                   symmetric ? none() : wrap(std::move(zero)));
 }
