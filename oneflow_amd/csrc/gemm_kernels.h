@@ -242,7 +242,7 @@ __device__ __forceinline__ void wait_vmem_all() { wait_vmem_le<0>(); }
 // rows [0, ROWS) x 128 bytes of tile kt of a row-major byte matrix -> swizzled LDS tile.  Rows are
 // `ld` bytes, a multiple of 16 but not of 128: of the last tile of such a ragged matrix the pieces
 // past the end of a row are not requested, their lanes write zeros to LDS instead (both operands
-// do so, or one does and the other is finite there: the products add 0).  RAGGED is a flag of the
+// do so, or one does and the other's elements there are zeros too: the products add 0).  RAGGED is a flag of the
 // kernel: the same test made at run time cost 8 % of 2048 x 11008 x 4096 (registers).
 template<bool RAGGED, int ROWS, int NWAVES>
 __device__ __forceinline__ void async_tile(const uint8_t* __restrict__ g, int64_t ld, int row0,
@@ -308,9 +308,11 @@ struct B2Dequant {
     typedef typename std::conditional<BITS == 4 && ZMODE == 0, uint16_t, uint32_t>::type Slot;
     Slot s[kChunks];
     Slot z[kChunks];
+    uint32_t past;  // RAGGED: bit i, chunk i lies past the end of its row
   };
   static __device__ __forceinline__ void load(const Params& p, int n0, int kt, int, int, int tid,
                                               Regs& r, uint8_t*) {
+    if (RAGGED) r.past = 0;
 #pragma unroll
     for (int i = 0; i < kChunks; ++i) {
       const int q = tid + i * NT;
@@ -318,9 +320,10 @@ struct B2Dequant {
       int row = n0 + q / kChunksPerRow;
       row = row < p.N ? row : p.N - 1;
       const int c = q % kChunksPerRow;
-      // past the end of a ragged row: its first chunk again (finite, and x is zero there)
+      // past the end of a ragged row: its first chunk again, expanded with a scale of zero
       const int byte = kt * kCodeBytesPerRow + c * 16;
       const bool in_row = !RAGGED || byte < (int)p.ldw;
+      if (RAGGED && !in_row) r.past |= 1u << i;
       r.v[i] = *reinterpret_cast<const u32x4*>(p.w + (int64_t)row * p.ldw + (in_row ? byte : 0));
       const int k = in_row ? kt * 64 + c * kElemsPerChunk : 0;
       const int64_t si = (int64_t)row * p.G + k / p.group_size;
@@ -340,9 +343,14 @@ struct B2Dequant {
       const int c = q % kChunksPerRow;
       uint8_t* rowp = lds + row * kStageRow;
       const int sw = swizzle_key(row);
-      const float sc = raw16_to_float<T>((uint16_t)r.s[i]);
+      float sc = raw16_to_float<T>((uint16_t)r.s[i]);
       float zc = 0.f;
       if (ZMODE == 2) zc = raw16_to_float<T>((uint16_t)r.z[i]);
+      if (RAGGED && (r.past >> i & 1u) != 0) {
+        // w~ = 0: x is zero there too, but zero times a code that overflows T under its scale is NaN
+        sc = 0.f;
+        zc = 0.f;
+      }
       if (ZMODE == 1) zc = TT<T>::round(-(float)((1 << (BITS - 1)) - 1) * sc);
       if constexpr (BITS == 8) {
         u32x4 o0, o1;

@@ -216,7 +216,7 @@ gemm_wr(WrParams p) {
       const int c = o - kXOps;
       const uint8_t* src = wr_uniform(wbase + (int64_t)gs * (kCB * KH));
       uint32_t off = woff[c];
-      // past the end of a ragged row: its first bytes of this step's piece 0 (finite; x is zero)
+      // past the end of a ragged row: its first bytes of this step's piece 0 (their scale is zero)
       if (RAGGED && gs * (kCB * KH) + wk[c] >= row_bytes) off -= (uint32_t)wk[c];
       async_copy16_unordered(src, off, st + kXBytes + (wave * kCodeOps + c) * 1024);
     }
@@ -267,11 +267,18 @@ gemm_wr(WrParams p) {
     const uint8_t* cp = smem + buf * kStage + kXBytes + wave * (kCodeOps * 1024) + lane * 16;
 #pragma unroll
     for (int o = 0; o < kCodeOps; ++o) dst[o] = *reinterpret_cast<const u32x4*>(cp + o * 1024);
-    int g = group_of((step0 + t) * (KH * 64) + kh * 64 + half * 32) - g0;
-    g = g < ng ? g : 0;  // (past the panel or K: not used, or x is zero and the scale finite)
+    const int k = (step0 + t) * (KH * 64) + kh * 64 + half * 32;
+    int g = group_of(k) - g0;
+    g = g < ng ? g : 0;  // (past the panel or K: not used, or the zero scale below)
     sd = TT<T>::load(reinterpret_cast<const S*>(sl) + g * BN + col);
     zd = 0.f;
     if (ZMODE == 2) zd = TT<T>::load(reinterpret_cast<const S*>(zl) + g * BN + col);
+    if (RAGGED && k >= p.K) {
+      // w~ = 0 past the end of a row: x is zero there too, but zero times a code that overflows T
+      // under somebody's scale would be NaN
+      sd = 0.f;
+      zd = 0.f;
+    }
     if (ZMODE == 1) zd = TT<T>::round(-(float)((1 << (BITS - 1)) - 1) * sd);
   };
   auto read_x = [&](int buf, int j, u32x4 (&dst)[TM]) {

@@ -13,8 +13,9 @@
 //
 // K is any multiple of a lane's share of a chunk (LK = 32 4-bit or 16 8-bit elements), so a lane's
 // share lies inside or outside the row as a whole.  In the last chunk of a ragged row (a K shard
-// of 43 groups of 64, say) the lanes beyond K re-read the row's first bytes and meet zeros of x:
-// nothing out of bounds is read and their products add 0.  Before, such rows went to the
+// of 43 groups of 64, say) the lanes beyond K re-read the row's first bytes, expand them with a scale
+// and a zero point of 0 (a w~ that overflows T would turn the zero of x it meets into NaN) and meet
+// zeros of x: nothing out of bounds is read and their products add 0.  Before, such rows went to the
 // one-wave-per-row fallback (2 layers of 4352 / 14624 columns, groups of 32, 3 rows of x: 836 us).
 #pragma once
 
@@ -240,11 +241,14 @@ gemv_rows_body(int block, const uint16_t* __restrict__ x, const uint8_t* __restr
           const int c = 2 * pair + u;
           if (c < nchunks) {
             int k0 = c * CK + kb * LK;
-            k0 = k0 < K ? k0 : 0;
+            const bool in_row = k0 < K;
+            k0 = in_row ? k0 : 0;
             const int grp = gs_shift >= 0 ? (k0 >> gs_shift) : (k0 / group_size);
-            const float s = TT<T>::load(reinterpret_cast<const S*>(sl) + srow + grp);
+            float s = TT<T>::load(reinterpret_cast<const S*>(sl) + srow + grp);
             float z = 0.f;
             if (ZMODE == kZeroAsym) z = TT<T>::load(reinterpret_cast<const S*>(zl) + srow + grp);
+            s = in_row ? s : 0.f;
+            z = in_row ? z : 0.f;
             if (ZMODE == kZeroSymU) z = TT<T>::round(-(float)((1 << (BITS - 1)) - 1) * s);
             if constexpr (BITS == 4) {
 #pragma unroll
@@ -352,7 +356,8 @@ gemv_rows_grouped(GemvGroup g, int M, int K, int group_size, int gs_shift, int r
 // the reduction area, which is used only after the k loop.
 //
 // Scales.  The scales (and zeros) of the block's rows are copied to LDS for panel_chunks chunks at a
-// time: all of K unless long rows of short groups leave no room for it.
+// time: all of K unless long rows of short groups leave no room for it.  A row of the panel ends with a
+// zero, the scale of a lane past the end of K.
 // ---------------------------------------------------------------------------------------------
 template<int BITS, int MT>
 struct RowsMtX {
@@ -391,11 +396,12 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
   if (rows_blk <= 0) return;
   const int ntiles = (rows_blk + 15) >> 4;
 
-  // LDS: [the waves' x buffers | red NWAVES*MT*256 f32][scales rows_per_block*panel_groups, padded
-  //      to 16 B][zeros (asymmetric)]
+  // LDS: [the waves' x buffers | red NWAVES*MT*256 f32][scales rows_per_block*(panel_groups + 1),
+  //      padded to 16 B][zeros (asymmetric)]
   typedef RowsMtX<BITS, MT> XB;
   float* red = reinterpret_cast<float*>(smem);
-  const int panel_bytes = (rows_per_block * panel_groups * 2 + 15) & ~15;
+  const int pitch = panel_groups + 1;
+  const int panel_bytes = (rows_per_block * pitch * 2 + 15) & ~15;
   constexpr size_t kRedBytes = (size_t)NWAVES * MT * 256 * 4;
   constexpr size_t kFront = (size_t)NWAVES * XB::kWaveBytes > kRedBytes
                                 ? (size_t)NWAVES * XB::kWaveBytes : kRedBytes;
@@ -456,13 +462,16 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
     g0 = gs_shift >= 0 ? (first_chunk * CK) >> gs_shift : (first_chunk * CK) / group_size;
     const int ng = G - g0 < panel_groups ? G - g0 : panel_groups;
     copy_scale_panel<NT, ZMODE == kZeroAsym, false>(sblk + g0, zblk + g0, G, rows_blk, rows_blk, ng,
-                                                    panel_groups, sl, zl, tid);
+                                                    pitch, sl, zl, tid);
+    if (tid < rows_per_block) {  // (at most 64 rows)
+      sl[tid * pitch + panel_groups] = 0;
+      if (ZMODE == kZeroAsym) zl[tid * pitch + panel_groups] = 0;
+    }
     __syncthreads();
   };
 
   auto work = [&](const u32x4 (&cur)[NTL], u32x4 (&nxt)[NTL]) {
-    int k0 = c * CK + kb * LK;
-    k0 = k0 < K ? k0 : 0;
+    const int k0 = c * CK + kb * LK;
     if ((c + 1) * CK > K) {  // (the same for every lane: the last chunk of a ragged row)
 #pragma unroll
       for (int i = 0; i < XB::kReqs; ++i) {
@@ -479,11 +488,11 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
     request_x(c + NWAVES);
     request_codes(c + NWAVES, nxt);
     int grp = (gs_shift >= 0 ? (k0 >> gs_shift) : (k0 / group_size)) - g0;
-    grp = grp < 0 ? 0 : grp;  // (a lane past the end of a row: any scale, its x is zero)
+    grp = k0 < K ? grp : panel_groups;
     float s[NTL], z[NTL];
 #pragma unroll
     for (int t = 0; t < NTL; ++t) {
-      const int at = (t * 16 + r) * panel_groups + grp;
+      const int at = (t * 16 + r) * pitch + grp;
       s[t] = TT<T>::load(reinterpret_cast<const S*>(sl) + at);
       z[t] = 0.f;
       if (ZMODE == kZeroAsym) z[t] = TT<T>::load(reinterpret_cast<const S*>(zl) + at);
@@ -725,7 +734,7 @@ inline size_t gemv_rows_mt_lds_bytes(int nwaves, int mt, int bits, int rows_per_
   const size_t red = (size_t)nwaves * mt * 256 * 4;
   const size_t xb = (size_t)nwaves * mt * 16 * ((bits == 4 ? 256 : 128) + 16);
   return (xb > red ? xb : red)
-         + (size_t)(asym ? 2 : 1) * ((rows_per_block * panel_groups * 2 + 15) & ~15);
+         + (size_t)(asym ? 2 : 1) * ((rows_per_block * (panel_groups + 1) * 2 + 15) & ~15);
 }
 
 inline size_t gemv_rows_lds_bytes(int nwaves, int M, int K, int group_size, int rows_per_block,

@@ -88,3 +88,52 @@ def test_matmul_quant_ragged_k(m, n, k):
                                           H.to_torch(b_scale), None, torch.float16))
     acc = a.astype(np.float64) @ b.astype(np.float64).T
     assert np.array_equal(got, (acc.astype(np.float32) * (a_scale[0] * b_scale)[None]).astype(np.float16))
+
+
+def _overflowing_weight(n, k, g, num_bits, symmetric, qdt, t, rng):
+    """Codes around zero, and three rows in which a product code * scale overflows T:
+      row 0  only if the codes of the row's last 128 elements met the scale of its first group
+      row 1  in its first group, row 2 where its last 128 elements begin: the results are infinite"""
+    signed = qdt == np.int8
+    neutral = 0 if signed or not symmetric else 2 ** (num_bits - 1) - 1
+    most = -2 ** (num_bits - 1) if signed else 2 ** num_bits - 1
+    # (neutral + 1) * huge is finite, most * huge is not
+    huge = {("f16", 4): (8000.0, 9000.0), ("f16", 8): (511.0, 515.0),
+            ("bf16", 4): (4.2e37,), ("bf16", 8): (2.6e36,)}[t, num_bits][signed]
+    codes = (neutral + rng.integers(-1 if symmetric else 0, 2, size=(n, k))).astype(qdt)
+    scale = np.full((n, k // g), 0.01, np.float32)
+    tail = (k - 1) // 128 * 128
+    codes[:3] = neutral
+    codes[0, 5] = neutral + 1
+    codes[0, tail:] = most
+    scale[0, 0] = huge
+    codes[1, 7] = most
+    scale[1, 0] = huge
+    codes[2, tail + 3] = most
+    scale[2, tail // g] = huge
+    w = H.pack_int4(codes) if num_bits == 4 else codes
+    zero = None if symmetric else H.as_T(np.zeros_like(scale), t)
+    return w, H.as_T(scale, t), zero
+
+
+@pytest.mark.parametrize("n,k,g", [(70, 288, 32), (33, 160, 32), (150, 2752, 64), (40, 9248, 32)])
+@pytest.mark.parametrize("m", [1, 3, 16, 17, 40, 64, 65, 130, 300])
+@pytest.mark.parametrize("t", ["f16", "bf16"])
+def test_linear_ragged_k_overflowing_products(m, n, k, g, t):
+    """What a kernel multiplies past the end of a row is zero whatever the weights hold: a finite
+    result stays finite, an infinite one infinite (with NaN in neither)."""
+    rng = np.random.Generator(np.random.PCG64(m * 13 + n + k))
+    x = rng.uniform(0.25, 1.0, size=(m, k)) * rng.choice([-1.0, 1.0], size=(m, k))
+    x = H.as_T(x.astype(np.float32), t)
+    for num_bits, symmetric, qdt in VARIANTS:
+        if t == "bf16" and qdt == np.int8:
+            continue  # no product there overflows: 2^(b-1) * s has to be finite in fp32
+        w, scale, zero = _overflowing_weight(n, k, g, num_bits, symmetric, qdt, t, rng)
+        ref = O.to_f32(O.fused_linear(x, w, scale, zero, None, num_bits, symmetric, 1, g))
+        assert np.isinf(ref[:, 1:3]).all() and np.isfinite(np.delete(ref, [1, 2], 1)).all()
+        got = O.to_f32(_linear(x, w, scale, zero, None, num_bits, symmetric, g))
+        what = f"{t} b{num_bits} m={m} n={n} k={k} {symmetric} {qdt}"
+        assert np.array_equal(got[:, 1:3], ref[:, 1:3]), what
+        # one product and sums of tiny ones in row 0: one rounding of T either way
+        assert np.allclose(got[:, 0], ref[:, 0], rtol=2.0 ** (-9 if t == "f16" else -6), atol=0), what
+        H.assert_linear_parity(H.as_T(got[:, 3:], t), H.as_T(ref[:, 3:], t), t, what)
