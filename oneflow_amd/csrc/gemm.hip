@@ -230,7 +230,8 @@ double slices_us(const LinearArgs& a, int64_t s) {
 // A step was timed per tile on symmetric fp16 4-bit codes (m = 32..384, n = 4096, one slice); what it
 // converts in the shadow of the matrix instructions no longer hides where the type and the zero point
 // make that longer: 1.65 times the step for bf16 with a zero point, 1.3 for fp16, 1.2 for bf16 without.
-double wr_plan_us(const LinearArgs& a, WrPlan* plan) {
+// Without a workspace the sums of slices have nowhere to go: the tile that is best with one slice.
+double wr_plan_us(const LinearArgs& a, bool have_workspace, WrPlan* plan) {
   double best = 1e30;
   if (a.m <= 16 || a.m >= 1024) return best;
   if (a.group_size % 32 != 0 || a.k % 32 != 0) return best;
@@ -266,6 +267,7 @@ double wr_plan_us(const LinearArgs& a, WrPlan* plan) {
       }
     };
     consider(1);
+    if (!have_workspace) continue;
     // steps / s falls, the sums grow with s: least where the two are equal, or where the chip is full
     int most = 256 / blocks < steps / 2 ? 256 / blocks : steps / 2;
     most = most < 16 ? most : 16;
@@ -275,21 +277,6 @@ double wr_plan_us(const LinearArgs& a, WrPlan* plan) {
     if (s >= 2 && s < most) consider(s + 1);
   }
   return best;
-}
-
-// gemm_wr or gemm_core2 on its tile of 256 x 128, whose k-tile of 64 takes about 1.12 us: that one
-// converts a code once per block where gemm_wr does once per wave, so with bf16 zero points and several
-// tiles of rows it keeps up (m = 900, n = k = 4096: 53 us against 58).
-bool wr_plan(const LinearArgs& a, WrPlan* plan) {
-  const double us = wr_plan_us(a, plan);
-  if (us >= 1e30) return false;
-  if (a.m > 128) {
-    const int64_t s = wq_splits(a);
-    const int64_t blocks = ((a.m + 255) / 256) * ((a.n + 127) / 128) * s;
-    const double rounds = (double)((blocks + 255) / 256);
-    if (4 + rounds * ((a.k + 63) / 64 / s) * 1.12 + slices_us(a, s) < us) return false;
-  }
-  return true;
 }
 
 size_t wq_partial_bytes(const LinearArgs& a) {
@@ -310,6 +297,21 @@ size_t wr_partial_bytes(const LinearArgs& a, const WrPlan& plan) {
 
 }  // namespace
 
+// gemm_wr or gemm_core2 on its tile of 256 x 128, whose k-tile of 64 takes about 1.12 us: that one
+// converts a code once per block where gemm_wr does once per wave, so with bf16 zero points and several
+// tiles of rows it keeps up (m = 900, n = k = 4096: 53 us against 58).
+bool gemm_wr_plan(const LinearArgs& a, bool have_workspace, WrPlan* plan) {
+  const double us = wr_plan_us(a, have_workspace, plan);
+  if (us >= 1e30) return false;
+  if (a.m > 128) {
+    const int64_t s = have_workspace ? wq_splits(a) : 1;
+    const int64_t blocks = ((a.m + 255) / 256) * ((a.n + 127) / 128) * s;
+    const double rounds = (double)((blocks + 255) / 256);
+    if (4 + rounds * ((a.k + 63) / 64 / s) * 1.12 + slices_us(a, s) < us) return false;
+  }
+  return true;
+}
+
 // Two passes pay once m is large: the in-tile path converts every weight tile once per 256 rows
 // of x (8 times at m = 2048) and that conversion, not the MFMAs, bounds it; converting the weight
 // once into the workspace and running the copy-fed GEMM on it is what the reference functor does
@@ -318,29 +320,25 @@ size_t gemm_wq_workspace_bytes(const LinearArgs& a) {
   if (!gemm_wq_supported(a)) return 0;
   if (a.m >= 1024) return (size_t)a.n * (size_t)a.k * 2;
   WrPlan plan;
-  if (wr_plan(a, &plan)) return wr_partial_bytes(a, plan);
+  if (gemm_wr_plan(a, true, &plan)) return wr_partial_bytes(a, plan);
   return wq_partial_bytes(a);
 }
 
-// The streaming kernel's rival for 16 < m <= 64: what gemm_wr is expected to take with a workspace.
+// The streaming kernel's rival for 16 < m <= 64: what gemm_wr is expected to take.
 double gemm_wr_us(const LinearArgs& a, bool have_workspace) {
-  WrPlan plan{kWr32x128, 1};
-  const double us = wr_plan_us(a, &plan);
-  return plan.splits > 1 && !have_workspace ? 1e30 : us;
+  WrPlan plan;
+  return wr_plan_us(a, have_workspace, &plan);
 }
 
 int launch_gemm_wq(hipStream_t st, const LinearArgs& a, void* workspace, size_t workspace_bytes) {
   const size_t need = gemm_wq_workspace_bytes(a);
   const bool have_ws =
       need != 0 && workspace != nullptr && workspace_bytes >= need && ofq_aligned16(workspace);
-  {
-    WrPlan plan;
-    if (wr_plan(a, &plan)) {
-      if (!have_ws) plan.splits = 1;
-      float* partials = static_cast<float*>(workspace);
-      return a.t_dtype == OFQ_F16 ? launch_gemm_wr_f16(st, a, plan, partials)
-                                  : launch_gemm_wr_bf16(st, a, plan, partials);
-    }
+  WrPlan plan;
+  if (gemm_wr_plan(a, have_ws, &plan)) {
+    float* partials = static_cast<float*>(workspace);
+    return a.t_dtype == OFQ_F16 ? launch_gemm_wr_f16(st, a, plan, partials)
+                                : launch_gemm_wr_bf16(st, a, plan, partials);
   }
   if (have_ws && a.m < 1024) {
     float* partials = static_cast<float*>(workspace);
