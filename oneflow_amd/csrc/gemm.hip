@@ -220,16 +220,30 @@ bool gemm_wq_supported(const LinearArgs& a) {
 
 namespace {
 
-double slices_us(const LinearArgs& a, int64_t s) {
-  return s > 1 ? 4 + 8e-6 * s * a.m * a.n / 6.5 : 0.0;
+// Expected times in us, fitted to 84 000 timings (n from 512 to 32000, half of them odd, k from 512 to 14336,
+// 17 <= m <= 1020, both types, both widths, with and without a zero point, groups of 32, 64 and 128, weights
+// not in cache).  They are within 18 % of the measured time for 98 of 100 plans; the plan chosen takes
+// about 1 % longer than the fastest one in the mean.
+//
+// `blocks` blocks on `slots` places: a k-step costs `alone` us where a block has the chip to itself and
+// `full` where every place is taken (the copies share the L2s, the matrix cores a clock).
+double rounds_us(int blocks, int slots, double alone, double full) {
+  const int rest = blocks % slots;
+  return blocks / slots * full + (rest != 0 ? alone + (full - alone) * rest / slots : 0.0);
 }
 
+inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
+
+inline bool has_zero_term(const LinearArgs& a) { return !a.symmetric || !a.w_signed; }
+
 // Tile and K slices of gemm_wr for 16 < m < 1024 (fewer rows stream, more are worth a converted copy of
-// the weight), by the time a plan is expected to take in us: 4 to the first step, the steps of a block,
-// and for slices 4 (second launch, end of the first) plus their fp32 sums out and back at 6.5 TB/s.
-// A step was timed per tile on symmetric fp16 4-bit codes (m = 32..384, n = 4096, one slice); what it
-// converts in the shadow of the matrix instructions no longer hides where the type and the zero point
-// make that longer: 1.65 times the step for bf16 with a zero point, 1.3 for fp16, 1.2 for bf16 without.
+// the weight) by the least expected time:
+//   the start, and 1.9 per 4096 scales (and zeros) that a block copies first;
+//   the steps, measured with symmetric fp16 4-bit codes; others take longer to expand, which the taller
+//   tiles hide better; a K that is not whole steps costs 1.4 times as much (the copies of such a
+//   kernel are all waited for); 8-bit codes that a single block reads are bound by the stream of them;
+//   the end: the output, 16-bit stores one by one where n is not whole pieces of 16 bytes, or for slices
+//   the second launch and their fp32 sums out and back at 5.2 TB/s.
 // Without a workspace the sums of slices have nowhere to go: the tile that is best with one slice.
 double wr_plan_us(const LinearArgs& a, bool have_workspace, WrPlan* plan) {
   double best = 1e30;
@@ -240,26 +254,38 @@ double wr_plan_us(const LinearArgs& a, bool have_workspace, WrPlan* plan) {
   struct Tile {
     WrTile tile;
     int bm, bn, step_k;
-    double step_us;
-    bool any_bits;
+    int above;  // up to so many rows the tile before does the same in less time
+    double start, alone, full;
+    bool any_bits, tall;
   };
-  static const Tile tiles[] = {{kWr32x128, 32, 128, 128, 0.54, true},
-                               {kWr64x128, 64, 128, 128, 0.68, true},
-                               {kWr96x128, 96, 128, 128, 0.77, false},
-                               {kWr128x256, 128, 256, 64, 0.72, true},
-                               {kWr192x256, 192, 256, 64, 0.88, false}};
-  const bool zero = !a.symmetric || !a.w_signed;
-  const bool bf = a.t_dtype == OFQ_BF16;
-  const double convert = zero ? (bf ? 1.65 : 1.3) : (bf ? 1.2 : 1.0);
+  static const Tile tiles[] = {{kWr32x128, 32, 128, 128, 0, 4.0, 0.43, 0.55, true, false},
+                               {kWr64x128, 64, 128, 128, 32, 4.5, 0.46, 0.69, true, false},
+                               {kWr96x128, 96, 128, 128, 64, 4.8, 0.51, 0.84, false, false},
+                               {kWr128x256, 128, 256, 64, 0, 5.1, 0.53, 0.88, true, true},
+                               {kWr192x256, 192, 256, 64, 128, 5.0, 0.72, 1.06, false, true}};
+  // [tall][8-bit][bf16][zero term]
+  static const double convert[2][2][2][2] = {{{{1.00, 1.08}, {1.04, 1.36}}, {{1.33, 1.33}, {1.35, 1.58}}},
+                                             {{{1.00, 1.03}, {1.00, 1.21}}, {{1.10, 1.11}, {1.13, 1.33}}}};
+  constexpr int kCUs = 256;
+  const bool zero = has_zero_term(a);
+  const double scales_us = 1.9 / 4096 * (a.symmetric ? 1 : 2) / a.group_size;  // per column and k
+  const double mn = 1e-6 * (double)a.m * a.n;
+  // us for the sums of one slice, in whole 32 x 32 tiles
+  const double slice_us = 8e-6 / 5.2 * 1024 * ceil_div(a.m, 32) * ceil_div(a.n, 32)
+                          + (a.n % 4 != 0 ? 0.17 * mn : 0.0);
+  const double store_us = a.n % 8 != 0 ? 0.4 + 2.1 * mn : 0.0;
   for (const Tile& t : tiles) {
-    if (!t.any_bits && a.bits != 4) continue;
-    const int blocks = (int)(((a.m + t.bm - 1) / t.bm) * ((a.n + t.bn - 1) / t.bn));
-    const int steps = (int)((a.k + t.step_k - 1) / t.step_k);
-    const double step_us = t.step_us * convert;
+    if (a.m <= t.above || (!t.any_bits && a.bits != 4)) continue;
+    const int blocks = ceil_div(a.m, t.bm) * ceil_div(a.n, t.bn);
+    const int steps = ceil_div(a.k, t.step_k);
+    const double c = convert[t.tall][a.bits == 8][a.t_dtype == OFQ_BF16][zero] * (a.k % t.step_k != 0 ? 1.4 : 1.0);
+    const double full = t.full * (a.bits == 8 && !t.tall && a.m <= t.bm ? 1.1 : 1.0);
     auto consider = [&](int s) {
-      const int per = (steps + s - 1) / s;
-      s = (steps + per - 1) / per;  // no empty last slice
-      const double us = 4 + (blocks * s + 255) / 256 * per * step_us + slices_us(a, s);
+      const int per = ceil_div(steps, s);
+      s = ceil_div(steps, per);  // no empty last slice
+      const double us = t.start + 0.5 * mn + per * c * rounds_us(blocks * s, kCUs, t.alone, full)
+                        + ceil_div(blocks * s, kCUs) * (per * t.step_k * t.bn * scales_us)
+                        + (s > 1 ? 1.9 + s * slice_us : store_us);
       if (us < best) {
         best = us;
         plan->tile = t.tile;
@@ -269,19 +295,52 @@ double wr_plan_us(const LinearArgs& a, bool have_workspace, WrPlan* plan) {
     consider(1);
     if (!have_workspace) continue;
     // steps / s falls, the sums grow with s: least where the two are equal, or where the chip is full
-    int most = 256 / blocks < steps / 2 ? 256 / blocks : steps / 2;
+    int most = kCUs / blocks < steps / 2 ? kCUs / blocks : steps / 2;
     most = most < 16 ? most : 16;
     if (most < 2) continue;
-    const int s = (int)std::sqrt(steps * step_us / (8e-6 * a.m * a.n / 6.5));
+    const int s = (int)std::sqrt((steps * full * c + a.k * t.bn * scales_us) / slice_us);
     consider(s < 2 ? 2 : (s > most ? most : s));
-    if (s >= 2 && s < most) consider(s + 1);
+    if (s < most) {
+      consider(s < 2 ? 3 : s + 1);
+      consider(most);
+    }
   }
   return best;
+}
+
+// The same for gemm_core2 on the tiles and slices that launch_wq_variant takes above 64 rows.  It
+// expands a code once per block where gemm_wr does once per wave: what is expanded hardly matters, and
+// with 8-bit codes or a zero point and several tiles of rows it is the faster one (fp16 8-bit 700 x
+// 13824 x 5120: 130 us, 177 there).
+double wq_us(const LinearArgs& a, int splits) {
+  const double c = (has_zero_term(a) ? 1.06 : 0.97) * (a.k % 64 != 0 ? 1.18 : 1.0);
+  const int n128 = ceil_div(a.n, 128);
+  double round;
+  if (a.m > 128) {
+    const bool wide = splits == 1 && pick_tile_width(a.m, a.n, false) == 192;
+    const int blocks = ceil_div(a.m, 256) * (wide ? ceil_div(a.n, 192) : n128) * splits;
+    round = rounds_us(blocks, 256, wide ? 1.40 : 1.02, wide ? 1.73 : 1.24);
+  } else if (splits > 1) {
+    round = rounds_us(n128 * splits, 256, 0.53, 0.93);
+  } else if (n128 < 192) {
+    round = rounds_us(ceil_div(a.n, 32), 768, 0.43, 0.90);
+  } else {
+    round = rounds_us(n128, 512, 0.95, 1.30);
+  }
+  const double mn = 1e-6 * (double)a.m * a.n;
+  return 3.2 + 0.5 * mn + ceil_div(ceil_div(a.k, 64), splits) * c * round
+         + (splits > 1 ? 4.1 + splits * mn * (8 / 7.4 + (a.n % 8 != 0 ? 1.35 : 0.0))
+                       : (a.n % 8 != 0 ? 0.5 + 1.5 * mn : 0.0));
 }
 
 size_t wq_partial_bytes(const LinearArgs& a) {
   const int splits = wq_splits(a);
   return splits > 1 ? (size_t)splits * (size_t)a.m * (size_t)a.n * 4 : 0;
+}
+
+// what launch_gemm_wq uses for a problem that is not gemm_wr's: the converted weight, or fp32 sums
+size_t wq_bytes(const LinearArgs& a) {
+  return a.m >= 1024 ? (size_t)a.n * (size_t)a.k * 2 : wq_partial_bytes(a);
 }
 
 // fp32 sums of the slices in whole 32 x 32 tiles, rounded up to whole [m, n] matrices of them; never
@@ -297,19 +356,10 @@ size_t wr_partial_bytes(const LinearArgs& a, const WrPlan& plan) {
 
 }  // namespace
 
-// gemm_wr or gemm_core2 on its tile of 256 x 128, whose k-tile of 64 takes about 1.12 us: that one
-// converts a code once per block where gemm_wr does once per wave, so with bf16 zero points and several
-// tiles of rows it keeps up (m = 900, n = k = 4096: 53 us against 58).
 bool gemm_wr_plan(const LinearArgs& a, bool have_workspace, WrPlan* plan) {
   const double us = wr_plan_us(a, have_workspace, plan);
   if (us >= 1e30) return false;
-  if (a.m > 128) {
-    const int64_t s = have_workspace ? wq_splits(a) : 1;
-    const int64_t blocks = ((a.m + 255) / 256) * ((a.n + 127) / 128) * s;
-    const double rounds = (double)((blocks + 255) / 256);
-    if (4 + rounds * ((a.k + 63) / 64 / s) * 1.12 + slices_us(a, s) < us) return false;
-  }
-  return true;
+  return a.m <= 64 || us <= wq_us(a, have_workspace ? wq_splits(a) : 1);
 }
 
 // Two passes pay once m is large: the in-tile path converts every weight tile once per 256 rows
@@ -318,24 +368,26 @@ bool gemm_wr_plan(const LinearArgs& a, bool have_workspace, WrPlan* plan) {
 // for m > 8 (oneflow/core/functional/impl/quantization.cpp:341-350).
 size_t gemm_wq_workspace_bytes(const LinearArgs& a) {
   if (!gemm_wq_supported(a)) return 0;
-  if (a.m >= 1024) return (size_t)a.n * (size_t)a.k * 2;
   WrPlan plan;
-  if (gemm_wr_plan(a, true, &plan)) return wr_partial_bytes(a, plan);
-  return wq_partial_bytes(a);
+  return gemm_wr_plan(a, true, &plan) ? wr_partial_bytes(a, plan) : wq_bytes(a);
 }
 
-// The streaming kernel's rival for 16 < m <= 64: what gemm_wr is expected to take.
-double gemm_wr_us(const LinearArgs& a, bool have_workspace) {
-  WrPlan plan;
-  return wr_plan_us(a, have_workspace, &plan);
+// The streaming kernel's rival for 16 < m <= 64: what gemm_wr is expected to take, `two_launches` us more
+// if it slices K.
+double gemm_wr_us(const LinearArgs& a, bool have_workspace, double two_launches) {
+  WrPlan plan{kWr32x128, 1};
+  const double us = wr_plan_us(a, have_workspace, &plan);
+  return plan.splits > 1 ? us + two_launches : us;
 }
 
 int launch_gemm_wq(hipStream_t st, const LinearArgs& a, void* workspace, size_t workspace_bytes) {
-  const size_t need = gemm_wq_workspace_bytes(a);
+  WrPlan plan;
+  bool wr = gemm_wr_plan(a, true, &plan);
+  const size_t need = wr ? wr_partial_bytes(a, plan) : wq_bytes(a);
   const bool have_ws =
       need != 0 && workspace != nullptr && workspace_bytes >= need && ofq_aligned16(workspace);
-  WrPlan plan;
-  if (gemm_wr_plan(a, have_ws, &plan)) {
+  if (need != 0 && !have_ws) wr = gemm_wr_plan(a, false, &plan);
+  if (wr) {
     float* partials = static_cast<float*>(workspace);
     return a.t_dtype == OFQ_F16 ? launch_gemm_wr_f16(st, a, plan, partials)
                                 : launch_gemm_wr_bf16(st, a, plan, partials);

@@ -24,11 +24,12 @@
 // w~ = T(T(q) * s) + z with the reference's roundings (dequant_regs.h), products and sums in fp32 in
 // the matrix core, one rounding of the result.
 //
-// What bounds it: for tall tiles the matrix cores with the conversions in their shadow (a step of
-// 192 x 256 x 64 on symmetric fp16 4-bit codes: 0.88 us, 1.8 PFLOP/s over the chip; taken back to one
-// block of vector instructions behind the matrix instructions it took 1.05), for flat ones the fixed
-// 8 us of two launches, the pipeline's start and the partial sums.  Before and after (gemm_core2
-// above 64 rows, gemv_rows_mt below), us, fp16 4-bit:
+// What bounds it: for tall tiles the matrix cores with the conversions in their shadow and, once every CU
+// has a block, what the blocks share: a step of 192 x 256 x 64 on symmetric fp16 4-bit codes takes 0.72 us
+// in a block that is alone and 1.06 us in each of 256 (6.3 MFLOP a step: 1.5 PFLOP/s over the chip).  For
+// flat tiles the fixed 6 us of two launches and the pipeline's start, the scales (1.9 us per 4096 of them,
+// before the first step) and the partial sums.  The steps of every tile: wr_plan_us in gemm.hip.  Before
+// and after (gemm_core2 above 64 rows, gemv_rows_mt below), us, fp16 4-bit:
 //   64 x 4096 x 11008   28.2 -> 17.2     333 x 4096 x 11008          59.6 -> 47.7
 //   64 x 32000 x 4096   46.2 -> 28.1     640 x 8192 x 8192 (zero)   143.7 -> 107.9
 //   128 x 11008 x 4096  29.5 -> 23.7     900 x 11008 x 4096 (zero)  103.7 -> 88.4

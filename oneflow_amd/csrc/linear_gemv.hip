@@ -833,24 +833,37 @@ bool gemv_mt_supported(const LinearArgs& a) {
 
 }  // namespace
 
-// Every block of gemv_rows_mt reads all of x, from L2: that, with a part per weight tile, is the time
-// of a turn of its waves over their chunks (us, measured for n = 4096, 11008 and 32000 at m = 32 and
-// 64, within 15 %).  gemm_wr reads x once per 128 rows of weights but starts a second kernel where
-// it slices K; it has to win by 2.5 us, what its second launch costs the host and cold weights its
-// slices.  So long rows of weights leave the streaming kernel (64 x 4096 x 11008: 27.6 us here, 18 there) and
-// n = 11008 of k = 4096 stays (19.0 us here, 19.4 there).
+// Expected time of gemv_rows_mt in us, within 25 % of the measured one for 98 of 100 shapes (those of
+// wr_plan_us with up to 64 rows).  A round of blocks starts and ends (4.25, the scales, the output); a turn of
+// a block's waves over their chunks takes a part per tile of weights expanded, one per row of weights
+// read and one per row of x read (every block reads all of x, from L2).
+static double gemv_mt_us(const LinearArgs& a) {
+  const bool b4 = a.bits == 4;
+  const int nw = a.m <= 32 ? 12 : 8;
+  const int ck = b4 ? 128 : 64;
+  int rows = (int)((a.n + 255) / 256);
+  rows = rows < 16 ? 16 : (rows > 16 * kRowsMaxTiles ? 16 * kRowsMaxTiles : rows);
+  const int grid = (int)((a.n + rows - 1) / rows), tiles = (rows + 15) / 16;
+  const int turns = (int)(((a.k + ck - 1) / ck + nw - 1) / nw);
+  // bf16 with a zero point has the longest conversion
+  const double longer = b4 && a.t_dtype == OFQ_BF16 && !(a.symmetric && a.w_signed) ? 1.21 : 1.0;
+  const double turn_us = b4 ? 0.26 + (0.50 * tiles + 0.20 * rows / 16) * longer + 0.0020 * a.m * nw
+                            : 0.10 + 0.26 * tiles + 0.31 * rows / 16 + 0.0009 * a.m * nw;
+  const int rest = grid % 256, rounds = (grid + 255) / 256;
+  const double scales = (double)a.k / a.group_size * rows * (a.symmetric ? 1 : 2);
+  return rounds * (4.25 + 1.4 / 4096 * scales) - 0.8 + 2.3e-6 * a.m * a.n
+         + turns * turn_us * (grid / 256 + (rest != 0 ? 0.83 + 0.17 * rest / 256 : 0.0));
+}
+
+// gemm_wr reads x once per 128 rows of weights, but starts a second kernel where it slices K: so long
+// rows of weights leave the streaming kernel (64 x 4096 x 11008 fp16: 27.6 us here, 17.4 there) and n =
+// 11008 of k = 4096 stays (19.0 us here, 19.4 there).  Below 12.5 us the second launch and the workspace
+// have to be won back as well: there the host, 3 us for the two, is what bounds a call that is not replayed
+// from a graph.
 bool gemv_mt_preferred(const LinearArgs& a, bool have_workspace) {
   if (!gemv_mt_supported(a)) return false;
-  const int nw = a.m <= 32 ? 12 : 8;
-  const int ck = a.bits == 4 ? 128 : 64;
-  int64_t rows = (a.n + 255) / 256;
-  rows = rows < 16 ? 16 : (rows > 16 * kRowsMaxTiles ? 16 * kRowsMaxTiles : rows);
-  const int64_t grid = (a.n + rows - 1) / rows, tiles = (rows + 15) / 16;
-  const int64_t rounds = (grid + 255) / 256;
-  const int64_t turns = ((a.k + ck - 1) / ck + nw - 1) / nw;
-  double turn_us = a.bits == 4 ? 1.2 + 0.95 * tiles : 0.6 + 0.75 * tiles;
-  if (a.bits == 4 && a.t_dtype == OFQ_BF16 && !a.symmetric) turn_us *= 1.15;  // the longest conversion
-  return 2 + rounds * turns * turn_us < gemm_wr_us(a, have_workspace) + 2.5;
+  const double us = gemv_mt_us(a);
+  return us < gemm_wr_us(a, have_workspace, us < 12.5 ? 3.0 : 0.5);
 }
 
 int launch_gemv_mt(hipStream_t st, const LinearArgs& a) {
@@ -996,7 +1009,8 @@ extern "C" int ofq_fused_linear_gq(void* stream, const void* x, const void* w,
     const int rc = launch_gemv_wq(st, a);
     if (rc != OFQ_ERR_UNSUPPORTED) return rc;  // e.g. bf16 with an x too large to stage
   }
-  if (a.m > 16 && gemv_mt_preferred(a, workspace != nullptr && workspace_bytes >= gemm_wq_workspace_bytes(a))) {
+  if (a.m > 16 && a.m <= 64
+      && gemv_mt_preferred(a, workspace != nullptr && workspace_bytes >= gemm_wq_workspace_bytes(a))) {
     const int rc = launch_gemv_mt(st, a);
     if (rc != OFQ_ERR_UNSUPPORTED) return rc;
   }

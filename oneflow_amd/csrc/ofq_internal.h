@@ -41,8 +41,9 @@ struct WrPlan {
 // the plan that launch_gemm_wq takes with a workspace of gemm_wq_workspace_bytes() or without one (then of
 // one slice); false: not this kernel's problem
 bool gemm_wr_plan(const LinearArgs& a, bool have_workspace, WrPlan* plan);
-// expected time (us; 1e30: not this kernel's problem) of a problem of 16 < m <= 64 on it
-double gemm_wr_us(const LinearArgs& a, bool have_workspace);
+// expected time (us; 1e30: not this kernel's problem) of a problem of 16 < m <= 64 on it, with two_launches
+// added if it takes two
+double gemm_wr_us(const LinearArgs& a, bool have_workspace, double two_launches);
 int launch_gemm_wr_f16(hipStream_t st, const LinearArgs& a, const WrPlan& plan, float* partials);
 int launch_gemm_wr_bf16(hipStream_t st, const LinearArgs& a, const WrPlan& plan, float* partials);
 
