@@ -229,9 +229,11 @@ gemm_wr(WrParams p) {
 #pragma unroll
   for (int t = 0; t < NSTAGE - 1; ++t) issue(t, t);
 
-  // ---- scales of the block's columns in LDS, [group][column] -----------------------------------
+  // ---- scales of the block's columns in LDS, [group][column], and a row of zeros behind them: the scale
+  //      past the end of K, where x is zero but a code might overflow T under a group's scale, and
+  //      infinity times zero is NaN ------------------------------------------------------------------
   uint16_t* sl = reinterpret_cast<uint16_t*>(smem + NSTAGE * kStage);
-  uint16_t* zl = sl + p.panel_groups * BN;
+  uint16_t* zl = sl + (p.panel_groups + 1) * BN;
   int g0 = 0, ng = 0;  // groups in the panel
   auto group_of = [&](int k) { return (int)__umulhi((uint32_t)k, p.group_magic); };
   auto fill_panel = [&](int t) {
@@ -241,6 +243,10 @@ gemm_wr(WrParams p) {
     copy_scale_panel<NT, ZMODE == 2, true>(p.scale + (int64_t)n0 * p.G + g0,
                                            p.zero + (int64_t)n0 * p.G + g0, p.G, BN, p.N - n0, ng,
                                            BN, sl, zl, tid);
+    if (RAGGED && tid < BN) {
+      sl[p.panel_groups * BN + tid] = 0;
+      if (ZMODE == 2) zl[p.panel_groups * BN + tid] = 0;
+    }
     __syncthreads();
   };
 
@@ -268,18 +274,11 @@ gemm_wr(WrParams p) {
     const uint8_t* cp = smem + buf * kStage + kXBytes + wave * (kCodeOps * 1024) + lane * 16;
 #pragma unroll
     for (int o = 0; o < kCodeOps; ++o) dst[o] = *reinterpret_cast<const u32x4*>(cp + o * 1024);
-    const int k = (step0 + t) * (KH * 64) + kh * 64 + half * 32;
-    int g = group_of(k) - g0;
-    g = g < ng ? g : 0;  // (past the panel or K: not used, or the zero scale below)
+    int g = group_of((step0 + t) * (KH * 64) + kh * 64 + half * 32) - g0;
+    g = g < ng ? g : (RAGGED ? p.panel_groups : 0);  // (past the panel: not used)
     sd = TT<T>::load(reinterpret_cast<const S*>(sl) + g * BN + col);
     zd = 0.f;
     if (ZMODE == 2) zd = TT<T>::load(reinterpret_cast<const S*>(zl) + g * BN + col);
-    if (RAGGED && k >= p.K) {
-      // w~ = 0 past the end of a row: x is zero there too, but zero times a code that overflows T
-      // under somebody's scale would be NaN
-      sd = 0.f;
-      zd = 0.f;
-    }
     if (ZMODE == 1) zd = TT<T>::round(-(float)((1 << (BITS - 1)) - 1) * sd);
   };
   auto read_x = [&](int buf, int j, u32x4 (&dst)[TM]) {

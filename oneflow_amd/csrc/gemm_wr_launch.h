@@ -48,7 +48,7 @@ int launch_wr_cfg(hipStream_t st, const LinearArgs& a, const WrPlan& plan, float
     int64_t groups = (int64_t)p.panel_steps * kStepK / a.group_size + 2;
     if (groups > p.G) groups = p.G;
     p.panel_groups = (int)groups;
-    lds = kStages + (size_t)groups * per_group;
+    lds = kStages + (size_t)(groups + 1) * per_group;  // and the row of zeros
     if (lds <= 160u * 1024u) break;
     if (p.panel_steps == 1) return OFQ_ERR_UNSUPPORTED;
     p.panel_steps = (p.panel_steps + 1) / 2;
