@@ -286,10 +286,6 @@ struct B2Copy {
   static __device__ __forceinline__ void store_part(const Params&, const Regs&, uint8_t*, int, int) {}
 };
 
-__device__ const uint16_t kZero16[1] = {0};
-// (said to be global memory, or a choice between two of them becomes a flat load)
-typedef const __attribute__((address_space(1))) uint16_t* GlobalU16;
-
 // Groupwise-quantised weights: codes are loaded as stored
 // ([N, K*bits/8] bytes) two k-tiles ahead, and turned into T when written to the swizzled LDS tile.
 template<bool RAGGED, typename T, int BITS, bool SIGNED, int ZMODE, int BN, int NT>
@@ -312,9 +308,11 @@ struct B2Dequant {
     typedef typename std::conditional<BITS == 4 && ZMODE == 0, uint16_t, uint32_t>::type Slot;
     Slot s[kChunks];
     Slot z[kChunks];
+    uint32_t past;  // RAGGED: bit i, chunk i lies past the end of its row
   };
   static __device__ __forceinline__ void load(const Params& p, int n0, int kt, int, int, int tid,
                                               Regs& r, uint8_t*) {
+    if (RAGGED) r.past = 0;
 #pragma unroll
     for (int i = 0; i < kChunks; ++i) {
       const int q = tid + i * NT;
@@ -322,15 +320,15 @@ struct B2Dequant {
       int row = n0 + q / kChunksPerRow;
       row = row < p.N ? row : p.N - 1;
       const int c = q % kChunksPerRow;
-      // past the end of a ragged row: its first chunk again with a scale of zero (x is zero there too,
-      // but zero times a code that overflows T under its scale would be NaN)
+      // past the end of a ragged row: its first chunk again, expanded with a scale of zero
       const int byte = kt * kCodeBytesPerRow + c * 16;
       const bool in_row = !RAGGED || byte < (int)p.ldw;
+      if (RAGGED && !in_row) r.past |= 1u << i;
       r.v[i] = *reinterpret_cast<const u32x4*>(p.w + (int64_t)row * p.ldw + (in_row ? byte : 0));
       const int k = in_row ? kt * 64 + c * kElemsPerChunk : 0;
       const int64_t si = (int64_t)row * p.G + k / p.group_size;
-      r.s[i] = *(in_row ? (GlobalU16)(p.scale + si) : (GlobalU16)kZero16);
-      if (ZMODE == 2) r.z[i] = *(in_row ? (GlobalU16)(p.zero + si) : (GlobalU16)kZero16);
+      r.s[i] = reinterpret_cast<const uint16_t*>(p.scale)[si];
+      if (ZMODE == 2) r.z[i] = reinterpret_cast<const uint16_t*>(p.zero)[si];
     }
   }
   // dequantise and store a quarter of the thread's chunks (all of them when there are fewer)
@@ -345,9 +343,14 @@ struct B2Dequant {
       const int c = q % kChunksPerRow;
       uint8_t* rowp = lds + row * kStageRow;
       const int sw = swizzle_key(row);
-      const float sc = raw16_to_float<T>((uint16_t)r.s[i]);
+      float sc = raw16_to_float<T>((uint16_t)r.s[i]);
       float zc = 0.f;
       if (ZMODE == 2) zc = raw16_to_float<T>((uint16_t)r.z[i]);
+      if (RAGGED && (r.past >> i & 1u) != 0) {
+        // w~ = 0: x is zero there too, but zero times a code that overflows T under its scale is NaN
+        sc = 0.f;
+        zc = 0.f;
+      }
       if (ZMODE == 1) zc = TT<T>::round(-(float)((1 << (BITS - 1)) - 1) * sc);
       if constexpr (BITS == 8) {
         u32x4 o0, o1;
