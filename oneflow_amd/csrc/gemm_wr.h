@@ -136,10 +136,9 @@ gemm_wr(WrParams p) {
   constexpr int kCodeOps = kCB / 32;                 // copies of a wave's codes per step
   constexpr int kXBytes = BM * kStageRow * KH;
   constexpr int kStage = (int)wr_stage_bytes<BITS, TM, WN, KH>();
-  // copies of x per step: KH * TM * 4 of 1 KB over W waves, the first kXRem of which take one more
-  constexpr int kXAll = kXBytes / 1024;
-  constexpr int kXMin = kXAll / W, kXRem = kXAll % W;
-  constexpr int kXOps = kXMin + (kXRem != 0 ? 1 : 0);
+  // copies of x per step: KH * TM * 4 of 1 KB over W waves
+  static_assert(kXBytes % (W * 1024) == 0, "every wave issues as many copies: its waits are one constant");
+  constexpr int kXOps = kXBytes / (W * 1024);
   constexpr int kOps = kXOps + kCodeOps;
   // vector instructions between two matrix instructions: a quarter step's conversion over TM slots
   constexpr int kDequant = TT<T>::dtype == OFQ_BF16 ? (ZMODE == 0 ? 26 : 46) : (ZMODE == 0 ? 22 : 26);
@@ -179,7 +178,7 @@ gemm_wr(WrParams p) {
   int xk[kXOps];  // byte of the row within the step
 #pragma unroll
   for (int o = 0; o < kXOps; ++o) {
-    const int q = o * W + wave < kXAll ? o * W + wave : 0;
+    const int q = o * W + wave;
     const int sub = q / (BM / 8);                 // which 64-element piece of the step
     const int rel = (q % (BM / 8)) * 8 + (lane >> 3);
     int row = m0 + rel;
@@ -206,7 +205,6 @@ gemm_wr(WrParams p) {
     const uint32_t st = lds0 + (uint32_t)buf * kStage;
     if (o < kXOps) {
       const int q = o * W + wave;
-      if (kXRem != 0 && o == kXMin && wave >= kXRem) return;
       const uint8_t* src = wr_uniform(xbase + (int64_t)gs * (kStageRow * KH));
       if (!RAGGED || gs * (kStageRow * KH) + xk[o] < K2) {
         async_copy16_unordered(src, xoff[o], st + q * 1024);
@@ -297,10 +295,8 @@ gemm_wr(WrParams p) {
   auto step = [&](int t) {
     // stages up to t + 1 are complete: all but the copies of the NSTAGE - 3 younger ones (none may be
     // left in flight where a ragged K's last stage has fewer copies)
-    if (RAGGED || NSTAGE == 3) {
+    if (RAGGED) {
       wr_wait_and_barrier<0>();
-    } else if (kXRem != 0 && wave >= kXRem) {
-      wr_wait_and_barrier<(kOps - 1) * (NSTAGE - 3)>();
     } else {
       wr_wait_and_barrier<kOps * (NSTAGE - 3)>();
     }
