@@ -343,15 +343,13 @@ size_t wq_bytes(const LinearArgs& a) {
   return a.m >= 1024 ? (size_t)a.n * (size_t)a.k * 2 : wq_partial_bytes(a);
 }
 
-// fp32 sums of the slices in whole 32 x 32 tiles, rounded up to whole [m, n] matrices of them; never
-// less than what gemm_core2's slices take, so that a problem that has few tiles has a workspace
+// fp32 sums of the slices in whole 32 x 32 tiles, rounded up to whole [m, n] matrices: the unit in which
+// the query has always counted slices
 size_t wr_partial_bytes(const LinearArgs& a, const WrPlan& plan) {
+  if (plan.splits == 1) return 0;
   const size_t mn = (size_t)a.m * (size_t)a.n * 4;
-  const size_t least = a.m > 64 ? wq_partial_bytes(a) : 0;
-  if (plan.splits == 1) return least;
-  const size_t tiles = (size_t)plan.splits * ((a.m + 31) / 32) * ((a.n + 31) / 32) * 4096;
-  const size_t need = (tiles + mn - 1) / mn * mn;
-  return need > least ? need : least;
+  const size_t tiles = (size_t)plan.splits * ceil_div(a.m, 32) * ceil_div(a.n, 32) * 4096;
+  return (tiles + mn - 1) / mn * mn;
 }
 
 }  // namespace

@@ -59,3 +59,20 @@ def test_with_a_workspace_no_slice_is_empty(m):
             steps = -(-k // step)
             per = -(-steps // plan.splits)
             assert (plan.splits - 1) * per < steps
+
+
+@pytest.mark.parametrize("m", [17, 64, 65, 200, 1000])
+@pytest.mark.parametrize("n,k", [(600, 1024), (4096, 11008), (32000, 4096), (11008, 4096), (1001, 2112)])
+def test_the_workspace_is_what_the_slices_take(m, n, k):
+    """No slices, no workspace; else whole 32 x 32 tiles of fp32 sums and less than one [m, n] more."""
+    for bits, symmetric in ((4, True), (8, False)):
+        plan = _plan(m, n, k, bits, symmetric, _lib.F16, workspace=True, group=32)
+        if plan is None:
+            continue
+        need = _lib.lib().ofq_fused_linear_gq_workspace_bytes(
+            _lib.I8 if symmetric else _lib.U8, _lib.F16, bits, symmetric, 1, 32, m, n, k)
+        if need == 0:  # one slice, or left to the streaming kernel
+            assert plan.splits == 1 or m <= 64
+            continue
+        tiles = plan.splits * -(-m // 32) * -(-n // 32) * 4096
+        assert plan.splits > 1 and tiles <= need < tiles + 4 * m * n, (m, n, k, plan.splits, need)
