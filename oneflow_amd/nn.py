@@ -197,6 +197,14 @@ class QuantizedLinear(torch.nn.Module):
                 f"num_bits={self.num_bits}, symmetric={self.symmetric}, group_size={self.group_size}")
 
 
+def _packed(m):
+    """(weight, weight_scale, weight_zero, bias) of a ``QuantizedLinear`` or of any object with these
+    attributes (``weight_zero`` only if it is not symmetric)."""
+    if isinstance(m, QuantizedLinear):
+        return m._packed()
+    return m.weight, m.weight_scale, getattr(m, "weight_zero", None), m.bias
+
+
 class QuantizedGLU(torch.nn.Module):
     """``y = (x W^T + b) * act(x V^T + c)`` over two ``QuantizedLinear`` weights of equal shape
     (``hidden`` = W, b and ``gate`` = V, c) through ``_C.fused_glu_with_groupwise_quantized_weight``
@@ -217,10 +225,11 @@ class QuantizedGLU(torch.nn.Module):
                    QuantizedLinear.from_float(gate_linear, **quant_args), activation)
 
     def forward(self, x):
-        modules = self._modules
-        h, g = modules["hidden"], modules["gate"]
-        w, w_scale, w_zero, b = h._packed()
-        v, v_scale, v_zero, c = g._packed()
+        modules = self._modules  # (Module.__getattr__ costs 0.4 us; a member need not be a module)
+        h = modules["hidden"] if "hidden" in modules else self.hidden
+        g = modules["gate"] if "gate" in modules else self.gate
+        w, w_scale, w_zero, b = _packed(h)
+        v, v_scale, v_zero, c = _packed(g)
         return _native.fused_glu(x, w, w_scale, w_zero, b, v, v_scale, v_zero, c, self.activation,
                                  h.num_bits, h.symmetric, 1, h.group_size)
 
@@ -239,8 +248,9 @@ class GroupedQuantizedLinear(torch.nn.Module):
         self.linears = torch.nn.ModuleList(linears)
 
     def forward(self, x):
-        ls = list(self._modules["linears"]._modules.values())
-        ws, scales, zeros, biases = zip(*[m._packed() for m in ls])
+        modules = self._modules
+        ls = list(modules["linears"] if "linears" in modules else self.linears)
+        ws, scales, zeros, biases = zip(*[_packed(m) for m in ls])
         if any(b is None for b in biases):
             if not all(b is None for b in biases):
                 raise ValueError("either every linear has a bias or none")

@@ -164,3 +164,32 @@ def test_quantized_linear_drops_a_stale_decode_copy():
     mod._set_decode_copy(fake)
     mod.weight = torch.ones_like(mod.weight)   # reassigned
     assert mod._decode_copy() is None
+
+
+class _Packed(torch.nn.Module):
+    """What a member of QuantizedGLU / GroupedQuantizedLinear has to have, and nothing more."""
+
+    in_features, out_features, num_bits, symmetric, group_size = 64, 8, 8, True, 64
+
+    def __init__(self):
+        super().__init__()
+        self.weight, self.weight_scale = _w(dtype=torch.int8), torch.ones((8, 1), dtype=torch.float16)
+        self.bias = None
+
+
+def test_modules_take_members_of_other_classes():
+    x = torch.zeros((2, 64), dtype=torch.float16)
+    plain = type("Plain", (), {k: v for k, v in vars(_Packed).items() if k[0] != "_"})()
+    for k, v in vars(_Packed()).items():
+        if k in ("weight", "weight_scale", "bias"):
+            setattr(plain, k, v)
+    for hidden, gate in ((_Packed(), _Packed()), (plain, plain)):
+        # every attribute has been found when the native function refuses tensors of the CPU
+        with pytest.raises(CheckFailedError, match="tensors must live on the GPU"):
+            flow.nn.QuantizedGLU(hidden, gate)(x)
+    grouped = flow.nn.GroupedQuantizedLinear([_Packed(), _Packed()])
+    with pytest.raises(CheckFailedError, match="tensors must live on the GPU"):
+        grouped(x)
+    grouped.linears = torch.nn.Sequential(_Packed())
+    with pytest.raises(CheckFailedError, match="tensors must live on the GPU"):
+        grouped(x)
