@@ -69,6 +69,16 @@ int launch_plain(hipStream_t st, const LinearArgs& a, const void* wt) {
     return launch_core2<MF, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
                                                                   a.n, (a.k + 63) / 64);
   }
+  if constexpr (RG) {  // (why: launch_pp)
+    if (width == 192) {
+      return launch_core2<MF, B2Copy<RG, 192, 512>, EP, 256, 192, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
+                                                                    a.n, (a.k + 63) / 64);
+    }
+    if (width == 256) {
+      return launch_core2<MF, B2Copy<RG, 256, 512>, EP, 256, 256, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
+                                                                    a.n, (a.k + 63) / 64);
+    }
+  }
   return std::is_same<T, f16>::value
              ? launch_gemm_pp_f16(st, a.x, wt, a.bias, a.out, a.m, a.n, a.k, width)
              : launch_gemm_pp_bf16(st, a.x, wt, a.bias, a.out, a.m, a.n, a.k, width);
@@ -636,6 +646,11 @@ int launch_mq(hipStream_t st, const void* a, const BCopyParams& bp, const float*
   const int width = pick_tile_width(m, n, true);
   if (width == 128) {
     return launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a, k, bp, ep, m, n, kt);
+  }
+  if constexpr (RG) {  // (why: launch_pp)
+    if (width == 192) {
+      return launch_core2<MfmaI8, B2Copy<RG, 192, 512>, EP, 256, 192, 4, 2>(st, a, k, bp, ep, m, n, kt);
+    }
   }
   return launch_gemm_pp_i8(st, a, bp.b, a_scale, b_scale, bias, out, TT<T>::dtype, m, n, k, width);
 }

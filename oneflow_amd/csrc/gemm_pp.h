@@ -182,25 +182,37 @@ int launch_pp_tile(hipStream_t st, const void* a, const void* b, int64_t row_byt
   return ofq_check_launch();
 }
 
-// width: what pick_tile_width says, 192 or more.  Tiles of 128 columns stay with gemm_core2: a slot
-// of four matrix instructions here is too short for the fetch beside it (1100 x 4096 x 4096: int8 33.3 us
-// there, 35.2 here, bf16 57.3 and 60.9; two k-steps a slot here, which at 192 and 256 columns is slower
-// than one: bf16 1024 x 11008 x 4096 82.0 against 78.2).  gemm_core2 against this kernel in bf16:
-// 192 columns 1024 x 11008 x 4096 80.4 -> 78.2, 256 columns 4096 x 4096 x 4096 107.8 -> 105.0,
-// 384 columns 4096 x 5000 x 4096 140.2 -> 134.9.
+// width: what pick_tile_width says.  This kernel against gemm_core2, time over time in the mean of 1200 random
+// problems (m to 8192, n to 32000, k to 14336; p. 95 is 2 to 5 % above the mean):
+//              rows of whole k-tiles: up to 16, 48, more    ragged rows: the same
+//   int8  192    0.99  0.99  0.98                           1.01  1.02  1.05
+//         256    0.98  0.97  0.93                           0.99  1.00  1.01
+//         384    0.98  0.97  0.94                           0.94  0.86  0.85
+//   fp16  192    0.99  0.98  0.97                           1.03  1.05  1.07
+//         256    0.99  0.97  0.95                           1.00  1.01  1.03
+//         384    0.99  0.97  0.95                           0.93  0.85  0.82
+//   bf16  192    1.00  0.99  0.96                           1.03  1.04  1.06
+//         256    0.99  0.96  0.94                           1.00  1.01  1.05
+//         384    0.98  0.97  0.95                           0.92  0.85  0.81
+// So ragged rows at 192 columns, and at 256 in 16 bits, stay with gemm_core2 (whose kernel for ragged rows
+// runs out of registers at 384 columns and nowhere else).  So do tiles of 128 columns: a slot of four
+// matrix instructions is too short for the fetch beside it (1100 x 4096 x 4096: int8 33.3 us there, 35.2
+// here, bf16 57.3 and 60.9).
 template<class MF, class EP>
 int launch_pp(hipStream_t st, const void* a, const void* b, int64_t row_bytes,
               const typename EP::Params& ep, int64_t M, int64_t N, int width) {
-#define OFQ_PP(BN)                                                                     \
-  return row_bytes % kStageRow != 0                                                    \
-             ? launch_pp_tile<MF, true, EP, BN>(st, a, b, row_bytes, ep, M, N)         \
-             : launch_pp_tile<MF, false, EP, BN>(st, a, b, row_bytes, ep, M, N)
-  switch (width) {
-    case 384: OFQ_PP(384);
-    case 256: OFQ_PP(256);
-    default: OFQ_PP(192);
+  constexpr bool kInt8 = std::is_same<MF, MfmaI8>::value;
+  const bool ragged = row_bytes % kStageRow != 0;
+  if (width == 384) {
+    return ragged ? launch_pp_tile<MF, true, EP, 384>(st, a, b, row_bytes, ep, M, N)
+                  : launch_pp_tile<MF, false, EP, 384>(st, a, b, row_bytes, ep, M, N);
   }
-#undef OFQ_PP
+  if (width == 256) {
+    if (!ragged) return launch_pp_tile<MF, false, EP, 256>(st, a, b, row_bytes, ep, M, N);
+    if constexpr (kInt8) return launch_pp_tile<MF, true, EP, 256>(st, a, b, row_bytes, ep, M, N);
+  }
+  if (width == 192 && !ragged) return launch_pp_tile<MF, false, EP, 192>(st, a, b, row_bytes, ep, M, N);
+  return OFQ_ERR_UNSUPPORTED;
 }
 
 }  // namespace

@@ -47,8 +47,9 @@ double gemm_wr_us(const LinearArgs& a, bool have_workspace, double two_launches)
 int launch_gemm_wr_f16(hipStream_t st, const LinearArgs& a, const WrPlan& plan, float* partials);
 int launch_gemm_wr_bf16(hipStream_t st, const LinearArgs& a, const WrPlan& plan, float* partials);
 
-// Copy-fed GEMMs for more than 128 rows (gemm_pp.h) on tiles of 256 x width (192, 256 or 384); the linear's with the
-// weight already in the dtype of x.
+// Copy-fed GEMMs for more than 128 rows (gemm_pp.h) on tiles of 256 x width (384, 256 or 192; rows that are
+// not a multiple of 128 bytes 384 only, or 256 in int8); the linear's with the weight already in the dtype
+// of x.
 int launch_gemm_pp_f16(hipStream_t st, const void* x, const void* w, const void* bias, void* out,
                        int64_t m, int64_t n, int64_t k, int width);
 int launch_gemm_pp_bf16(hipStream_t st, const void* x, const void* w, const void* bias, void* out,
