@@ -354,12 +354,15 @@ size_t wq_bytes(const LinearArgs& a) {
 }
 
 // fp32 sums of the slices in whole 32 x 32 tiles, rounded up to whole [m, n] matrices: the unit in which
-// the query has always counted slices
+// the query has always counted slices.  Above 64 rows never less than gemm_core2's slices take, the size
+// that callers know for these problems.
 size_t wr_partial_bytes(const LinearArgs& a, const WrPlan& plan) {
   if (plan.splits == 1) return 0;
   const size_t mn = (size_t)a.m * (size_t)a.n * 4;
   const size_t tiles = (size_t)plan.splits * ceil_div(a.m, 32) * ceil_div(a.n, 32) * 4096;
-  return (tiles + mn - 1) / mn * mn;
+  const size_t need = (tiles + mn - 1) / mn * mn;
+  const size_t known = a.m > 64 ? wq_partial_bytes(a) : 0;
+  return need > known ? need : known;
 }
 
 }  // namespace
