@@ -8,10 +8,11 @@
 //       dequantised once and a copy-fed GEMM runs on it;
 //   (2) matmul_quant: int8 x int8 -> int32 MFMA with a per-row/per-tensor scale epilogue.
 //
-// All are instances of one byte-oriented core (gemm_kernels.h).  A tile row is always 128 bytes
-// of K (64 fp16/bf16 or 128 int8 elements), a k-step of the 32x32 MFMA consumes 32 of those bytes
-// per row (16 bytes per lane), so the same LDS layout and fragment addressing serve every type.
-// This file only picks tile shapes and fills parameter blocks.
+// Three kernels share one layout: a tile row is always 128 bytes of K (64 fp16/bf16 or 128 int8
+// elements), a k-step of the 32x32 MFMA consumes 32 of those bytes per row (16 bytes per lane), whatever
+// the type.  gemm_core2 (gemm_kernels.h) serves both operations, gemm_pp (gemm_pp.h) their copy-fed
+// tiles of 256 rows, gemm_wr (gemm_wr.h) 17 to 1023 rows with the weights packed up to the registers.
+// This file only chooses kernel, tile and slices and fills parameter blocks.
 #include <cmath>
 
 #include "gemm_kernels.h"

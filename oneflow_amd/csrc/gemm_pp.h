@@ -46,12 +46,13 @@ __device__ __forceinline__ void copy_pieces(const uint8_t* __restrict__ a_kt,
 // (group 0 in its last multiplying slot, group 1 in its last fetching one).
 //
 // What bounds it: the clock that the chip gives matrix instructions on random operands, then the copies.
-// 8192 x 11008 x 4096, 256 x 384 tiles, kernel alone: int8 314 us (2.36 PTOP/s; groups in step 365, no
-// copies 290, no epilogue 277, neither fetches nor copies 270), bf16 550 us (1.35 PFLOP/s; no copies 454,
-// no fetches 525, no epilogue 526).  2048 rows: int8 82 us (in step 97), bf16 141.  Measured and not
-// taken: waves of 128 x 96 (fewer LDS reads: 314 / 563 us), copies spread over more slots (312 / 558) or
-// requested before the fetches (320 / 564), rows of 64 bytes in a ring of four stages (three in flight:
-// 355 / 621, half lines cost more than the distance gives), non-temporal stores (within 1.5 %).
+// 8192 x 11008 x 4096 on 256 x 384 tiles, launches in a row: int8 341 us (2.17 POP/s; gemm_core2 371), bf16
+// 572 us (1.29 PFLOP/s; 646); 2048 rows: int8 87 us (89), bf16 146 (150); among a pass's other kernels 374
+// and 163.  Taken apart when it was built, in runs whose whole took int8 314 us and bf16 550: groups in
+// step 365, no copies 290 / 454, no epilogue 277 / 526, no fetches - / 525, neither fetches nor copies 270.
+// In the same runs, and not taken: waves of 128 x 96 (fewer LDS reads: 314 / 563), copies spread over more
+// slots (312 / 558) or requested before the fetches (320 / 564), rows of 64 bytes in a ring of four stages
+// (three in flight: 355 / 621, half lines cost more than the distance gives), non-temporal stores (1.5 %).
 template<class MF, bool RAGGED, class EP, int BN>
 __global__ void __launch_bounds__(512)
 gemm_pp(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int64_t ld,

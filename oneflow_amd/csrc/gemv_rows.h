@@ -340,9 +340,12 @@ gemv_rows_grouped(GemvGroup g, int M, int K, int group_size, int gs_shift, int r
 // c = wave, wave + NWAVES, ... and, per chunk, every 16-row weight tile of the block.  Sums stay in
 // registers and are folded through LDS one weight tile at a time.  No barrier inside the k loop.
 //
-// What bounds it: every block reads all of x from L2, 256 * m * k * 2 bytes at about 11 TB/s, so the
-// time follows the chunks per wave (64 x 4096 x 11008 fp16: 27.6 us for 23 MB of weights); the dispatch
-// leaves long rows of weights to gemm_wr for that.  Everything a chunk needs, its MT * 16 rows x 2 CK
+// What bounds it: no unit of the chip, but two waves a SIMD that wait.  At 48 x 11008 x 4096 (fp16, zero
+// point, 17.9 us) a wave waits for memory 36 % of its life and for an issue slot 33 %; the vector units are
+// busy 42 % of the time, LDS 23 %, the matrix cores 12 %, and L2 hands out about 9 TB/s (every block reads all
+// of x: 100 MB).  A chunk costs a wave its turn through request, LDS, conversion and product whatever m
+// is, so the time follows the chunks per wave (64 x 4096 x 11008 fp16: 27.6 us for 23 MB of weights); the
+// dispatch leaves long rows of weights to gemm_wr for that.  Everything a chunk needs, its MT * 16 rows x 2 CK
 // bytes of x and its NTL weight tiles, is requested while the chunk before is worked on (one weight tile
 // in flight took 20.3 us at 64 x 11008 x 4096 where this takes 19.0, and 26.1 against 21.2 at 48 rows
 // of 8-bit codes).  The requests are unconditional and straight line (a tile past the block's rows

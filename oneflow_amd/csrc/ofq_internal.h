@@ -24,9 +24,9 @@ struct LinearArgs {
 
 // MFMA GEMM with in-tile dequantisation; groups along K.  Returns OFQ_ERR_UNSUPPORTED when the
 // shape does not meet the kernel's tiling constraints (caller falls back).
-// With a workspace of gemm_wq_workspace_bytes() (non-zero for large m only) the weight is
-// dequantised once into it and a copy-fed GEMM runs on the result; without one the in-tile path
-// is used.
+// With a workspace of gemm_wq_workspace_bytes() K is cut into slices (m < 1024, where the tiles do not fill
+// the chip) or the weight is dequantised once into it and a copy-fed GEMM runs on the result (from 1024
+// rows on); without one a block walks all of K, on packed weights.
 bool gemm_wq_supported(const LinearArgs& a);
 size_t gemm_wq_workspace_bytes(const LinearArgs& a);
 int launch_gemm_wq(hipStream_t st, const LinearArgs& a, void* workspace, size_t workspace_bytes);
@@ -78,8 +78,8 @@ int launch_gemv_m1_any(hipStream_t st, const LinearArgs& a);
 bool gemv_wq_supported(const LinearArgs& a);
 int launch_gemv_wq(hipStream_t st, const LinearArgs& a);
 
-// 16 < m <= 64 without a workspace: the decode kernel's row split with several 16-row tiles of x
-// per weight tile.  Not where gemm_wr is expected to take clearly less.
+// 16 < m <= 64: the decode kernel's row split with several 16-row tiles of x per weight tile, without a
+// workspace.  Not where gemm_wr is expected to take less.
 bool gemv_mt_preferred(const LinearArgs& a, bool have_workspace);
 int launch_gemv_mt(hipStream_t st, const LinearArgs& a);
 
