@@ -833,7 +833,7 @@ bool gemv_mt_supported(const LinearArgs& a) {
 
 }  // namespace
 
-// Expected time of gemv_rows_mt in us, within 25 % of the measured one for 98 of 100 shapes (those of
+// Expected time of gemv_rows_mt in us, within 27 % of the measured one for 98 of 100 shapes (those of
 // wr_plan_us with up to 64 rows).  A round of blocks starts and ends (4.25, the scales, the output); a turn of
 // a block's waves over their chunks takes a part per tile of weights expanded, one per row of weights
 // read and one per row of x read (every block reads all of x, from L2).
