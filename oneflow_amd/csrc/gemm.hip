@@ -89,39 +89,52 @@ int launch_plain(hipStream_t st, const LinearArgs& a, const void* wt) {
 // slices that run as separate blocks, each writing fp32 partial sums of the whole output tile to
 // its slice of the workspace; splitk_finalize adds the slices in order (so the result does not
 // depend on scheduling), adds the bias and rounds to T once.
-template<typename T, int VEC>
+//
+// Four outputs a thread at a flat index of [M, N], the last thread's four end with the last output (M N >= 4;
+// what two threads compute is the same).  Rows of N and slices of M N elements begin at any element.
+template<typename V, typename E>
+__device__ __forceinline__ V sum_slices4(const E* __restrict__ part, int64_t MN, int splits) {
+  typedef V any __attribute__((aligned(4)));
+  constexpr int U = 4;  // slices requested together
+  V sum = *reinterpret_cast<const any*>(part);
+  for (int s0 = 1; s0 < splits; s0 += U) {
+    V v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      v[u] = *reinterpret_cast<const any*>(part + (int64_t)(s0 + u < splits ? s0 + u : splits - 1) * MN);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (s0 + u < splits) sum += v[u];
+  }
+  return sum;
+}
+template<typename T, typename F>
+__device__ __forceinline__ void store_folded4(typename TT<T>::storage* __restrict__ out, int n, int N,
+                                              F value) {
+  typename TT<T>::storage o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    TT<T>::store(&o[e], value(e, n));
+    if (++n == N) n = 0;
+  }
+  if constexpr (sizeof(o) == 8) {
+    *reinterpret_cast<u32x2_any*>(out) = *reinterpret_cast<const u32x2*>(o);
+  } else {
+    *reinterpret_cast<u32x4_any*>(out) = *reinterpret_cast<const u32x4*>(o);
+  }
+}
+
+template<typename T>
 __global__ void __launch_bounds__(256)
 splitk_finalize(const float* __restrict__ part, const typename TT<T>::storage* __restrict__ bias,
-                typename TT<T>::storage* __restrict__ out, int64_t MN, int N, int splits) {
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VEC;
+                typename TT<T>::storage* __restrict__ out, uint32_t MN, uint32_t N, int splits) {
+  uint32_t i = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= MN) return;
-  float acc[VEC];
-  if constexpr (VEC == 4) {
-    const f32x4 v = *reinterpret_cast<const f32x4*>(part + i);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] = v[e];
-    for (int sidx = 1; sidx < splits; ++sidx) {
-      const f32x4 u = *reinterpret_cast<const f32x4*>(part + (int64_t)sidx * MN + i);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] += u[e];
-    }
-  } else {
-    acc[0] = part[i];
-    for (int sidx = 1; sidx < splits; ++sidx) acc[0] += part[(int64_t)sidx * MN + i];
-  }
-  const int n = (int)(i % N);  // VEC divides N: the VEC elements share a row
-  typename TT<T>::storage o[VEC];
-#pragma unroll
-  for (int e = 0; e < VEC; ++e) {
-    float v = acc[e];
-    if (bias != nullptr) v += TT<T>::load(bias + n + e);
-    TT<T>::store(&o[e], v);
-  }
-  if constexpr (VEC == 4) {
-    *reinterpret_cast<u32x2*>(out + i) = *reinterpret_cast<const u32x2*>(o);
-  } else {
-    out[i] = o[0];
-  }
+  i = i < MN - 4 ? i : MN - 4;
+  const f32x4 acc = sum_slices4<f32x4>(part + i, MN, splits);
+  store_folded4<T>(out + i, (int)(i % N), (int)N, [&](int e, int n) {
+    return bias != nullptr ? acc[e] + TT<T>::load(bias + n) : acc[e];
+  });
 }
 
 // Slices of K for the in-tile path: as many as still fit the blocks into one resident round
@@ -171,13 +184,8 @@ int launch_wq_variant(hipStream_t st, const LinearArgs& a, float* partials, int 
     }
     if (rc != OFQ_OK) return rc;
     const int64_t mn = a.m * a.n;
-    if (a.n % 4 == 0) {
-      splitk_finalize<T, 4><<<(unsigned)((mn / 4 + 255) / 256), 256, 0, st>>>(
-          partials, ep.bias, ep.out, mn, (int)a.n, splits);
-    } else {
-      splitk_finalize<T, 1><<<(unsigned)((mn + 255) / 256), 256, 0, st>>>(
-          partials, ep.bias, ep.out, mn, (int)a.n, splits);
-    }
+    splitk_finalize<T><<<(unsigned)((mn + 1023) / 1024), 256, 0, st>>>(
+        partials, ep.bias, ep.out, (uint32_t)mn, (uint32_t)a.n, splits);
     return ofq_check_launch();
   }
   // 256x128 tiles on 8 waves when there are enough rows of x to fill them, else 128x128 on 4
@@ -253,8 +261,8 @@ inline bool has_zero_term(const LinearArgs& a) { return !a.symmetric || !a.w_sig
 //   the steps, measured with symmetric fp16 4-bit codes; others take longer to expand, which the taller
 //   tiles hide better; a K that is not whole steps costs 1.4 times as much (the copies of such a
 //   kernel are all waited for); 8-bit codes that a single block reads are bound by the stream of them;
-//   the end: the output, 16-bit stores one by one where n is not whole pieces of 16 bytes, or for slices
-//   the second launch and their fp32 sums out and back at 5.2 TB/s.
+//   the end: the output, whose rows begin anywhere in a line where n is not whole pieces of 16 bytes, or for
+//   slices the second launch and their fp32 sums out and back at 5.2 TB/s.
 // Without a workspace the sums of slices have nowhere to go: the tile that is best with one slice.
 double wr_plan_us(const LinearArgs& a, bool have_workspace, WrPlan* plan) {
   double best = 1e30;
@@ -282,9 +290,8 @@ double wr_plan_us(const LinearArgs& a, bool have_workspace, WrPlan* plan) {
   const double scales_us = 1.9 / 4096 * (a.symmetric ? 1 : 2) / a.group_size;  // per column and k
   const double mn = 1e-6 * (double)a.m * a.n;
   // us for the sums of one slice, in whole 32 x 32 tiles
-  const double slice_us = 8e-6 / 5.2 * 1024 * ceil_div(a.m, 32) * ceil_div(a.n, 32)
-                          + (a.n % 4 != 0 ? 0.17 * mn : 0.0);
-  const double store_us = a.n % 8 != 0 ? 0.4 + 2.1 * mn : 0.0;
+  const double slice_us = 8e-6 / 5.2 * 1024 * ceil_div(a.m, 32) * ceil_div(a.n, 32);
+  const double store_us = a.n % 8 != 0 ? 0.35 * mn : 0.0;
   for (const Tile& t : tiles) {
     if (a.m <= t.above || (!t.any_bits && a.bits != 4)) continue;
     const int blocks = ceil_div(a.m, t.bm) * ceil_div(a.n, t.bn);
@@ -340,8 +347,7 @@ double wq_us(const LinearArgs& a, int splits) {
   }
   const double mn = 1e-6 * (double)a.m * a.n;
   return 3.2 + 0.5 * mn + ceil_div(ceil_div(a.k, 64), splits) * c * round
-         + (splits > 1 ? 4.1 + splits * mn * (8 / 7.4 + (a.n % 8 != 0 ? 1.35 : 0.0))
-                       : (a.n % 8 != 0 ? 0.5 + 1.5 * mn : 0.0));
+         + (splits > 1 ? 4.1 + splits * mn * 8 / 6.5 : (a.n % 8 != 0 ? 0.2 * mn : 0.0));
 }
 
 size_t wq_partial_bytes(const LinearArgs& a) {
@@ -463,13 +469,8 @@ int launch_plain_split(hipStream_t st, const LinearArgs& a, const void* wt, floa
   const int64_t mn = a.m * a.n;
   const S* bias = static_cast<const S*>(a.bias);
   S* out = static_cast<S*>(a.out);
-  if (a.n % 4 == 0) {
-    splitk_finalize<T, 4><<<(unsigned)((mn / 4 + 255) / 256), 256, 0, st>>>(partials, bias, out, mn,
-                                                                          (int)a.n, splits);
-  } else {
-    splitk_finalize<T, 1><<<(unsigned)((mn + 255) / 256), 256, 0, st>>>(partials, bias, out, mn,
-                                                                      (int)a.n, splits);
-  }
+  splitk_finalize<T><<<(unsigned)((mn + 1023) / 1024), 256, 0, st>>>(partials, bias, out, (uint32_t)mn,
+                                                                     (uint32_t)a.n, splits);
   return ofq_check_launch();
 }
 
@@ -565,36 +566,21 @@ int mq_splits(int64_t m, int64_t n, int64_t k) {
 
 // adds the int32 slices (integer addition: any order gives the same sum) and applies the
 // epilogue of EpScale
-template<typename T, int VEC>
+template<typename T>
 __global__ void __launch_bounds__(256)
 splitk_finalize_i32(const int* __restrict__ part, const float* __restrict__ a_scale,
                     const float* __restrict__ b_scale,
                     const typename TT<T>::storage* __restrict__ bias,
-                    typename TT<T>::storage* __restrict__ out, int64_t MN, int N, int splits) {
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VEC;
+                    typename TT<T>::storage* __restrict__ out, uint32_t MN, uint32_t N, int splits) {
+  uint32_t i = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= MN) return;
-  int acc[VEC];
-  if constexpr (VEC == 4) {
-    const i32x4 v = *reinterpret_cast<const i32x4*>(part + i);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] = v[e];
-    for (int sidx = 1; sidx < splits; ++sidx) {
-      const i32x4 u = *reinterpret_cast<const i32x4*>(part + (int64_t)sidx * MN + i);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] += u[e];
-    }
-  } else {
-    acc[0] = part[i];
-    for (int sidx = 1; sidx < splits; ++sidx) acc[0] += part[(int64_t)sidx * MN + i];
-  }
-  const int n = (int)(i % N);  // VEC divides N: the VEC elements share a row
+  i = i < MN - 4 ? i : MN - 4;
+  const i32x4 acc = sum_slices4<i32x4>(part + i, MN, splits);
   const float sa = a_scale[0];
-#pragma unroll
-  for (int e = 0; e < VEC; ++e) {
-    float r = (float)acc[e] * (sa * b_scale[n + e]);
-    if (bias != nullptr) r = r + TT<T>::load(bias + n + e);
-    TT<T>::store(out + i + e, r);
-  }
+  store_folded4<T>(out + i, (int)(i % N), (int)N, [&](int e, int n) {
+    const float r = (float)acc[e] * (sa * b_scale[n]);
+    return bias != nullptr ? r + TT<T>::load(bias + n) : r;
+  });
 }
 
 template<bool RG, typename T>
@@ -616,13 +602,9 @@ int launch_mq_split(hipStream_t st, const void* a, const BCopyParams& bp, const 
   if (rc != OFQ_OK) return rc;
   const int64_t mn = m * n;
   const int* pi = reinterpret_cast<const int*>(partials);
-  if (n % 4 == 0) {
-    splitk_finalize_i32<T, 4><<<(unsigned)((mn / 4 + 255) / 256), 256, 0, st>>>(
-        pi, a_scale, b_scale, static_cast<const S*>(bias), static_cast<S*>(out), mn, (int)n, splits);
-  } else {
-    splitk_finalize_i32<T, 1><<<(unsigned)((mn + 255) / 256), 256, 0, st>>>(
-        pi, a_scale, b_scale, static_cast<const S*>(bias), static_cast<S*>(out), mn, (int)n, splits);
-  }
+  splitk_finalize_i32<T><<<(unsigned)((mn + 1023) / 1024), 256, 0, st>>>(
+      pi, a_scale, b_scale, static_cast<const S*>(bias), static_cast<S*>(out), (uint32_t)mn, (uint32_t)n,
+      splits);
   return ofq_check_launch();
 }
 

@@ -97,8 +97,8 @@ __device__ __forceinline__ void wr_store_tile(const f32x16& acc, uint8_t* lds, u
     const int m = m0 + row, n = n0 + piece * 8;
     if (m < M) {
       uint16_t* dst = out + (int64_t)m * N + n;
-      if ((N & 7) == 0) {
-        if (n < N) *reinterpret_cast<u32x4*>(dst) = v;
+      if (n + 8 <= N) {
+        *reinterpret_cast<u32x4_any*>(dst) = v;
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -446,8 +446,8 @@ gemm_wr_fold(const float* __restrict__ part, const uint16_t* __restrict__ bias,
   const int m = m0 + row, n = n0 + piece * 4;
   if (m < M) {
     uint16_t* dst = out + (int64_t)m * N + n;
-    if ((N & 3) == 0) {
-      if (n < N) *reinterpret_cast<u32x2*>(dst) = v;
+    if (n + 4 <= N) {
+      *reinterpret_cast<u32x2_any*>(dst) = v;
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {

@@ -23,6 +23,10 @@ typedef int i32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+// 8 and 16 bytes at the address of any element, for rows that are not whole 16-byte pieces: one vector
+// store all the same (amdhsa runs gfx950 in unaligned access mode; the type tells the compiler).
+typedef u32x2 u32x2_any __attribute__((aligned(2)));
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
 
 constexpr int kWave = 64;
 
