@@ -8,7 +8,8 @@
 //                      matmul_wx = x w~^T + b, matmul_vx = x v~^T + c (both stored in T),
 //                      y = matmul_wx * act(matmul_vx), the activation evaluated in fp32 on the
 //                      widened gate and rounded to T, the product rounded to T.
-// For m <= 16 the linears of one call run as a single launch of the decode kernel; otherwise
+// For m <= 16 the linears of one call, and a gated unit with its gating, run as a single launch of a
+// decode kernel; otherwise
 // they run one after the other through the op's own entry point.
 #include "ofq_device.h"
 #include "ofq_internal.h"
@@ -256,8 +257,8 @@ extern "C" int ofq_fused_glu_gq(void* stream, const void* x, const void* w, cons
     a[1].zero = v_zero;
     a[1].bias = c;
     a[1].out = matmul_vx;
-    // decode, fp16, 4-bit codes: both linears and the gating as one launch
-    if (m <= 16 && t_dtype == OFQ_F16 && decode_args_ok(a[0]) && decode_args_ok(a[1])
+    // decode: both linears and the gating as one launch
+    if (m <= 16 && t_dtype != OFQ_F32 && decode_args_ok(a[0]) && decode_args_ok(a[1])
         && ofq_aligned16(y)) {
       rc = launch_gemv_glu(st, a[0], a[1], y, activation);
       if (rc != OFQ_ERR_UNSUPPORTED) return rc;

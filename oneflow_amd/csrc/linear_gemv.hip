@@ -316,6 +316,20 @@ bool rows_supported(const LinearArgs& a) {
          && (a.symmetric || !a.w_signed);
 }
 
+// the ring kernel, where it is the faster one (gemv_ring_launch.h)
+int launch_ring(hipStream_t st, const LinearArgs* pr, int count, bool glu, void* y, int act) {
+  const LinearArgs& a = pr[0];
+  for (int i = 0; i < count; ++i) {
+    const LinearArgs& b = pr[i];
+    if (!rows_supported(b) || b.t_dtype != a.t_dtype || b.bits != a.bits || b.w_signed != a.w_signed
+        || b.symmetric != a.symmetric || b.group_size != a.group_size || b.m != a.m || b.k != a.k) {
+      return OFQ_ERR_UNSUPPORTED;
+    }
+  }
+  return a.t_dtype == OFQ_BF16 ? launch_gemv_ring_bf16(st, pr, count, glu, y, act)
+                               : launch_gemv_ring_f16(st, pr, count, glu, y, act);
+}
+
 template<typename T, int NW>
 int launch_rows_t(hipStream_t st, const LinearArgs& a, int grid, int rpb, size_t lds,
                   bool staged) {
@@ -337,6 +351,10 @@ int launch_rows_t(hipStream_t st, const LinearArgs& a, int grid, int rpb, size_t
 
 // OFQ_ERR_UNSUPPORTED when x does not fit the block's registers and LDS
 int launch_rows(hipStream_t st, const LinearArgs& a) {
+  {
+    const int rc = launch_ring(st, &a, 1, false, nullptr, 0);
+    if (rc != OFQ_ERR_UNSUPPORTED) return rc;
+  }
   constexpr int kCUs = 256;
   const int64_t max_rows = 16 * kRowsMaxTiles;
   int64_t grid = kCUs;
@@ -700,15 +718,8 @@ int launch_w4p_glu_inst(hipStream_t st, const LinearArgs& a, const GluArgs& glu,
   return ofq_check_launch();
 }
 
-}  // namespace
-
-int launch_gemv_glu(hipStream_t st, const LinearArgs& a, const LinearArgs& g, void* y, int act) {
-  {
-    const int rc = launch_gemv_m1_glu(st, a, g, y, act);
-    if (rc != OFQ_ERR_UNSUPPORTED) return rc;
-  }
+int launch_w4p_glu(hipStream_t st, const LinearArgs& a, const LinearArgs& g, void* y, int act) {
   if (!w4p_supported(a) || !w4p_supported(g)) return OFQ_ERR_UNSUPPORTED;
-  if (g.n != a.n || g.k != a.k || g.m != a.m || g.x != a.x) return OFQ_ERR_UNSUPPORTED;
   constexpr int kCUs = 256;
   const bool exact = !(a.symmetric && a.w_signed);
   // A block walks the same rows of both weights.  First choice: up to 64 rows of each per block,
@@ -770,6 +781,18 @@ int launch_gemv_glu(hipStream_t st, const LinearArgs& a, const LinearArgs& g, vo
   return OFQ_ERR_UNSUPPORTED;
 }
 
+}  // namespace
+
+int launch_gemv_glu(hipStream_t st, const LinearArgs& a, const LinearArgs& g, void* y, int act) {
+  int rc = launch_gemv_m1_glu(st, a, g, y, act);
+  if (rc != OFQ_ERR_UNSUPPORTED) return rc;
+  if (g.n != a.n || g.k != a.k || g.m != a.m || g.x != a.x) return OFQ_ERR_UNSUPPORTED;
+  rc = launch_w4p_glu(st, a, g, y, act);
+  if (rc != OFQ_ERR_UNSUPPORTED) return rc;
+  const LinearArgs both[2] = {a, g};
+  return launch_ring(st, both, 2, true, y, act);
+}
+
 int launch_gemv_grouped(hipStream_t st, const LinearArgs* pr, int count) {
   if (count < 1 || count > kGemvMaxProblems) return OFQ_ERR_UNSUPPORTED;
   {
@@ -790,6 +813,10 @@ int launch_gemv_grouped(hipStream_t st, const LinearArgs* pr, int count) {
   }
   if (all_w4p) {
     const int rc = launch_w4p_grouped(st, pr, count);
+    if (rc != OFQ_ERR_UNSUPPORTED) return rc;
+  }
+  if (count > 1) {
+    const int rc = launch_ring(st, pr, count, false, nullptr, 0);
     if (rc != OFQ_ERR_UNSUPPORTED) return rc;
   }
   int rpb = 0;

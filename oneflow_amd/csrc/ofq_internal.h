@@ -102,6 +102,11 @@ int launch_gemv_grouped(hipStream_t st, const LinearArgs* problems, int count);
 // not fit (caller runs the linears and the gating separately).
 int launch_gemv_glu(hipStream_t st, const LinearArgs& a, const LinearArgs& g, void* y, int act);
 
+// The ring kernel (gemv_ring.h) on one linear of up to 16 rows of x, on several that share m, k, dtype and
+// quantisation attributes, or on the two of a gated unit (glu: problems 0 and 1, then y = out0 * act(out1)).
+int launch_gemv_ring_f16(hipStream_t st, const LinearArgs* problems, int count, bool glu, void* y, int act);
+int launch_gemv_ring_bf16(hipStream_t st, const LinearArgs* problems, int count, bool glu, void* y, int act);
+
 // matmul_quant with few rows of a (m <= 64; k a multiple of 64): int8 MFMA with the weights
 // streamed once.
 bool matmul_quant_rows_supported(int64_t m, int64_t n, int64_t k);
