@@ -59,13 +59,6 @@ struct RingArgs {
   int phases;
   uint32_t m_magic;  // ceil(2^32 / M)
 };
-struct RingMat {
-  const uint8_t* w;
-  const uint16_t* scale;
-  const uint16_t* zero;
-  const uint16_t* bias;
-  uint16_t* out;
-};
 
 // bytes of LDS of the scales of one matrix
 __host__ __device__ inline int ring_scale_bytes(int rows_per_block, int G) {
@@ -127,7 +120,7 @@ __device__ __forceinline__ float ring_sum(const float* src, int M, int tr) {
 
 template<typename T, int BITS, bool SIGNED, int ZMODE, int TR, int TL, int NMAT>
 __device__ __forceinline__ void
-gemv_ring_body(int block, const uint16_t* __restrict__ x, const RingMat (&mats)[NMAT], int N,
+gemv_ring_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[NMAT], int N,
                uint16_t* __restrict__ y, int act, const RingArgs& p) {
   typedef typename TT<T>::storage S;
   static_assert(sizeof(S) == 2, "16-bit element types");
@@ -229,7 +222,7 @@ gemv_ring_body(int block, const uint16_t* __restrict__ x, const RingMat (&mats)[
   auto copy_scales = [&]() {
 #pragma unroll
     for (int i = 0; i < NMAT * kRegions; ++i) {
-      const RingMat& mt = mats[i / kRegions];
+      const RowsMat& mt = mats[i / kRegions];
       const uint8_t* src = reinterpret_cast<const uint8_t*>(i % kRegions == 0 ? mt.scale : mt.zero)
                            + (s_first - s_shift);
       const int nops = (s_bytes + 1023) >> 10;
@@ -438,8 +431,8 @@ gemv_ring_body(int block, const uint16_t* __restrict__ x, const RingMat (&mats)[
 
 template<typename T, int BITS, bool SIGNED, int ZMODE, int TR, int TL>
 __global__ void __launch_bounds__(kRingWaves * 64)
-gemv_ring(const uint16_t* __restrict__ x, RingMat mat, int N, RingArgs p) {
-  const RingMat mats[1] = {mat};
+gemv_ring(const uint16_t* __restrict__ x, RowsMat mat, int N, RingArgs p) {
+  const RowsMat mats[1] = {mat};
   gemv_ring_body<T, BITS, SIGNED, ZMODE, TR, TL, 1>((int)blockIdx.x, x, mats, N, nullptr, 0, p);
 }
 // Several linears of the same m, k and quantisation: the grid is the concatenation of their blocks.
@@ -447,7 +440,7 @@ template<typename T, int BITS, bool SIGNED, int ZMODE, int TR, int TL>
 __global__ void __launch_bounds__(kRingWaves * 64)
 gemv_ring_grouped(GemvGroup g, RingArgs p) {
   const GemvProblem pr = select_problem(g, (int)blockIdx.x);
-  const RingMat mats[1] = {{pr.w, static_cast<const uint16_t*>(pr.scale), static_cast<const uint16_t*>(pr.zero),
+  const RowsMat mats[1] = {{pr.w, static_cast<const uint16_t*>(pr.scale), static_cast<const uint16_t*>(pr.zero),
                             static_cast<const uint16_t*>(pr.bias), static_cast<uint16_t*>(pr.out)}};
   gemv_ring_body<T, BITS, SIGNED, ZMODE, TR, TL, 1>((int)blockIdx.x - pr.first_block,
                                                     static_cast<const uint16_t*>(pr.x), mats, pr.N,
@@ -457,9 +450,9 @@ gemv_ring_grouped(GemvGroup g, RingArgs p) {
 // of both weights.
 template<typename T, int BITS, bool SIGNED, int ZMODE, int TR, int TL>
 __global__ void __launch_bounds__(kRingWaves * 64)
-gemv_ring_glu(const uint16_t* __restrict__ x, RingMat hidden, RingMat gate, int N,
+gemv_ring_glu(const uint16_t* __restrict__ x, RowsMat hidden, RowsMat gate, int N,
               uint16_t* __restrict__ y, int act, RingArgs p) {
-  const RingMat mats[2] = {hidden, gate};
+  const RowsMat mats[2] = {hidden, gate};
   gemv_ring_body<T, BITS, SIGNED, ZMODE, TR, TL, 2>((int)blockIdx.x, x, mats, N, y, act, p);
 }
 

@@ -1,9 +1,8 @@
+// gemv_ring (gemv_ring.h) for fp16 activations.
 #include "gemv_ring_launch.h"
 
 namespace ofq {
 
-int launch_gemv_ring_f16(hipStream_t st, const LinearArgs* pr, int count, bool glu, void* y, int act) {
-  return launch_ring_t<f16>(st, pr, count, glu, y, act);
-}
+int launch_gemv_ring_f16(hipStream_t st, const LinearJob& job) { return launch_ring_t<f16>(st, job); }
 
 }  // namespace ofq

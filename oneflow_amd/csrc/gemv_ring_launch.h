@@ -99,12 +99,6 @@ inline bool ring_plan(const LinearArgs& a, const int64_t* rows, int count, int m
   return false;
 }
 
-inline RingMat ring_mat(const LinearArgs& a) {
-  return RingMat{static_cast<const uint8_t*>(a.w), static_cast<const uint16_t*>(a.scale),
-                 static_cast<const uint16_t*>(a.zero), static_cast<const uint16_t*>(a.bias),
-                 static_cast<uint16_t*>(a.out)};
-}
-
 // Where the ring is the faster one: 6000 random problems (m 1 .. 16, n 512 .. 32000, k 512 .. 14336, both types
 // and widths, groups of 32, 64, 128), time of the kernels that ran before over this one's:
 //   gated units                                   1.27 (5 of 100 below 1.08): two launches and the gating's
@@ -124,47 +118,32 @@ inline bool ring_preferred(const LinearArgs& a, bool one, const RingPlan& plan) 
   return a.m > 1 && p.rows_per_block <= 8 && turns >= 2;
 }
 
-// what is launched: one problem, several, or a gated unit's two
-struct RingJob {
-  const LinearArgs* pr;
-  int count;
-  bool glu;
-  void* y;
-  int act;
-};
-
 template<typename T, int BITS, bool SIGNED, int ZMODE, int TR, int TL>
-int launch_ring_inst(hipStream_t st, const RingJob& job, const RingPlan& plan) {
+int launch_ring_inst(hipStream_t st, const LinearJob& job, const RingPlan& plan) {
   const LinearArgs& a = job.pr[0];
   const uint16_t* x = static_cast<const uint16_t*>(a.x);
   static std::atomic<uint64_t> allowed{0}, allowed_grouped{0}, allowed_glu{0};  // devices: LDS limit raised
   if (job.glu) {
     auto kern = gemv_ring_glu<T, BITS, SIGNED, ZMODE, TR, TL>;
     if (!ofq_allow_dynamic_lds(reinterpret_cast<const void*>(kern), 160 * 1024, allowed_glu)) return OFQ_ERR_LAUNCH;
-    kern<<<plan.grid, kRingWaves * 64, plan.lds, st>>>(x, ring_mat(a), ring_mat(job.pr[1]), (int)a.n,
+    kern<<<plan.grid, kRingWaves * 64, plan.lds, st>>>(x, rows_mat(a), rows_mat(job.pr[1]), (int)a.n,
                                                        static_cast<uint16_t*>(job.y), job.act, plan.args);
   } else if (job.count > 1) {
     auto kern = gemv_ring_grouped<T, BITS, SIGNED, ZMODE, TR, TL>;
     if (!ofq_allow_dynamic_lds(reinterpret_cast<const void*>(kern), 160 * 1024, allowed_grouped)) return OFQ_ERR_LAUNCH;
     GemvGroup g{};
-    g.count = job.count;
-    int first = 0;
-    for (int i = 0; i < job.count; ++i) {
-      const LinearArgs& p = job.pr[i];
-      g.p[i] = GemvProblem{p.x, static_cast<const uint8_t*>(p.w), p.scale, p.zero, p.bias, p.out, (int)p.n, first};
-      first += (int)((p.n + plan.args.rows_per_block - 1) / plan.args.rows_per_block);
-    }
+    fill_group(g, job.pr, job.count, plan.args.rows_per_block);
     kern<<<plan.grid, kRingWaves * 64, plan.lds, st>>>(g, plan.args);
   } else {
     auto kern = gemv_ring<T, BITS, SIGNED, ZMODE, TR, TL>;
     if (!ofq_allow_dynamic_lds(reinterpret_cast<const void*>(kern), 160 * 1024, allowed)) return OFQ_ERR_LAUNCH;
-    kern<<<plan.grid, kRingWaves * 64, plan.lds, st>>>(x, ring_mat(a), (int)a.n, plan.args);
+    kern<<<plan.grid, kRingWaves * 64, plan.lds, st>>>(x, rows_mat(a), (int)a.n, plan.args);
   }
   return ofq_check_launch();
 }
 
 template<typename T, int BITS, bool SIGNED, int ZMODE>
-int launch_ring_variant(hipStream_t st, const RingJob& job, const RingPlan& plan) {
+int launch_ring_variant(hipStream_t st, const LinearJob& job, const RingPlan& plan) {
 #define OFQ_L(TRV, TLV) \
   if (plan.tr == TRV && plan.tl == TLV) return launch_ring_inst<T, BITS, SIGNED, ZMODE, TRV, TLV>(st, job, plan);
   OFQ_L(8, 1) OFQ_L(8, 2) OFQ_L(8, 3) OFQ_L(8, 4)
@@ -174,16 +153,15 @@ int launch_ring_variant(hipStream_t st, const RingJob& job, const RingPlan& plan
 }
 
 template<typename T>
-int launch_ring_t(hipStream_t st, const LinearArgs* pr, int count, bool glu, void* y, int act) {
-  const LinearArgs& a = pr[0];
+int launch_ring_t(hipStream_t st, const LinearJob& job) {
+  const LinearArgs& a = job.pr[0];
   int64_t rows[kGemvMaxProblems];
-  const int lists = glu ? 1 : count;
-  for (int i = 0; i < lists; ++i) rows[i] = pr[i].n;
+  const int lists = job.glu ? 1 : job.count;
+  for (int i = 0; i < lists; ++i) rows[i] = job.pr[i].n;
   RingPlan plan;
-  if (!ring_plan(a, rows, lists, glu ? 2 : 1, &plan) || !ring_preferred(a, count == 1, plan)) {
+  if (!ring_plan(a, rows, lists, job.glu ? 2 : 1, &plan) || !ring_preferred(a, job.count == 1, plan)) {
     return OFQ_ERR_UNSUPPORTED;
   }
-  const RingJob job{pr, count, glu, y, act};
   const int zmode = !a.symmetric ? kZeroAsym : (a.w_signed ? kZeroNone : kZeroSymU);
 #define OFQ_V(B, SG, ZM)                              \
   if (a.bits == B && a.w_signed == SG && zmode == ZM) \

@@ -22,6 +22,7 @@
 #include "dequant_regs.h"
 #include "gemv_kernels.h"
 #include "ofq_device.h"
+#include "ofq_internal.h"
 #include "scale_panel.h"
 
 namespace ofq {
@@ -362,6 +363,34 @@ gemv_rows_grouped(GemvGroup g, int M, int K, int group_size, int gs_shift, int r
 // time: all of K unless long rows of short groups leave no room for it.  A row of the panel ends with a
 // zero, the scale of a lane past the end of K.
 // ---------------------------------------------------------------------------------------------
+struct RowsMat {  // a weight and what belongs to it
+  const uint8_t* w;
+  const uint16_t* scale;
+  const uint16_t* zero;
+  const uint16_t* bias;
+  uint16_t* out;
+};
+inline RowsMat rows_mat(const LinearArgs& a) {
+  return RowsMat{static_cast<const uint8_t*>(a.w), static_cast<const uint16_t*>(a.scale),
+                 static_cast<const uint16_t*>(a.zero), static_cast<const uint16_t*>(a.bias),
+                 static_cast<uint16_t*>(a.out)};
+}
+inline void fill_group(GemvGroup& g, const LinearArgs* pr, int count, int rpb) {
+  g.count = count;
+  int first = 0;
+  for (int i = 0; i < count; ++i) {
+    g.p[i].x = pr[i].x;
+    g.p[i].w = static_cast<const uint8_t*>(pr[i].w);
+    g.p[i].scale = pr[i].scale;
+    g.p[i].zero = pr[i].zero;
+    g.p[i].bias = pr[i].bias;
+    g.p[i].out = pr[i].out;
+    g.p[i].N = (int)pr[i].n;
+    g.p[i].first_block = first;
+    first += (int)((pr[i].n + rpb - 1) / rpb);
+  }
+}
+
 template<int BITS, int MT>
 struct RowsMtX {
   static constexpr int CK = BITS == 4 ? 128 : 64;
@@ -373,12 +402,17 @@ struct RowsMtX {
   static constexpr int kWaveBytes = MT * 16 * kPitch;
 };
 
-template<typename T, int BITS, bool SIGNED, int ZMODE, int NWAVES, int MT, int NTL>
-__global__ void __launch_bounds__(NWAVES * 64)
-gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
-             const uint16_t* __restrict__ scale, const uint16_t* __restrict__ zero,
-             const uint16_t* __restrict__ bias, uint16_t* __restrict__ out, int M, int N, int K,
-             int group_size, int gs_shift, int rows_per_block, int panel_chunks, int panel_groups) {
+// NTL: weight tiles of a matrix in a block; NMAT = 2: the two weights of a gated unit, whose blocks own the same
+// rows of both and form y = hidden * act(gate) from the rounded sums.  One launch for q/k/v or for a gated unit
+// instead of one each and the gating's: 5840 random layers of 17 to 64 rows of x (k 1024 to 6000) take 1 / 2.35
+// of the time for three linears of k, k/c, k/c rows (each alone is bound by its launch and one short turn
+// of the waves), 7 300 gated units 1 / 1.28 (those of 100 MB and more the same).  Where that is expected to
+// take longer than one by one (3 % of the gated units): launch_gemv_mt_several.
+template<typename T, int BITS, bool SIGNED, int ZMODE, int NWAVES, int MT, int NTL, int NMAT>
+__device__ __forceinline__ void
+gemv_rows_mt_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[NMAT], int N,
+                  uint16_t* __restrict__ y, int act, int M, int K, int group_size, int gs_shift,
+                  int rows_per_block, int panel_chunks, int panel_groups) {
   typedef typename TT<T>::storage S;
   static_assert(sizeof(S) == 2, "16-bit element types");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -393,14 +427,14 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15;
   const int kb = lane >> 4;
-  const int row0 = blockIdx.x * rows_per_block;
+  const int row0 = block * rows_per_block;
   int rows_blk = N - row0;
   if (rows_blk > rows_per_block) rows_blk = rows_per_block;
   if (rows_blk <= 0) return;
   const int ntiles = (rows_blk + 15) >> 4;
 
   // LDS: [the waves' x buffers | red NWAVES*MT*256 f32][scales rows_per_block*(panel_groups + 1),
-  //      padded to 16 B][zeros (asymmetric)]
+  //      padded to 16 B, of every matrix][zeros (asymmetric)]
   typedef RowsMtX<BITS, MT> XB;
   float* red = reinterpret_cast<float*>(smem);
   const int pitch = panel_groups + 1;
@@ -409,23 +443,26 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
   constexpr size_t kFront = (size_t)NWAVES * XB::kWaveBytes > kRedBytes
                                 ? (size_t)NWAVES * XB::kWaveBytes : kRedBytes;
   uint16_t* sl = reinterpret_cast<uint16_t*>(smem + kFront);
-  uint16_t* zl = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(sl) + panel_bytes);
+  const int panel = panel_bytes / 2;  // 16-bit values from one matrix's to the next one's
+  uint16_t* zl = sl + NMAT * panel;
   uint8_t* xbuf = smem + (size_t)wave * XB::kWaveBytes;
 
-  const uint8_t* wblk = w + (int64_t)row0 * row_bytes;
+  const uint8_t* wblk[NMAT];
+#pragma unroll
+  for (int mat = 0; mat < NMAT; ++mat) wblk[mat] = mats[mat].w + (int64_t)row0 * row_bytes;
   uint32_t roff[NTL];  // of this lane's row of every tile
 #pragma unroll
   for (int t = 0; t < NTL; ++t) {
     const int row_l = t * 16 + r;
     roff[t] = row_l < rows_blk ? (uint32_t)row_l * (uint32_t)row_bytes : 0u;
   }
-  auto request_codes = [&](int c, u32x4 (&dst)[NTL]) {  // (a chunk past the end re-reads chunk 0)
+  auto request_codes = [&](int c, u32x4 (&dst)[NMAT * NTL]) {  // (a chunk past the end re-reads chunk 0)
     int off = c * 64 + kb * 16;
     off = off < row_bytes ? off : 0;
 #pragma unroll
-    for (int t = 0; t < NTL; ++t) {
+    for (int t = 0; t < NMAT * NTL; ++t) {
       dst[t] = __builtin_nontemporal_load(
-          reinterpret_cast<const u32x4*>(wblk + roff[t] + (uint32_t)off));
+          reinterpret_cast<const u32x4*>(wblk[t / NTL] + roff[t % NTL] + (uint32_t)off));
     }
   };
   // request i of a chunk covers rows kRowsPerReq * i + lane / kLanesPerRow, 16 bytes per lane; rows
@@ -447,33 +484,36 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
                                               + (uint32_t)off);
     }
   };
-  f32x4 acc[NTL][MT];
+  f32x4 acc[NMAT * NTL][MT];
 #pragma unroll
-  for (int t = 0; t < NTL; ++t)
+  for (int t = 0; t < NMAT * NTL; ++t)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   int c = wave;
-  u32x4 code_a[NTL], code_b[NTL];
+  u32x4 code_a[NMAT * NTL], code_b[NMAT * NTL];
   request_x(c);
   request_codes(c, code_a);
 
-  const uint16_t* sblk = scale + (int64_t)row0 * G;
-  const uint16_t* zblk = ZMODE == kZeroAsym ? zero + (int64_t)row0 * G : sblk;
   int g0 = 0;  // first group of the panel
   auto fill_panel = [&](int first_chunk) {
     g0 = gs_shift >= 0 ? (first_chunk * CK) >> gs_shift : (first_chunk * CK) / group_size;
     const int ng = G - g0 < panel_groups ? G - g0 : panel_groups;
-    copy_scale_panel<NT, ZMODE == kZeroAsym, false>(sblk + g0, zblk + g0, G, rows_blk, rows_blk, ng,
-                                                    pitch, sl, zl, tid);
-    if (tid < rows_per_block) {  // (at most 64 rows)
-      sl[tid * pitch + panel_groups] = 0;
-      if (ZMODE == kZeroAsym) zl[tid * pitch + panel_groups] = 0;
+#pragma unroll
+    for (int mat = 0; mat < NMAT; ++mat) {
+      const uint16_t* sblk = mats[mat].scale + (int64_t)row0 * G + g0;
+      const uint16_t* zblk = ZMODE == kZeroAsym ? mats[mat].zero + (int64_t)row0 * G + g0 : sblk;
+      copy_scale_panel<NT, ZMODE == kZeroAsym, false>(sblk, zblk, G, rows_blk, rows_blk, ng, pitch,
+                                                      sl + mat * panel, zl + mat * panel, tid);
+      if (tid < rows_per_block) {  // (at most 64 rows)
+        sl[mat * panel + tid * pitch + panel_groups] = 0;
+        if (ZMODE == kZeroAsym) zl[mat * panel + tid * pitch + panel_groups] = 0;
+      }
     }
     __syncthreads();
   };
 
-  auto work = [&](const u32x4 (&cur)[NTL], u32x4 (&nxt)[NTL]) {
+  auto work = [&](const u32x4 (&cur)[NMAT * NTL], u32x4 (&nxt)[NMAT * NTL]) {
     const int k0 = c * CK + kb * LK;
     if ((c + 1) * CK > K) {  // (the same for every lane: the last chunk of a ragged row)
 #pragma unroll
@@ -492,10 +532,10 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
     request_codes(c + NWAVES, nxt);
     int grp = (gs_shift >= 0 ? (k0 >> gs_shift) : (k0 / group_size)) - g0;
     grp = k0 < K ? grp : panel_groups;
-    float s[NTL], z[NTL];
+    float s[NMAT * NTL], z[NMAT * NTL];
 #pragma unroll
-    for (int t = 0; t < NTL; ++t) {
-      const int at = (t * 16 + r) * pitch + grp;
+    for (int t = 0; t < NMAT * NTL; ++t) {
+      const int at = t / NTL * panel + (t % NTL * 16 + r) * pitch + grp;
       s[t] = TT<T>::load(reinterpret_cast<const S*>(sl) + at);
       z[t] = 0.f;
       if (ZMODE == kZeroAsym) z[t] = TT<T>::load(reinterpret_cast<const S*>(zl) + at);
@@ -511,8 +551,8 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
           xa[mt] = *reinterpret_cast<const u32x4*>(xl + mt * 16 * XB::kPitch + j * 16);
         }
 #pragma unroll
-        for (int t = 0; t < NTL; ++t) {
-          if (t < ntiles) {
+        for (int t = 0; t < NMAT * NTL; ++t) {
+          if (t % NTL < ntiles) {
             const u32x4 b = dequant8_b4<T, SIGNED, ZMODE>(cur[t][j], s[t], z[t]);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) acc[t][mt] = MfmaK32<T>::mma(xa[mt], b, acc[t][mt]);
@@ -527,8 +567,8 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
         xa[mt][1] = *reinterpret_cast<const u32x4*>(xl + mt * 16 * XB::kPitch + 16);
       }
 #pragma unroll
-      for (int t = 0; t < NTL; ++t) {
-        if (t < ntiles) {
+      for (int t = 0; t < NMAT * NTL; ++t) {
+        if (t % NTL < ntiles) {
           u32x4 b0, b1;
           dequant16_b8<T, SIGNED, ZMODE>(cur[t], s[t], z[t], b0, b1);
 #pragma unroll
@@ -554,31 +594,93 @@ gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
 
   // fold, one weight tile at a time: red[wave][m (MT*16)][n (16)]
   __syncthreads();  // the reduction area overlays the x buffers of other waves
+  constexpr int kOuts = (MT * 256 + NT - 1) / NT;  // of a tile, a thread's
 #pragma unroll
   for (int t = 0; t < NTL; ++t) {
     if (t < ntiles) {
-      if (t > 0) __syncthreads();  // the previous tile's sums have been read
+      S first[kOuts];  // what the first matrix gives
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
+      for (int mat = 0; mat < NMAT; ++mat) {
+        if (t + mat > 0) __syncthreads();  // the previous tile's sums have been read
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int m = mt * 16 + 4 * kb + v;
-          red[(wave * (MT * 16) + m) * 16 + r] = acc[t][mt][v];
-        }
-      __syncthreads();
-      for (int o = tid; o < M * 16; o += NT) {
-        float sum = 0.f;
+        for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int wv = 0; wv < NWAVES; ++wv) sum += red[wv * (MT * 256) + o];
-        const int m = o >> 4;
-        const int row_l = t * 16 + (o & 15);
-        if (row_l < rows_blk) {
-          if (bias != nullptr) sum += TT<T>::load(reinterpret_cast<const S*>(bias) + row0 + row_l);
-          TT<T>::store(reinterpret_cast<S*>(out) + (int64_t)m * N + row0 + row_l, sum);
+          for (int v = 0; v < 4; ++v) {
+            const int m = mt * 16 + 4 * kb + v;
+            red[(wave * (MT * 16) + m) * 16 + r] = acc[mat * NTL + t][mt][v];
+          }
+        __syncthreads();
+        auto output = [&](int o) {
+          const int row_l = t * 16 + (o & 15);
+          S res = S();
+          if (row_l < rows_blk) {
+            float sum = 0.f;
+#pragma unroll
+            for (int wv = 0; wv < NWAVES; ++wv) sum += red[wv * (MT * 256) + o];
+            if (mats[mat].bias != nullptr) {
+              sum += TT<T>::load(reinterpret_cast<const S*>(mats[mat].bias) + row0 + row_l);
+            }
+            TT<T>::store(&res, sum);
+            reinterpret_cast<S*>(mats[mat].out)[(int64_t)(o >> 4) * N + row0 + row_l] = res;
+          }
+          return res;
+        };
+        if constexpr (NMAT == 1) {
+          for (int o = tid; o < M * 16; o += NT) output(o);
+        } else {
+#pragma unroll
+          for (int i = 0; i < kOuts; ++i) {
+            const int o = tid + i * NT;
+            if (o < M * 16) {
+              const S res = output(o);
+              const int row_l = t * 16 + (o & 15);
+              if (mat == 0) {
+                first[i] = res;
+              } else if (row_l < rows_blk) {
+                const float a = TT<T>::round(glu_activation(TT<T>::load(&res), act));
+                TT<T>::store(reinterpret_cast<S*>(y) + (int64_t)(o >> 4) * N + row0 + row_l,
+                             TT<T>::load(&first[i]) * a);
+              }
+            }
+          }
         }
       }
     }
   }
+}
+
+template<typename T, int BITS, bool SIGNED, int ZMODE, int NWAVES, int MT, int NTL>
+__global__ void __launch_bounds__(NWAVES * 64)
+gemv_rows_mt(const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
+             const uint16_t* __restrict__ scale, const uint16_t* __restrict__ zero,
+             const uint16_t* __restrict__ bias, uint16_t* __restrict__ out, int M, int N, int K,
+             int group_size, int gs_shift, int rows_per_block, int panel_chunks, int panel_groups) {
+  const RowsMat mats[1] = {{w, scale, zero, bias, out}};
+  gemv_rows_mt_body<T, BITS, SIGNED, ZMODE, NWAVES, MT, NTL, 1>(
+      (int)blockIdx.x, x, mats, N, nullptr, 0, M, K, group_size, gs_shift, rows_per_block,
+      panel_chunks, panel_groups);
+}
+// several linears of the same m, k and quantisation: the grid is the concatenation of their blocks
+template<typename T, int BITS, bool SIGNED, int ZMODE, int NWAVES, int MT, int NTL>
+__global__ void __launch_bounds__(NWAVES * 64)
+gemv_rows_mt_grouped(GemvGroup g, int M, int K, int group_size, int gs_shift, int rows_per_block,
+                     int panel_chunks, int panel_groups) {
+  const GemvProblem pr = select_problem(g, (int)blockIdx.x);
+  const RowsMat mats[1] = {{pr.w, static_cast<const uint16_t*>(pr.scale), static_cast<const uint16_t*>(pr.zero),
+                            static_cast<const uint16_t*>(pr.bias), static_cast<uint16_t*>(pr.out)}};
+  gemv_rows_mt_body<T, BITS, SIGNED, ZMODE, NWAVES, MT, NTL, 1>(
+      (int)blockIdx.x - pr.first_block, static_cast<const uint16_t*>(pr.x), mats, pr.N, nullptr, 0, M,
+      K, group_size, gs_shift, rows_per_block, panel_chunks, panel_groups);
+}
+template<typename T, int BITS, bool SIGNED, int ZMODE, int NWAVES, int MT, int NTL>
+__global__ void __launch_bounds__(NWAVES * 64)
+gemv_rows_mt_glu(const uint16_t* __restrict__ x, RowsMat hidden, RowsMat gate,
+                 uint16_t* __restrict__ y, int act, int M, int N, int K, int group_size, int gs_shift,
+                 int rows_per_block, int panel_chunks, int panel_groups) {
+  const RowsMat mats[2] = {hidden, gate};
+  gemv_rows_mt_body<T, BITS, SIGNED, ZMODE, NWAVES, MT, NTL, 2>(
+      (int)blockIdx.x, x, mats, N, y, act, M, K, group_size, gs_shift, rows_per_block, panel_chunks,
+      panel_groups);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -733,11 +835,11 @@ inline size_t gemv_rows_f32_lds_bytes(int nwaves, int K, int group_size, int row
 }
 
 inline size_t gemv_rows_mt_lds_bytes(int nwaves, int mt, int bits, int rows_per_block,
-                                     int panel_groups, bool asym) {
+                                     int panel_groups, bool asym, int matrices) {
   const size_t red = (size_t)nwaves * mt * 256 * 4;
   const size_t xb = (size_t)nwaves * mt * 16 * ((bits == 4 ? 256 : 128) + 16);
   return (xb > red ? xb : red)
-         + (size_t)(asym ? 2 : 1) * ((rows_per_block * (panel_groups + 1) * 2 + 15) & ~15);
+         + (size_t)(matrices * (asym ? 2 : 1)) * ((rows_per_block * (panel_groups + 1) * 2 + 15) & ~15);
 }
 
 inline size_t gemv_rows_lds_bytes(int nwaves, int M, int K, int group_size, int rows_per_block,

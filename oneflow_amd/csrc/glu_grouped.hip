@@ -8,8 +8,8 @@
 //                      matmul_wx = x w~^T + b, matmul_vx = x v~^T + c (both stored in T),
 //                      y = matmul_wx * act(matmul_vx), the activation evaluated in fp32 on the
 //                      widened gate and rounded to T, the product rounded to T.
-// For m <= 16 the linears of one call, and a gated unit with its gating, run as a single launch of a
-// decode kernel; otherwise
+// Up to 64 rows of x the linears of one call, and a gated unit with its gating, run as a single launch of
+// a streaming kernel where it takes their shapes; otherwise
 // they run one after the other through the op's own entry point.
 #include "ofq_device.h"
 #include "ofq_internal.h"
@@ -124,12 +124,12 @@ int run_single(void* stream, const LinearArgs& a) {
                              a.group_dim, a.group_size, a.m, a.n, a.k, nullptr, 0);
 }
 
-// the argument checks of the single op that the decode kernel relies on
+// the argument checks of the single op that the kernels of up to 64 rows of x rely on
 bool decode_args_ok(const LinearArgs& a) {
   if (a.x == nullptr || a.w == nullptr || a.scale == nullptr || a.out == nullptr) return false;
   if (a.symmetric != (a.zero == nullptr)) return false;
   if (!a.symmetric && a.w_signed) return false;
-  if (a.m < 1 || a.m > 16 || a.n < 1 || a.k < 1 || a.group_size < 1) return false;
+  if (a.m < 1 || a.m > 64 || a.n < 1 || a.k < 1 || a.group_size < 1) return false;
   if (a.k % a.group_size != 0) return false;
   const int64_t i32max = 0x7FFFFFFF;
   if (a.m * a.k > i32max || a.n * a.k > i32max || a.m * a.n > i32max) return false;
@@ -146,7 +146,10 @@ int run_group(void* stream, const LinearArgs* pr, int count) {
     bool ok = chunk > 1;
     for (int i = 0; ok && i < chunk; ++i) ok = decode_args_ok(pr[done + i]);
     int rc = OFQ_ERR_UNSUPPORTED;
-    if (ok) rc = launch_gemv_grouped(st, pr + done, chunk);
+    if (ok) {
+      rc = pr[done].m <= 16 ? launch_gemv_grouped(st, pr + done, chunk)
+                            : launch_gemv_mt_several(st, pr + done, chunk, false, nullptr, 0);
+    }
     if (rc == OFQ_ERR_UNSUPPORTED) {
       for (int i = 0; i < chunk; ++i) {
         rc = run_single(stream, pr[done + i]);
@@ -257,10 +260,11 @@ extern "C" int ofq_fused_glu_gq(void* stream, const void* x, const void* w, cons
     a[1].zero = v_zero;
     a[1].bias = c;
     a[1].out = matmul_vx;
-    // decode: both linears and the gating as one launch
-    if (m <= 16 && t_dtype != OFQ_F32 && decode_args_ok(a[0]) && decode_args_ok(a[1])
+    // up to 64 rows of x: both linears and the gating as one launch
+    if (m <= 64 && t_dtype != OFQ_F32 && decode_args_ok(a[0]) && decode_args_ok(a[1])
         && ofq_aligned16(y)) {
-      rc = launch_gemv_glu(st, a[0], a[1], y, activation);
+      rc = m <= 16 ? launch_gemv_glu(st, a[0], a[1], y, activation)
+                   : launch_gemv_mt_several(st, a, 2, true, y, activation);
       if (rc != OFQ_ERR_UNSUPPORTED) return rc;
     }
     rc = run_group(stream, a, 2);

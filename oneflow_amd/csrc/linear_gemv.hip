@@ -317,17 +317,16 @@ bool rows_supported(const LinearArgs& a) {
 }
 
 // the ring kernel, where it is the faster one (gemv_ring_launch.h)
-int launch_ring(hipStream_t st, const LinearArgs* pr, int count, bool glu, void* y, int act) {
-  const LinearArgs& a = pr[0];
-  for (int i = 0; i < count; ++i) {
-    const LinearArgs& b = pr[i];
+int launch_ring(hipStream_t st, const LinearJob& job) {
+  const LinearArgs& a = job.pr[0];
+  for (int i = 0; i < job.count; ++i) {
+    const LinearArgs& b = job.pr[i];
     if (!rows_supported(b) || b.t_dtype != a.t_dtype || b.bits != a.bits || b.w_signed != a.w_signed
         || b.symmetric != a.symmetric || b.group_size != a.group_size || b.m != a.m || b.k != a.k) {
       return OFQ_ERR_UNSUPPORTED;
     }
   }
-  return a.t_dtype == OFQ_BF16 ? launch_gemv_ring_bf16(st, pr, count, glu, y, act)
-                               : launch_gemv_ring_f16(st, pr, count, glu, y, act);
+  return a.t_dtype == OFQ_BF16 ? launch_gemv_ring_bf16(st, job) : launch_gemv_ring_f16(st, job);
 }
 
 template<typename T, int NW>
@@ -352,7 +351,7 @@ int launch_rows_t(hipStream_t st, const LinearArgs& a, int grid, int rpb, size_t
 // OFQ_ERR_UNSUPPORTED when x does not fit the block's registers and LDS
 int launch_rows(hipStream_t st, const LinearArgs& a) {
   {
-    const int rc = launch_ring(st, &a, 1, false, nullptr, 0);
+    const int rc = launch_ring(st, LinearJob{&a, 1, false, nullptr, 0});
     if (rc != OFQ_ERR_UNSUPPORTED) return rc;
   }
   constexpr int kCUs = 256;
@@ -458,53 +457,40 @@ int launch_gemv_variant(hipStream_t st, const LinearArgs& a) {
 }
 
 // ---- 16 < m <= 64: several tiles of x per weight tile -----------------------------------------
-struct RowsMtPlan {
-  int grid, rows_per_block, panel_chunks, panel_groups;
-  size_t lds;
-};
-
-template<typename T, int BITS, bool SIGNED, int ZMODE, int NW, int MT, int NTL>
-int launch_rows_mt_inst(hipStream_t st, const LinearArgs& a, const RowsMtPlan& p) {
-  auto kern = gemv_rows_mt<T, BITS, SIGNED, ZMODE, NW, MT, NTL>;
-  static std::atomic<uint64_t> lds_allowed{0};  // devices on which the kernel's LDS limit is raised
-  if (!ofq_allow_dynamic_lds(reinterpret_cast<const void*>(kern), 160 * 1024, lds_allowed)) return OFQ_ERR_LAUNCH;
-  kern<<<p.grid, NW * 64, p.lds, st>>>(
-      static_cast<const uint16_t*>(a.x), static_cast<const uint8_t*>(a.w),
-      static_cast<const uint16_t*>(a.scale), static_cast<const uint16_t*>(a.zero),
-      static_cast<const uint16_t*>(a.bias), static_cast<uint16_t*>(a.out), (int)a.m, (int)a.n,
-      (int)a.k, (int)a.group_size, ilog2_exact(a.group_size), p.rows_per_block, p.panel_chunks,
-      p.panel_groups);
-  return ofq_check_launch();
-}
-
-template<typename T, int NW, int MT>
-int launch_rows_mt_t(hipStream_t st, const LinearArgs& a, const RowsMtPlan& p) {
-  const int zmode = !a.symmetric ? kZeroAsym : (a.w_signed ? kZeroNone : kZeroSymU);
-#define OFQ_R(B, SG, ZM)                                                                     \
-  if (a.bits == B && a.w_signed == SG && zmode == ZM)                                        \
-    return p.rows_per_block <= 16   ? launch_rows_mt_inst<T, B, SG, ZM, NW, MT, 1>(st, a, p) \
-           : p.rows_per_block <= 32 ? launch_rows_mt_inst<T, B, SG, ZM, NW, MT, 2>(st, a, p) \
-                                    : launch_rows_mt_inst<T, B, SG, ZM, NW, MT, 4>(st, a, p);
-  OFQ_R(4, true, kZeroNone)
-  OFQ_R(4, false, kZeroSymU)
-  OFQ_R(4, false, kZeroAsym)
-  OFQ_R(8, true, kZeroNone)
-  OFQ_R(8, false, kZeroSymU)
-  OFQ_R(8, false, kZeroAsym)
-#undef OFQ_R
-  return OFQ_ERR_UNSUPPORTED;
-}
-
-template<typename T>
-int launch_rows_mt(hipStream_t st, const LinearArgs& a) {
+// Rows per block (of each matrix) and blocks: one round of blocks, one per CU, if a block's rows are then at
+// most the kernel's weight tiles.
+constexpr int kMtGluTiles = 2;  // of each of the two weights
+void rows_mt_split(const LinearJob& job, int* rpb, int64_t* grid) {
   constexpr int kCUs = 256;
-  const int64_t max_rows = 16 * kRowsMaxTiles;
-  int64_t grid = kCUs;
-  if ((a.n + grid - 1) / grid > max_rows) grid = (a.n + max_rows - 1) / max_rows;
+  const int lists = job.glu ? 1 : job.count;
+  const int max_rows = 16 * (job.glu ? kMtGluTiles : kRowsMaxTiles);
+  int64_t total = 0;
+  for (int i = 0; i < lists; ++i) total += job.pr[i].n;
+  auto blocks_at = [&](int r) {
+    int64_t b = 0;
+    for (int i = 0; i < lists; ++i) b += (job.pr[i].n + r - 1) / r;
+    return b;
+  };
+  int64_t rows = (total + kCUs - 1) / kCUs;
+  if (rows < 16) rows = 16;
+  if (job.glu && rows > max_rows) {  // whole rounds
+    const int64_t rounds = (rows + max_rows - 1) / max_rows;
+    rows = (total + kCUs * rounds - 1) / (kCUs * rounds);
+  }
+  if (rows > max_rows) rows = max_rows;
+  int r = (int)rows;
+  while (r < max_rows && blocks_at(r) > kCUs && total <= (int64_t)kCUs * max_rows) ++r;
+  *rpb = r;
+  *grid = blocks_at(r);
+}
+
+int launch_rows_mt(hipStream_t st, const LinearJob& job) {
+  const LinearArgs& a = job.pr[0];
   RowsMtPlan p;
-  p.rows_per_block = (int)((a.n + grid - 1) / grid);
-  if (p.rows_per_block < 16) p.rows_per_block = 16;
-  p.grid = (int)((a.n + p.rows_per_block - 1) / p.rows_per_block);
+  int64_t grid;
+  rows_mt_split(job, &p.rows_per_block, &grid);
+  if (grid > 0x7FFFFFFF) return OFQ_ERR_UNSUPPORTED;
+  p.grid = (int)grid;
   // 12 waves for two tiles of x, 8 for three and four (the x buffers and the registers of the
   // requests in flight)
   const int mt = (int)((a.m + 15) / 16);
@@ -519,14 +505,11 @@ int launch_rows_mt(hipStream_t st, const LinearArgs& a) {
     const int64_t groups = ((int64_t)p.panel_chunks * ck) / a.group_size + 2;
     const int64_t all = a.k / a.group_size;
     p.panel_groups = (int)(groups < all ? groups : all);
-    p.lds = gemv_rows_mt_lds_bytes(nw, mt, a.bits, p.rows_per_block, p.panel_groups, !a.symmetric);
+    p.lds = gemv_rows_mt_lds_bytes(nw, mt, a.bits, p.rows_per_block, p.panel_groups, !a.symmetric,
+                                   job.glu ? 2 : 1);
     if (p.lds <= 160u * 1024u) break;
   }
-  switch (mt) {
-    case 2: return launch_rows_mt_t<T, 12, 2>(st, a, p);
-    case 3: return launch_rows_mt_t<T, 8, 3>(st, a, p);
-    default: return launch_rows_mt_t<T, 8, 4>(st, a, p);
-  }
+  return a.t_dtype == OFQ_BF16 ? launch_gemv_mt_bf16(st, job, p) : launch_gemv_mt_f16(st, job, p);
 }
 
 // ---- fp32 activations -------------------------------------------------------------------------
@@ -646,22 +629,6 @@ int64_t grouped_split(const LinearArgs* pr, int count, int max_rows, int* rpb_ou
   if (rpb > max_rows) rpb = max_rows;
   *rpb_out = rpb;
   return blocks_at(rpb);
-}
-
-void fill_group(GemvGroup& g, const LinearArgs* pr, int count, int rpb) {
-  g.count = count;
-  int first = 0;
-  for (int i = 0; i < count; ++i) {
-    g.p[i].x = pr[i].x;
-    g.p[i].w = static_cast<const uint8_t*>(pr[i].w);
-    g.p[i].scale = pr[i].scale;
-    g.p[i].zero = pr[i].zero;
-    g.p[i].bias = pr[i].bias;
-    g.p[i].out = pr[i].out;
-    g.p[i].N = (int)pr[i].n;
-    g.p[i].first_block = first;
-    first += (int)((pr[i].n + rpb - 1) / rpb);
-  }
 }
 
 // fp16, 4-bit codes, groups in multiples of 128: the kernel of the single-problem fast path
@@ -790,7 +757,7 @@ int launch_gemv_glu(hipStream_t st, const LinearArgs& a, const LinearArgs& g, vo
   rc = launch_w4p_glu(st, a, g, y, act);
   if (rc != OFQ_ERR_UNSUPPORTED) return rc;
   const LinearArgs both[2] = {a, g};
-  return launch_ring(st, both, 2, true, y, act);
+  return launch_ring(st, LinearJob{both, 2, true, y, act});
 }
 
 int launch_gemv_grouped(hipStream_t st, const LinearArgs* pr, int count) {
@@ -816,7 +783,7 @@ int launch_gemv_grouped(hipStream_t st, const LinearArgs* pr, int count) {
     if (rc != OFQ_ERR_UNSUPPORTED) return rc;
   }
   if (count > 1) {
-    const int rc = launch_ring(st, pr, count, false, nullptr, 0);
+    const int rc = launch_ring(st, LinearJob{pr, count, false, nullptr, 0});
     if (rc != OFQ_ERR_UNSUPPORTED) return rc;
   }
   int rpb = 0;
@@ -864,13 +831,19 @@ bool gemv_mt_supported(const LinearArgs& a) {
 // wr_plan_us with up to 64 rows).  A round of blocks starts and ends (4.25, the scales, the output); a turn of
 // a block's waves over their chunks takes a part per tile of weights expanded, one per row of weights
 // read and one per row of x read (every block reads all of x, from L2).
-static double gemv_mt_us(const LinearArgs& a) {
+static double gemv_mt_us(const LinearJob& job) {
+  const LinearArgs& a = job.pr[0];
   const bool b4 = a.bits == 4;
   const int nw = a.m <= 32 ? 12 : 8;
   const int ck = b4 ? 128 : 64;
-  int rows = (int)((a.n + 255) / 256);
-  rows = rows < 16 ? 16 : (rows > 16 * kRowsMaxTiles ? 16 * kRowsMaxTiles : rows);
-  const int grid = (int)((a.n + rows - 1) / rows), tiles = (rows + 15) / 16;
+  int rows;
+  int64_t blocks;
+  rows_mt_split(job, &rows, &blocks);
+  const int matrices = job.glu ? 2 : 1;
+  const int grid = (int)blocks, tiles = matrices * ((rows + 15) / 16);
+  int64_t outputs = 0;
+  for (int i = 0; i < job.count; ++i) outputs += a.m * job.pr[i].n;
+  rows *= matrices;
   const int turns = (int)(((a.k + ck - 1) / ck + nw - 1) / nw);
   // bf16 with a zero point has the longest conversion
   const double longer = b4 && a.t_dtype == OFQ_BF16 && !(a.symmetric && a.w_signed) ? 1.21 : 1.0;
@@ -878,7 +851,7 @@ static double gemv_mt_us(const LinearArgs& a) {
                             : 0.10 + 0.26 * tiles + 0.31 * rows / 16 + 0.0009 * a.m * nw;
   const int rest = grid % 256, rounds = (grid + 255) / 256;
   const double scales = (double)a.k / a.group_size * rows * (a.symmetric ? 1 : 2);
-  return rounds * (4.25 + 1.4 / 4096 * scales) - 0.8 + 2.3e-6 * a.m * a.n
+  return rounds * (4.25 + 1.4 / 4096 * scales) - 0.8 + 2.3e-6 * outputs
          + turns * turn_us * (grid / 256 + (rest != 0 ? 0.83 + 0.17 * rest / 256 : 0.0));
 }
 
@@ -889,12 +862,34 @@ static double gemv_mt_us(const LinearArgs& a) {
 // from a graph.
 bool gemv_mt_preferred(const LinearArgs& a, bool have_workspace) {
   if (!gemv_mt_supported(a)) return false;
-  const double us = gemv_mt_us(a);
+  const double us = gemv_mt_us(LinearJob{&a, 1, false, nullptr, 0});
   return us < gemm_wr_us(a, have_workspace, us < 12.5 ? 3.0 : 0.5);
 }
 
 int launch_gemv_mt(hipStream_t st, const LinearArgs& a) {
-  return a.t_dtype == OFQ_BF16 ? launch_rows_mt<bf16>(st, a) : launch_rows_mt<f16>(st, a);
+  const LinearJob job{&a, 1, false, nullptr, 0};
+  return launch_rows_mt(st, job);
+}
+
+// Against one launch per problem (without a workspace: the entry points of several linears and gated units
+// have none), each by its own best kernel, and the gating's.
+int launch_gemv_mt_several(hipStream_t st, const LinearArgs* pr, int count, bool glu, void* y, int act) {
+  if (count < 2 || count > kGemvMaxProblems) return OFQ_ERR_UNSUPPORTED;
+  const LinearArgs& a = pr[0];
+  const LinearJob job{pr, count, glu, y, act};
+  double apart = glu ? 4.0 : 0.0;
+  for (int i = 0; i < count; ++i) {
+    const LinearArgs& b = pr[i];
+    if (!gemv_mt_supported(b) || b.t_dtype != a.t_dtype || b.bits != a.bits || b.w_signed != a.w_signed
+        || b.symmetric != a.symmetric || b.group_size != a.group_size || b.m != a.m || b.k != a.k
+        || (glu && (b.x != a.x || b.n != a.n))) {
+      return OFQ_ERR_UNSUPPORTED;
+    }
+    const double mt = gemv_mt_us(LinearJob{&b, 1, false, nullptr, 0}), wr = gemm_wr_us(b, false, 0.0);
+    apart += mt < wr ? mt : wr;
+  }
+  if (gemv_mt_us(job) > apart) return OFQ_ERR_UNSUPPORTED;
+  return launch_rows_mt(st, job);
 }
 
 bool gemv_wq_supported(const LinearArgs& a) {

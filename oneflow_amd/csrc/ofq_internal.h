@@ -82,6 +82,9 @@ int launch_gemv_wq(hipStream_t st, const LinearArgs& a);
 // workspace.  Not where gemm_wr is expected to take less.
 bool gemv_mt_preferred(const LinearArgs& a, bool have_workspace);
 int launch_gemv_mt(hipStream_t st, const LinearArgs& a);
+// several of them, or a gated unit's two with y = out0 * act(out1), in one launch where that is expected to
+// take less than one by one; else OFQ_ERR_UNSUPPORTED
+int launch_gemv_mt_several(hipStream_t st, const LinearArgs* problems, int count, bool glu, void* y, int act);
 
 // Groups along N (group_dim = 0), fp16 / bf16: the streaming kernel with one scale per k (any m,
 // 64 rows of x per pass over the weights), and for m > 64 with a workspace of
@@ -102,10 +105,25 @@ int launch_gemv_grouped(hipStream_t st, const LinearArgs* problems, int count);
 // not fit (caller runs the linears and the gating separately).
 int launch_gemv_glu(hipStream_t st, const LinearArgs& a, const LinearArgs& g, void* y, int act);
 
-// The ring kernel (gemv_ring.h) on one linear of up to 16 rows of x, on several that share m, k, dtype and
-// quantisation attributes, or on the two of a gated unit (glu: problems 0 and 1, then y = out0 * act(out1)).
-int launch_gemv_ring_f16(hipStream_t st, const LinearArgs* problems, int count, bool glu, void* y, int act);
-int launch_gemv_ring_bf16(hipStream_t st, const LinearArgs* problems, int count, bool glu, void* y, int act);
+// What one launch of a streaming kernel works on: one linear, several that share m, k, dtype and quantisation
+// attributes, or the two of a gated unit (problems 0 and 1 of equal n and x, then y = out0 * act(out1)).
+struct LinearJob {
+  const LinearArgs* pr;
+  int count;
+  bool glu;
+  void* y;
+  int act;
+};
+// The ring kernel (gemv_ring.h), up to 16 rows of x; OFQ_ERR_UNSUPPORTED where it is not the faster one.
+int launch_gemv_ring_f16(hipStream_t st, const LinearJob& job);
+int launch_gemv_ring_bf16(hipStream_t st, const LinearJob& job);
+// gemv_rows_mt (gemv_rows.h), 17 to 64 rows of x
+struct RowsMtPlan {
+  int grid, rows_per_block, panel_chunks, panel_groups;
+  size_t lds;
+};
+int launch_gemv_mt_f16(hipStream_t st, const LinearJob& job, const RowsMtPlan& plan);
+int launch_gemv_mt_bf16(hipStream_t st, const LinearJob& job, const RowsMtPlan& plan);
 
 // matmul_quant with few rows of a (m <= 64; k a multiple of 64): int8 MFMA with the weights
 // streamed once.

@@ -1,7 +1,8 @@
-"""The streaming kernel whose operands all come by counted copies (one linear, several, a gated unit) for 1 to
-16 rows of x: tiles of 8 and 16 rows with partial last ones, rows of K that end inside a chunk and inside a
+"""The streaming kernels for one linear, several and a gated unit.  Up to 16 rows of x, the one whose operands
+all come by counted copies: tiles of 8 and 16 rows with partial last ones, rows of K that end inside a chunk and inside a
 step, groups that are not powers of two, scale arrays that end inside a 16-byte piece, every split of the
-waves over tiles and K, and x that passes LDS in parts.
+waves over tiles and K, and x that passes LDS in parts.  17 to 64 rows: two, three and four tiles of x, one
+and two tiles of rows of each weight of a gated unit, one to four of several linears.
 
 |result - exact| <= one rounding to the dtype + (k + 2) fp32 roundings of the running sum of |x| |w~|, and w~ is
 formed exactly as groupwise_dequantize forms it."""
@@ -57,7 +58,9 @@ def test_one(m, n, k, g, dtype):
 
 
 @pytest.mark.parametrize("m,k,g,ns", [(1, 96, 32, (7, 1, 300)), (5, 1696, 32, (1111, 139, 139)), (8, 4128, 96, (4096, 17, 9)),
-                                      (9, 736, 32, (515, 16, 33)), (16, 1568, 32, (9000, 2)), (16, 64, 32, (40, 4099, 17)), (4, 11040, 32, (700, 300))])
+                                      (9, 736, 32, (515, 16, 33)), (17, 1696, 32, (1111, 139, 139)),
+                                      (33, 1184, 32, (4097, 9, 1030)), (64, 544, 32, (9000, 2200)),
+                                      (49, 224, 32, (16000, 40)), (40, 480, 96, (300, 301, 5)), (16, 1568, 32, (9000, 2)), (16, 64, 32, (40, 4099, 17)), (4, 11040, 32, (700, 300))])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_several(m, k, g, ns, dtype):
     import oneflow_amd as flow
@@ -75,7 +78,8 @@ def test_several(m, k, g, ns, dtype):
 
 @pytest.mark.parametrize("m,n,k,g", [(1, 37, 96, 32), (2, 700, 1184, 32), (8, 4671, 480, 96), (7, 9001, 224, 32),
                                      (9, 1030, 1568, 32), (16, 11008, 160, 32), (8, 300, 11040, 32),
-                                     (4, 30000, 64, 64)])
+                                     (4, 30000, 64, 64), (17, 1030, 1184, 32), (32, 5021, 480, 96), (33, 37, 2208, 32),
+                                     (48, 9001, 160, 32), (49, 2700, 544, 32), (64, 14001, 96, 32)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_gated_unit(m, n, k, g, dtype):
     """Both linears and y = hidden * relu(gate), whose only roundings are the two of T; nothing past the outputs."""
