@@ -150,6 +150,24 @@ def test_moving_average_observer_sequence(scheme, formula, dt):
     assert float(obs.moving_max[0]) == 0.0
 
 
+@pytest.mark.parametrize("slices", [1, 2, 64, 65, 256, 257, 1023, 1025, 3841, 4096, 4097, 5121])
+@pytest.mark.parametrize("dt", ["float32", "float64"])
+def test_moving_average_observer_finds_an_extreme_in_any_slice(slices, dt):
+    """One block folds the extremes of slices of 4096 elements: the largest and the smallest value
+    in the first, the last and other slices, exactly (an extreme is a copy of an element)."""
+    import torch
+    import oneflow_amd as flow
+    x = torch.zeros(slices * 4096 - 5, dtype=getattr(torch, dt), device="cuda")
+    st = torch.zeros(1, dtype=torch.int64, device="cuda")
+    for hi, lo in {(0, slices - 1), (slices - 1, 0), (slices // 2, slices // 3),
+                   (min(1024, slices - 1), min(4096, slices - 1))}:
+        x[hi * 4096 + 7], x[lo * 4096 + 4000] = 3.25, -7.5
+        mmax, mmin = torch.zeros(1, dtype=x.dtype, device="cuda"), torch.zeros(1, dtype=x.dtype, device="cuda")
+        flow._C.moving_average_min_max_observer(x, st, mmax, mmin, True, 1, "google", 8, "affine", 0.95)
+        assert (float(mmax[0]), float(mmin[0])) == (3.25, -7.5), (hi, lo)
+        x[hi * 4096 + 7] = x[lo * 4096 + 4000] = 0.0
+
+
 def test_moving_average_observer_large_and_checks():
     import torch
     import oneflow_amd as flow
