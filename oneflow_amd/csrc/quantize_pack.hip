@@ -56,6 +56,30 @@ __device__ __forceinline__ uint32_t group_max_u32(uint32_t m, int L) {
   return m;
 }
 
+// eight codes in the low bits of c (8 of them in two words, or 4 in one)
+template<int BITS>
+__device__ __forceinline__ void pack_codes8(const uint32_t (&c)[8], uint32_t (&w)[2]) {
+  auto bytes4 = [](uint32_t b0, uint32_t b1, uint32_t b2, uint32_t b3) {
+    return __builtin_amdgcn_perm(b1, b0, 0x0c0c0400u) | __builtin_amdgcn_perm(b3, b2, 0x04000c0cu);
+  };
+  if (BITS == 8) {
+    w[0] = bytes4(c[0], c[1], c[2], c[3]);
+    w[1] = bytes4(c[4], c[5], c[6], c[7]);
+  } else {
+    uint32_t p[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) p[b] = (c[2 * b] << 4) | (c[2 * b + 1] & 0xF);
+    w[0] = bytes4(p[0], p[1], p[2], p[3]);
+  }
+}
+
+// v / d from the rounded reciprocal of d, corrected twice with the exact remainder
+__device__ __forceinline__ float corrected_quotient(float v, float d, float recip) {
+  float q = v * recip;
+  q = __builtin_fmaf(__builtin_fmaf(-d, q, v), recip, q);
+  return __builtin_fmaf(__builtin_fmaf(-d, q, v), recip, q);
+}
+
 // Codes of 8 symmetric 16-bit values in 4 bytes (4 bit) or 8, for a group whose largest magnitude lies
 // well inside the exponent range: the bits a division and rint give, with fewer instructions.
 //  - v / sc and absmax / (2^(b-1) - 1) are the product with the reciprocal, corrected once with the exact
@@ -77,24 +101,55 @@ __device__ __forceinline__ void quant_codes8(u32x4 raw, float sc, uint32_t (&w)[
     if (!SIGNED) q = q + kOffset;
     c[e] = __builtin_bit_cast(uint32_t, q + 12582912.0f);
   }
-  auto bytes4 = [](uint32_t b0, uint32_t b1, uint32_t b2, uint32_t b3) {
-    return __builtin_amdgcn_perm(b1, b0, 0x0c0c0400u) | __builtin_amdgcn_perm(b3, b2, 0x04000c0cu);
-  };
-  if (BITS == 8) {
-    w[0] = bytes4(c[0], c[1], c[2], c[3]);
-    w[1] = bytes4(c[4], c[5], c[6], c[7]);
-  } else {
-    uint32_t p[4];
+  pack_codes8<BITS>(c, w);
+}
+
+// The same for 8 asymmetric values: (v - mn) / sc in fp32, rounded half to even.  `recip` is the rounded reciprocal
+// of sc, whose significand is not all ones: a quotient that is corrected with its exact remainder until it is
+// within one ulp, and once more, is then the correctly rounded one (Markstein).  A quotient that underflows on the
+// way is far below 1/2.
+template<typename T, int BITS>
+__device__ __forceinline__ void quant_codes8_asym(u32x4 raw, float mn, float sc, float recip,
+                                                  uint32_t (&w)[2]) {
+  uint32_t c[8];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) p[b] = (c[2 * b] << 4) | (c[2 * b + 1] & 0xF);
-    w[0] = bytes4(p[0], p[1], p[2], p[3]);
+  for (int e = 0; e < 8; ++e) {
+    const float d = raw16_to_float<T>((uint16_t)(raw[e / 2] >> (16 * (e & 1)))) - mn;
+    c[e] = __builtin_bit_cast(uint32_t, corrected_quotient(d, sc, recip) + 12582912.0f);
   }
+  pack_codes8<BITS>(c, w);
+}
+
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+// 16-bit floating-point patterns <-> unsigned integers in the same order (-0 below +0, NaNs outermost)
+__device__ __forceinline__ u16x2 ordered_keys(uint32_t two) {
+  typedef short i16x2 __attribute__((ext_vector_type(2)));
+  const i16x2 sign = __builtin_bit_cast(i16x2, two) >> 15;
+  return __builtin_bit_cast(u16x2, two ^ (__builtin_bit_cast(uint32_t, sign) | 0x80008000u));
+}
+__device__ __forceinline__ uint16_t key_pattern(uint32_t key) {
+  return (uint16_t)(key ^ ((key & 0x8000u) != 0 ? 0x8000u : 0xFFFFu));
+}
+
+// both halves' largest values of L consecutive lanes (a power of two; all lanes of the wave take part)
+__device__ __forceinline__ u16x2 group_max_u16x2(u16x2 m, int L) {
+  auto fold = [&](int other) { m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, other)); };
+  auto bits = [&]() { return __builtin_bit_cast(int, m); };
+  if (L >= 2) fold(__builtin_amdgcn_update_dpp(0, bits(), 0xB1, 0xF, 0xF, false));    // quad_perm [1,0,3,2]
+  if (L >= 4) fold(__builtin_amdgcn_update_dpp(0, bits(), 0x4E, 0xF, 0xF, false));    // quad_perm [2,3,0,1]
+  if (L >= 8) fold(__builtin_amdgcn_update_dpp(0, bits(), 0x141, 0xF, 0xF, false));   // row_half_mirror
+  if (L >= 16) fold(__builtin_amdgcn_update_dpp(0, bits(), 0x140, 0xF, 0xF, false));  // row_mirror
+  if (L >= 32) fold(__shfl_xor(bits(), 16, kWave));
+  if (L >= 64) fold(__shfl_xor(bits(), 32, kWave));
+  return m;
 }
 
 // groups along K, g = 8 * L with L a power of two <= 64, rows 16-byte aligned.  Bound by its vector
 // instructions until symmetric 16-bit groups took their largest magnitude as an integer maximum of bit
 // patterns and the codes from quant_codes8: 11008 x 4096 fp16 to 4 bit, groups of 128, 27.7 -> 20.1 us
-// (5.6 TB/s).  Four packs a thread, all requested first, had made it 31.5 us: it was not short of requests.
+// (5.6 TB/s); asymmetric groups the extremes as two integer maxima in one register and the codes from
+// quant_codes8_asym: the same shape, 31.5 -> 25.3 us (4.5 TB/s); 4096 x 4096 13.5 -> 12.3.  Four packs a thread, all requested first, had made it 31.5 us: it was not short of requests.
 template<typename T, bool SYM, bool SIGNED, int BITS>
 __global__ void __launch_bounds__(256)
 quantize_pack_rows(const typename TT<T>::storage* __restrict__ x, uint8_t* __restrict__ q,
@@ -116,7 +171,6 @@ quantize_pack_rows(const typename TT<T>::storage* __restrict__ x, uint8_t* __res
   }
   if constexpr (SYM && sizeof(S) == 2) {
     const u32x4 bits = *reinterpret_cast<const u32x4*>(raw);
-    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
     u16x2 m2 = __builtin_bit_cast(u16x2, bits[0] & 0x7FFF7FFFu);
 #pragma unroll
     for (int i = 1; i < 4; ++i)
@@ -133,6 +187,40 @@ quantize_pack_rows(const typename TT<T>::storage* __restrict__ x, uint8_t* __res
       quant_codes8<T, SIGNED, BITS>(bits, sc, w);
       if (!live) return;
       if (l == 0) TT<T>::store(&scale[grp], sc);
+      if (BITS == 8) {
+        *reinterpret_cast<u32x2*>(q + base) = u32x2{w[0], w[1]};
+      } else {
+        *reinterpret_cast<uint32_t*>(q + (base >> 1)) = w[0];
+      }
+      return;
+    }
+  }
+  if constexpr (!SYM && sizeof(S) == 2) {
+    const u32x4 bits = *reinterpret_cast<const u32x4*>(raw);
+    u16x2 hi = ordered_keys(bits[0]), lo = hi;
+#pragma unroll
+    for (int i = 1; i < 4; ++i) {
+      const u16x2 key = ordered_keys(bits[i]);
+      hi = __builtin_elementwise_max(hi, key);
+      lo = __builtin_elementwise_min(lo, key);
+    }
+    const uint16_t top = hi[0] > hi[1] ? hi[0] : hi[1], low = lo[0] < lo[1] ? lo[0] : lo[1];
+    const u16x2 ends = group_max_u16x2(u16x2{top, (uint16_t)~low}, L);
+    const uint32_t key_max = ends[0], key_min = (uint16_t)~ends[1];
+    // finite (fp16), of magnitudes up to 2^60 (bf16); NaN and infinity lie outside
+    constexpr uint32_t kMost = TT<T>::dtype == OFQ_F16 ? 0x7BFFu : 0x5D80u;
+    const float mx = raw16_to_float<T>(key_pattern(key_max)), mn = raw16_to_float<T>(key_pattern(key_min));
+    constexpr float kMax = (float)((1 << BITS) - 1);
+    const float sc = corrected_quotient(mx - mn, kMax, 1.0f / kMax);
+    if (key_max <= (0x8000u | kMost) && key_min >= (0x7FFFu - kMost) && sc >= 0x1p-60f
+        && (__builtin_bit_cast(uint32_t, sc) & 0x7FFFFFu) != 0x7FFFFFu) {
+      uint32_t w[2];
+      quant_codes8_asym<T, BITS>(bits, mn, sc, 1.0f / sc, w);
+      if (!live) return;
+      if (l == 0) {
+        TT<T>::store(&scale[grp], sc);
+        TT<T>::store(&zero[grp], mn);
+      }
       if (BITS == 8) {
         *reinterpret_cast<u32x2*>(q + base) = u32x2{w[0], w[1]};
       } else {

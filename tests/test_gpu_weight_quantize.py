@@ -69,6 +69,38 @@ def test_symmetric_fp16_groups_of_arbitrary_bit_patterns(bits, signed):
     assert np.array_equal(s.view(np.uint16)[rows], sr.view(np.uint16)[rows])
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("g", [8, 16, 32, 64, 128, 256, 512])
+@pytest.mark.parametrize("t", ["f16", "bf16"])
+def test_asymmetric_16bit_groups_of_arbitrary_bit_patterns(t, g, bits):
+    """Asymmetric quantisation of 16-bit weights finds the extremes in integers and divides through
+    a twice corrected multiplication with the reciprocal, where the scale's range allows it: groups of
+    random bit patterns (every exponent, subnormals, both zeros, the largest values), groups of nearly
+    equal values, constant groups and infinities, against the oracle's `(x - min) / scale`, bit for bit."""
+    rng = np.random.default_rng(g + bits)
+    rows = 2 ** 18 // g + 3
+    p = rng.integers(0, 65536, size=(rows, g)).astype(np.uint16)
+    exponent, top = (0x7C00, 10) if t == "f16" else (0x7F80, 7)
+    p[(p & exponent) == exponent] &= np.uint16(0xFFFF ^ (1 << top))  # no infinity and no NaN yet
+    p[rows // 8:] = (p[rows // 8:] & np.uint16(0xFFFF ^ exponent)) | (
+        rng.integers(1, exponent >> top, size=(rows - rows // 8, 1)).astype(np.uint16) << np.uint16(top))
+    p[rows // 4:rows // 2] &= np.uint16(0x7FFF)                      # one sign
+    p[rows // 2:rows // 2 + 50] |= np.uint16(0x8000)
+    p[rows // 2 + 50:rows // 2 + 60] &= np.uint16(0xFFFF ^ 0x7E)     # few distinct values
+    p[0], p[1], p[2] = 0, p[2, 0], 0x8000                            # constant groups
+    p[3, 0], p[4, 1], p[5, 2] = exponent, 0x8000 | exponent, 1       # infinities; one subnormal
+    x = p.view(np.float16) if t == "f16" else p
+    qr, sr, zr = O.groupwise_quantize(x, bits, False, 1, g, False)
+    q, s, z = _run(x, bits, False, 1, g, False)
+    wide = O.to_f32(x)
+    with np.errstate(over="ignore"):
+        keep = np.isfinite(wide.max(1) - wide.min(1))  # elsewhere the codes come from inf / inf
+    assert keep.sum() > rows * 0.8 and not keep[3:5].any()
+    assert np.array_equal(s.view(np.uint16), sr.view(np.uint16))
+    assert np.array_equal(O.to_f32(z)[keep], O.to_f32(zr)[keep])
+    assert np.array_equal(q.view(np.uint8)[keep], qr.view(np.uint8)[keep])
+
+
 def test_constant_and_zero_groups_and_ties():
     """scale 0 groups get the code of value 0; exact .5 quotients round to even."""
     x = np.zeros((4, 64), np.float32)
