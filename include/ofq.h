@@ -266,6 +266,17 @@ int ofq_fused_layer_norm_quantization(void* stream, const void* x, const void* g
                                       float* zero_point, int t_dtype, int64_t rows, int64_t cols,
                                       double epsilon, int quantization_bit, int statistics,
                                       void* workspace, size_t workspace_bytes);
+/*
+ * The same for fp16 and bf16 rows of any multiple of 8 up to 16384 elements, gamma and beta each optional,
+ * 16-byte aligned (codes: 8); codes and scale carry the bits of the two ops here as well.  Any other case
+ * returns OFQ_ERR_UNSUPPORTED.  Same workspace.
+ */
+int ofq_fused_layer_norm_quantization_any_row(void* stream, const void* x, const void* gamma,
+                                              const void* beta, void* codes, float* scale,
+                                              float* zero_point, int t_dtype, int64_t rows,
+                                              int64_t cols, double epsilon, int quantization_bit,
+                                              int statistics, void* workspace,
+                                              size_t workspace_bytes);
 
 /*
  * groupwise_quantize: the producer of the weight format of the two ops above.

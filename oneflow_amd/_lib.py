@@ -55,6 +55,8 @@ SIGNATURES = {
                                                          ctypes.c_double, _i, _i, _vp, _sz]),
     "ofq_fused_layer_norm_quantization": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i64, _i64,
                                                ctypes.c_double, _i, _i, _vp, _sz]),
+    "ofq_fused_layer_norm_quantization_any_row": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i64, _i64,
+                                                       ctypes.c_double, _i, _i, _vp, _sz]),
     "ofq_fused_layer_norm_quantization_workspace_bytes": (_sz, [_i, _i64, _i64]),
     "ofq_grouped_linear_gq": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i,
                                    _i, _i, _i64]),

@@ -736,6 +736,7 @@ ln_observer_finalize(const float* __restrict__ part, int64_t n, int bits,
 //           again -- from L2 where the first kernel left them: the same wave of the same block
 //           took them there --, forms y with the stored statistics exactly as the first kernel
 //           did, and quantises it the way quantize_half_to_bytes_kernel does.
+// Up to 8 rows go to ln_quant_rows below, which needs one launch.
 // The codes are those of fused_layer_norm_min_max_observer followed by quantization (symmetric,
 // per layer) of its y, bit for bit; traffic is x once from HBM, x once more from L2 and the codes
 // (25 MB at 2048 x 4096 where the two ops move 58.7 MB).
@@ -773,6 +774,60 @@ struct LnRowF16 {
     return t;
   }
 };
+
+// How the codes of one tensor follow from its scale s = absmax / upper: rint(y / s), clamped, NaN -> 0.
+//  kLnDivide : the division and the clamp, for any s
+//  kLnFast2  : s within 2^+-60: the product with the reciprocal, corrected twice (div_of_half_value)
+//  kLnFast1  : 8 bits and the same s: corrected once, which gives the same bits for every |y| <= absmax
+//              (quantize_pack.hip, quant_codes8: all fp16 pairs compared; bf16 significands are among them, and
+//              a quotient that underflows on the way rounds to 0)
+// A fast quotient lies within the codes (y is finite: an infinite one makes the scale infinite), so that
+// adding 1.5 * 2^23 leaves the code in the low byte; a NaN that came from a 16-bit value has zeros there.
+enum { kLnDivide, kLnFast2, kLnFast1 };
+__device__ __forceinline__ int ln_code_mode(float s, int bits) {
+  const float mag = __builtin_fabsf(s);
+  return !(mag >= 0x1p-60f && mag <= 0x1p60f) ? kLnDivide : bits == 8 ? kLnFast1 : kLnFast2;
+}
+template<typename T, int MODE>
+__device__ __forceinline__ u32x2 ln_codes8(u32x4 y, float s, float recip, int lo, int hi) {
+  RawPack<T> r;
+  r.q[0] = y;
+  float v[8];
+  widen<T>(r, v);
+  uint32_t words[2];
+#pragma unroll
+  for (int e4 = 0; e4 < 8; e4 += 4) {
+    uint32_t b[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float a = v[e4 + j];
+      if constexpr (MODE == kLnDivide) {
+        const float t = __builtin_rintf(a / s);
+        int c;
+        asm("v_cvt_i32_f32 %0, %1" : "=v"(c) : "v"(t));  // saturates; NaN -> 0
+        b[j] = (uint32_t)clamp_i32(c, lo, hi);
+      } else {
+        float q = a * recip;
+        q = __builtin_fmaf(__builtin_fmaf(-s, q, a), recip, q);
+        if (MODE == kLnFast2) q = __builtin_fmaf(__builtin_fmaf(-s, q, a), recip, q);
+        b[j] = __builtin_bit_cast(uint32_t, q + 12582912.0f);
+      }
+    }
+    words[e4 / 4] = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u)
+                    | __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu);
+  }
+  return u32x2{words[0], words[1]};
+}
+
+// f(constant) for the mode of this scale, taken once per wave: inside a loop every quotient would be computed
+// and one selected
+template<typename F>
+__device__ __forceinline__ void ln_with_mode(float s, int bits, F&& f) {
+  const int mode = ln_code_mode(s, bits);
+  if (mode == kLnFast1) f(std::integral_constant<int, kLnFast1>());
+  else if (mode == kLnFast2) f(std::integral_constant<int, kLnFast2>());
+  else f(std::integral_constant<int, kLnDivide>());
+}
 
 template<int NP, bool EXACT>
 __global__ void __launch_bounds__(kLnqBlock)
@@ -953,14 +1008,9 @@ ln_quant_second(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gam
     *zero_point = 0.0f;
   }
   if (!active) return;
-  // quantisation of quantize_half_to_bytes_kernel, symmetric scheme
-  const float mag = __builtin_fabsf(s);
-  const bool recip_ok = mag >= 0x1p-60f && mag <= 0x1p60f;
-  const float recip = recip_ok ? 1.0f / s : 0.f;
+  const float recip = 1.0f / s;
   const int hi = (int)upper, lo = -hi - 1;
-  // (the branch on the scale's range is taken once per wave: inside the loop both quotients
-  // would be computed for every element and one of them selected)
-  auto walk = [&](auto fast) {
+  ln_with_mode(s, bits, [&](auto mode) {
     for (int64_t row = gw; row < rows; row += nwaves) {
       if (row != gw) {
         const uint16_t* xr = x + row * kCols + pack0 * 512 + lane * 8;
@@ -984,41 +1034,342 @@ ln_quant_second(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gam
         // (held as four packed registers: otherwise the affine is emitted element by element)
         u32x4 yb = __builtin_bit_cast(u32x4, prm.out(d, inv, i, params, lane));
         asm volatile("" : "+v"(yb[0]), "+v"(yb[1]), "+v"(yb[2]), "+v"(yb[3]));
-        const f16x8 y = __builtin_bit_cast(f16x8, yb);
-        uint32_t words[2];
-#pragma unroll
-        for (int e4 = 0; e4 < 8; e4 += 4) {
-          uint32_t b[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float v = (float)y[e4 + j];
-            float q;
-            if constexpr (decltype(fast)::value) {
-              // (y is finite here: an infinite y makes the scale infinite, which is the other
-              // branch)
-              q = div_of_finite_half_value(v, s, recip);
-            } else {
-              q = v / s;
-            }
-            const float t = __builtin_rintf(q);
-            int c;
-            asm("v_cvt_i32_f32 %0, %1" : "=v"(c) : "v"(t));  // saturates; NaN -> 0
-            b[j] = (uint32_t)clamp_i32(c, lo, hi);
-          }
-          const uint32_t lo2 = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u);
-          const uint32_t hi2 = __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu);
-          words[e4 / 4] = lo2 | hi2;
-        }
-        const u32x2 w2 = {words[0], words[1]};
+        const u32x2 w2 = ln_codes8<f16, decltype(mode)::value>(yb, s, recip, lo, hi);
         __builtin_nontemporal_store(w2, reinterpret_cast<u32x2*>(cr + i * 512));
       }
     }
-  };
-  if (recip_ok) {
-    walk(std::true_type());
+  });
+}
+
+// ---------------------------------------------------------------------------------------------
+// The same composition for fp16 and bf16 rows of any 8 * n elements up to 16384, gamma and beta each
+// optional.  A row is taken by WPR waves: one (the arithmetic of ln_observer_wave_rows; DOT: the
+// fp16 row sum of ln_observer_wave_full) or four (that of ln_observer_rows), so scale and codes carry
+// the bits of the two ops.
+//   ln_quant_rows<ONE = false> + ln_quant_codes : two launches; y is formed twice and never stored
+//   ln_quant_rows<ONE = true>                   : one launch of one block, for as many rows as it
+//     holds (8, or 4 of more than 4096 elements): the rows wait in registers for the block's maximum
+// Time of a call of the two ops and of this: 1 x 2432 fp16 13.0 -> 6.4 us, 8 x 1280 bf16 13.6 -> 6.2, 64 x 6080
+// fp16 13.3 -> 9.2, 1024 x 6080 19.1 -> 14.0, 4096 x 4096 bf16 44 -> 36 (host-bound up to some hundred rows:
+// three launches and two allocations became one or two launches).  Many rows are bound by the vector units
+// of both kernels: 8192 x 2432 fp16 17.9 + 16.0 us, where their traffic takes about 14.
+// ---------------------------------------------------------------------------------------------
+constexpr int ln_rows_per_block(int wpr, bool one) { return wpr == 1 ? 8 : one ? 4 : 1; }
+
+template<typename T>
+__device__ __forceinline__ RawPack<T> load_pack(const uint16_t* p) {
+  return load_raw<T>(reinterpret_cast<const typename TT<T>::storage*>(p));
+}
+
+// y of 8 elements from their deviations x - mean, as ln_observer_wave_rows forms it
+template<typename T>
+__device__ __forceinline__ u32x4 ln_out8(const float* d, float inv, bool has_gamma, const RawPack<T>& g,
+                                         bool has_beta, const RawPack<T>& b) {
+  if constexpr (TT<T>::dtype == OFQ_F16) {
+    f16x8 t;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) t[e] = (f16)normalised<f16>(d[e], inv);
+    if (has_gamma) t = t * __builtin_bit_cast(f16x8, g.q[0]);
+    if (has_beta) t = t + __builtin_bit_cast(f16x8, b.q[0]);
+    u32x4 bits = __builtin_bit_cast(u32x4, t);
+    // (held as four packed registers: otherwise the affine is emitted element by element)
+    asm volatile("" : "+v"(bits[0]), "+v"(bits[1]), "+v"(bits[2]), "+v"(bits[3]));
+    return bits;
   } else {
-    walk(std::false_type());
+    float gf[8], bf[8], o[8];
+    if (has_gamma) widen<T>(g, gf);
+    if (has_beta) widen<T>(b, bf);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float t = normalised<T>(d[e], inv);
+      if (has_gamma) t = TT<T>::round(t * gf[e]);
+      if (has_beta) t = TT<T>::round(t + bf[e]);
+      o[e] = t;
+    }
+    return narrow<T>(o).q[0];
   }
+}
+
+// the largest |y| seen, NaN passed over: fp16 in eight packed maxima, bf16 in one float
+template<typename T>
+struct LnAbsMax {
+  f16x8 packed = {(f16)0.0f, (f16)0.0f, (f16)0.0f, (f16)0.0f, (f16)0.0f, (f16)0.0f, (f16)0.0f, (f16)0.0f};
+  float one = 0.0f;
+  __device__ __forceinline__ void take(u32x4 y) {
+    if constexpr (TT<T>::dtype == OFQ_F16) {
+      const u32x4 ab = {y[0] & 0x7FFF7FFFu, y[1] & 0x7FFF7FFFu, y[2] & 0x7FFF7FFFu, y[3] & 0x7FFF7FFFu};
+      packed = __builtin_elementwise_max(packed, __builtin_bit_cast(f16x8, ab));
+    } else {
+      RawPack<T> r;
+      r.q[0] = y;
+      float v[8];
+      widen<T>(r, v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) one = fmaxf(one, fabsf(v[e]));
+    }
+  }
+  __device__ __forceinline__ float value() const {
+    float m = one;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) m = fmaxf(m, (float)packed[e]);
+    return m;
+  }
+};
+
+// the sum over the WPR waves of a row, in the order of block_reduce (every thread of the block calls it)
+template<int WPR, typename V>
+__device__ __forceinline__ V row_sum(V v, V* smem) {
+  v = wave_reduce(v, OpSum());
+  if constexpr (WPR == 1) return v;
+  const int wave = threadIdx.x / kWave;
+  __syncthreads();
+  if ((threadIdx.x & (kWave - 1)) == 0) smem[wave] = v;
+  __syncthreads();
+  const int w0 = wave / WPR * WPR;
+  V r = smem[w0];
+#pragma unroll
+  for (int i = 1; i < WPR; ++i) r = r + smem[w0 + i];
+  return r;
+}
+
+template<typename T, int NP, int WPR, bool DOT, bool EXACT, bool ONE>
+__global__ void __launch_bounds__(ln_rows_per_block(WPR, ONE) * WPR * kWave)
+ln_quant_rows(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma,
+              const uint16_t* __restrict__ beta, float* __restrict__ block_absmax,
+              float* __restrict__ stats, int8_t* __restrict__ codes, float* __restrict__ scale,
+              float* __restrict__ zero_point, int64_t rows, int cols, double eps64, int bits) {
+  constexpr int kRows = ln_rows_per_block(WPR, ONE);
+  constexpr int kWaves = kRows * WPR;
+  constexpr int kStep = WPR * kWave;  // packs between two of a thread
+  __shared__ float smem[kWaves];
+  __shared__ double smem64[EXACT ? kWaves : 1];
+  const float eps = (float)eps64;
+  const int t = threadIdx.x % kStep;
+  const int npacks = cols / 8;
+  const int per_block = ONE ? kRows : (int)blockDim.x / kStep;
+  const int64_t first = (int64_t)blockIdx.x * per_block + threadIdx.x / kStep;
+  const int64_t stride = (int64_t)gridDim.x * per_block;
+  // rows of a block in turns that all its threads take (row_sum holds barriers); a thread whose row lies past
+  // the last one reads nothing
+  const int64_t turns = ONE ? 1 : (rows - (int64_t)blockIdx.x * per_block + stride - 1) / stride;
+  // gamma and beta: one copy in LDS for the rows of a block, or in the registers of the only row's threads
+  constexpr bool kShared = kRows > 1;
+  __shared__ u32x4 params[kShared ? 2 * NP * kStep : 1];
+  RawPack<T> gr[kShared ? 1 : NP], br[kShared ? 1 : NP], v[NP];
+  bool in[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    in[i] = t + i * kStep < npacks;
+    if constexpr (!kShared) {
+      if (in[i] && gamma) gr[i] = load_pack<T>(gamma + (t + i * kStep) * 8);
+      if (in[i] && beta) br[i] = load_pack<T>(beta + (t + i * kStep) * 8);
+    }
+  }
+  auto request = [&](int64_t row) {
+    const uint16_t* xr = x + (row < rows ? row : 0) * cols;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      if (in[i] && row < rows) v[i] = load_pack<T>(xr + (t + i * kStep) * 8);
+      else v[i].q[0] = u32x4{0u, 0u, 0u, 0u};
+    }
+  };
+  request(first);
+  if constexpr (kShared) {
+    for (int p = threadIdx.x; p < npacks; p += blockDim.x) {
+      if (gamma) params[p] = load_pack<T>(gamma + p * 8).q[0];
+      if (beta) params[NP * kStep + p] = load_pack<T>(beta + p * 8).q[0];
+    }
+    __syncthreads();
+  }
+  // The row is held in storage format and widened again in every pass: without the empty asm the compiler
+  // keeps the widened floats too, twice the registers (176 to 240 of them for rows of 4096).
+  auto hold_pack = [](RawPack<T>& r) {
+    u32x4 h = r.q[0];
+    asm volatile("" : "+v"(h[0]), "+v"(h[1]), "+v"(h[2]), "+v"(h[3]));
+    r.q[0] = h;
+  };
+  auto hold = [&]() {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) hold_pack(v[i]);
+  };
+  LnAbsMax<T> amax8;
+  float mean = 0.0f, inv = 0.0f;
+  for (int64_t turn = 0; turn < turns; ++turn) {
+    const int64_t row = first + turn * stride;
+    const bool live = row < rows;
+    if (turn != 0) request(row);
+    // (an element past the row adds a zero to the sum and, skipped, nothing to the squares)
+    float sum = 0.0f;
+    double sum64 = 0.0;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      float f[8];
+      widen<T>(v[i], f);
+      if constexpr (EXACT) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum64 += (double)f[e];
+      } else if constexpr (DOT) {
+        uint32_t ones_bits = 0x3c003c00u;  // (1, 1) held in a register, see ln_observer_wave_full
+        asm volatile("" : "+v"(ones_bits));
+        const f16x2 ones = __builtin_bit_cast(f16x2, ones_bits);
+        const f16x8 h = __builtin_bit_cast(f16x8, v[i].q[0]);
+        sum = __builtin_amdgcn_fdot2(__builtin_shufflevector(h, h, 0, 1), ones, sum, false);
+        sum = __builtin_amdgcn_fdot2(__builtin_shufflevector(h, h, 2, 3), ones, sum, false);
+        sum = __builtin_amdgcn_fdot2(__builtin_shufflevector(h, h, 4, 5), ones, sum, false);
+        sum = __builtin_amdgcn_fdot2(__builtin_shufflevector(h, h, 6, 7), ones, sum, false);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum += f[e];
+      }
+    }
+    if constexpr (EXACT) {
+      sum64 = row_sum<WPR>(sum64, smem64);
+      hold();
+      const double mean64 = sum64 / (double)cols;
+      double q = 0.0;
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        if (!in[i]) continue;
+        float f[8];
+        widen<T>(v[i], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const double d = (double)f[e] - mean64;
+          q = __builtin_fma(d, d, q);
+        }
+      }
+      q = row_sum<WPR>(q, smem64);
+      mean = (float)mean64;
+      inv = exact_inv(q, (double)cols, eps64);
+    } else {
+      sum = row_sum<WPR>(sum, smem);
+      hold();
+      mean = sum / (float)cols;
+      float m2 = 0.0f;
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        if (!in[i]) continue;
+        float f[8];
+        widen<T>(v[i], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float d = f[e] - mean;
+          m2 = __builtin_fmaf(d, d, m2);
+        }
+      }
+      m2 = row_sum<WPR>(m2, smem);
+      const float var = fmaxf(m2 / (float)cols, 0.0f);
+      inv = 1.0f / __builtin_sqrtf(var + eps);
+    }
+    hold();
+    if constexpr (!ONE) {
+      if (t == 0 && live) {
+        stats[2 * row] = mean;
+        stats[2 * row + 1] = inv;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      if (!in[i] || !live) continue;
+      float d[8];
+      widen<T>(v[i], d);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) d[e] = d[e] - mean;
+      RawPack<T> g, b;
+      if constexpr (kShared) {
+        g.q[0] = params[t + i * kStep];
+        b.q[0] = params[NP * kStep + t + i * kStep];
+      } else {
+        hold_pack(gr[i]), hold_pack(br[i]);  // (or their floats are kept over the turns)
+        g = gr[i], b = br[i];
+      }
+      const u32x4 y = ln_out8<T>(d, inv, gamma != nullptr, g, beta != nullptr, b);
+      amax8.take(y);
+      if constexpr (ONE) v[i].q[0] = y;
+    }
+  }
+  const float amax = block_reduce(amax8.value(), OpMax(), smem);
+  if constexpr (!ONE) {
+    if (threadIdx.x == 0) block_absmax[blockIdx.x] = amax;
+  } else {
+    const float upper = (float)(1 << (bits - 1)) - 1.0f;
+    const float s = amax / upper;
+    if (threadIdx.x == 0) {
+      *scale = s;
+      *zero_point = 0.0f;
+    }
+    if (first >= rows) return;
+    const float recip = 1.0f / s;
+    const int hi = (int)upper, lo = -hi - 1;
+    ln_with_mode(s, bits, [&](auto mode) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        if (!in[i]) continue;
+        *reinterpret_cast<u32x2*>(codes + first * cols + (t + i * kStep) * 8) =
+            ln_codes8<T, decltype(mode)::value>(v[i].q[0], s, recip, lo, hi);
+      }
+    });
+  }
+}
+
+// Codes from the statistics of ln_quant_rows.  A thread keeps one pack of gamma and of beta and walks the rows
+// blockIdx.y, + gridDim.y, ..., U of them requested at once; every block folds the partial maxima into the
+// scale by itself.
+constexpr int kLnCodesBlock = 256;
+template<typename T, int U>
+__global__ void __launch_bounds__(kLnCodesBlock)
+ln_quant_codes(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma,
+               const uint16_t* __restrict__ beta, const float* __restrict__ part, int nparts,
+               const float* __restrict__ stats, int8_t* __restrict__ codes, float* __restrict__ scale,
+               float* __restrict__ zero_point, int64_t rows, int cols, int bits) {
+  __shared__ float smem[kLnCodesBlock / kWave];
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  const bool in = p < cols / 8;
+  const int at = in ? p * 8 : 0;
+  RawPack<T> v[U], g, b;
+  float mean[U], inv[U];
+  auto request = [&](int64_t row0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t row = row0 + u * (int64_t)gridDim.y;
+      const int64_t r = row < rows ? row : blockIdx.y;
+      v[u] = load_pack<T>(x + r * cols + at);
+      mean[u] = stats[2 * r];
+      inv[u] = stats[2 * r + 1];
+    }
+  };
+  float amax = 0.0f;
+  for (int i = threadIdx.x; i < nparts; i += blockDim.x) amax = fmaxf(amax, part[i]);
+  request(blockIdx.y);
+  if (gamma) g = load_pack<T>(gamma + at);
+  if (beta) b = load_pack<T>(beta + at);
+  amax = block_reduce(amax, OpMax(), smem);
+  const float upper = (float)(1 << (bits - 1)) - 1.0f;
+  const float s = amax / upper;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+    *scale = s;
+    *zero_point = 0.0f;
+  }
+  if (!in) return;
+  const float recip = 1.0f / s;
+  const int hi = (int)upper, lo = -hi - 1;
+  ln_with_mode(s, bits, [&](auto mode) {
+    for (int64_t row0 = blockIdx.y; row0 < rows; row0 += U * (int64_t)gridDim.y) {
+      if (row0 != blockIdx.y) request(row0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t row = row0 + u * (int64_t)gridDim.y;
+        if (row >= rows) break;
+        float d[8];
+        widen<T>(v[u], d);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) d[e] = d[e] - mean[u];
+        const u32x4 y = ln_out8<T>(d, inv[u], gamma != nullptr, g, beta != nullptr, b);
+        *reinterpret_cast<u32x2*>(codes + row * cols + at) =
+            ln_codes8<T, decltype(mode)::value>(y, s, recip, lo, hi);
+      }
+    }
+  });
 }
 
 // host-side rounding of a float to T (round to nearest even)
@@ -1232,19 +1583,92 @@ extern "C" int ofq_fused_skip_layer_norm_min_max_observer(
                   workspace_bytes);
 }
 
+
+namespace ofq {
+namespace {
+
+struct LnQuantArgs {
+  const uint16_t *x, *gamma, *beta;
+  float *part, *stats;
+  int8_t* codes;
+  float *scale, *zero_point;
+  int64_t rows;
+  int cols;
+  double eps;
+  int bits;
+};
+
+template<typename T, int NP, int WPR, bool DOT, bool EXACT>
+void launch_ln_quant_rows(hipStream_t st, const LnQuantArgs& a) {
+  constexpr int kOne = ln_rows_per_block(WPR, true), kMany = ln_rows_per_block(WPR, false);
+  // more than two bf16 rows of four waves keep one CU busy longer than a second launch costs (4 x 8192:
+  // 10.6 us a call in one launch, 9.2 in two; 8 x 4096, a wave to a row: 10.5 and 12.1)
+  constexpr int kMostOne = TT<T>::dtype == OFQ_BF16 && WPR > 1 ? kOne / 2 : kOne;
+  if constexpr (NP * WPR <= 16) {
+    if (a.rows <= kMostOne) {
+      ln_quant_rows<T, NP, WPR, DOT, EXACT, true><<<1, kOne * WPR * kWave, 0, st>>>(
+          a.x, a.gamma, a.beta, a.part, a.stats, a.codes, a.scale, a.zero_point, a.rows, a.cols, a.eps, a.bits);
+      return;
+    }
+  }
+  if constexpr (!DOT) {
+    // a row to a block until every CU has one, to a SIMD until those have one, then 16 waves per CU
+    const int per_block = a.rows <= 256 ? 1 : a.rows <= 1024 && kMany > 4 ? 4 : kMany;
+    const int64_t blocks = (a.rows + per_block - 1) / per_block, most = 4096 / (kMany * WPR);
+    const int grid = (int)(blocks < most ? blocks : most);
+    ln_quant_rows<T, NP, WPR, false, EXACT, false><<<grid, per_block * WPR * kWave, 0, st>>>(
+        a.x, a.gamma, a.beta, a.part, a.stats, a.codes, a.scale, a.zero_point, a.rows, a.cols, a.eps, a.bits);
+    const int packs = a.cols / 8;
+    const int bx = (packs + kLnCodesBlock - 1) / kLnCodesBlock;
+    const int threads = ((packs + bx - 1) / bx + kWave - 1) / kWave * kWave;
+    const int most_y = 8192 / (bx * threads / kWave);
+    if (a.rows <= most_y) {
+      ln_quant_codes<T, 1><<<dim3(bx, (unsigned)a.rows), threads, 0, st>>>(
+          a.x, a.gamma, a.beta, a.part, grid, a.stats, a.codes, a.scale, a.zero_point, a.rows, a.cols, a.bits);
+    } else {
+      const int64_t turns = (a.rows + 4 * (int64_t)most_y - 1) / (4 * (int64_t)most_y);
+      const unsigned by = (unsigned)((a.rows + 4 * turns - 1) / (4 * turns));
+      ln_quant_codes<T, 4><<<dim3(bx, by), threads, 0, st>>>(
+          a.x, a.gamma, a.beta, a.part, grid, a.stats, a.codes, a.scale, a.zero_point, a.rows, a.cols, a.bits);
+    }
+  }
+}
+
+template<typename T, bool EXACT>
+void launch_ln_quant_any(hipStream_t st, const LnQuantArgs& a) {
+  const int packs = a.cols / 8;
+  if (packs <= kWave) launch_ln_quant_rows<T, 1, 1, false, EXACT>(st, a);
+  else if (packs <= 2 * kWave) launch_ln_quant_rows<T, 2, 1, false, EXACT>(st, a);
+  else if (packs <= 4 * kWave) launch_ln_quant_rows<T, 4, 1, false, EXACT>(st, a);
+  else if (packs <= 8 * kWave) launch_ln_quant_rows<T, 8, 1, false, EXACT>(st, a);
+  else if (packs <= 16 * kWave) launch_ln_quant_rows<T, 4, 4, false, EXACT>(st, a);
+  else launch_ln_quant_rows<T, 8, 4, false, EXACT>(st, a);
+}
+
+// the shapes ln_quant_first and ln_quant_second take
+bool ln_quant_full(const void* x, const void* gamma, const void* beta, const void* codes, int t_dtype,
+                   int64_t cols) {
+  const int64_t np = cols / 512;
+  return t_dtype == OFQ_F16 && gamma != nullptr && beta != nullptr && cols % 512 == 0
+         && (np == 1 || np == 2 || np == 4 || np == 8) && ofq_aligned16(x) && ofq_aligned16(gamma)
+         && ofq_aligned16(beta) && (reinterpret_cast<uintptr_t>(codes) & 7u) == 0;
+}
+
+}  // namespace
+}  // namespace ofq
+
 extern "C" size_t ofq_fused_layer_norm_quantization_workspace_bytes(int, int64_t rows, int64_t) {
   // [partial maxima: rows floats, padded to 16 bytes][(mean, inv) of every row]
   return rows > 0 ? (((size_t)rows * sizeof(float) + 15) & ~(size_t)15) + (size_t)rows * 2 * sizeof(float)
                   : 0;
 }
 
-extern "C" int ofq_fused_layer_norm_quantization(void* stream, const void* x, const void* gamma,
-                                                 const void* beta, void* codes, float* scale,
-                                                 float* zero_point, int t_dtype, int64_t rows,
-                                                 int64_t cols, double epsilon, int quantization_bit,
-                                                 int statistics, void* workspace,
-                                                 size_t workspace_bytes) {
-  using namespace ofq;
+namespace ofq {
+namespace {
+
+int ln_quant(void* stream, const void* x, const void* gamma, const void* beta, void* codes, float* scale,
+             float* zero_point, int t_dtype, int64_t rows, int64_t cols, double epsilon, int quantization_bit,
+             int statistics, void* workspace, size_t workspace_bytes, bool any_row) {
   OFQ_RETURN_IF(quantization_bit <= 1 || quantization_bit > 8, OFQ_ERR_BAD_ATTR);
   OFQ_RETURN_IF(statistics != OFQ_LN_STATS_FP32 && statistics != OFQ_LN_STATS_FP64,
                 OFQ_ERR_BAD_ATTR);
@@ -1259,12 +1683,11 @@ extern "C" int ofq_fused_layer_norm_quantization(void* stream, const void* x, co
                     || !ofq_aligned16(workspace),
                 OFQ_ERR_WORKSPACE);
   // the shapes the register-resident row kernels take; everything else is the two ops in a row
-  const int np = (int)(cols / 512);
-  if (t_dtype != OFQ_F16 || gamma == nullptr || beta == nullptr || cols % 512 != 0
-      || !(np == 1 || np == 2 || np == 4 || np == 8) || !ofq_aligned16(x) || !ofq_aligned16(gamma)
-      || !ofq_aligned16(beta) || (reinterpret_cast<uintptr_t>(codes) & 7u) != 0) {
-    return OFQ_ERR_UNSUPPORTED;
-  }
+  const bool full = ln_quant_full(x, gamma, beta, codes, t_dtype, cols);
+  const bool rows8 = t_dtype != OFQ_F32 && cols % 8 == 0 && cols <= 16384 && ofq_aligned16(x)
+                     && ofq_aligned16(gamma) && ofq_aligned16(beta)
+                     && (reinterpret_cast<uintptr_t>(codes) & 7u) == 0;
+  OFQ_RETURN_IF(!(full || (any_row && rows8)), OFQ_ERR_UNSUPPORTED);
   hipStream_t st = static_cast<hipStream_t>(stream);
   float* part = static_cast<float*>(workspace);
   float* stats = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace)
@@ -1272,13 +1695,39 @@ extern "C" int ofq_fused_layer_norm_quantization(void* stream, const void* x, co
   const uint16_t* xs = static_cast<const uint16_t*>(x);
   const uint16_t* gs = static_cast<const uint16_t*>(gamma);
   const uint16_t* bs = static_cast<const uint16_t*>(beta);
+  const bool exact = statistics == OFQ_LN_STATS_FP64;
+  const int np = (int)(cols / 512);
+  const LnQuantArgs args = {xs, gs, bs, part, stats, static_cast<int8_t*>(codes), scale, zero_point, rows,
+                            (int)cols, epsilon, quantization_bit};
+  if (!full) {
+    if (t_dtype == OFQ_F16) {
+      if (exact) launch_ln_quant_any<f16, true>(st, args);
+      else launch_ln_quant_any<f16, false>(st, args);
+    } else {
+      if (exact) launch_ln_quant_any<bf16, true>(st, args);
+      else launch_ln_quant_any<bf16, false>(st, args);
+    }
+    return ofq_check_launch();
+  }
+  if (rows <= ln_rows_per_block(1, true)) {
+#define OFQ_LNQ(NPV)                                                  \
+  if (exact) launch_ln_quant_rows<f16, NPV, 1, true, true>(st, args); \
+  else launch_ln_quant_rows<f16, NPV, 1, true, false>(st, args);
+    switch (np) {
+      case 1: OFQ_LNQ(1) break;
+      case 2: OFQ_LNQ(2) break;
+      case 4: OFQ_LNQ(4) break;
+      default: OFQ_LNQ(8) break;
+    }
+#undef OFQ_LNQ
+    return ofq_check_launch();
+  }
   // one row per wave up to 16 waves per CU, beyond that the waves walk the rows; both kernels
   // use the same grid, so a row meets the same wave of the same block twice
   const int64_t waves = rows < 256 * 16 ? rows : 256 * 16;
   constexpr int kWavesPerBlock = kLnqBlock / kWave;
   const int grid = (int)((waves + kWavesPerBlock - 1) / kWavesPerBlock);
   const int64_t nparts = grid;  // one partial maximum per block of the first kernel (<= 512)
-  const bool exact = statistics == OFQ_LN_STATS_FP64;
   // parts of a row in the second kernel: enough waves for 16 per CU where the rows allow it
   int split = 1;
   while (split < 4 && split * 2 <= np && waves * split * 2 <= 256 * 16) split *= 2;
@@ -1304,6 +1753,27 @@ extern "C" int ofq_fused_layer_norm_quantization(void* stream, const void* x, co
 #undef OFQ_LNQ1
 #undef OFQ_LNQ2
   return ofq_check_launch();
+}
+
+}  // namespace
+}  // namespace ofq
+
+extern "C" int ofq_fused_layer_norm_quantization(void* stream, const void* x, const void* gamma,
+                                                 const void* beta, void* codes, float* scale,
+                                                 float* zero_point, int t_dtype, int64_t rows,
+                                                 int64_t cols, double epsilon, int quantization_bit,
+                                                 int statistics, void* workspace,
+                                                 size_t workspace_bytes) {
+  return ofq::ln_quant(stream, x, gamma, beta, codes, scale, zero_point, t_dtype, rows, cols, epsilon,
+                       quantization_bit, statistics, workspace, workspace_bytes, false);
+}
+
+extern "C" int ofq_fused_layer_norm_quantization_any_row(
+    void* stream, const void* x, const void* gamma, const void* beta, void* codes, float* scale,
+    float* zero_point, int t_dtype, int64_t rows, int64_t cols, double epsilon, int quantization_bit,
+    int statistics, void* workspace, size_t workspace_bytes) {
+  return ofq::ln_quant(stream, x, gamma, beta, codes, scale, zero_point, t_dtype, rows, cols, epsilon,
+                       quantization_bit, statistics, workspace, workspace_bytes, true);
 }
 
 extern "C" int ofq_fused_layer_norm_min_max_observer_stats(

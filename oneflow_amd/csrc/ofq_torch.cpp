@@ -933,7 +933,7 @@ PyObject* layer_norm_quantization(PyObject* const* args) {
   {
     const Tensor ws = workspace(ws_bytes, x);
     rc = unlocked(
-        ofq_fused_layer_norm_quantization, st, ptr(x_), ptr(g_), ptr(b_), ptr(codes), ps, pz, td,
+        ofq_fused_layer_norm_quantization_any_row, st, ptr(x_), ptr(g_), ptr(b_), ptr(codes), ps, pz, td,
         rows, cols, epsilon, (int)bit, stats, ptr(ws), ws_bytes);
   }
   if (rc == OFQ_ERR_UNSUPPORTED) {
@@ -949,7 +949,7 @@ PyObject* layer_norm_quantization(PyObject* const* args) {
         ofq_quantization, st, ptr(y), ps, pz, ptr(codes), td, OFQ_I8, y.numel(), 1, (int)bit,
         OFQ_SCHEME_SYMMETRIC, OFQ_FORMULA_GOOGLE, OFQ_ZP_FLOAT));
   } else {
-    check_status("ofq_fused_layer_norm_quantization", rc);
+    check_status("ofq_fused_layer_norm_quantization_any_row", rc);
   }
   return tuple_of(wrap(std::move(codes)), wrap(std::move(scale)), wrap(std::move(zero_point)));
 }

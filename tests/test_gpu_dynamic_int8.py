@@ -140,6 +140,38 @@ def test_layer_norm_quantization_equals_the_two_ops(rows, cols, exact):
         assert np.array_equal(H.to_numpy(codes), O.quantize_to_int8(y_ref, s_ref, 8))
 
 
+@pytest.mark.parametrize("t", ["f16", "bf16"])
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("rows,cols", [
+    (1, 8), (8, 24), (9, 512), (3, 520), (8, 1000), (5, 1024), (33, 1280), (8, 2048), (4, 2432), (7, 4096),
+    (8, 4088), (9, 4096), (5000, 1544), (4, 4104), (5, 8192), (1, 6080), (300, 6080), (4100, 4160), (2, 8200),
+    (21, 16384), (40000, 64), (3, 16392), (6, 1001)])
+def test_layer_norm_quantization_any_row(t, exact, rows, cols):
+    """Rows of any length: one launch for the few rows a block holds, two launches above that, the two
+    ops for what neither takes.  Identical codes and scale to the two ops, with the parameters
+    present, absent or one of them, with a row that holds an infinity or a NaN, and with y = 0."""
+    import oneflow_amd as flow
+    import torch
+    x, gamma, beta = _cfg5_inputs(rows, cols, t)
+    xt, gt, bt = H.to_torch(x), H.to_torch(gamma), H.to_torch(beta)
+    xt[rows // 2] += 40.0
+    zeros = torch.zeros_like(gt)
+    cases = [(xt, gt, bt), (xt, None, None), (xt, gt, None), (xt, None, bt), (xt, zeros, zeros)]
+    if rows > 1:
+        for bad in (float("nan"), float("inf")):
+            xb = xt.clone()
+            xb[rows - 1, cols // 2] = bad
+            cases.append((xb, gt, bt))
+    xc = xt.clone()
+    xc[0] = 0.0  # a constant row
+    for xi, g, b in cases + [(xc, gt, bt)]:
+        y, s, z = flow._C.fused_layer_norm_min_max_observer(xi, g, b, 1e-5, 8, exact_statistics=exact)
+        want = flow._C.quantization(y, s, z, "google", 8, "symmetric", out_dtype=torch.int8)
+        codes, s2, z2 = flow._C.fused_layer_norm_quantization(xi, g, b, 1e-5, 8, exact_statistics=exact)
+        assert torch.equal(s.view(torch.int32), s2.view(torch.int32)) and z2.item() == 0.0
+        assert torch.equal(codes, want)
+
+
 @pytest.mark.parametrize("bits", [2, 5, 8])
 def test_layer_norm_quantization_bit_widths_and_a_zero_row_tensor(bits):
     import oneflow_amd as flow
