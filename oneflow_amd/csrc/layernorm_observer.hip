@@ -14,7 +14,8 @@
 // 1 KB per wave instruction) and kept in registers for the three uses (sum, squared deviations,
 // normalise); the reductions are cross-lane only, so no barrier and no LDS is involved and the
 // waves of a CU drift apart, which overlaps one wave's loads with another's stores.  Longer rows
-// use one block per row.  The absmax of the stored values goes to the workspace (one float per
+// use one block per row; up to 8 rows of a 16-bit type share one block, which needs no second launch
+// (ln_quant_rows).  The absmax of the stored values goes to the workspace (one float per
 // wave or per row) and a second one-wave launch folds them and divides.
 #include <atomic>
 #include <type_traits>
@@ -1043,16 +1044,17 @@ ln_quant_second(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gam
 
 // ---------------------------------------------------------------------------------------------
 // The same composition for fp16 and bf16 rows of any 8 * n elements up to 16384, gamma and beta each
-// optional.  A row is taken by WPR waves: one (the arithmetic of ln_observer_wave_rows; DOT: the
-// fp16 row sum of ln_observer_wave_full) or four (that of ln_observer_rows), so scale and codes carry
+// optional.  A row is taken by WPR waves: one (the arithmetic of ln_observer_wave_rows; FULL:
+// rows of 512 * NP elements, fp16 with the row sum of ln_observer_wave_full) or four (that of ln_observer_rows), so scale and codes carry
 // the bits of the two ops.
-//   ln_quant_rows<ONE = false> + ln_quant_codes : two launches; y is formed twice and never stored
-//   ln_quant_rows<ONE = true>                   : one launch of one block, for as many rows as it
-//     holds (8, or 4 of more than 4096 elements): the rows wait in registers for the block's maximum
-// Time of a call of the two ops and of this: 1 x 2432 fp16 13.0 -> 6.4 us, 8 x 1280 bf16 13.6 -> 6.2, 64 x 6080
-// fp16 13.3 -> 9.2, 1024 x 6080 19.1 -> 14.0, 4096 x 4096 bf16 44 -> 36 (host-bound up to some hundred rows:
+//   ln_quant_rows<kLnStats> + ln_quant_codes : two launches; y is formed twice and never stored
+//   ln_quant_rows<kLnCodes>                  : one launch of one block, for as many rows as it holds
+//     (8, or 4 of more than 4096 elements): the rows wait in registers for the block's maximum
+// Time of a call of the two ops and of this: 1 x 2432 fp16 13.0 -> 6.4 us, 8 x 1280 bf16 13.6 -> 6.4, 64 x 6080
+// fp16 13.3 -> 9.2, 1024 x 6080 19.1 -> 14.0, 4096 x 4096 bf16 44 -> 31 (host-bound up to some hundred rows:
 // three launches and two allocations became one or two launches).  Many rows are bound by the vector units
-// of both kernels: 8192 x 2432 fp16 17.9 + 16.0 us, where their traffic takes about 14.
+// of both kernels: 8192 x 2432 fp16 17.8 + 15.3 us, where their traffic takes about 14.
+// ln_quant_rows<OUT = kLnY> is also the observer of few rows, with or without a residual input.
 // ---------------------------------------------------------------------------------------------
 constexpr int ln_rows_per_block(int wpr, bool one) { return wpr == 1 ? 8 : one ? 4 : 1; }
 
@@ -1061,32 +1063,65 @@ __device__ __forceinline__ RawPack<T> load_pack(const uint16_t* p) {
   return load_raw<T>(reinterpret_cast<const typename TT<T>::storage*>(p));
 }
 
+// 8 floats rounded to bf16, two to an instruction; the packed values, and optionally the floats again
+__device__ __forceinline__ u32x4 round8_bf16(float* f, bool again) {
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{f[2 * i], f[2 * i + 1]}, bf2));
+    asm volatile("" : "+v"(w));  // (or the pair is converted one by one where it is widened again)
+    r[i] = w;
+    if (again) {
+      f[2 * i] = __builtin_bit_cast(float, w << 16);
+      f[2 * i + 1] = __builtin_bit_cast(float, w & 0xFFFF0000u);
+    }
+  }
+  return r;
+}
+
+// What stands for an absent parameter or residual input, so that nothing is decided per element: gamma 1; beta +0
+// next to a gamma (the reference adds its default beta 0: -0 becomes +0) and else -0, which leaves every value as
+// it is; +0 for a residual input
+template<typename T>
+__device__ __forceinline__ uint32_t ln_ones() {
+  return TT<T>::dtype == OFQ_F16 ? 0x3C003C00u : 0x3F803F80u;
+}
+template<typename T>
+__device__ __forceinline__ RawPack<T> ln_pack_or(const uint16_t* p, int64_t at, uint32_t absent) {
+  RawPack<T> r;
+  r.q[0] = u32x4{absent, absent, absent, absent};
+  if (p) r = load_pack<T>(p + at);
+  return r;
+}
+
 // y of 8 elements from their deviations x - mean, as ln_observer_wave_rows forms it
 template<typename T>
-__device__ __forceinline__ u32x4 ln_out8(const float* d, float inv, bool has_gamma, const RawPack<T>& g,
-                                         bool has_beta, const RawPack<T>& b) {
+__device__ __forceinline__ u32x4 ln_out8(const float* d, float inv, const RawPack<T>& g, const RawPack<T>& b) {
   if constexpr (TT<T>::dtype == OFQ_F16) {
     f16x8 t;
 #pragma unroll
     for (int e = 0; e < 8; ++e) t[e] = (f16)normalised<f16>(d[e], inv);
-    if (has_gamma) t = t * __builtin_bit_cast(f16x8, g.q[0]);
-    if (has_beta) t = t + __builtin_bit_cast(f16x8, b.q[0]);
+    t = t * __builtin_bit_cast(f16x8, g.q[0]);
+    t = t + __builtin_bit_cast(f16x8, b.q[0]);
     u32x4 bits = __builtin_bit_cast(u32x4, t);
     // (held as four packed registers: otherwise the affine is emitted element by element)
     asm volatile("" : "+v"(bits[0]), "+v"(bits[1]), "+v"(bits[2]), "+v"(bits[3]));
     return bits;
   } else {
-    float gf[8], bf[8], o[8];
-    if (has_gamma) widen<T>(g, gf);
-    if (has_beta) widen<T>(b, bf);
+    float gf[8], bf[8], t[8];
+    widen<T>(g, gf);
+    widen<T>(b, bf);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float t = normalised<T>(d[e], inv);
-      if (has_gamma) t = TT<T>::round(t * gf[e]);
-      if (has_beta) t = TT<T>::round(t + bf[e]);
-      o[e] = t;
-    }
-    return narrow<T>(o).q[0];
+    for (int e = 0; e < 8; ++e) t[e] = d[e] * inv;
+    round8_bf16(t, true);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) t[e] = t[e] * gf[e];
+    round8_bf16(t, true);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) t[e] = t[e] + bf[e];
+    return round8_bf16(t, false);
   }
 }
 
@@ -1132,12 +1167,48 @@ __device__ __forceinline__ V row_sum(V v, V* smem) {
   return r;
 }
 
-template<typename T, int NP, int WPR, bool DOT, bool EXACT, bool ONE>
-__global__ void __launch_bounds__(ln_rows_per_block(WPR, ONE) * WPR * kWave)
+// the residual inputs of skip_layer_norm, see SkipArgs
+struct LnSkip16 {
+  const uint16_t *bias, *skip;
+  float alpha;
+};
+
+// 8 elements of the residual sum in place of those of x: b bias, s skip
+template<typename T>
+__device__ __forceinline__ void ln_add_skip(RawPack<T>& v, float alpha, const RawPack<T>& s,
+                                            const RawPack<T>& b) {
+  if constexpr (TT<T>::dtype == OFQ_F16) {  // (native fp16 arithmetic, see ln_observer_wave_full)
+    const f16x8 xb = __builtin_bit_cast(f16x8, v.q[0]) + __builtin_bit_cast(f16x8, b.q[0]);
+    v.q[0] = __builtin_bit_cast(u32x4, xb + __builtin_bit_cast(f16x8, s.q[0]) * (f16)alpha);
+  } else {
+    float fx[8], fb[8], fs[8];
+    widen<T>(v, fx);
+    widen<T>(b, fb);
+    widen<T>(s, fs);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      fx[e] = fx[e] + fb[e];
+      fs[e] = fs[e] * alpha;
+    }
+    round8_bf16(fx, true);
+    round8_bf16(fs, true);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) fx[e] = fx[e] + fs[e];
+    v.q[0] = round8_bf16(fx, false);
+  }
+}
+
+// What a launch leaves: (mean, inv) of the rows and a maximum per block, or, of one block, codes or y
+enum { kLnStats, kLnCodes, kLnY };
+
+template<typename T, int NP, int WPR, bool FULL, bool EXACT, int OUT, bool SKIP>
+__global__ void __launch_bounds__(ln_rows_per_block(WPR, OUT != kLnStats) * WPR * kWave)
 ln_quant_rows(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma,
               const uint16_t* __restrict__ beta, float* __restrict__ block_absmax,
-              float* __restrict__ stats, int8_t* __restrict__ codes, float* __restrict__ scale,
-              float* __restrict__ zero_point, int64_t rows, int cols, double eps64, int bits) {
+              float* __restrict__ stats, void* __restrict__ out, float* __restrict__ scale,
+              float* __restrict__ zero_point, int64_t rows, int cols, double eps64, int bits, LnSkip16 sk) {
+  constexpr bool ONE = OUT != kLnStats;
+  static_assert(ONE || !SKIP, "the residual variant has one block");
   constexpr int kRows = ln_rows_per_block(WPR, ONE);
   constexpr int kWaves = kRows * WPR;
   constexpr int kStep = WPR * kWave;  // packs between two of a thread
@@ -1155,14 +1226,17 @@ ln_quant_rows(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma
   // gamma and beta: one copy in LDS for the rows of a block, or in the registers of the only row's threads
   constexpr bool kShared = kRows > 1;
   __shared__ u32x4 params[kShared ? 2 * NP * kStep : 1];
+  const uint32_t no_beta = gamma ? 0u : 0x80008000u;
   RawPack<T> gr[kShared ? 1 : NP], br[kShared ? 1 : NP], v[NP];
   bool in[NP];
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    in[i] = t + i * kStep < npacks;
+    in[i] = FULL || t + i * kStep < npacks;
     if constexpr (!kShared) {
-      if (in[i] && gamma) gr[i] = load_pack<T>(gamma + (t + i * kStep) * 8);
-      if (in[i] && beta) br[i] = load_pack<T>(beta + (t + i * kStep) * 8);
+      if (in[i]) {
+        gr[i] = ln_pack_or<T>(gamma, (t + i * kStep) * 8, ln_ones<T>());
+        br[i] = ln_pack_or<T>(beta, (t + i * kStep) * 8, no_beta);
+      }
     }
   }
   auto request = [&](int64_t row) {
@@ -1174,21 +1248,32 @@ ln_quant_rows(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma
     }
   };
   request(first);
+  RawPack<T> sr[SKIP ? NP : 1], br1[SKIP ? NP : 1];
+  if constexpr (SKIP) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      if (in[i] && first < rows) {
+        sr[i] = ln_pack_or<T>(sk.skip, first * cols + (t + i * kStep) * 8, 0u);
+        br1[i] = ln_pack_or<T>(sk.bias, (t + i * kStep) * 8, 0u);
+      }
+    }
+  }
   if constexpr (kShared) {
     for (int p = threadIdx.x; p < npacks; p += blockDim.x) {
-      if (gamma) params[p] = load_pack<T>(gamma + p * 8).q[0];
-      if (beta) params[NP * kStep + p] = load_pack<T>(beta + p * 8).q[0];
+      params[p] = ln_pack_or<T>(gamma, p * 8, ln_ones<T>()).q[0];
+      params[NP * kStep + p] = ln_pack_or<T>(beta, p * 8, no_beta).q[0];
     }
     __syncthreads();
   }
-  // The row is held in storage format and widened again in every pass: without the empty asm the compiler
-  // keeps the widened floats too, twice the registers (176 to 240 of them for rows of 4096).
+  // The rows of many blocks are held in storage format and widened again in every pass: without the empty asm
+  // the compiler keeps the widened floats too, twice the registers (176 to 240 of them for rows of 4096).
   auto hold_pack = [](RawPack<T>& r) {
     u32x4 h = r.q[0];
     asm volatile("" : "+v"(h[0]), "+v"(h[1]), "+v"(h[2]), "+v"(h[3]));
     r.q[0] = h;
   };
   auto hold = [&]() {
+    if constexpr (ONE && !(EXACT && WPR > 1)) return;
 #pragma unroll
     for (int i = 0; i < NP; ++i) hold_pack(v[i]);
   };
@@ -1198,6 +1283,12 @@ ln_quant_rows(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma
     const int64_t row = first + turn * stride;
     const bool live = row < rows;
     if (turn != 0) request(row);
+    if constexpr (SKIP) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        if (in[i] && live) ln_add_skip<T>(v[i], sk.alpha, sr[i], br1[i]);
+      }
+    }
     // (an element past the row adds a zero to the sum and, skipped, nothing to the squares)
     float sum = 0.0f;
     double sum64 = 0.0;
@@ -1208,7 +1299,7 @@ ln_quant_rows(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma
       if constexpr (EXACT) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) sum64 += (double)f[e];
-      } else if constexpr (DOT) {
+      } else if constexpr (FULL && TT<T>::dtype == OFQ_F16) {
         uint32_t ones_bits = 0x3c003c00u;  // (1, 1) held in a register, see ln_observer_wave_full
         asm volatile("" : "+v"(ones_bits));
         const f16x2 ones = __builtin_bit_cast(f16x2, ones_bits);
@@ -1283,9 +1374,12 @@ ln_quant_rows(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma
         hold_pack(gr[i]), hold_pack(br[i]);  // (or their floats are kept over the turns)
         g = gr[i], b = br[i];
       }
-      const u32x4 y = ln_out8<T>(d, inv, gamma != nullptr, g, beta != nullptr, b);
+      const u32x4 y = ln_out8<T>(d, inv, g, b);
       amax8.take(y);
-      if constexpr (ONE) v[i].q[0] = y;
+      if constexpr (OUT == kLnCodes) v[i].q[0] = y;
+      if constexpr (OUT == kLnY) {
+        *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(out) + row * cols + (t + i * kStep) * 8) = y;
+      }
     }
   }
   const float amax = block_reduce(amax8.value(), OpMax(), smem);
@@ -1298,7 +1392,8 @@ ln_quant_rows(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma
       *scale = s;
       *zero_point = 0.0f;
     }
-    if (first >= rows) return;
+    if (OUT != kLnCodes || first >= rows) return;
+    int8_t* codes = static_cast<int8_t*>(out);
     const float recip = 1.0f / s;
     const int hi = (int)upper, lo = -hi - 1;
     ln_with_mode(s, bits, [&](auto mode) {
@@ -1341,8 +1436,8 @@ ln_quant_codes(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamm
   float amax = 0.0f;
   for (int i = threadIdx.x; i < nparts; i += blockDim.x) amax = fmaxf(amax, part[i]);
   request(blockIdx.y);
-  if (gamma) g = load_pack<T>(gamma + at);
-  if (beta) b = load_pack<T>(beta + at);
+  g = ln_pack_or<T>(gamma, at, ln_ones<T>());
+  b = ln_pack_or<T>(beta, at, gamma ? 0u : 0x80008000u);
   amax = block_reduce(amax, OpMax(), smem);
   const float upper = (float)(1 << (bits - 1)) - 1.0f;
   const float s = amax / upper;
@@ -1364,7 +1459,7 @@ ln_quant_codes(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamm
         widen<T>(v[u], d);
 #pragma unroll
         for (int e = 0; e < 8; ++e) d[e] = d[e] - mean[u];
-        const u32x4 y = ln_out8<T>(d, inv[u], gamma != nullptr, g, beta != nullptr, b);
+        const u32x4 y = ln_out8<T>(d, inv[u], g, b);
         *reinterpret_cast<u32x2*>(codes + row * cols + at) =
             ln_codes8<T, decltype(mode)::value>(y, s, recip, lo, hi);
       }
@@ -1388,6 +1483,83 @@ float round_to_T_host(float v) {
   return v;
 }
 
+struct LnQuantArgs {
+  const uint16_t *x, *gamma, *beta;
+  float *part, *stats;
+  void* out;
+  float *scale, *zero_point;
+  int64_t rows;
+  int cols;
+  double eps;
+  int bits;
+};
+
+// Rows that one block takes; 0 for rows longer than it takes.  One launch of 4 x 4096, 8 x 4096 and 4 x 8192 fp16
+// rows with a residual input is 5.0, 6.6 and 7.1 us, the row kernel and the fold 4.1 + 1.4, 4.6 + 1.4 and
+// 7.3 + 1.5 with a gap between them and 2.3 us of the host for the second launch.  For y of long bf16 rows, which
+// take more of the one CU's vector units, it ends earlier: 4 x 4096 6.6, 8 x 4096 8.9 and 4 x 8192 9.8 us
+// against 6.4 + 1.2, 7.1 + 1.4 and 7.7 + 1.2.
+template<typename T>
+constexpr int ln_one_block_rows(int packs, int out) {
+  const int rows = packs <= 8 * kWave ? ln_rows_per_block(1, true)
+                   : packs <= 16 * kWave ? ln_rows_per_block(4, true) : 0;
+  return TT<T>::dtype == OFQ_BF16 && out == kLnY && packs > 4 * kWave ? rows / 2 : rows;
+}
+
+template<typename T, int NP, int WPR, bool FULL, bool EXACT, int OUT, bool SKIP>
+void launch_ln_one_block(hipStream_t st, const LnQuantArgs& a, const LnSkip16& sk) {
+  ln_quant_rows<T, NP, WPR, FULL, EXACT, OUT, SKIP><<<1, ln_rows_per_block(WPR, true) * WPR * kWave, 0, st>>>(
+      a.x, a.gamma, a.beta, a.part, a.stats, a.out, a.scale, a.zero_point, a.rows, a.cols, a.eps, a.bits, sk);
+}
+
+// fp16 rows are full only with both parameters, as for ln_observer_wave_full, whose sums those are
+template<typename T, bool EXACT, int OUT, bool SKIP>
+void ln_one_block(hipStream_t st, const LnQuantArgs& a, const LnSkip16& sk) {
+  const int packs = a.cols / 8;
+  const bool full = (a.cols == 512 || a.cols == 1024 || a.cols == 2048 || a.cols == 4096)
+                    && (TT<T>::dtype != OFQ_F16 || (a.gamma != nullptr && a.beta != nullptr));
+#define OFQ_LN_ONE(NPV)                                                                \
+  if (full) launch_ln_one_block<T, NPV, 1, true, EXACT, OUT, SKIP>(st, a, sk);         \
+  else launch_ln_one_block<T, NPV, 1, false, EXACT, OUT, SKIP>(st, a, sk)
+  if (packs <= kWave) {
+    OFQ_LN_ONE(1);
+  } else if (packs <= 2 * kWave) {
+    OFQ_LN_ONE(2);
+  } else if (packs <= 4 * kWave) {
+    OFQ_LN_ONE(4);
+  } else if (packs <= 8 * kWave) {
+    OFQ_LN_ONE(8);
+  } else {
+    launch_ln_one_block<T, 4, 4, false, EXACT, OUT, SKIP>(st, a, sk);
+  }
+#undef OFQ_LN_ONE
+}
+
+template<typename T, int NP, int WPR, bool EXACT>
+void launch_ln_quant_rows(hipStream_t st, const LnQuantArgs& a) {
+  constexpr int kMany = ln_rows_per_block(WPR, false);
+  // a row to a block until every CU has one, to a SIMD until those have one, then 16 waves per CU
+  int8_t* codes = static_cast<int8_t*>(a.out);
+  const int per_block = a.rows <= 256 ? 1 : a.rows <= 1024 && kMany > 4 ? 4 : kMany;
+  const int64_t blocks = (a.rows + per_block - 1) / per_block, most = 4096 / (kMany * WPR);
+  const int grid = (int)(blocks < most ? blocks : most);
+  ln_quant_rows<T, NP, WPR, false, EXACT, kLnStats, false><<<grid, per_block * WPR * kWave, 0, st>>>(
+      a.x, a.gamma, a.beta, a.part, a.stats, codes, a.scale, a.zero_point, a.rows, a.cols, a.eps, a.bits, LnSkip16{});
+  const int packs = a.cols / 8;
+  const int bx = (packs + kLnCodesBlock - 1) / kLnCodesBlock;
+  const int threads = ((packs + bx - 1) / bx + kWave - 1) / kWave * kWave;
+  const int most_y = 8192 / (bx * threads / kWave);
+  if (a.rows <= most_y) {
+    ln_quant_codes<T, 1><<<dim3(bx, (unsigned)a.rows), threads, 0, st>>>(
+        a.x, a.gamma, a.beta, a.part, grid, a.stats, codes, a.scale, a.zero_point, a.rows, a.cols, a.bits);
+  } else {
+    const int64_t turns = (a.rows + 4 * (int64_t)most_y - 1) / (4 * (int64_t)most_y);
+    const unsigned by = (unsigned)((a.rows + 4 * turns - 1) / (4 * turns));
+    ln_quant_codes<T, 4><<<dim3(bx, by), threads, 0, st>>>(
+        a.x, a.gamma, a.beta, a.part, grid, a.stats, codes, a.scale, a.zero_point, a.rows, a.cols, a.bits);
+  }
+}
+
 template<typename T, bool SKIP, bool EXACT>
 int launch(hipStream_t st, const void* x, const void* gamma, const void* beta, void* y,
            float* scale, float* zero_point, int64_t rows, int64_t cols, double eps, int bits,
@@ -1406,6 +1578,16 @@ int launch(hipStream_t st, const void* x, const void* gamma, const void* beta, v
                       && ofq_aligned16(gamma) && ofq_aligned16(beta) && ofq_aligned16(bias)
                       && ofq_aligned16(skip) && (cols * sizeof(S)) % 16 == 0;
   const int64_t npacks = cols / 8;
+  if constexpr (sizeof(S) == 2) {
+    // as many rows as one block holds need no second launch
+    if (vec_ok && npacks <= 16 * kWave && rows <= ln_one_block_rows<T>((int)npacks, kLnY)) {
+      const auto u16 = [](const void* p) { return static_cast<const uint16_t*>(p); };
+      const LnQuantArgs a = {u16(x), u16(gamma), u16(beta), nullptr, nullptr, y, scale, zero_point, rows,
+                             (int)cols, eps, bits};
+      ln_one_block<T, EXACT, kLnY, SKIP>(st, a, LnSkip16{u16(bias), u16(skip), sk.alpha});
+      return ofq_check_launch();
+    }
+  }
   int64_t nparts = rows;
   constexpr int kWavesPerBlock = kLnBlock / kWave;
   // fp32 rows beyond 2048 elements would not fit a lane's registers at two waves per SIMD
@@ -1587,62 +1769,16 @@ extern "C" int ofq_fused_skip_layer_norm_min_max_observer(
 namespace ofq {
 namespace {
 
-struct LnQuantArgs {
-  const uint16_t *x, *gamma, *beta;
-  float *part, *stats;
-  int8_t* codes;
-  float *scale, *zero_point;
-  int64_t rows;
-  int cols;
-  double eps;
-  int bits;
-};
-
-template<typename T, int NP, int WPR, bool DOT, bool EXACT>
-void launch_ln_quant_rows(hipStream_t st, const LnQuantArgs& a) {
-  constexpr int kOne = ln_rows_per_block(WPR, true), kMany = ln_rows_per_block(WPR, false);
-  // more than two bf16 rows of four waves keep one CU busy longer than a second launch costs (4 x 8192:
-  // 10.6 us a call in one launch, 9.2 in two; 8 x 4096, a wave to a row: 10.5 and 12.1)
-  constexpr int kMostOne = TT<T>::dtype == OFQ_BF16 && WPR > 1 ? kOne / 2 : kOne;
-  if constexpr (NP * WPR <= 16) {
-    if (a.rows <= kMostOne) {
-      ln_quant_rows<T, NP, WPR, DOT, EXACT, true><<<1, kOne * WPR * kWave, 0, st>>>(
-          a.x, a.gamma, a.beta, a.part, a.stats, a.codes, a.scale, a.zero_point, a.rows, a.cols, a.eps, a.bits);
-      return;
-    }
-  }
-  if constexpr (!DOT) {
-    // a row to a block until every CU has one, to a SIMD until those have one, then 16 waves per CU
-    const int per_block = a.rows <= 256 ? 1 : a.rows <= 1024 && kMany > 4 ? 4 : kMany;
-    const int64_t blocks = (a.rows + per_block - 1) / per_block, most = 4096 / (kMany * WPR);
-    const int grid = (int)(blocks < most ? blocks : most);
-    ln_quant_rows<T, NP, WPR, false, EXACT, false><<<grid, per_block * WPR * kWave, 0, st>>>(
-        a.x, a.gamma, a.beta, a.part, a.stats, a.codes, a.scale, a.zero_point, a.rows, a.cols, a.eps, a.bits);
-    const int packs = a.cols / 8;
-    const int bx = (packs + kLnCodesBlock - 1) / kLnCodesBlock;
-    const int threads = ((packs + bx - 1) / bx + kWave - 1) / kWave * kWave;
-    const int most_y = 8192 / (bx * threads / kWave);
-    if (a.rows <= most_y) {
-      ln_quant_codes<T, 1><<<dim3(bx, (unsigned)a.rows), threads, 0, st>>>(
-          a.x, a.gamma, a.beta, a.part, grid, a.stats, a.codes, a.scale, a.zero_point, a.rows, a.cols, a.bits);
-    } else {
-      const int64_t turns = (a.rows + 4 * (int64_t)most_y - 1) / (4 * (int64_t)most_y);
-      const unsigned by = (unsigned)((a.rows + 4 * turns - 1) / (4 * turns));
-      ln_quant_codes<T, 4><<<dim3(bx, by), threads, 0, st>>>(
-          a.x, a.gamma, a.beta, a.part, grid, a.stats, a.codes, a.scale, a.zero_point, a.rows, a.cols, a.bits);
-    }
-  }
-}
-
 template<typename T, bool EXACT>
 void launch_ln_quant_any(hipStream_t st, const LnQuantArgs& a) {
   const int packs = a.cols / 8;
-  if (packs <= kWave) launch_ln_quant_rows<T, 1, 1, false, EXACT>(st, a);
-  else if (packs <= 2 * kWave) launch_ln_quant_rows<T, 2, 1, false, EXACT>(st, a);
-  else if (packs <= 4 * kWave) launch_ln_quant_rows<T, 4, 1, false, EXACT>(st, a);
-  else if (packs <= 8 * kWave) launch_ln_quant_rows<T, 8, 1, false, EXACT>(st, a);
-  else if (packs <= 16 * kWave) launch_ln_quant_rows<T, 4, 4, false, EXACT>(st, a);
-  else launch_ln_quant_rows<T, 8, 4, false, EXACT>(st, a);
+  if (a.rows <= ln_one_block_rows<T>(packs, kLnCodes)) ln_one_block<T, EXACT, kLnCodes, false>(st, a, LnSkip16{});
+  else if (packs <= kWave) launch_ln_quant_rows<T, 1, 1, EXACT>(st, a);
+  else if (packs <= 2 * kWave) launch_ln_quant_rows<T, 2, 1, EXACT>(st, a);
+  else if (packs <= 4 * kWave) launch_ln_quant_rows<T, 4, 1, EXACT>(st, a);
+  else if (packs <= 8 * kWave) launch_ln_quant_rows<T, 8, 1, EXACT>(st, a);
+  else if (packs <= 16 * kWave) launch_ln_quant_rows<T, 4, 4, EXACT>(st, a);
+  else launch_ln_quant_rows<T, 8, 4, EXACT>(st, a);
 }
 
 // the shapes ln_quant_first and ln_quant_second take
@@ -1697,7 +1833,7 @@ int ln_quant(void* stream, const void* x, const void* gamma, const void* beta, v
   const uint16_t* bs = static_cast<const uint16_t*>(beta);
   const bool exact = statistics == OFQ_LN_STATS_FP64;
   const int np = (int)(cols / 512);
-  const LnQuantArgs args = {xs, gs, bs, part, stats, static_cast<int8_t*>(codes), scale, zero_point, rows,
+  const LnQuantArgs args = {xs, gs, bs, part, stats, codes, scale, zero_point, rows,
                             (int)cols, epsilon, quantization_bit};
   if (!full) {
     if (t_dtype == OFQ_F16) {
@@ -1709,17 +1845,9 @@ int ln_quant(void* stream, const void* x, const void* gamma, const void* beta, v
     }
     return ofq_check_launch();
   }
-  if (rows <= ln_rows_per_block(1, true)) {
-#define OFQ_LNQ(NPV)                                                  \
-  if (exact) launch_ln_quant_rows<f16, NPV, 1, true, true>(st, args); \
-  else launch_ln_quant_rows<f16, NPV, 1, true, false>(st, args);
-    switch (np) {
-      case 1: OFQ_LNQ(1) break;
-      case 2: OFQ_LNQ(2) break;
-      case 4: OFQ_LNQ(4) break;
-      default: OFQ_LNQ(8) break;
-    }
-#undef OFQ_LNQ
+  if (rows <= ln_one_block_rows<f16>((int)(cols / 8), kLnCodes)) {
+    if (exact) ln_one_block<f16, true, kLnCodes, false>(st, args, LnSkip16{});
+    else ln_one_block<f16, false, kLnCodes, false>(st, args, LnSkip16{});
     return ofq_check_launch();
   }
   // one row per wave up to 16 waves per CU, beyond that the waves walk the rows; both kernels

@@ -172,6 +172,36 @@ def test_layer_norm_quantization_any_row(t, exact, rows, cols):
         assert torch.equal(codes, want)
 
 
+@pytest.mark.parametrize("t", ["f16", "bf16"])
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("cols", [8, 504, 512, 1024, 1288, 2048, 2432, 4096, 4104, 8192, 8200])
+def test_observer_of_few_rows_equals_that_of_many(t, exact, cols):
+    """Up to 8 rows (4 of more than 4096 elements) are normalised by one block, which also folds the
+    scale; the same rows among 32 take the row kernels and a second launch.  A row's y does not depend on
+    the others, so it agrees bit for bit; the scale is that of the rows themselves."""
+    import oneflow_amd as flow
+    import torch
+    x, gamma, beta = _cfg5_inputs(32, cols, t)
+    xt, gt, bt = H.to_torch(x), H.to_torch(gamma), H.to_torch(beta)
+    bias = (0.5 * torch.randn(cols, generator=torch.Generator().manual_seed(3))).to(xt.dtype).cuda()
+    skip = torch.randn(32, cols, generator=torch.Generator().manual_seed(4)).to(xt.dtype).cuda()
+    bits = lambda y: y.view(torch.int16)  # noqa: E731
+    scale_of = lambda y: np.float32(y.float().abs().max().item()) / np.float32(127)  # noqa: E731
+    for rows in (1, 2, 3, 4, 5, 7, 8, 9):
+        for g, b in ((gt, bt), (gt, None), (None, bt), (None, None)):
+            few = flow._C.fused_layer_norm_min_max_observer(xt[:rows], g, b, 1e-5, 8, exact_statistics=exact)
+            many = flow._C.fused_layer_norm_min_max_observer(xt, g, b, 1e-5, 8, exact_statistics=exact)
+            assert torch.equal(bits(few[0]), bits(many[0][:rows])), (rows, g is None, b is None)
+            assert float(few[1]) == scale_of(many[0][:rows]) and few[2].item() == 0.0
+        for p, s in ((bias, skip), (None, skip), (bias, None)):
+            few = flow._C.fused_skip_layer_norm_min_max_observer(
+                xt[:rows], gt, bt, p, None if s is None else s[:rows], 1e-5, 0.37, 8, exact_statistics=exact)
+            many = flow._C.fused_skip_layer_norm_min_max_observer(xt, gt, bt, p, s, 1e-5, 0.37, 8,
+                                                                  exact_statistics=exact)
+            assert torch.equal(bits(few[0]), bits(many[0][:rows])), (rows, p is None, s is None)
+            assert float(few[1]) == scale_of(many[0][:rows])
+
+
 @pytest.mark.parametrize("bits", [2, 5, 8])
 def test_layer_norm_quantization_bit_widths_and_a_zero_row_tensor(bits):
     import oneflow_amd as flow
