@@ -484,6 +484,83 @@ void rows_mt_split(const LinearJob& job, int* rpb, int64_t* grid) {
   *grid = blocks_at(r);
 }
 
+// The split of gemv_ring_mt, or false where scales, rings and x do not fit LDS.  One block per CU and round; the
+// workers' split over tiles and K by the longest wave's steps: of a step, each tile's expansion and products, and
+// what it takes whatever it has of them, x among it.
+bool ring_mt_plan(const LinearJob& job, RingMtPlan* plan) {
+  const LinearArgs& a = job.pr[0];
+  constexpr int kCUs = 256, kLds = 160 * 1024, kMaxTl = 3, kWorkers = 12;
+  const int lists = job.glu ? 1 : job.count, matrices = job.glu ? 2 : 1;
+  const int ck = a.bits == 4 ? 128 : 64;
+  const int64_t G = a.k / a.group_size;
+  const int regions = matrices * (a.symmetric ? 1 : 2);
+  const int64_t steps = (a.k + ck - 1) / ck;
+  const int64_t step_x = a.m * ck * 2;
+  if (G * 2 * 16 > kLds) return false;
+  int64_t total = 0;
+  for (int i = 0; i < lists; ++i) total += job.pr[i].n;
+  auto blocks_at = [&](int64_t r) {
+    int64_t b = 0;
+    for (int i = 0; i < lists; ++i) b += (job.pr[i].n + r - 1) / r;
+    return b;
+  };
+  for (int64_t rounds = 1; rounds <= 512; rounds *= 2) {
+    const int64_t want = kCUs * rounds;
+    int64_t rpb = (total + want - 1) / want;
+    if (rpb > 16 * kMaxTl * kWorkers) continue;
+    if (rpb < 16) rpb = 16;
+    while (blocks_at(rpb) > want && rpb < 16 * kMaxTl * kWorkers) ++rpb;
+    const int64_t nvt = matrices * ((rpb + 15) / 16);
+    const int64_t scales = (regions * ((rpb * G * 2 + 16 + 15) & ~15) + 1023) & ~(int64_t)1023;
+    double best = 1e30;
+    for (int wk = kWorkers; wk >= 1; --wk) {
+      if (kWorkers % wk != 0) continue;
+      const int64_t tl = (nvt + kWorkers / wk - 1) / (kWorkers / wk);
+      if (tl > kMaxTl) continue;
+      const int64_t xbuf = (wk * step_x + 1023) & ~(int64_t)1023;
+      if (xbuf > 64 * 1024) continue;  // kRingMtCopies
+      const int most = tl == 1 ? 3 : (tl == 2 ? 2 : 1);
+      int buffers = 4, depth = 0;
+      for (; buffers >= 2; --buffers) {
+        const int64_t left = kLds - scales - buffers * xbuf;
+        depth = left < 0 ? 0 : (int)(left / (kWorkers * tl * 1024));
+        depth = depth < most ? depth : most;
+        if (depth >= (most < 2 || buffers == 2 ? 1 : 2)) break;
+      }
+      if (buffers < 2) continue;
+      const size_t red = (size_t)nvt * wk * a.m * 64;
+      if (red > kLds) continue;
+      const int64_t phases = (steps + wk - 1) / wk;
+      const double cost = phases * (tl + 0.2 + 0.1 * ((a.m + 15) / 16) + 0.5);
+      if (cost < best) {
+        best = cost;
+        plan->tl = (int)tl;
+        plan->wk = wk;
+        plan->depth = depth;
+        plan->buffers = buffers;
+        plan->phases = (int)phases;
+        plan->lds = (size_t)(scales + kWorkers * depth * tl * 1024 + buffers * xbuf);
+        if (red > plan->lds) plan->lds = red;
+      }
+    }
+    if (best >= 1e30) continue;
+    const int64_t grid = blocks_at(rpb);
+    if (grid > 0x7FFFFFFF) return false;
+    plan->grid = (int)grid;
+    plan->rows_per_block = (int)rpb;
+    return true;
+  }
+  return false;
+}
+
+int launch_ring_mt(hipStream_t st, const LinearJob& job, const RingMtPlan& plan) {
+  const LinearArgs& a = job.pr[0];
+  if (a.t_dtype == OFQ_BF16) {
+    return a.bits == 4 ? launch_gemv_ring_mt_bf16_b4(st, job, plan) : launch_gemv_ring_mt_bf16_b8(st, job, plan);
+  }
+  return a.bits == 4 ? launch_gemv_ring_mt_f16_b4(st, job, plan) : launch_gemv_ring_mt_f16_b8(st, job, plan);
+}
+
 int launch_rows_mt(hipStream_t st, const LinearJob& job) {
   const LinearArgs& a = job.pr[0];
   RowsMtPlan p;
@@ -831,7 +908,7 @@ bool gemv_mt_supported(const LinearArgs& a) {
 // wr_plan_us with up to 64 rows).  A round of blocks starts and ends (4.25, the scales, the output); a turn of
 // a block's waves over their chunks takes a part per tile of weights expanded, one per row of weights
 // read and one per row of x read (every block reads all of x, from L2).
-static double gemv_mt_us(const LinearJob& job) {
+static double rows_mt_us(const LinearJob& job) {
   const LinearArgs& a = job.pr[0];
   const bool b4 = a.bits == 4;
   const int nw = a.m <= 32 ? 12 : 8;
@@ -855,20 +932,61 @@ static double gemv_mt_us(const LinearJob& job) {
          + turns * turn_us * (grid / 256 + (rest != 0 ? 0.83 + 0.17 * rest / 256 : 0.0));
 }
 
+// Expected time of gemv_ring_mt in us, within 18 % of the measured one for 96 of 100 (500 random problems of 17 to
+// 64 rows: linears of 512 to 32000 x 512 to 14336, several of a layer, gated units).  A round of blocks starts
+// and ends; a phase (a step of every wave) takes a part per tile of its waves expanded and one per row
+// of x that every wave reads from LDS.
+static double ring_mt_us(const LinearJob& job, const RingMtPlan& plan) {
+  const LinearArgs& a = job.pr[0];
+  const bool b4 = a.bits == 4;
+  const int matrices = job.glu ? 2 : 1;
+  const int rounds = (plan.grid + 255) / 256;
+  const double tiles = matrices * ((plan.rows_per_block + 15) / 16);
+  double outputs = 0;
+  for (int i = 0; i < job.count; ++i) outputs += (double)a.m * job.pr[i].n;
+  const double scales = (double)(a.k / a.group_size) * plan.rows_per_block * matrices * (a.symmetric ? 1 : 2);
+  // bf16 with a zero point has the longest conversion
+  const double expanded = plan.tl * (b4 && a.t_dtype == OFQ_BF16 && !a.symmetric ? 1.2 : 1.0);
+  const double reads = tiles * plan.wk * a.m;  // rows of a chunk of x, 256 bytes of them with 4-bit codes
+  const double phase = b4 ? 0.075 + 0.53 * expanded + 0.00088 * reads : 0.21 + 0.30 * expanded + 0.00045 * reads;
+  return rounds * (5.7 + 0.75 / 4096 * scales + plan.phases * phase) + 1.4e-6 * outputs;
+}
+
+// The faster of the two streaming kernels for a job: gemv_rows_mt, whose waves copy x for themselves, or
+// gemv_ring_mt, which starts 1.5 us later and takes less per byte.  One and two tiles of rows a block are the
+// former's (time over gemv_ring_mt's 0.78 and 0.91; 48 x 4096 x 4096 fp16 4-bit: 9.3 us, 11.5 there); from three
+// on a tenth less expected picks no problem of 300 that takes more than 1 % longer (64 x 11008 x 4096: 18.7 -> 16.1 us;
+// two weights of 9952 x 3584 at 31 rows, bf16 with a zero point: 39 -> 25, of 10880 x 4096 at 45, 8 bits: 43 -> 26).
+static double gemv_mt_us(const LinearJob& job, bool* ring, RingMtPlan* plan) {
+  const double rows = rows_mt_us(job);
+  *ring = ring_mt_plan(job, plan) && (job.glu ? 2 : 1) * ((plan->rows_per_block + 15) / 16) >= 3;
+  const double us = *ring ? ring_mt_us(job, *plan) : rows;
+  *ring = us < 0.9 * rows;
+  return *ring ? us * 1.05 : rows;
+}
+static int launch_mt_job(hipStream_t st, const LinearJob& job, bool ring, const RingMtPlan& plan) {
+  return ring ? launch_ring_mt(st, job, plan) : launch_rows_mt(st, job);
+}
+
 // gemm_wr reads x once per 128 rows of weights, but starts a second kernel where it slices K: so long
-// rows of weights leave the streaming kernel (64 x 4096 x 11008 fp16: 27.6 us here, 17.4 there) and n =
-// 11008 of k = 4096 stays (19.0 us here, 19.4 there).  Below 12.5 us the second launch and the workspace
+// rows of weights leave the streaming kernels (64 x 4096 x 11008 fp16: 27.6 us here, 17.4 there) and n =
+// 11008 of k = 4096 stays (16.4 us here, 19.4 there).  Below 12.5 us the second launch and the workspace
 // have to be won back as well: there the host, 3 us for the two, is what bounds a call that is not replayed
 // from a graph.
 bool gemv_mt_preferred(const LinearArgs& a, bool have_workspace) {
   if (!gemv_mt_supported(a)) return false;
-  const double us = gemv_mt_us(LinearJob{&a, 1, false, nullptr, 0});
+  bool ring;
+  RingMtPlan plan;
+  const double us = gemv_mt_us(LinearJob{&a, 1, false, nullptr, 0}, &ring, &plan);
   return us < gemm_wr_us(a, have_workspace, us < 12.5 ? 3.0 : 0.5);
 }
 
 int launch_gemv_mt(hipStream_t st, const LinearArgs& a) {
   const LinearJob job{&a, 1, false, nullptr, 0};
-  return launch_rows_mt(st, job);
+  bool ring;
+  RingMtPlan plan;
+  gemv_mt_us(job, &ring, &plan);
+  return launch_mt_job(st, job, ring, plan);
 }
 
 // Against one launch per problem (without a workspace: the entry points of several linears and gated units
@@ -878,6 +996,8 @@ int launch_gemv_mt_several(hipStream_t st, const LinearArgs* pr, int count, bool
   const LinearArgs& a = pr[0];
   const LinearJob job{pr, count, glu, y, act};
   double apart = glu ? 4.0 : 0.0;
+  bool ring;
+  RingMtPlan plan;
   for (int i = 0; i < count; ++i) {
     const LinearArgs& b = pr[i];
     if (!gemv_mt_supported(b) || b.t_dtype != a.t_dtype || b.bits != a.bits || b.w_signed != a.w_signed
@@ -885,11 +1005,12 @@ int launch_gemv_mt_several(hipStream_t st, const LinearArgs* pr, int count, bool
         || (glu && (b.x != a.x || b.n != a.n))) {
       return OFQ_ERR_UNSUPPORTED;
     }
-    const double mt = gemv_mt_us(LinearJob{&b, 1, false, nullptr, 0}), wr = gemm_wr_us(b, false, 0.0);
+    const double mt = gemv_mt_us(LinearJob{&b, 1, false, nullptr, 0}, &ring, &plan), wr = gemm_wr_us(b, false, 0.0);
     apart += mt < wr ? mt : wr;
   }
-  if (gemv_mt_us(job) > apart) return OFQ_ERR_UNSUPPORTED;
-  return launch_rows_mt(st, job);
+  const double us = gemv_mt_us(job, &ring, &plan);
+  if (us > apart) return OFQ_ERR_UNSUPPORTED;
+  return launch_mt_job(st, job, ring, plan);
 }
 
 bool gemv_wq_supported(const LinearArgs& a) {

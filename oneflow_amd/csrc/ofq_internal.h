@@ -124,6 +124,15 @@ struct RowsMtPlan {
 };
 int launch_gemv_mt_f16(hipStream_t st, const LinearJob& job, const RowsMtPlan& plan);
 int launch_gemv_mt_bf16(hipStream_t st, const LinearJob& job, const RowsMtPlan& plan);
+// gemv_ring_mt (gemv_ring_mt.h), 17 to 64 rows of x
+struct RingMtPlan {
+  int grid, rows_per_block, tl, wk, depth, buffers, phases;
+  size_t lds;
+};
+int launch_gemv_ring_mt_f16_b4(hipStream_t st, const LinearJob& job, const RingMtPlan& plan);
+int launch_gemv_ring_mt_f16_b8(hipStream_t st, const LinearJob& job, const RingMtPlan& plan);
+int launch_gemv_ring_mt_bf16_b4(hipStream_t st, const LinearJob& job, const RingMtPlan& plan);
+int launch_gemv_ring_mt_bf16_b8(hipStream_t st, const LinearJob& job, const RingMtPlan& plan);
 
 // matmul_quant with few rows of a (m <= 64; k a multiple of 64): int8 MFMA with the weights
 // streamed once.

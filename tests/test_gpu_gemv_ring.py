@@ -57,6 +57,47 @@ def test_one(m, n, k, g, dtype):
         _check(out, x, weight, g, bits, symmetric, (m, n, k, g, bits, symmetric, qdt, dtype))
 
 
+# 17 to 64 rows of x and three tiles of rows a block or more: two, three and four tiles of x with partial last ones,
+# one to three tiles of rows a wave, two to four buffers of x, one to six phases with K ending inside them
+MANY_TILES = [(31, 21517, 1184, 32), (20, 30011, 544, 32), (48, 17003, 1184, 32), (33, 28100, 480, 96),
+              (64, 20999, 1056, 32), (49, 9001, 2208, 32), (64, 32003, 96, 32)]
+
+
+@pytest.mark.parametrize("m,n,k,g", MANY_TILES)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_many_tiles(m, n, k, g, dtype):
+    test_one(m, n, k, g, dtype)
+
+
+@pytest.mark.parametrize("m,k,g,ns", [(40, 2016, 32, (16000, 40)), (64, 1184, 32, (9000, 2200, 2200))])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_many_tiles_several(m, k, g, ns, dtype):
+    test_several(m, k, g, ns, dtype)
+
+
+@pytest.mark.parametrize("m,n,k,g", [(32, 9001, 1184, 32), (33, 11003, 480, 96), (48, 6001, 2208, 32),
+                                     (64, 14001, 544, 32), (49, 9001, 1056, 32), (20, 30000, 160, 32)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_many_tiles_gated_unit(m, n, k, g, dtype):
+    test_gated_unit(m, n, k, g, dtype)
+
+
+def test_many_tiles_an_infinite_x_stays_in_its_row():
+    import oneflow_amd as flow
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    m, n, k, g = 49, 9001, 2208, 32
+    x = torch.randn(m, k, generator=gen, device="cuda").half()
+    w, scale, _, bias = _weight(gen, n, k, g, 4, True, torch.int8, torch.float16)
+    run = lambda a: flow._C.fused_linear_with_groupwise_quantized_weight(  # noqa: E731
+        a, w, scale, b=bias, num_bits=4, symmetric=True, group_dim=1, group_size=g)
+    plain = run(x)
+    x2 = x.clone()
+    x2[48, k - 1] = float("inf")
+    out = run(x2)
+    assert torch.equal(out[:48], plain[:48])
+    assert not bool(torch.isfinite(out[48][(w[:, -1] & 15) != 0]).any())
+
+
 @pytest.mark.parametrize("m,k,g,ns", [(1, 96, 32, (7, 1, 300)), (5, 1696, 32, (1111, 139, 139)), (8, 4128, 96, (4096, 17, 9)),
                                       (9, 736, 32, (515, 16, 33)), (17, 1696, 32, (1111, 139, 139)),
                                       (33, 1184, 32, (4097, 9, 1030)), (64, 544, 32, (9000, 2200)),
