@@ -118,9 +118,9 @@ int ofq_groupwise_dequantize(void* stream, const void* in, const void* scale, co
  *   differ in the last bits of the output.
  * Any m is accepted (the reference kernel has no m limit either, :473,590).
  * workspace: optional.  With a buffer of ofq_fused_linear_gq_workspace_bytes() (0 for m <= 16) the
- *   problem may be cut along K into blocks that leave fp32 partial sums there (16 < m < 1024), or,
- *   for m >= 1024 (n*k*sizeof(T)), the weight is dequantised once into it and a copy-fed MFMA GEMM
- *   runs on the result (the functor's own m > 8 decomposition); with NULL or a smaller buffer the
+ *   problem may be cut along K into blocks that leave fp32 partial sums there (m > 16), or,
+ *   for m >= 1024 (n*k*sizeof(T), or the partial sums where they take more), the weight is dequantised once into it
+ *   and a copy-fed MFMA GEMM runs on the result (the functor's own m > 8 decomposition); with NULL or a smaller buffer the
  *   weights are expanded inside the GEMM and a block walks all of K (same results up to fp32
  *   summation order, slower).  With group_dim 0 it is n*k*sizeof(T) for m > 64 (same decomposition;
  *   plus fp32 partial sums of K slices when there are few output tiles); without it the streaming
@@ -358,7 +358,7 @@ int ofq_matmul_quant(void* stream, const void* a, const void* b, const float* a_
 /*
  * The same op with an optional workspace (the op's tmp_buffer).  ofq_matmul_quant_workspace_bytes()
  * is non-zero when 64 < m and the 128-wide output tiles alone would leave most CUs without a
- * block: K is then cut into up to 8 slices that run as separate blocks, each writing its int32
+ * block: where that is the faster way, K is then cut into up to 8 slices that run as separate blocks, each writing its int32
  * partial sums to the workspace (splits * m * n * 4 bytes), and a second kernel adds the slices
  * (integer addition: the result does not depend on the order) and applies the epilogue.  Same
  * bits as ofq_matmul_quant, which is this call with workspace NULL.

@@ -11,7 +11,7 @@
 // Three kernels share one layout: a tile row is always 128 bytes of K (64 fp16/bf16 or 128 int8
 // elements), a k-step of the 32x32 MFMA consumes 32 of those bytes per row (16 bytes per lane), whatever
 // the type.  gemm_core2 (gemm_kernels.h) serves both operations, gemm_pp (gemm_pp.h) their copy-fed
-// tiles of 256 rows, gemm_wr (gemm_wr.h) 17 to 1023 rows with the weights packed up to the registers.
+// tiles of 256 rows, gemm_wr (gemm_wr.h) 17 rows and more with the weights packed up to the registers.
 // This file only chooses kernel, tile and slices and fills parameter blocks.
 #include <cmath>
 
@@ -21,27 +21,85 @@
 
 namespace ofq {
 
-// Width of the weight tile under a 256-row tile of x.  The blocks run in rounds of one per CU;
-// a round costs about in proportion to the tile width, so the candidate with the smallest
-// (rounds x width) wins, the wider one on a tie (less L2 -> LDS traffic per MFMA).  384 (waves
-// 4 x 2, 64 x 192 per wave: 12 MFMAs per 8 fragment reads) is open to the copy-fed GEMMs only and
-// runs about a tenth faster per column than the narrower tiles on random operands (2048 x 11008
-// x 4096 bf16: 163 us against 182 us for 352-wide tiles on 8 x 1 waves, whose waves read 12
-// fragments per 11 MFMAs), which its cost is credited with; 192 turns the 258 or 344 tiles of
-// m = 768 / 1024 at n = 11008 (two rounds of 128-wide tiles, the second nearly empty) into one
-// round of 174 / 232: 160 -> 115 us in-tile.
-int pick_tile_width(int64_t m, int64_t n, bool allow_wide) {
+// Width of the weight tile under a 256-row tile of x in the in-tile path.  The blocks run in rounds of one per
+// CU; a round costs about in proportion to the tile width, so the one with the smaller (rounds x width) wins,
+// the wider one on a tie (less L2 -> LDS traffic per MFMA): 192 turns the 258 or 344 tiles of m = 768 /
+// 1024 at n = 11008 (two rounds of 128-wide tiles, the second nearly empty) into one round of 174 / 232:
+// 160 -> 115 us.
+int pick_tile_width(int64_t m, int64_t n) {
   const int64_t m_tiles = (m + 255) / 256;
   auto cost = [&](int64_t bn) { return ((m_tiles * ((n + bn - 1) / bn) + 255) / 256) * bn; };
-  int best = 128;
-  if (cost(192) <= cost(best)) best = 192;
-  // 256 x 256 (copy-fed operands only): one round of 256 blocks where 128-wide tiles take two
-  // (int8 4096 x 4096 x 4096: 101 -> 87 us; bf16 4096 x 4096 x 11008 behind the dequantised
-  // weight: 410 -> 331 us, 8192 rows 1050 -> 750 us)
-  if (allow_wide && cost(256) <= cost(best)) best = 256;
-  if (allow_wide && cost(384) * 9 <= cost(best) * 10) best = 384;
-  return best;
+  return cost(192) <= cost(128) ? 192 : 128;
 }
+
+namespace {
+
+inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
+
+// The GEMMs whose operands are both copied (int8, and 16-bit behind a converted weight): their tiles, and the
+// expected time in us of one on m x n outputs and kt k-tiles of 128 bytes,
+//   start + outputs * m n / 10^6 + kt * (alone + share * b/256 + round * ceil(b/256) + pair * ceil(b/512))
+// with b blocks: tiles from 256 rows on run one block a CU (rounds of 256), those of 128 two, those of 64 more.
+// Fitted to 250 (int8, 65 <= m <= 8192) and 384 (16 bits, 1024 <= m <= 4096) random problems with 512 to 14336 and to
+// 32000 columns, k from 512 to 8192 and to 14336, each timed on every tile: within 12 % of the measured time for 90 of
+// 100, 64 x 64 tiles within 18 %.  The tile of the least expected time took 1.5 % longer than the best one in the
+// mean; rules by ranges of m and block counts, which this replaces, 15 % (int8) and 11 % (16 bits), most of it on
+// weights with few columns, whose 256-row tiles fill a part of the chip: int8 839 x 2054 x 1664 21.1 -> 8.4 us (64 x
+// 64 tiles), 1265 x 1120 x 1280 18.1 -> 7.1.
+enum CopyTile { kCopy64, kCopy128, kCopy256x128, kCopy256x192, kCopy256x256, kCopy256x384, kCopyTiles };
+struct TileCost {
+  int bm, bn;
+  double start, outputs, alone, share, round, pair;
+};
+const TileCost kCopyCost[2][2][kCopyTiles] = {  // [int8][ragged k]
+    {{{64, 64, 5.1, 0.17, 0.088, 0.194, 0.038, 0.0},
+      {128, 128, 4.3, 0.73, 0.0, 0.189, 0.013, 0.534},
+      {256, 128, 5.8, 0.71, 0.0, 0.203, 0.778, 0.0},
+      {256, 192, 8.6, 0.70, 0.0, 0.303, 0.887, 0.0},
+      {256, 256, 10.6, 0.75, 0.0, 0.469, 0.952, 0.0},
+      {256, 384, 13.9, 0.66, 0.0, 0.617, 1.324, 0.0}},
+     {{64, 64, 4.5, 0.37, 0.139, 0.151, 0.115, 0.0},
+      {128, 128, 4.4, 0.47, 0.0, 0.174, 0.204, 0.466},
+      {256, 128, 4.1, 0.84, 0.0, 0.027, 1.042, 0.0},
+      {256, 192, 8.0, 0.54, 0.0, 0.316, 1.100, 0.0},
+      {256, 256, 9.9, 0.66, 0.0, 0.382, 1.310, 0.0},
+      {256, 384, 14.6, 0.54, 0.0, 0.586, 1.697, 0.0}}},
+    {{{64, 64, 3.0, 0.54, 0.0, 0.077, 0.0, 0.271},
+      {128, 128, 3.4, 0.71, 0.0, 0.170, 0.177, 0.277},
+      {256, 128, 5.2, 0.77, 0.0, 0.256, 0.684, 0.0},
+      {256, 192, 9.2, 0.61, 0.0, 0.351, 0.816, 0.0},
+      {256, 256, 11.3, 0.59, 0.0, 0.457, 0.941, 0.0},
+      {256, 384, 13.7, 0.44, 0.0, 0.699, 1.329, 0.0}},
+     {{64, 64, 3.3, 0.41, 0.074, 0.071, 0.078, 0.219},
+      {128, 128, 4.0, 0.52, 0.0, 0.239, 0.247, 0.290},
+      {256, 128, 5.7, 0.81, 0.0, 0.221, 0.837, 0.0},
+      {256, 192, 9.4, 0.71, 0.0, 0.187, 1.044, 0.0},
+      {256, 256, 11.7, 0.55, 0.0, 0.206, 1.318, 0.0},
+      {256, 384, 14.4, 0.68, 0.0, 0.160, 1.728, 0.0}}}};
+
+double tile_us(const TileCost& c, int64_t m, int64_t n, int64_t kt, int splits = 1) {
+  const double b = (double)((m + c.bm - 1) / c.bm) * (double)((n + c.bn - 1) / c.bn) * splits;
+  return c.start + c.outputs * 1e-6 * (double)m * n
+         + kt * (c.alone + c.share * b / 256 + c.round * std::ceil(b / 256) + c.pair * std::ceil(b / 512));
+}
+CopyTile pick_copy_tile(bool int8, int64_t m, int64_t n, int64_t row_bytes, double* us) {
+  const TileCost* cost = kCopyCost[int8][row_bytes % 128 != 0];
+  int best = 0;
+  double best_us = 1e300;
+  for (int i = 0; i < kCopyTiles; ++i) {
+    double t = tile_us(cost[i], m, n, (row_bytes + 127) / 128);
+    // (int8 on long rows: up to 1.4 of what is expected, 434 x 2263 x 7168 31 us for 23, where slices take 26)
+    if (int8 && i == kCopy64 && row_bytes > 32 * 128) t *= 1.15;
+    if (t < best_us) {
+      best = i;
+      best_us = t;
+    }
+  }
+  if (us != nullptr) *us = best_us;
+  return (CopyTile)best;
+}
+
+}  // namespace
 
 namespace {
 
@@ -57,29 +115,26 @@ int launch_plain(hipStream_t st, const LinearArgs& a, const void* wt) {
   typename EP::Params ep;
   ep.bias = static_cast<const S*>(a.bias);
   ep.out = static_cast<S*>(a.out);
-  // 256-row tiles that would leave a quarter of the CUs without a block, where 128 x 128 tiles
-  // give 192 to 512 blocks: those, on 8 waves (1024 x 4096 x 4096)
-  const int64_t b256 = ((a.m + 255) / 256) * ((a.n + 127) / 128);
-  const int64_t b128 = ((a.m + 127) / 128) * ((a.n + 127) / 128);
-  if (b256 < 192 && b128 >= 192 && b128 <= 512) {
-    return launch_core2<MF, B2Copy<RG, 128, 512>, EP, 128, 128, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                  a.n, (a.k + 63) / 64);
-  }
-  const int width = pick_tile_width(a.m, a.n, true);
-  if (width == 128) {
-    return launch_core2<MF, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                  a.n, (a.k + 63) / 64);
+  const int64_t kt = (a.k + 63) / 64;
+  const CopyTile tile = pick_copy_tile(false, a.m, a.n, a.k * 2, nullptr);
+  switch (tile) {
+    case kCopy64:
+      return launch_core2<MF, B2Copy<RG, 64, 256>, EP, 64, 64, 2, 2>(st, a.x, a.k * 2, bp, ep, a.m, a.n, kt);
+    case kCopy128:
+      return launch_core2<MF, B2Copy<RG, 128, 512>, EP, 128, 128, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m, a.n, kt);
+    case kCopy256x128:
+      return launch_core2<MF, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m, a.n, kt);
+    default: break;
   }
   if constexpr (RG) {  // (why: launch_pp)
-    if (width == 192) {
-      return launch_core2<MF, B2Copy<RG, 192, 512>, EP, 256, 192, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                    a.n, (a.k + 63) / 64);
+    if (tile == kCopy256x192) {
+      return launch_core2<MF, B2Copy<RG, 192, 512>, EP, 256, 192, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m, a.n, kt);
     }
-    if (width == 256) {
-      return launch_core2<MF, B2Copy<RG, 256, 512>, EP, 256, 256, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m,
-                                                                    a.n, (a.k + 63) / 64);
+    if (tile == kCopy256x256) {
+      return launch_core2<MF, B2Copy<RG, 256, 512>, EP, 256, 256, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m, a.n, kt);
     }
   }
+  const int width = kCopyCost[0][RG][tile].bn;
   return std::is_same<T, f16>::value
              ? launch_gemm_pp_f16(st, a.x, wt, a.bias, a.out, a.m, a.n, a.k, width)
              : launch_gemm_pp_bf16(st, a.x, wt, a.bias, a.out, a.m, a.n, a.k, width);
@@ -190,7 +245,7 @@ int launch_wq_variant(hipStream_t st, const LinearArgs& a, float* partials, int 
   }
   // 256x128 tiles on 8 waves when there are enough rows of x to fill them, else 128x128 on 4
   if (a.m > 128) {
-    if (pick_tile_width(a.m, a.n, false) == 192) {
+    if (pick_tile_width(a.m, a.n) == 192) {
       return launch_core2<MF, B2Dequant<RG, T, BITS, SIGNED, ZMODE, 192, 512>, EP, 256, 192, 4, 2>(
           st, a.x, a.k * 2, bp, ep, a.m, a.n, (a.k + 63) / 64);
     }
@@ -251,12 +306,9 @@ double rounds_us(int blocks, int slots, double alone, double full) {
   return blocks / slots * full + (rest != 0 ? alone + (full - alone) * rest / slots : 0.0);
 }
 
-inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
-
 inline bool has_zero_term(const LinearArgs& a) { return !a.symmetric || !a.w_signed; }
 
-// Tile and K slices of gemm_wr for 16 < m < 1024 (fewer rows stream, more are worth a converted copy of
-// the weight) by the least expected time:
+// Tile and K slices of gemm_wr for more than 16 rows (fewer stream) by the least expected time:
 //   the start, and 1.9 per 4096 scales (and zeros) that a block copies first;
 //   the steps, measured with symmetric fp16 4-bit codes; others take longer to expand, which the taller
 //   tiles hide better; a K that is not whole steps costs 1.4 times as much (the copies of such a
@@ -266,7 +318,7 @@ inline bool has_zero_term(const LinearArgs& a) { return !a.symmetric || !a.w_sig
 // Without a workspace the sums of slices have nowhere to go: the tile that is best with one slice.
 double wr_plan_us(const LinearArgs& a, bool have_workspace, WrPlan* plan) {
   double best = 1e30;
-  if (a.m <= 16 || a.m >= 1024) return best;
+  if (a.m <= 16) return best;
   if (a.group_size % 32 != 0 || a.k % 32 != 0) return best;
   // k / group_size as a multiply-high by ceil(2^32 / group_size) is exact up to here
   if ((a.group_size & (a.group_size - 1)) != 0 && a.k * a.group_size >= ((int64_t)1 << 32)) return best;
@@ -335,7 +387,7 @@ double wq_us(const LinearArgs& a, int splits) {
   const int n128 = ceil_div(a.n, 128);
   double round;
   if (a.m > 128) {
-    const bool wide = splits == 1 && pick_tile_width(a.m, a.n, false) == 192;
+    const bool wide = splits == 1 && pick_tile_width(a.m, a.n) == 192;
     const int blocks = ceil_div(a.m, 256) * (wide ? ceil_div(a.n, 192) : n128) * splits;
     round = rounds_us(blocks, 256, wide ? 1.40 : 1.02, wide ? 1.73 : 1.24);
   } else if (splits > 1) {
@@ -372,22 +424,40 @@ size_t wr_partial_bytes(const LinearArgs& a, const WrPlan& plan) {
   return need > known ? need : known;
 }
 
+// Two passes for m >= 1024: the weight converted once at the rate of a large copy, and the copy-fed GEMM on it
+// (within 10 % for 90 of 100 of 384 problems with m to 4096).
+double two_pass_us(const LinearArgs& a) {
+  const double nk = (double)a.n * a.k;
+  double us;
+  pick_copy_tile(false, a.m, a.n, a.k * 2, &us);
+  return us + 2.2 + nk * (2 + a.bits / 8.0 + (a.symmetric ? 2.0 : 4.0) / a.group_size) / 5.9e6;
+}
+
 }  // namespace
 
+// From 1024 rows on against the converted weight, with 1.1 of gemm_wr's expected time (it is 5 % short there in the
+// mean): few columns or little K for the rows leave gemm_wr ahead, whose slices fill the chip and which does not write the
+// weight out (1105 x 863 x 7296 fp16 8-bit 121 -> 32 us, 1024 x 4096 x 11008 4-bit 140 -> 107).  Without a
+// workspace the weights of so many rows stay with gemm_core2's in-tile path.
 bool gemm_wr_plan(const LinearArgs& a, bool have_workspace, WrPlan* plan) {
+  if (a.m >= 1024 && !have_workspace) return false;
   const double us = wr_plan_us(a, have_workspace, plan);
   if (us >= 1e30) return false;
+  if (a.m >= 1024) return us * 1.1 < two_pass_us(a);
   return a.m <= 64 || us <= wq_us(a, have_workspace ? wq_splits(a) : 1);
 }
 
 // Two passes pay once m is large: the in-tile path converts every weight tile once per 256 rows
 // of x (8 times at m = 2048) and that conversion, not the MFMAs, bounds it; converting the weight
 // once into the workspace and running the copy-fed GEMM on it is what the reference functor does
-// for m > 8 (oneflow/core/functional/impl/quantization.cpp:341-350).
+// for m > 8 (oneflow/core/functional/impl/quantization.cpp:341-350).  From 1024 rows on never less than the
+// converted weight, the size that callers know for these problems.
 size_t gemm_wq_workspace_bytes(const LinearArgs& a) {
   if (!gemm_wq_supported(a)) return 0;
   WrPlan plan;
-  return gemm_wr_plan(a, true, &plan) ? wr_partial_bytes(a, plan) : wq_bytes(a);
+  if (!gemm_wr_plan(a, true, &plan)) return wq_bytes(a);
+  const size_t need = wr_partial_bytes(a, plan);
+  return a.m >= 1024 && need < wq_bytes(a) ? wq_bytes(a) : need;
 }
 
 // The streaming kernel's rival for 16 < m <= 64: what gemm_wr is expected to take, `two_launches` us more
@@ -402,9 +472,14 @@ int launch_gemm_wq(hipStream_t st, const LinearArgs& a, void* workspace, size_t 
   WrPlan plan;
   bool wr = gemm_wr_plan(a, true, &plan);
   const size_t need = wr ? wr_partial_bytes(a, plan) : wq_bytes(a);
-  const bool have_ws =
-      need != 0 && workspace != nullptr && workspace_bytes >= need && ofq_aligned16(workspace);
-  if (need != 0 && !have_ws) wr = gemm_wr_plan(a, false, &plan);
+  auto fits = [&](size_t bytes) {
+    return bytes != 0 && workspace != nullptr && workspace_bytes >= bytes && ofq_aligned16(workspace);
+  };
+  bool have_ws = fits(need);
+  if (need != 0 && !have_ws) {
+    wr = gemm_wr_plan(a, false, &plan);
+    have_ws = a.m >= 1024 && fits(wq_bytes(a));  // too little for the slices, enough for the converted weight
+  }
   if (wr) {
     float* partials = static_cast<float*>(workspace);
     return a.t_dtype == OFQ_F16 ? launch_gemm_wr_f16(st, a, plan, partials)
@@ -516,45 +591,27 @@ static constexpr int64_t kMatmulQuantRowsMaxM = 64;
 namespace ofq {
 namespace {
 
-// K slices of the int8 GEMM when its 128-wide tiles alone would leave most CUs without a block:
-// as many as still fit one resident round (256x128 tiles: one block per CU; 128x128: two), each
-// at least 4 k-tiles of 128.
-// Tiles below 256 rows, one launch, no K slices and no workspace, for the int8 GEMM on rows of up
-// to 6144 codes (a block's k loop costs about 0.4 us per 128-byte k-tile whatever the tile, so
-// on long rows K slices win again: 256 x 4096 x 11008 46.9 us against 27.8 us):
-//  - 64 x 64 tiles (4 waves) when there are 128 to 768 of them: they alone fill the chip
-//    (256 x 4096 x 4096: 256 blocks) and no partial sum leaves it -- 13.3 us against 18.7 us with
-//    slices; 128 rows 12.6 against 15.1, 512 rows 18.7 against 24.5, 768 rows 24.9 against 34.9,
-//    256 x 11008 x 4096 23.1 against 33.1;
-//  - 128 x 128 tiles on 8 waves when the 256-row tiles would leave a quarter of the CUs without
-//    a block and these give 192 to 512 blocks (1024 x 4096 x 4096: 28.7 against 36.3 us,
-//    512 x 11008 x 4096: 40.5 against 48.3 us).
-enum MqTile { kMqTileDefault = 0, kMqTile64 = 64, kMqTile128 = 128 };
-MqTile mq_tile(int64_t m, int64_t n, int64_t k) {
-  if (m <= kMatmulQuantRowsMaxM || k > 6144) return kMqTileDefault;
+// K slices for which the workspace query makes room, the size that callers know: where the 128-wide tiles of the int8
+// GEMM alone would leave most CUs without a block, as many as fit one resident round (256x128 tiles: one
+// block per CU; 128x128: two), each at least 4 k-tiles of 128.
+int mq_room(int64_t m, int64_t n, int64_t k) {
   const int64_t t64 = ((m + 63) / 64) * ((n + 63) / 64);
-  if (m <= 768 && t64 >= 128 && t64 <= 768) return kMqTile64;
   const int64_t b256 = ((m + 255) / 256) * ((n + 127) / 128);
   const int64_t b128 = ((m + 127) / 128) * ((n + 127) / 128);
-  if (b256 < 192 && b128 >= 192 && b128 <= 512) return kMqTile128;
-  return kMqTileDefault;
-}
-
-int mq_splits(int64_t m, int64_t n, int64_t k) {
-  if (mq_tile(m, n, k) != kMqTileDefault) return 1;
+  if (m > kMatmulQuantRowsMaxM && k <= 6144) {
+    if (m <= 768 && t64 >= 128 && t64 <= 768) return 1;
+    if (b256 < 192 && b128 >= 192 && b128 <= 512) return 1;
+  }
   // long rows (k >= 8192) already pay for slices from 33 rows of a on: 4096 x 11008 at m = 64
   // streams in 33 us and runs in 22 us as slices
   if (m <= (k >= 8192 ? kMatmulQuantRowsMaxM / 2 : kMatmulQuantRowsMaxM)) return 1;
-  int64_t bm = m > 128 ? 256 : 128;
+  int64_t blocks = m > 128 ? b256 : b128;
   int64_t slots = m > 128 ? 256 : 512;
   // up to 512 rows on a weight with few column tiles: 128-row tiles and fewer, longer slices
-  // write half the partial sums (256 x 4096 x 4096: 21.2 -> 18.8 us, 128 rows: 18.2 -> 15.1 us)
-  const bool few_tiles = m <= 512 && ((m + 127) / 128) * ((n + 127) / 128) <= 128;
-  if (few_tiles) {
-    bm = 128;
+  if (m <= 512 && b128 <= 128) {
+    blocks = b128;
     slots = m <= 128 ? 128 : 256;
   }
-  const int64_t blocks = ((m + bm - 1) / bm) * ((n + 127) / 128);
   int64_t s = slots / blocks;
   const int64_t kt = (k + 127) / 128;
   if (s > 8) s = 8;
@@ -562,6 +619,42 @@ int mq_splits(int64_t m, int64_t n, int64_t k) {
   if (s < 1) s = 1;
   while (s > 1 && ((kt + s - 1) / s) * (s - 1) >= kt) --s;  // no empty last slice
   return (int)s;
+}
+
+// Tile and slices by the least expected time (kCopyCost), with at most `most` slices: one slice on any tile, or
+// several of 128 x 128 or 256 x 128 tiles in one resident round, whose int32 sums and second launch cost 2 to 4 us and
+// 1.6 to 2 us per 10^6 sums.
+struct MqPlan {
+  CopyTile tile;
+  int splits;
+};
+MqPlan mq_plan(int64_t m, int64_t n, int64_t k, int most) {
+  // up to 64 rows (k >= 8192) the rival streams; the slices of the query are the ones that were measured against it
+  if (m <= kMatmulQuantRowsMaxM && most > 1) return MqPlan{kCopy128, most};
+  static const TileCost kSliced[2][2] = {{{128, 128, 5.5, 1.13, 0.0, 0.147, 0.0, 0.445},
+                                          {256, 128, 7.2, 1.33, 0.0, 0.178, 0.646, 0.0}},
+                                         {{128, 128, 5.9, 1.31, 0.0, 0.178, 0.033, 0.494},
+                                          {256, 128, 7.4, 1.52, 0.0, 0.084, 0.826, 0.0}}};
+  static const double kSums[2][2] = {{1.98, 1.57}, {1.72, 1.59}};  // us per 10^6 of a slice
+  MqPlan plan{kCopy64, 1};
+  double best;
+  plan.tile = pick_copy_tile(true, m, n, k, &best);
+  const int64_t kt = (k + 127) / 128;
+  const int ragged = k % 128 != 0;
+  for (int s = 2; s <= most; ++s) {
+    const int64_t per = (kt + s - 1) / s;
+    if (per < 2 || per * (s - 1) >= kt) continue;
+    for (int i = 0; i < 2; ++i) {
+      const TileCost& c = kSliced[ragged][i];
+      if ((int64_t)ceil_div(m, c.bm) * ceil_div(n, c.bn) * s > (i == 0 ? 512 : 256)) continue;
+      const double us = tile_us(c, m, n, per, s) + kSums[ragged][i] * s * 1e-6 * (double)m * n;
+      if (us < best) {
+        best = us;
+        plan = MqPlan{i == 0 ? kCopy128 : kCopy256x128, s};
+      }
+    }
+  }
+  return plan;
 }
 
 // adds the int32 slices (integer addition: any order gives the same sum) and applies the
@@ -586,13 +679,13 @@ splitk_finalize_i32(const int* __restrict__ part, const float* __restrict__ a_sc
 template<bool RG, typename T>
 int launch_mq_split(hipStream_t st, const void* a, const BCopyParams& bp, const float* a_scale,
                     const float* b_scale, const void* bias, void* out, int64_t m, int64_t n,
-                    int64_t k, float* partials, int splits) {
+                    int64_t k, float* partials, const MqPlan& plan) {
   typedef typename TT<T>::storage S;
+  const int splits = plan.splits;
   EpPartialI32::Params pp;
   pp.out = partials;
   int rc;
-  const bool few_tiles = m <= 512 && ((m + 127) / 128) * ((n + 127) / 128) <= 128;  // as mq_splits
-  if (m > 128 && !few_tiles) {
+  if (plan.tile == kCopy256x128) {
     rc = launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EpPartialI32, 256, 128, 4, 2>(st, a, k, bp, pp, m,
                                                                              n, (k + 127) / 128, splits);
   } else {
@@ -611,7 +704,8 @@ int launch_mq_split(hipStream_t st, const void* a, const BCopyParams& bp, const 
 // one launch, no K slices
 template<bool RG, typename T>
 int launch_mq(hipStream_t st, const void* a, const BCopyParams& bp, const float* a_scale,
-              const float* b_scale, const void* bias, void* out, int64_t m, int64_t n, int64_t k) {
+              const float* b_scale, const void* bias, void* out, int64_t m, int64_t n, int64_t k,
+              CopyTile tile) {
   typedef EpScale<T> EP;
   typename EP::Params ep;
   ep.a_scale = a_scale;
@@ -619,25 +713,19 @@ int launch_mq(hipStream_t st, const void* a, const BCopyParams& bp, const float*
   ep.bias = static_cast<const typename TT<T>::storage*>(bias);
   ep.out = static_cast<typename TT<T>::storage*>(out);
   const int64_t kt = (k + 127) / 128;
-  const MqTile tile = mq_tile(m, n, k);
-  if (tile == kMqTile64) {
-    return launch_core2<MfmaI8, B2Copy<RG, 64, 256>, EP, 64, 64, 2, 2>(st, a, k, bp, ep, m, n, kt);
-  }
-  if (tile == kMqTile128) {
-    return launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EP, 128, 128, 4, 2>(st, a, k, bp, ep, m, n, kt);
-  }
-  if (m <= 128) {
-    return launch_core2<MfmaI8, B2Copy<RG, 128, 256>, EP, 128, 128, 2, 2>(st, a, k, bp, ep, m, n, kt);
-  }
-  const int width = pick_tile_width(m, n, true);
-  if (width == 128) {
-    return launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a, k, bp, ep, m, n, kt);
+  switch (tile) {
+    case kCopy64: return launch_core2<MfmaI8, B2Copy<RG, 64, 256>, EP, 64, 64, 2, 2>(st, a, k, bp, ep, m, n, kt);
+    case kCopy128: return launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EP, 128, 128, 4, 2>(st, a, k, bp, ep, m, n, kt);
+    case kCopy256x128:
+      return launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a, k, bp, ep, m, n, kt);
+    default: break;
   }
   if constexpr (RG) {  // (why: launch_pp)
-    if (width == 192) {
+    if (tile == kCopy256x192) {
       return launch_core2<MfmaI8, B2Copy<RG, 192, 512>, EP, 256, 192, 4, 2>(st, a, k, bp, ep, m, n, kt);
     }
   }
+  const int width = kCopyCost[1][RG][tile].bn;
   return launch_gemm_pp_i8(st, a, bp.b, a_scale, b_scale, bias, out, TT<T>::dtype, m, n, k, width);
 }
 
@@ -646,7 +734,7 @@ int launch_mq(hipStream_t st, const void* a, const BCopyParams& bp, const float*
 
 extern "C" size_t ofq_matmul_quant_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
-  const int splits = ofq::mq_splits(m, n, k);
+  const int splits = ofq::mq_room(m, n, k);
   return splits > 1 ? (size_t)splits * (size_t)m * (size_t)n * 4 : 0;
 }
 
@@ -684,13 +772,17 @@ extern "C" int ofq_matmul_quant_ws(void* stream, const void* a, const void* b, c
   bp.b = static_cast<const uint8_t*>(b);
   bp.ldb = k;
   bp.N = (int)n;
+  MqPlan plan = mq_plan(m, n, k, 1);
   {
-    const int splits = mq_splits(m, n, k);
-    const size_t need = (size_t)splits * (size_t)m * (size_t)n * 4;
-    if (splits > 1 && workspace != nullptr && workspace_bytes >= need && ofq_aligned16(workspace)) {
+    const int room = mq_room(m, n, k);
+    const size_t need = (size_t)room * (size_t)m * (size_t)n * 4;
+    if (room > 1 && workspace != nullptr && workspace_bytes >= need && ofq_aligned16(workspace)) {
+      plan = mq_plan(m, n, k, room);
+    }
+    if (plan.splits > 1) {
       float* part = static_cast<float*>(workspace);
 #define OFQ_MQS(RG, T)                                                                           \
-  return launch_mq_split<RG, T>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, part, splits)
+  return launch_mq_split<RG, T>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, part, plan)
       if (k % 128 != 0) {
         switch (out_dtype) {
           case OFQ_F16: OFQ_MQS(true, f16);
@@ -712,14 +804,14 @@ extern "C" int ofq_matmul_quant_ws(void* stream, const void* a, const void* b, c
   }
   if (k % 128 != 0) {
     switch (out_dtype) {
-      case OFQ_F16: return launch_mq<true, f16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k);
-      case OFQ_BF16: return launch_mq<true, bf16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k);
-      default: return launch_mq<true, float>(st, a, bp, a_scale, b_scale, bias, out, m, n, k);
+      case OFQ_F16: return launch_mq<true, f16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, plan.tile);
+      case OFQ_BF16: return launch_mq<true, bf16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, plan.tile);
+      default: return launch_mq<true, float>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, plan.tile);
     }
   }
   switch (out_dtype) {
-    case OFQ_F16: return launch_mq<false, f16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k);
-    case OFQ_BF16: return launch_mq<false, bf16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k);
-    default: return launch_mq<false, float>(st, a, bp, a_scale, b_scale, bias, out, m, n, k);
+    case OFQ_F16: return launch_mq<false, f16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, plan.tile);
+    case OFQ_BF16: return launch_mq<false, bf16>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, plan.tile);
+    default: return launch_mq<false, float>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, plan.tile);
   }
 }

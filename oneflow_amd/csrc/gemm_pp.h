@@ -183,7 +183,7 @@ int launch_pp_tile(hipStream_t st, const void* a, const void* b, int64_t row_byt
   return ofq_check_launch();
 }
 
-// width: what pick_tile_width says.  This kernel against gemm_core2, time over time in the mean of 1200 random
+// width: what pick_copy_tile says.  This kernel against gemm_core2, time over time in the mean of 1200 random
 // problems (m to 8192, n to 32000, k to 14336; p. 95 is 2 to 5 % above the mean):
 //              rows of whole k-tiles: up to 16, 48, more    ragged rows: the same
 //   int8  192    0.99  0.99  0.98                           1.01  1.02  1.05

@@ -1097,7 +1097,7 @@ extern "C" size_t ofq_fused_linear_gq_workspace_bytes(int w_dtype, int t_dtype, 
   a.k = k;
   if (gemv_wq_supported(a) || gemv_m1_any_supported(a) || gemv_mt_preferred(a, true)) return 0;
   if (group_dim == 0) return gemm_gn_workspace_bytes(a);
-  return gemm_wq_workspace_bytes(a);  // K slices below 1024 rows, the converted weight from there on
+  return gemm_wq_workspace_bytes(a);  // K slices, from 1024 rows on at least the converted weight
 }
 
 extern "C" int ofq_fused_linear_gq(void* stream, const void* x, const void* w,

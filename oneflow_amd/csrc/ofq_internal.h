@@ -24,9 +24,9 @@ struct LinearArgs {
 
 // MFMA GEMM with in-tile dequantisation; groups along K.  Returns OFQ_ERR_UNSUPPORTED when the
 // shape does not meet the kernel's tiling constraints (caller falls back).
-// With a workspace of gemm_wq_workspace_bytes() K is cut into slices (m < 1024, where the tiles do not fill
-// the chip) or the weight is dequantised once into it and a copy-fed GEMM runs on the result (from 1024
-// rows on); without one a block walks all of K, on packed weights.
+// With a workspace of gemm_wq_workspace_bytes() K is cut into slices where the tiles do not fill the chip, or,
+// from 1024 rows on and where that is expected to take less, the weight is dequantised once into it and a copy-fed GEMM
+// runs on the result; without one a block walks all of K, on packed weights.
 bool gemm_wq_supported(const LinearArgs& a);
 size_t gemm_wq_workspace_bytes(const LinearArgs& a);
 int launch_gemm_wq(hipStream_t st, const LinearArgs& a, void* workspace, size_t workspace_bytes);
