@@ -172,6 +172,26 @@ def test_layer_norm_quantization_any_row(t, exact, rows, cols):
         assert torch.equal(codes, want)
 
 
+@pytest.mark.parametrize("rows", [9, 255, 256, 257, 1023, 1025, 4099, 16383, 16384, 16389, 40003])
+def test_layer_norm_observer_folds_every_row(rows):
+    """One partial maximum a row: the scale is that of the largest |y| whichever row holds it (one row is an impulse,
+    whose normalised peak is the largest there is)."""
+    import torch
+    import oneflow_amd as flow
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    cols = 33  # rows that a block each takes
+    x = torch.rand(rows, cols, generator=gen, device="cuda")
+    for row in sorted({0, 1, 3, 4, 63, 64, 255, 256, 257, 1023, 1024, 4095, 4096, 16383, 16384, rows // 2,
+                       rows - 4, rows - 3, rows - 2, rows - 1}):
+        if 0 <= row < rows:
+            t = x.clone()
+            t[row] = 0
+            t[row, 5] = 1
+            y, scale, zero = flow._C.fused_layer_norm_min_max_observer(t, None, None)
+            assert float(y.abs().max()) == float(y[row].abs().max())
+            assert torch.equal(scale.view(-1)[0], y.abs().max() / 127) and float(zero) == 0, row
+
+
 @pytest.mark.parametrize("t", ["f16", "bf16"])
 @pytest.mark.parametrize("exact", [False, True])
 @pytest.mark.parametrize("cols", [8, 504, 512, 1024, 1288, 2048, 2432, 4096, 4104, 8192, 8200])
