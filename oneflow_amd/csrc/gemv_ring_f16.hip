@@ -3,6 +3,8 @@
 
 namespace ofq {
 
-int launch_gemv_ring_f16(hipStream_t st, const LinearJob& job) { return launch_ring_t<f16>(st, job); }
+int launch_gemv_ring_f16(hipStream_t st, const LinearJob& job, const RingPlan& plan) {
+  return launch_ring_t<f16>(st, job, plan);
+}
 
 }  // namespace ofq

@@ -30,6 +30,7 @@
 //     to T.
 #include <atomic>
 #include "gemv_kernels.h"
+#include "gemv_ring.h"
 #include "gemv_rows.h"
 #include "ofq_device.h"
 #include "ofq_internal.h"
@@ -316,25 +317,117 @@ bool rows_supported(const LinearArgs& a) {
          && (a.symmetric || !a.w_signed);
 }
 
-// the ring kernel, where it is the faster one (gemv_ring_launch.h)
-int launch_ring(hipStream_t st, const LinearJob& job) {
+// The split of gemv_ring for a job, or false where scales, rings and x do not fit LDS.
+//
+// One block per CU and round; the waves' split over tiles and K by the longest wave's turns, a turn being a
+// tile's expansion and products and a step's share of reading x (about half of that).
+bool ring_plan(const LinearJob& job, RingPlan* plan) {
+  const LinearArgs& a = job.pr[0];
+  const int lists = job.glu ? 1 : job.count, matrices = job.glu ? 2 : 1;
+  const int ck = a.bits == 4 ? 128 : 64, rec = ck * 2;
+  const int G = (int)(a.k / a.group_size);
+  const int regions = matrices * (a.symmetric ? 1 : 2);
+  const int M = (int)a.m;
+  const int tr = M <= 8 ? 8 : 16, sub = tr == 8 ? 2 : 1;
+  const int steps = (int)((a.k + ck * sub - 1) / (ck * sub));
+  constexpr int kCUs = 256, kLds = 160 * 1024;
+  int64_t total = 0;
+  for (int i = 0; i < lists; ++i) total += job.pr[i].n;
+  auto blocks_at = [&](int rpb) {
+    int64_t b = 0;
+    for (int i = 0; i < lists; ++i) b += (job.pr[i].n + rpb - 1) / rpb;
+    return b;
+  };
+  for (int rounds = 1; rounds <= 512; rounds *= 2) {
+    const int64_t want = (int64_t)kCUs * rounds;
+    int64_t rpb64 = (total + want - 1) / want;
+    if (rpb64 > 512) continue;
+    int rpb = (int)rpb64 < tr ? tr : (int)rpb64;
+    while (blocks_at(rpb) > want && rpb < 512) ++rpb;
+    // not more tiles than the rows need: the last tile of every block full
+    const int ntiles = (rpb + tr - 1) / tr;
+    const int nvt = matrices * ntiles;
+    const int scales = (regions * ring_scale_bytes(rpb, G) + 1023) & ~1023;
+    double best = 1e30;
+    for (int wk_shift = 4; wk_shift >= 0; --wk_shift) {
+      const int wk = 1 << wk_shift, groups = kRingWaves >> wk_shift;
+      const int tl = (nvt + groups - 1) / groups;
+      if (tl > kRingMaxTiles) continue;
+      const int depth = tl == 1 ? 3 : (tl == 2 ? 2 : 1);
+      const int budget = kLds - scales - kRingWaves * depth * tl * 1024;
+      const int step_x = sub * M * rec;
+      if (budget < 1024) continue;
+      int phase_steps = steps, phases = 1;
+      if ((int64_t)steps * step_x > budget / 1024 * 1024) {
+        phase_steps = (budget / 2 / 1024 * 1024) / step_x / wk * wk;
+        if (phase_steps < wk) continue;
+        phases = (steps + phase_steps - 1) / phase_steps;
+        phase_steps = ((steps + phases - 1) / phases + wk - 1) / wk * wk;
+        phases = (steps + phase_steps - 1) / phase_steps;
+      }
+      const int xbuf = (phase_steps * step_x + 1023) & ~1023;
+      size_t lds = (size_t)scales + kRingWaves * depth * tl * 1024 + (size_t)xbuf * (phases > 1 ? 2 : 1);
+      const size_t red = ((size_t)nvt << wk_shift) * M * 16 * 4;
+      if (red > lds) lds = red;
+      if (lds > kLds) continue;
+      const int turns = phases == 1 ? (steps + wk - 1) / wk : phases * (phase_steps / wk);
+      const double cost = turns * (tl + 0.5) + 1.0 * (phases - 1);
+      if (cost < best) {
+        best = cost;
+        plan->tr = tr;
+        plan->tl = tl;
+        plan->lds = lds;
+        plan->wk_shift = wk_shift;
+        plan->phase_steps = phase_steps;
+        plan->phases = phases;
+      }
+    }
+    if (best >= 1e30) continue;
+    const int64_t grid = blocks_at(rpb);
+    if (grid > 0x7FFFFFFF) return false;
+    plan->grid = (int)grid;
+    plan->rows_per_block = rpb;
+    return true;
+  }
+  return false;
+}
+
+}  // namespace
+
+// Whether gemv_ring takes a job, and how.  (The plan comes last: its loops run for every call, and small calls are
+// bound by the host: 3 x 1560 x 1024 bf16 5.7 us with the plan, 5.3 before it.)
+// Where the ring is the faster one: 6000 random problems (m 1 .. 16, n 512 .. 32000, k 512 .. 14336, both types
+// and widths, groups of 32, 64, 128), time of the kernels that ran before over this one's:
+//   gated units                                   1.27 (5 of 100 below 1.08): two launches and the gating's
+//   several linears                               1.14 (5 of 100 below 0.97)
+//   one linear of more than 16 rows a block, or of whole turns of waves over short blocks   1.14
+// and where it is not: one row of x of up to 4096 elements (0.87: gemv_m1_any), one linear of one 16-row tile a
+// block (0.96: gemv_rows, whose requests land in registers, has nothing to balance there), and more than 8 rows
+// of x that pass LDS in four parts or more (1.0, down to 0.75).
+bool gemv_ring_choice(const LinearJob& job, RingPlan* plan) {
   const LinearArgs& a = job.pr[0];
   for (int i = 0; i < job.count; ++i) {
     const LinearArgs& b = job.pr[i];
     if (!rows_supported(b) || b.t_dtype != a.t_dtype || b.bits != a.bits || b.w_signed != a.w_signed
         || b.symmetric != a.symmetric || b.group_size != a.group_size || b.m != a.m || b.k != a.k) {
-      return OFQ_ERR_UNSUPPORTED;
+      return false;
     }
   }
-  // What ring_preferred would say of one linear with at most 16 rows a block, without the plan, whose loops the host
-  // runs for every call: small calls are bound by the host (3 x 1560 x 1024 bf16: 5.7 us with the plan, 5.3 before it).
   if (job.count == 1) {
-    const int64_t rows = (a.n + 255) / 256;
-    if (a.m == 1 && a.k <= 4096) return OFQ_ERR_UNSUPPORTED;
-    const bool turns = a.k > 16 * 2 * (a.bits == 4 ? 128 : 64);  // 16 waves take more than a step each
-    if (rows <= 16 && !(a.m > 1 && a.m <= 8 && rows <= 8 && turns)) return OFQ_ERR_UNSUPPORTED;
+    const int64_t rows = (a.n + 255) / 256;  // of a block
+    if (a.m == 1 && a.k <= 4096) return false;
+    const bool turns = a.k > kRingWaves * 2 * (a.bits == 4 ? 128 : 64);  // the waves take more than a step each
+    if (rows <= 16 && !(a.m > 1 && a.m <= 8 && rows <= 8 && turns)) return false;
   }
-  return a.t_dtype == OFQ_BF16 ? launch_gemv_ring_bf16(st, job) : launch_gemv_ring_f16(st, job);
+  return ring_plan(job, plan) && !(a.m > 8 && plan->phases >= 4);
+}
+
+namespace {
+
+int launch_ring(hipStream_t st, const LinearJob& job) {
+  RingPlan plan;
+  if (!gemv_ring_choice(job, &plan)) return OFQ_ERR_UNSUPPORTED;
+  return job.pr[0].t_dtype == OFQ_BF16 ? launch_gemv_ring_bf16(st, job, plan) : launch_gemv_ring_f16(st, job, plan);
 }
 
 template<typename T, int NW>

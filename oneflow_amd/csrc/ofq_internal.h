@@ -114,9 +114,14 @@ struct LinearJob {
   void* y;
   int act;
 };
-// The ring kernel (gemv_ring.h), up to 16 rows of x; OFQ_ERR_UNSUPPORTED where it is not the faster one.
-int launch_gemv_ring_f16(hipStream_t st, const LinearJob& job);
-int launch_gemv_ring_bf16(hipStream_t st, const LinearJob& job);
+// The ring kernel (gemv_ring.h), up to 16 rows of x
+struct RingPlan {
+  int grid, rows_per_block, tr, tl, wk_shift, phase_steps, phases;
+  size_t lds;
+};
+bool gemv_ring_choice(const LinearJob& job, RingPlan* plan);
+int launch_gemv_ring_f16(hipStream_t st, const LinearJob& job, const RingPlan& plan);
+int launch_gemv_ring_bf16(hipStream_t st, const LinearJob& job, const RingPlan& plan);
 // gemv_rows_mt (gemv_rows.h), 17 to 64 rows of x
 struct RowsMtPlan {
   int grid, rows_per_block, panel_chunks, panel_groups;

@@ -1,0 +1,94 @@
+"""Which streaming kernel a linear, several of them or a gated unit are launched with, and how (host code of the
+library: no GPU)."""
+import ctypes
+import random
+
+import pytest
+
+from oneflow_amd import _lib
+from test_gemm_plan import LinearArgs
+
+LDS = 160 * 1024
+
+
+class LinearJob(ctypes.Structure):  # csrc/ofq_internal.h, as the plans below
+    _fields_ = [("pr", ctypes.POINTER(LinearArgs)), ("count", ctypes.c_int), ("glu", ctypes.c_bool),
+                ("y", ctypes.c_void_p), ("act", ctypes.c_int)]
+
+
+class RingPlan(ctypes.Structure):
+    _fields_ = ([(f, ctypes.c_int) for f in ("grid", "rows_per_block", "tr", "tl", "wk_shift", "phase_steps",
+                                             "phases")] + [("lds", ctypes.c_size_t)])
+
+
+def _job(ns, m, k, g, bits, symmetric, dtype, glu):
+    pr = (LinearArgs * len(ns))(*[
+        LinearArgs(t_dtype=dtype, w_signed=symmetric, bits=bits, symmetric=symmetric, group_dim=1, group_size=g,
+                   m=m, n=n, k=k) for n in ns])
+    return LinearJob(pr, len(ns), glu, None, 0)
+
+
+def ring_plan(ns, m, k, g, bits, symmetric, dtype=_lib.F16, glu=False):
+    """The plan of gemv_ring (1 to 16 rows of x), or None where another kernel serves."""
+    f = _lib.lib()["_ZN3ofq16gemv_ring_choiceERKNS_9LinearJobEPNS_8RingPlanE"]
+    f.restype, f.argtypes = ctypes.c_bool, [ctypes.POINTER(LinearJob), ctypes.POINTER(RingPlan)]
+    plan = RingPlan()
+    return plan if f(ctypes.byref(_job(ns, m, k, g, bits, symmetric, dtype, glu)), ctypes.byref(plan)) else None
+
+
+def _random_job(rng, m):
+    bits, g = rng.choice([4, 8]), rng.choice([32, 64, 96, 128])
+    k = g * rng.randint(1, 14336 // g)
+    mode = rng.choice(["one", "several", "glu"])
+    ns = [rng.randint(1, 32000)] if mode == "one" else [k, max(1, k // 4), max(1, k // 4)]
+    if mode == "glu":
+        ns = [rng.randint(1, 20000)] * 2
+    return ns, m, k, g, bits, rng.choice([True, False]), rng.choice([_lib.F16, _lib.BF16]), mode == "glu"
+
+
+def _scale_bytes(rows, groups):
+    return (rows * groups * 2 + 16 + 15) & ~15
+
+
+def test_every_plan_of_the_ring_is_what_the_kernel_assumes():
+    """All rows and all of K are covered, what the kernel lays out in LDS fits, and the counts that its waits
+    are written for are kept."""
+    rng, seen = random.Random(0), 0
+    for _ in range(20000):
+        job = ns, m, k, g, bits, symmetric, _, glu = _random_job(rng, rng.randint(1, 16))
+        p = ring_plan(*job)
+        if p is None:
+            continue
+        seen += 1
+        mats, lists = (2, ns[:1]) if glu else (1, ns)
+        ck = 128 if bits == 4 else 64
+        sub = 2 if m <= 8 else 1
+        steps, wk = -(-k // (ck * sub)), 1 << p.wk_shift
+        tiles = mats * -(-p.rows_per_block // p.tr)
+        depth = {1: 3, 2: 2, 3: 1, 4: 1}[p.tl]
+        assert p.tr == (8 if m <= 8 else 16), job
+        assert p.grid == sum(-(-n // p.rows_per_block) for n in lists), job
+        assert (16 >> p.wk_shift) * p.tl >= tiles, job
+        assert p.phases * p.phase_steps >= steps > (p.phases - 1) * p.phase_steps, job
+        assert p.phases == 1 or p.phase_steps % wk == 0, job
+        scales = mats * (1 if symmetric else 2) * _scale_bytes(p.rows_per_block, k // g)
+        x = (p.phase_steps * sub * m * ck * 2 + 1023) & ~1023
+        used = ((scales + 1023) & ~1023) + 16 * depth * p.tl * 1024 + x * (1 if p.phases == 1 else 2)
+        assert max(used, tiles * wk * m * 64) <= p.lds <= LDS, job
+    assert seen > 5000
+
+
+# (rows of the weights, rows of x, k, group, bits, symmetric, gated) -> served by gemv_ring
+@pytest.mark.parametrize("ns,m,k,g,bits,symmetric,glu,ring", [
+    ([11008], 8, 4096, 32, 4, True, False, True), ([11008], 12, 4096, 64, 8, False, False, True),
+    ([1024], 4, 8192, 64, 4, True, False, True),    # short blocks, whole turns of waves
+    ([1024], 4, 4096, 64, 4, True, False, False),   # the same, one turn
+    ([4096], 4, 4096, 64, 4, True, False, False),   # one 16-row tile a block
+    ([11008], 1, 4096, 64, 4, True, False, False), ([11008], 1, 4128, 32, 4, True, False, True),
+    ([8200], 16, 8192, 64, 8, True, False, False),  # more than 8 rows of x in four parts or more
+    ([4672] * 2, 3, 1536, 32, 8, False, True, True), ([4096, 1024, 1024], 4, 4096, 64, 4, True, False, True),
+    ([11008], 17, 4096, 64, 4, True, False, False),  # up to 16 rows of x
+    ([11008], 8, 4104, 24, 4, True, False, False)])  # groups of whole lanes
+def test_where_the_ring_serves(ns, m, k, g, bits, symmetric, glu, ring):
+    for dtype in (_lib.F16, _lib.BF16):
+        assert (ring_plan(ns, m, k, g, bits, symmetric, dtype, glu) is not None) == ring, dtype
