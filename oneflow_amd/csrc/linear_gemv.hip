@@ -1058,18 +1058,19 @@ static double ring_mt_us(const LinearJob& job, const RingMtPlan& plan) {
 // former's (time over gemv_ring_mt's 0.78 and 0.91; 48 x 4096 x 4096 fp16 4-bit: 9.3 us, 11.5 there); from three
 // on a tenth less expected picks no problem of 300 that takes more than 1 % longer (64 x 11008 x 4096: 18.7 -> 16.1 us;
 // two weights of 9952 x 3584 at 31 rows, bf16 with a zero point: 39 -> 25, of 10880 x 4096 at 45, 8 bits: 43 -> 26).
-static double gemv_mt_us(const LinearJob& job, bool* ring, RingMtPlan* plan) {
+void gemv_mt_choice(const LinearJob& job, MtChoice* choice) {
   const double rows = rows_mt_us(job);
   int64_t total = 0;
   for (int i = 0; i < (job.glu ? 1 : job.count); ++i) total += job.pr[i].n;
   const auto tiles = [&](int64_t rpb) { return (job.glu ? 2 : 1) * ((rpb + 15) / 16); };
-  *ring = tiles((total + 255) / 256) >= 3 && ring_mt_plan(job, plan) && tiles(plan->rows_per_block) >= 3;
-  const double us = *ring ? ring_mt_us(job, *plan) : rows;
-  *ring = us < 0.9 * rows;
-  return *ring ? us * 1.05 : rows;
+  RingMtPlan& plan = choice->plan;
+  choice->ring = tiles((total + 255) / 256) >= 3 && ring_mt_plan(job, &plan) && tiles(plan.rows_per_block) >= 3;
+  const double ring = choice->ring ? ring_mt_us(job, plan) : 0.0;
+  choice->ring = choice->ring && ring < 0.9 * rows;
+  choice->us = choice->ring ? ring * 1.05 : rows;
 }
-static int launch_mt_job(hipStream_t st, const LinearJob& job, bool ring, const RingMtPlan& plan) {
-  return ring ? launch_ring_mt(st, job, plan) : launch_rows_mt(st, job);
+static int launch_mt_job(hipStream_t st, const LinearJob& job, const MtChoice& choice) {
+  return choice.ring ? launch_ring_mt(st, job, choice.plan) : launch_rows_mt(st, job);
 }
 
 // gemm_wr reads x once per 128 rows of weights, but starts a second kernel where it slices K: so long
@@ -1077,20 +1078,14 @@ static int launch_mt_job(hipStream_t st, const LinearJob& job, bool ring, const 
 // 11008 of k = 4096 stays (16.4 us here, 19.4 there).  Below 12.5 us the second launch and the workspace
 // have to be won back as well: there the host, 3 us for the two, is what bounds a call that is not replayed
 // from a graph.
-bool gemv_mt_preferred(const LinearArgs& a, bool have_workspace) {
+bool gemv_mt_preferred(const LinearArgs& a, bool have_workspace, MtChoice* choice) {
   if (!gemv_mt_supported(a)) return false;
-  bool ring;
-  RingMtPlan plan;
-  const double us = gemv_mt_us(LinearJob{&a, 1, false, nullptr, 0}, &ring, &plan);
-  return us < gemm_wr_us(a, have_workspace, us < 12.5 ? 3.0 : 0.5);
+  gemv_mt_choice(LinearJob{&a, 1, false, nullptr, 0}, choice);
+  return choice->us < gemm_wr_us(a, have_workspace, choice->us < 12.5 ? 3.0 : 0.5);
 }
 
-int launch_gemv_mt(hipStream_t st, const LinearArgs& a) {
-  const LinearJob job{&a, 1, false, nullptr, 0};
-  bool ring;
-  RingMtPlan plan;
-  gemv_mt_us(job, &ring, &plan);
-  return launch_mt_job(st, job, ring, plan);
+int launch_gemv_mt(hipStream_t st, const LinearArgs& a, const MtChoice& choice) {
+  return launch_mt_job(st, LinearJob{&a, 1, false, nullptr, 0}, choice);
 }
 
 // Against one launch per problem (without a workspace: the entry points of several linears and gated units
@@ -1100,8 +1095,7 @@ int launch_gemv_mt_several(hipStream_t st, const LinearArgs* pr, int count, bool
   const LinearArgs& a = pr[0];
   const LinearJob job{pr, count, glu, y, act};
   double apart = glu ? 4.0 : 0.0;
-  bool ring;
-  RingMtPlan plan;
+  MtChoice choice;
   for (int i = 0; i < count; ++i) {
     const LinearArgs& b = pr[i];
     if (!gemv_mt_supported(b) || b.t_dtype != a.t_dtype || b.bits != a.bits || b.w_signed != a.w_signed
@@ -1109,12 +1103,13 @@ int launch_gemv_mt_several(hipStream_t st, const LinearArgs* pr, int count, bool
         || (glu && (b.x != a.x || b.n != a.n))) {
       return OFQ_ERR_UNSUPPORTED;
     }
-    const double mt = gemv_mt_us(LinearJob{&b, 1, false, nullptr, 0}, &ring, &plan), wr = gemm_wr_us(b, false, 0.0);
-    apart += mt < wr ? mt : wr;
+    gemv_mt_choice(LinearJob{&b, 1, false, nullptr, 0}, &choice);
+    const double wr = gemm_wr_us(b, false, 0.0);
+    apart += choice.us < wr ? choice.us : wr;
   }
-  const double us = gemv_mt_us(job, &ring, &plan);
-  if (us > apart) return OFQ_ERR_UNSUPPORTED;
-  return launch_mt_job(st, job, ring, plan);
+  gemv_mt_choice(job, &choice);
+  if (choice.us > apart) return OFQ_ERR_UNSUPPORTED;
+  return launch_mt_job(st, job, choice);
 }
 
 bool gemv_wq_supported(const LinearArgs& a) {
@@ -1199,7 +1194,8 @@ extern "C" size_t ofq_fused_linear_gq_workspace_bytes(int w_dtype, int t_dtype, 
   a.m = m;
   a.n = n;
   a.k = k;
-  if (gemv_wq_supported(a) || gemv_m1_any_supported(a) || gemv_mt_preferred(a, true)) return 0;
+  MtChoice choice;
+  if (gemv_wq_supported(a) || gemv_m1_any_supported(a) || gemv_mt_preferred(a, true, &choice)) return 0;
   if (group_dim == 0) return gemm_gn_workspace_bytes(a);
   return gemm_wq_workspace_bytes(a);  // K slices, from 1024 rows on at least the converted weight
 }
@@ -1256,9 +1252,10 @@ extern "C" int ofq_fused_linear_gq(void* stream, const void* x, const void* w,
     const int rc = launch_gemv_wq(st, a);
     if (rc != OFQ_ERR_UNSUPPORTED) return rc;  // e.g. bf16 with an x too large to stage
   }
+  MtChoice choice;
   if (a.m > 16 && a.m <= 64
-      && gemv_mt_preferred(a, workspace != nullptr && workspace_bytes >= gemm_wq_workspace_bytes(a))) {
-    const int rc = launch_gemv_mt(st, a);
+      && gemv_mt_preferred(a, workspace != nullptr && workspace_bytes >= gemm_wq_workspace_bytes(a), &choice)) {
+    const int rc = launch_gemv_mt(st, a, choice);
     if (rc != OFQ_ERR_UNSUPPORTED) return rc;
   }
   if (gemm_wq_supported(a)) return launch_gemm_wq(st, a, workspace, workspace_bytes);

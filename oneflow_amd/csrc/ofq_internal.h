@@ -78,10 +78,11 @@ int launch_gemv_m1_any(hipStream_t st, const LinearArgs& a);
 bool gemv_wq_supported(const LinearArgs& a);
 int launch_gemv_wq(hipStream_t st, const LinearArgs& a);
 
-// 16 < m <= 64: the decode kernel's row split with several 16-row tiles of x per weight tile, without a
-// workspace.  Not where gemm_wr is expected to take less.
-bool gemv_mt_preferred(const LinearArgs& a, bool have_workspace);
-int launch_gemv_mt(hipStream_t st, const LinearArgs& a);
+// 16 < m <= 64: the streaming kernels with several 16-row tiles of x per weight tile, without a
+// workspace.  Not where gemm_wr is expected to take less; `choice` is which of the two runs, and how.
+struct MtChoice;
+bool gemv_mt_preferred(const LinearArgs& a, bool have_workspace, MtChoice* choice);
+int launch_gemv_mt(hipStream_t st, const LinearArgs& a, const MtChoice& choice);
 // several of them, or a gated unit's two with y = out0 * act(out1), in one launch where that is expected to
 // take less than one by one; else OFQ_ERR_UNSUPPORTED
 int launch_gemv_mt_several(hipStream_t st, const LinearArgs* problems, int count, bool glu, void* y, int act);
@@ -134,6 +135,13 @@ struct RingMtPlan {
   int grid, rows_per_block, tl, wk, depth, buffers, phases;
   size_t lds;
 };
+// the faster of the two for a job, and its expected time
+struct MtChoice {
+  bool ring;  // gemv_ring_mt, by `plan`
+  RingMtPlan plan;
+  double us;
+};
+void gemv_mt_choice(const LinearJob& job, MtChoice* choice);
 int launch_gemv_ring_mt_f16_b4(hipStream_t st, const LinearJob& job, const RingMtPlan& plan);
 int launch_gemv_ring_mt_f16_b8(hipStream_t st, const LinearJob& job, const RingMtPlan& plan);
 int launch_gemv_ring_mt_bf16_b4(hipStream_t st, const LinearJob& job, const RingMtPlan& plan);
