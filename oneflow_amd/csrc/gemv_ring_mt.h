@@ -13,7 +13,7 @@
 // way from the barrier over x from LDS, the expansion and the products to the next one, and 5.7 us to start, load
 // the first x, fold and store.  A phase's x is read from LDS by every wave for its own tiles (0.09 us per 100 rows
 // of a 4-bit chunk), so more tiles of a wave cost less each.  Against gemv_rows_mt (us):
-//   fp16 4-bit  48 x 11008 x 4096 with a zero point  17.8 -> 16.0   64 x 11008 x 4096        18.7 -> 16.1
+//   fp16 4-bit  48 x 11008 x 4096 with a zero point  17.8 -> 16.0   64 x 11008 x 4096        20.6 -> 18.6
 //   fp16 4-bit  40 x 22000 x 2944   29.3 -> 18.2 (gemm_wr 19.9)     20 x 2 x 9216 x 3584     27.3 -> 18.7
 //   8 bits      56 x 2 x 12032 x 3968 bf16  51.4 -> 33.2            45 x 2 x 10880 x 4096 fp16  43.2 -> 26
 // Addresses of x made once instead of for every copy, and two to three buffers in flight: 48 x 11008 x 4096 21.2 -> 16.7.

@@ -1053,21 +1053,19 @@ static double ring_mt_us(const LinearJob& job, const RingMtPlan& plan) {
   return rounds * (5.7 + 0.75 / 4096 * scales + plan.phases * phase) + 1.4e-6 * outputs;
 }
 
-// The faster of the two streaming kernels for a job: gemv_rows_mt, whose waves copy x for themselves, or
-// gemv_ring_mt, which starts 1.5 us later and takes less per byte.  One and two tiles of rows a block are the
-// former's (time over gemv_ring_mt's 0.78 and 0.91; 48 x 4096 x 4096 fp16 4-bit: 9.3 us, 11.5 there); from three
-// on a tenth less expected picks no problem of 300 that takes more than 1 % longer (64 x 11008 x 4096: 18.7 -> 16.1 us;
-// two weights of 9952 x 3584 at 31 rows, bf16 with a zero point: 39 -> 25, of 10880 x 4096 at 45, 8 bits: 43 -> 26).
+// Which of the two streaming kernels takes a job, gemv_rows_mt, whose waves copy x for themselves, or gemv_ring_mt,
+// which starts 1.5 us later and takes less per byte.  Both timed on 6065 random jobs of 17 to 64 rows (linears of 512
+// to 32000 x 512 to 14336, several of a layer, gated units; weights from HBM): with three tiles of rows a block and
+// more gemv_ring_mt takes 0.78 of the time in the mean, 38 of 2310 more than 3 % longer (1.13 at worst, 36 x 8388 x
+// 512 8-bit); with one and two tiles 1.21 and 1.02 times.  (A comparison of expected times, with a tenth
+// to spare, turned 824 of the 2310 away: 64 x 11008 x 4096 fp16 4-bit 20.6 us, now 18.6, 56 rows 18.7 -> 16.6.)
 void gemv_mt_choice(const LinearJob& job, MtChoice* choice) {
-  const double rows = rows_mt_us(job);
   int64_t total = 0;
   for (int i = 0; i < (job.glu ? 1 : job.count); ++i) total += job.pr[i].n;
   const auto tiles = [&](int64_t rpb) { return (job.glu ? 2 : 1) * ((rpb + 15) / 16); };
   RingMtPlan& plan = choice->plan;
   choice->ring = tiles((total + 255) / 256) >= 3 && ring_mt_plan(job, &plan) && tiles(plan.rows_per_block) >= 3;
-  const double ring = choice->ring ? ring_mt_us(job, plan) : 0.0;
-  choice->ring = choice->ring && ring < 0.9 * rows;
-  choice->us = choice->ring ? ring * 1.05 : rows;
+  choice->us = choice->ring ? ring_mt_us(job, plan) * 1.05 : rows_mt_us(job);
 }
 static int launch_mt_job(hipStream_t st, const LinearJob& job, const MtChoice& choice) {
   return choice.ring ? launch_ring_mt(st, job, choice.plan) : launch_rows_mt(st, job);
@@ -1075,7 +1073,7 @@ static int launch_mt_job(hipStream_t st, const LinearJob& job, const MtChoice& c
 
 // gemm_wr reads x once per 128 rows of weights, but starts a second kernel where it slices K: so long
 // rows of weights leave the streaming kernels (64 x 4096 x 11008 fp16: 27.6 us here, 17.4 there) and n =
-// 11008 of k = 4096 stays (16.4 us here, 19.4 there).  Below 12.5 us the second launch and the workspace
+// 11008 of k = 4096 stays.  Below 12.5 us the second launch and the workspace
 // have to be won back as well: there the host, 3 us for the two, is what bounds a call that is not replayed
 // from a graph.
 bool gemv_mt_preferred(const LinearArgs& a, bool have_workspace, MtChoice* choice) {
@@ -1088,14 +1086,13 @@ int launch_gemv_mt(hipStream_t st, const LinearArgs& a, const MtChoice& choice) 
   return launch_mt_job(st, LinearJob{&a, 1, false, nullptr, 0}, choice);
 }
 
-// Against one launch per problem (without a workspace: the entry points of several linears and gated units
-// have none), each by its own best kernel, and the gating's.
+// One launch against one per problem, each by its own best kernel (without a workspace: the entry points of
+// several linears and gated units have none), and the gating's: 0.94 of the time at most on 2429 random layers, 0.53 in
+// the mean, with gemv_ring_mt where it takes them.  gemv_rows_mt on three tiles a block and more (rows of K whose
+// scales leave gemv_ring_mt no room) by expected times.
 int launch_gemv_mt_several(hipStream_t st, const LinearArgs* pr, int count, bool glu, void* y, int act) {
   if (count < 2 || count > kGemvMaxProblems) return OFQ_ERR_UNSUPPORTED;
   const LinearArgs& a = pr[0];
-  const LinearJob job{pr, count, glu, y, act};
-  double apart = glu ? 4.0 : 0.0;
-  MtChoice choice;
   for (int i = 0; i < count; ++i) {
     const LinearArgs& b = pr[i];
     if (!gemv_mt_supported(b) || b.t_dtype != a.t_dtype || b.bits != a.bits || b.w_signed != a.w_signed
@@ -1103,12 +1100,20 @@ int launch_gemv_mt_several(hipStream_t st, const LinearArgs* pr, int count, bool
         || (glu && (b.x != a.x || b.n != a.n))) {
       return OFQ_ERR_UNSUPPORTED;
     }
-    gemv_mt_choice(LinearJob{&b, 1, false, nullptr, 0}, &choice);
-    const double wr = gemm_wr_us(b, false, 0.0);
-    apart += choice.us < wr ? choice.us : wr;
   }
+  const LinearJob job{pr, count, glu, y, act};
+  MtChoice choice;
   gemv_mt_choice(job, &choice);
-  if (choice.us > apart) return OFQ_ERR_UNSUPPORTED;
+  if (!choice.ring) {
+    double apart = glu ? 4.0 : 0.0;
+    for (int i = 0; i < count; ++i) {
+      MtChoice one;
+      gemv_mt_choice(LinearJob{&pr[i], 1, false, nullptr, 0}, &one);
+      const double wr = gemm_wr_us(pr[i], false, 0.0);
+      apart += one.us < wr ? one.us : wr;
+    }
+    if (choice.us > apart) return OFQ_ERR_UNSUPPORTED;
+  }
   return launch_mt_job(st, job, choice);
 }
 

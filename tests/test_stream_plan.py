@@ -21,6 +21,15 @@ class RingPlan(ctypes.Structure):
                                              "phases")] + [("lds", ctypes.c_size_t)])
 
 
+class RingMtPlan(ctypes.Structure):
+    _fields_ = ([(f, ctypes.c_int) for f in ("grid", "rows_per_block", "tl", "wk", "depth", "buffers", "phases")]
+                + [("lds", ctypes.c_size_t)])
+
+
+class MtChoice(ctypes.Structure):
+    _fields_ = [("ring", ctypes.c_bool), ("plan", RingMtPlan), ("us", ctypes.c_double)]
+
+
 def _job(ns, m, k, g, bits, symmetric, dtype, glu):
     pr = (LinearArgs * len(ns))(*[
         LinearArgs(t_dtype=dtype, w_signed=symmetric, bits=bits, symmetric=symmetric, group_dim=1, group_size=g,
@@ -34,6 +43,15 @@ def ring_plan(ns, m, k, g, bits, symmetric, dtype=_lib.F16, glu=False):
     f.restype, f.argtypes = ctypes.c_bool, [ctypes.POINTER(LinearJob), ctypes.POINTER(RingPlan)]
     plan = RingPlan()
     return plan if f(ctypes.byref(_job(ns, m, k, g, bits, symmetric, dtype, glu)), ctypes.byref(plan)) else None
+
+
+def ring_mt_plan(ns, m, k, g, bits, symmetric, dtype=_lib.F16, glu=False):
+    """The plan of gemv_ring_mt (17 to 64 rows of x), or None where gemv_rows_mt is the streaming kernel."""
+    f = _lib.lib()["_ZN3ofq14gemv_mt_choiceERKNS_9LinearJobEPNS_8MtChoiceE"]
+    f.restype, f.argtypes = None, [ctypes.POINTER(LinearJob), ctypes.POINTER(MtChoice)]
+    choice = MtChoice()
+    f(ctypes.byref(_job(ns, m, k, g, bits, symmetric, dtype, glu)), ctypes.byref(choice))
+    return choice.plan if choice.ring else None
 
 
 def _random_job(rng, m):
@@ -92,3 +110,38 @@ def test_every_plan_of_the_ring_is_what_the_kernel_assumes():
 def test_where_the_ring_serves(ns, m, k, g, bits, symmetric, glu, ring):
     for dtype in (_lib.F16, _lib.BF16):
         assert (ring_plan(ns, m, k, g, bits, symmetric, dtype, glu) is not None) == ring, dtype
+
+
+def test_every_plan_of_17_to_64_rows_is_what_the_kernel_assumes():
+    rng, seen = random.Random(1), 0
+    for _ in range(20000):
+        job = ns, m, k, g, bits, symmetric, _, glu = _random_job(rng, rng.randint(17, 64))
+        p = ring_mt_plan(*job)
+        if p is None:
+            continue
+        seen += 1
+        mats, lists = (2, ns[:1]) if glu else (1, ns)
+        ck = 128 if bits == 4 else 64
+        steps, tiles = -(-k // ck), mats * -(-p.rows_per_block // 16)
+        assert tiles >= 3 and p.grid == sum(-(-n // p.rows_per_block) for n in lists), job
+        assert 12 % p.wk == 0 and 12 // p.wk * p.tl >= tiles and 1 <= p.tl <= 3, job
+        assert 1 <= p.depth and p.depth * p.tl <= 4 and 2 <= p.buffers <= 4, job
+        assert p.phases == -(-steps // p.wk), job
+        x = (p.wk * m * ck * 2 + 1023) & ~1023
+        assert x <= 64 * 1024, job  # what four waves copy in 16 copies each
+        scales = mats * (1 if symmetric else 2) * _scale_bytes(p.rows_per_block, k // g)
+        used = ((scales + 1023) & ~1023) + 12 * p.depth * p.tl * 1024 + p.buffers * x
+        assert max(used, tiles * p.wk * m * 64) <= p.lds <= LDS, job
+    assert seen > 3000
+
+
+@pytest.mark.parametrize("ns,m,k,g,bits,symmetric,glu,ring", [
+    ([11008], 48, 4096, 128, 4, True, False, True), ([11008], 48, 4096, 128, 4, False, False, True),
+    ([11008], 56, 4096, 128, 4, True, False, True), ([11008], 56, 4096, 128, 4, False, False, True),
+    ([11008], 64, 4096, 128, 4, True, False, True), ([11008], 64, 4096, 128, 4, False, False, True),
+    ([11008], 64, 4096, 128, 8, True, False, True), ([8192], 64, 4096, 128, 4, True, False, False),  # two tiles a block
+    ([4096], 17, 4096, 128, 4, True, False, False), ([4096] * 3, 33, 4096, 32, 4, True, False, True),
+    ([4096] * 2, 33, 4096, 32, 4, True, True, False), ([4352] * 2, 33, 4096, 32, 4, True, True, True)])
+def test_three_tiles_of_rows_a_block_and_more_are_the_copying_waves(ns, m, k, g, bits, symmetric, glu, ring):
+    for dtype in (_lib.F16, _lib.BF16):
+        assert (ring_mt_plan(ns, m, k, g, bits, symmetric, dtype, glu) is not None) == ring, dtype
