@@ -396,14 +396,21 @@ bool ring_plan(const LinearJob& job, RingPlan* plan) {
 
 // Whether gemv_ring takes a job, and how.  (The plan comes last: its loops run for every call, and small calls are
 // bound by the host: 3 x 1560 x 1024 bf16 5.7 us with the plan, 5.3 before it.)
-// Where the ring is the faster one: 6000 random problems (m 1 .. 16, n 512 .. 32000, k 512 .. 14336, both types
-// and widths, groups of 32, 64, 128), time of the kernels that ran before over this one's:
-//   gated units                                   1.27 (5 of 100 below 1.08): two launches and the gating's
-//   several linears                               1.14 (5 of 100 below 0.97)
-//   one linear of more than 16 rows a block, or of whole turns of waves over short blocks   1.14
-// and where it is not: one row of x of up to 4096 elements (0.87: gemv_m1_any), one linear of one 16-row tile a
-// block (0.96: gemv_rows, whose requests land in registers, has nothing to balance there), and more than 8 rows
-// of x that pass LDS in four parts or more (1.0, down to 0.75).
+// Time against the kernels that would run instead, on 12 400 random jobs (m 1 .. 16, n 512 .. 32000, k 512 .. 14336,
+// both types and widths, groups of 32, 64, 128, weights from HBM):
+//   gated units                                          0.75, none of 3000 longer: two launches and the gating's
+//   several linears                                      0.91, 28 of 2500 more than 3 % longer, 1.09 at worst
+//   one linear of more than 16 rows a block, or of whole turns of waves over short blocks
+//                                                        0.86, 109 of 4700 more than 3 % longer, 1.15 at worst
+// and where it is not the faster one:
+//   one row of x of up to 4096 elements                  1.15 (gemv_m1_any)
+//   one linear of one 16-row tile a block                1.04 (gemv_rows, whose requests land in registers, has nothing
+//                                                        to balance there)
+//   up to 8 rows of x, blocks of whole 16-row tiles:     one linear of 25 to 32 rows a block and 2 to 4 turns of
+//                                                        gemv_rows' waves 1.03 (0.9 to 1.25); several of 25 to 32 rows
+//                                                        and 2 turns 1.03 (0.95 to 1.1), of 9 to 16 rows, up to 3
+//                                                        rows of x and 2 turns and more 1.01 (to 1.08)
+//   more than 8 rows of x that pass LDS in four parts or more 1.0, up to 1.33
 bool gemv_ring_choice(const LinearJob& job, RingPlan* plan) {
   const LinearArgs& a = job.pr[0];
   for (int i = 0; i < job.count; ++i) {
@@ -413,11 +420,19 @@ bool gemv_ring_choice(const LinearJob& job, RingPlan* plan) {
       return false;
     }
   }
+  int64_t rows = 0;  // of a block
+  for (int i = 0; i < (job.glu ? 1 : job.count); ++i) rows += job.pr[i].n;
+  rows = (rows + 255) / 256;
+  const int tiles8 = (int)((rows + 7) / 8);
+  const int64_t turns = (a.k - 1) / (16 * (a.bits == 4 ? 128 : 64)) + 1;  // of gemv_rows' waves
+  // (fp16 with 4-bit codes and no zero point has the shortest expansion, in gemv_ring's own order)
+  const bool whole = a.m <= 8 && !(a.t_dtype == OFQ_F16 && a.bits == 4 && a.symmetric);
   if (job.count == 1) {
-    const int64_t rows = (a.n + 255) / 256;  // of a block
     if (a.m == 1 && a.k <= 4096) return false;
-    const bool turns = a.k > kRingWaves * 2 * (a.bits == 4 ? 128 : 64);  // the waves take more than a step each
-    if (rows <= 16 && !(a.m > 1 && a.m <= 8 && rows <= 8 && turns)) return false;
+    if (rows <= 16 && !(a.m > 1 && a.m <= 8 && rows <= 8 && turns > 2)) return false;
+    if (whole && tiles8 == 4 && turns >= 2 && turns <= 4) return false;
+  } else if (!job.glu && whole && ((tiles8 == 2 && turns >= 2 && a.m <= 3) || (tiles8 == 4 && turns == 2))) {
+    return false;
   }
   return ring_plan(job, plan) && !(a.m > 8 && plan->phases >= 4);
 }

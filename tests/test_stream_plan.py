@@ -105,6 +105,13 @@ def test_every_plan_of_the_ring_is_what_the_kernel_assumes():
     ([11008], 1, 4096, 64, 4, True, False, False), ([11008], 1, 4128, 32, 4, True, False, True),
     ([8200], 16, 8192, 64, 8, True, False, False),  # more than 8 rows of x in four parts or more
     ([4672] * 2, 3, 1536, 32, 8, False, True, True), ([4096, 1024, 1024], 4, 4096, 64, 4, True, False, True),
+    # blocks of whole 16-row tiles: 25 to 32 rows of one linear, 9 to 16 and 25 to 32 of several
+    ([8097], 5, 1664, 128, 8, False, False, False), ([8097], 5, 1024, 128, 8, False, False, True),
+    ([6949], 2, 5632, 128, 8, True, False, True), ([6949], 2, 4096, 128, 8, True, False, False),
+    ([8193], 5, 1664, 128, 8, False, False, True), ([8097], 9, 1664, 128, 8, False, False, True),
+    ([2176] * 3, 7, 2176, 32, 4, False, False, False), ([2176, 272, 272], 3, 2176, 64, 4, False, False, False),
+    ([2176, 272, 272], 4, 2176, 64, 4, False, False, True), ([2048, 256, 256], 3, 2048, 64, 4, False, False, True),
+    ([2560] * 3, 3, 4608, 64, 4, False, False, True),
     ([11008], 17, 4096, 64, 4, True, False, False),  # up to 16 rows of x
     ([11008], 8, 4104, 24, 4, True, False, False)])  # groups of whole lanes
 def test_where_the_ring_serves(ns, m, k, g, bits, symmetric, glu, ring):
@@ -145,3 +152,10 @@ def test_every_plan_of_17_to_64_rows_is_what_the_kernel_assumes():
 def test_three_tiles_of_rows_a_block_and_more_are_the_copying_waves(ns, m, k, g, bits, symmetric, glu, ring):
     for dtype in (_lib.F16, _lib.BF16):
         assert (ring_mt_plan(ns, m, k, g, bits, symmetric, dtype, glu) is not None) == ring, dtype
+
+
+def test_the_shortest_expansion_stays_with_the_ring():
+    """fp16 with 4-bit codes and no zero point, on blocks of whole 16-row tiles."""
+    for ns, m, k in (([6949], 2, 5632), ([2176] * 3, 7, 2176), ([2176, 272, 272], 3, 2176)):
+        assert ring_plan(ns, m, k, 64, 4, True, _lib.F16) is not None
+        assert ring_plan(ns, m, k, 64, 4, True, _lib.BF16) is None
