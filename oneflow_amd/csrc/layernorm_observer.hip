@@ -1277,9 +1277,24 @@ ln_quant_rows(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma
     }
   }
   if constexpr (kShared) {
-    for (int p = threadIdx.x; p < npacks; p += blockDim.x) {
-      params[p] = ln_pack_or<T>(gamma, p * 8, ln_ones<T>()).q[0];
-      params[NP * kStep + p] = ln_pack_or<T>(beta, p * 8, no_beta).q[0];
+    // all requested before the first is stored: a block of one wave, which takes NP packs of each, waited for
+    // memory NP times (10 x 4096 bf16 to codes 10.2 -> 9.0 us, 15 x 3784 fp16 10.2 -> 9.0)
+    RawPack<T> g[NP], b[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int p = threadIdx.x + i * blockDim.x;
+      if (p < npacks) {
+        g[i] = ln_pack_or<T>(gamma, p * 8, ln_ones<T>());
+        b[i] = ln_pack_or<T>(beta, p * 8, no_beta);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int p = threadIdx.x + i * blockDim.x;
+      if (p < npacks) {
+        params[p] = g[i].q[0];
+        params[NP * kStep + p] = b[i].q[0];
+      }
     }
     __syncthreads();
   }
