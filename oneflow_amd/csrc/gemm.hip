@@ -38,58 +38,62 @@ inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
 // The GEMMs whose operands are both copied (int8, and 16-bit behind a converted weight): their tiles, and the
 // expected time in us of one on m x n outputs and kt k-tiles of 128 bytes,
-//   start + outputs * m n / 10^6 + kt * (alone + share * b/256 + round * ceil(b/256) + pair * ceil(b/512))
-// with b blocks: tiles from 256 rows on run one block a CU (rounds of 256), those of 128 two, those of 64 more.
-// Fitted to 250 (int8, 65 <= m <= 8192) and 384 (16 bits, 1024 <= m <= 4096) random problems with 512 to 14336 and to
-// 32000 columns, k from 512 to 8192 and to 14336, each timed on every tile: within 12 % of the measured time for 90 of
-// 100, 64 x 64 tiles within 18 %.  The tile of the least expected time took 1.5 % longer than the best one in the
-// mean; rules by ranges of m and block counts, which this replaces, 15 % (int8) and 11 % (16 bits), most of it on
-// weights with few columns, whose 256-row tiles fill a part of the chip: int8 839 x 2054 x 1664 21.1 -> 8.4 us (64 x
-// 64 tiles), 1265 x 1120 x 1280 18.1 -> 7.1.
+//   start + outputs * m n / 10^6 + kt * (alone + share * b/256 + round * ceil(b/256) + pair * ceil(b/512)
+//                                        + four * ceil(b/1024))
+// with b blocks: tiles from 256 rows on run one block a CU (rounds of 256), those of 128 two, those of 64 four.
+// int8: fitted to 15 500 random products of 65 to 8192 rows, 512 to 14336 columns and k from 512 to 8192, half of them with
+// weights from HBM, half with two that take turns in cache, each timed on every tile: within 12 % of the measured time
+// for 90 of 100, 64 x 64 tiles within 22 %.  The tile of the least expected time takes 0.8 % longer than the best one in
+// the mean, 0.74 of what rules by ranges of m and block counts chose; 106 of the 15 500 take more than 3 % longer than
+// that (1.24 at worst, 64 x 64 tiles of some 1000 blocks).  Without the rounds of four, which long rows of 64 x 64
+// tiles show (114 x 13256 x 5824 47.2 us, now 38.9; 321 x 5816 x 2560 21.4, now 18.0; 613 x 3744 x 3456 25.9, now
+// 21.3), it was 275, up to 1.49.
+// 16 bits: fitted to 384 random problems of 1024 to 4096 rows, to 32000 columns and k to 14336; on 2900 others
+// 0.74 of what the rules chose, 14 more than 3 % longer (1.14 at worst, 1609 x 12072 x 576, where 384 columns are
+// the best tile and 192 the chosen one).
 enum CopyTile { kCopy64, kCopy128, kCopy256x128, kCopy256x192, kCopy256x256, kCopy256x384, kCopyTiles };
 struct TileCost {
   int bm, bn;
-  double start, outputs, alone, share, round, pair;
+  double start, outputs, alone, share, round, pair, four;
 };
 const TileCost kCopyCost[2][2][kCopyTiles] = {  // [int8][ragged k]
-    {{{64, 64, 5.1, 0.17, 0.088, 0.194, 0.038, 0.0},
-      {128, 128, 4.3, 0.73, 0.0, 0.189, 0.013, 0.534},
-      {256, 128, 5.8, 0.71, 0.0, 0.203, 0.778, 0.0},
-      {256, 192, 8.6, 0.70, 0.0, 0.303, 0.887, 0.0},
-      {256, 256, 10.6, 0.75, 0.0, 0.469, 0.952, 0.0},
-      {256, 384, 13.9, 0.66, 0.0, 0.617, 1.324, 0.0}},
-     {{64, 64, 4.5, 0.37, 0.139, 0.151, 0.115, 0.0},
-      {128, 128, 4.4, 0.47, 0.0, 0.174, 0.204, 0.466},
-      {256, 128, 4.1, 0.84, 0.0, 0.027, 1.042, 0.0},
-      {256, 192, 8.0, 0.54, 0.0, 0.316, 1.100, 0.0},
-      {256, 256, 9.9, 0.66, 0.0, 0.382, 1.310, 0.0},
-      {256, 384, 14.6, 0.54, 0.0, 0.586, 1.697, 0.0}}},
-    {{{64, 64, 3.0, 0.54, 0.0, 0.077, 0.0, 0.271},
-      {128, 128, 3.4, 0.71, 0.0, 0.170, 0.177, 0.277},
-      {256, 128, 5.2, 0.77, 0.0, 0.256, 0.684, 0.0},
-      {256, 192, 9.2, 0.61, 0.0, 0.351, 0.816, 0.0},
-      {256, 256, 11.3, 0.59, 0.0, 0.457, 0.941, 0.0},
-      {256, 384, 13.7, 0.44, 0.0, 0.699, 1.329, 0.0}},
-     {{64, 64, 3.3, 0.41, 0.074, 0.071, 0.078, 0.219},
-      {128, 128, 4.0, 0.52, 0.0, 0.239, 0.247, 0.290},
-      {256, 128, 5.7, 0.81, 0.0, 0.221, 0.837, 0.0},
-      {256, 192, 9.4, 0.71, 0.0, 0.187, 1.044, 0.0},
-      {256, 256, 11.7, 0.55, 0.0, 0.206, 1.318, 0.0},
-      {256, 384, 14.4, 0.68, 0.0, 0.160, 1.728, 0.0}}}};
+    {{{64, 64, 5.1, 0.17, 0.088, 0.194, 0.038, 0.0, 0.0},
+      {128, 128, 4.3, 0.73, 0.0, 0.189, 0.013, 0.534, 0.0},
+      {256, 128, 5.8, 0.71, 0.0, 0.203, 0.778, 0.0, 0.0},
+      {256, 192, 8.6, 0.70, 0.0, 0.303, 0.887, 0.0, 0.0},
+      {256, 256, 10.6, 0.75, 0.0, 0.469, 0.952, 0.0, 0.0},
+      {256, 384, 13.9, 0.66, 0.0, 0.617, 1.324, 0.0, 0.0}},
+     {{64, 64, 4.5, 0.37, 0.139, 0.151, 0.115, 0.0, 0.0},
+      {128, 128, 4.4, 0.47, 0.0, 0.174, 0.204, 0.466, 0.0},
+      {256, 128, 4.1, 0.84, 0.0, 0.027, 1.042, 0.0, 0.0},
+      {256, 192, 8.0, 0.54, 0.0, 0.316, 1.100, 0.0, 0.0},
+      {256, 256, 9.9, 0.66, 0.0, 0.382, 1.310, 0.0, 0.0},
+      {256, 384, 14.6, 0.54, 0.0, 0.586, 1.697, 0.0, 0.0}}},
+    {{{64, 64, 2.3, 0.45, 0.0, 0.129, 0.0, 0.0, 0.370},
+      {128, 128, 2.9, 0.60, 0.0, 0.203, 0.078, 0.477, 0.0},
+      {256, 128, 4.8, 0.66, 0.0, 0.323, 0.745, 0.0, 0.0},
+      {256, 192, 9.1, 0.45, 0.0, 0.404, 0.853, 0.0, 0.0},
+      {256, 256, 11.2, 0.36, 0.0, 0.503, 0.976, 0.0, 0.0},
+      {256, 384, 13.5, 0.33, 0.0, 0.606, 1.388, 0.0, 0.0}},
+     {{64, 64, 2.6, 0.43, 0.0, 0.138, 0.019, 0.003, 0.428},
+      {128, 128, 3.2, 0.56, 0.0, 0.228, 0.160, 0.471, 0.0},
+      {256, 128, 5.0, 0.68, 0.0, 0.261, 0.902, 0.0, 0.0},
+      {256, 192, 9.1, 0.44, 0.0, 0.381, 1.075, 0.0, 0.0},
+      {256, 256, 11.3, 0.37, 0.0, 0.402, 1.361, 0.0, 0.0},
+      {256, 384, 14.4, 0.31, 0.0, 0.498, 1.789, 0.0, 0.0}}}};
 
 double tile_us(const TileCost& c, int64_t m, int64_t n, int64_t kt, int splits = 1) {
   const double b = (double)((m + c.bm - 1) / c.bm) * (double)((n + c.bn - 1) / c.bn) * splits;
   return c.start + c.outputs * 1e-6 * (double)m * n
-         + kt * (c.alone + c.share * b / 256 + c.round * std::ceil(b / 256) + c.pair * std::ceil(b / 512));
+         + kt * (c.alone + c.share * b / 256 + c.round * std::ceil(b / 256) + c.pair * std::ceil(b / 512)
+                 + c.four * std::ceil(b / 1024));
 }
 CopyTile pick_copy_tile(bool int8, int64_t m, int64_t n, int64_t row_bytes, double* us) {
   const TileCost* cost = kCopyCost[int8][row_bytes % 128 != 0];
   int best = 0;
   double best_us = 1e300;
   for (int i = 0; i < kCopyTiles; ++i) {
-    double t = tile_us(cost[i], m, n, (row_bytes + 127) / 128);
-    // (int8 on long rows: up to 1.4 of what is expected, 434 x 2263 x 7168 31 us for 23, where slices take 26)
-    if (int8 && i == kCopy64 && row_bytes > 32 * 128) t *= 1.15;
+    const double t = tile_us(cost[i], m, n, (row_bytes + 127) / 128);
     if (t < best_us) {
       best = i;
       best_us = t;
@@ -621,9 +625,9 @@ int mq_room(int64_t m, int64_t n, int64_t k) {
   return (int)s;
 }
 
-// Tile and slices by the least expected time (kCopyCost), with at most `most` slices: one slice on any tile, or
-// several of 128 x 128 or 256 x 128 tiles in one resident round, whose int32 sums and second launch cost 2 to 4 us and
-// 1.6 to 2 us per 10^6 sums.
+// Tile and slices by the least expected time (kCopyCost), with at most `most` slices (what the workspace that callers
+// know has room for): one slice on any tile, or several of 128 x 128 or 256 x 128 tiles in one resident round,
+// whose int32 sums and second launch cost 2 us and 1.7 to 1.8 us per 10^6 sums.
 struct MqPlan {
   CopyTile tile;
   int splits;
@@ -631,11 +635,11 @@ struct MqPlan {
 MqPlan mq_plan(int64_t m, int64_t n, int64_t k, int most) {
   // up to 64 rows (k >= 8192) the rival streams; the slices of the query are the ones that were measured against it
   if (m <= kMatmulQuantRowsMaxM && most > 1) return MqPlan{kCopy128, most};
-  static const TileCost kSliced[2][2] = {{{128, 128, 5.5, 1.13, 0.0, 0.147, 0.0, 0.445},
-                                          {256, 128, 7.2, 1.33, 0.0, 0.178, 0.646, 0.0}},
-                                         {{128, 128, 5.9, 1.31, 0.0, 0.178, 0.033, 0.494},
-                                          {256, 128, 7.4, 1.52, 0.0, 0.084, 0.826, 0.0}}};
-  static const double kSums[2][2] = {{1.98, 1.57}, {1.72, 1.59}};  // us per 10^6 of a slice
+  static const TileCost kSliced[2][2] = {{{128, 128, 5.3, 0.0, 0.536, 0.215, 0.0, 0.0, 0.0},
+                                          {256, 128, 6.6, 0.0, 0.724, 0.288, 0.0, 0.0, 0.0}},
+                                         {{128, 128, 5.6, 0.0, 0.584, 0.327, 0.0, 0.0, 0.0},
+                                          {256, 128, 6.9, 0.0, 0.860, 0.286, 0.0, 0.0, 0.0}}};
+  static const double kSums[2][2] = {{1.80, 1.79}, {1.69, 1.79}};  // us per 10^6 of a slice
   MqPlan plan{kCopy64, 1};
   double best;
   plan.tile = pick_copy_tile(true, m, n, k, &best);
