@@ -147,6 +147,8 @@ def test_every_plan_of_17_to_64_rows_is_what_the_kernel_assumes():
     ([11008], 56, 4096, 128, 4, True, False, True), ([11008], 56, 4096, 128, 4, False, False, True),
     ([11008], 64, 4096, 128, 4, True, False, True), ([11008], 64, 4096, 128, 4, False, False, True),
     ([11008], 64, 4096, 128, 8, True, False, True), ([8192], 64, 4096, 128, 4, True, False, False),  # two tiles a block
+    ([9536], 44, 640, 64, 8, False, False, False), ([9536], 44, 1088, 64, 8, False, False, True),
+    ([9536], 44, 640, 64, 4, False, False, True), ([12300], 44, 640, 64, 8, False, False, True),
     ([4096], 17, 4096, 128, 4, True, False, False), ([4096] * 3, 33, 4096, 32, 4, True, False, True),
     ([4096] * 2, 33, 4096, 32, 4, True, True, False), ([4352] * 2, 33, 4096, 32, 4, True, True, True)])
 def test_three_tiles_of_rows_a_block_and_more_are_the_copying_waves(ns, m, k, g, bits, symmetric, glu, ring):
