@@ -5,6 +5,7 @@ import random
 
 import pytest
 
+import test_gpu_gemv_ring as ring_tests
 from oneflow_amd import _lib
 from test_gemm_plan import LinearArgs
 
@@ -161,3 +162,46 @@ def test_the_shortest_expansion_stays_with_the_ring():
     for ns, m, k in (([6949], 2, 5632), ([2176] * 3, 7, 2176), ([2176, 272, 272], 3, 2176)):
         assert ring_plan(ns, m, k, 64, 4, True, _lib.F16) is not None
         assert ring_plan(ns, m, k, 64, 4, True, _lib.BF16) is None
+
+
+def _kernels(ns, m, k, g, glu=False):
+    """What the variants of ring_tests run for one of its shapes; None stands for a kernel that is not a ring."""
+    mode = "gated" if glu else "one" if len(ns) == 1 else "several"
+    for bits, symmetric, _ in ring_tests.VARIANTS:
+        for dtype in (_lib.F16, _lib.BF16):
+            p = (ring_plan if m <= 16 else ring_mt_plan)(ns, m, k, g, bits, symmetric, dtype, glu)
+            if p is None:
+                yield None
+            elif m <= 16:
+                yield from ((p.tr, mode, p.tl), ("waves over K", 1 << p.wk_shift),
+                            ("x in parts", p.tr, mode, p.phases > 1))
+            else:
+                yield from ((-(-m // 16), "tiles of x", mode, p.tl), ("workers over K", p.wk),
+                            ("buffers", p.buffers), ("phases", min(p.phases, 3)))
+
+
+def test_the_gpu_tests_run_every_ring_kernel():
+    t, seen = ring_tests, set()
+    for m, n, k, g in t.ONE + t.MANY_TILES:
+        seen |= set(_kernels([n], m, k, g))
+    for m, k, g, ns in t.SEVERAL + t.MANY_TILES_SEVERAL:
+        seen |= set(_kernels(list(ns), m, k, g))
+    for m, n, k, g in t.GATED + t.MANY_TILES_GATED:
+        seen |= set(_kernels([n, n], m, k, g, True))
+    modes = ("one", "several", "gated")
+    want = {(tr, mode, tl) for tr in (8, 16) for mode in modes for tl in (1, 2, 3, 4)}
+    want |= {("waves over K", 1 << s) for s in range(5)}
+    want |= {("x in parts", tr, mode, parts) for tr in (8, 16) for mode in modes for parts in (False, True)}
+    want |= {(mt, "tiles of x", mode, tl) for mt in (2, 3, 4) for mode in modes for tl in (1, 2, 3)}
+    want |= {("workers over K", w) for w in (1, 2, 3, 4, 6, 12)}
+    want |= {("buffers", b) for b in (2, 3, 4)} | {("phases", p) for p in (1, 2, 3)}
+    assert want <= seen, sorted(want - seen, key=str)
+
+
+def test_the_gpu_tests_of_many_tiles_run_the_copying_waves():
+    t = ring_tests
+    jobs = [([n], m, k, g, False) for m, n, k, g in t.MANY_TILES]
+    jobs += [(list(ns), m, k, g, False) for m, k, g, ns in t.MANY_TILES_SEVERAL]
+    jobs += [([n, n], m, k, g, True) for m, n, k, g in t.MANY_TILES_GATED]
+    for job in jobs:
+        assert None not in set(_kernels(*job)), job
