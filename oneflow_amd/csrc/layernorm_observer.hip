@@ -1279,9 +1279,10 @@ ln_quant_rows(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma
   if constexpr (kShared) {
     // all requested before the first is stored: a block of one wave, which takes NP packs of each, waited for
     // memory NP times (10 x 4096 bf16 to codes 10.2 -> 9.0 us, 15 x 3784 fp16 10.2 -> 9.0)
-    RawPack<T> g[NP], b[NP];
+    constexpr int kTurns = ONE ? (NP + kRows - 1) / kRows : NP;
+    RawPack<T> g[kTurns], b[kTurns];
 #pragma unroll
-    for (int i = 0; i < NP; ++i) {
+    for (int i = 0; i < kTurns; ++i) {
       const int p = threadIdx.x + i * blockDim.x;
       if (p < npacks) {
         g[i] = ln_pack_or<T>(gamma, p * 8, ln_ones<T>());
@@ -1289,7 +1290,7 @@ ln_quant_rows(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma
       }
     }
 #pragma unroll
-    for (int i = 0; i < NP; ++i) {
+    for (int i = 0; i < kTurns; ++i) {
       const int p = threadIdx.x + i * blockDim.x;
       if (p < npacks) {
         params[p] = g[i].q[0];
