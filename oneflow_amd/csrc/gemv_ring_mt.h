@@ -9,10 +9,13 @@
 // counted asynchronous copies, up to three steps ahead: a wave's copies complete in order, so that codes from
 // HBM behind copies of x, or in front of them, would be waited for at every barrier -- hence the split.
 //
-// What bounds it: a phase (one step of every wave between two barriers) of 0.8 us where a wave has one tile, the
-// way from the barrier over x from LDS, the expansion and the products to the next one, and 5.7 us to start, load
-// the first x, fold and store.  A phase's x is read from LDS by every wave for its own tiles (0.09 us per 100 rows
-// of a 4-bit chunk), so more tiles of a wave cost less each.  Against gemv_rows_mt (us):
+// What bounds it: a phase (one step of every wave between two barriers), the way from the barrier over x from LDS,
+// the expansion and the products to the next one, and 5.5 us to start, load the first x, fold and store.  A phase takes
+// 1.3 to 1.5 us where a wave has one tile of 4-bit codes (n = 11008, weights from HBM: 8.2, 11.0 and 16.8 us for 2, 4
+// and 8 phases at 48 rows, 8.6, 11.5 and 18.4 at 64).  Its x is read from LDS by every wave for its own tiles, so more
+// tiles of a wave cost less each.  Waves wait for 60 % of their lives at 48 x 11008 x 4096, LDS is busy 38 % of the
+// time, more than half of that with conflicts of banks, vector units 47 %, matrix units 13 %, L2 serves 7 TB/s.
+// Against gemv_rows_mt (us):
 //   fp16 4-bit  48 x 11008 x 4096 with a zero point  17.8 -> 16.0   64 x 11008 x 4096        20.6 -> 18.6
 //   fp16 4-bit  40 x 22000 x 2944   29.3 -> 18.2 (gemm_wr 19.9)     20 x 2 x 9216 x 3584     27.3 -> 18.7
 //   8 bits      56 x 2 x 12032 x 3968 bf16  51.4 -> 33.2            45 x 2 x 10880 x 4096 fp16  43.2 -> 26
@@ -98,7 +101,7 @@ gemv_ring_mt_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mat
   const int ntiles = (rows_blk + 15) >> 4;  // per matrix
   const int nvt = NMAT * ntiles;
 
-  // LDS: [scales, zeros of every matrix][rings of the workers][two buffers of x]; the sums take the
+  // LDS: [scales, zeros of every matrix][rings of the workers][two to four buffers of x]; the sums take the
   //      place of all of it
   const int sreg = ring_scale_bytes(p.rows_per_block, G);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;

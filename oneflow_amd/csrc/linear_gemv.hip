@@ -1072,9 +1072,10 @@ static double ring_mt_us(const LinearJob& job, const RingMtPlan& plan) {
 // which starts 1.5 us later and takes less per byte.  Both timed on 6065 random jobs of 17 to 64 rows (linears of 512
 // to 32000 x 512 to 14336, several of a layer, gated units; weights from HBM): with three tiles of rows a block and
 // more gemv_ring_mt takes 0.78 of the time in the mean, 32 of 2290 more than 3 % longer (1.12 at worst, 21 x
-// 8380 x 10176 bf16 with a zero point); with one and two tiles 1.21 and 1.02 times, three tiles of 8-bit codes with K
-// up to 1024, a phase or two, 1.0 (to 1.16: 44 x 9536 x 640 7.8 us, 9.1 with gemv_ring_mt).  (A comparison of expected times, with a tenth
-// to spare, turned 824 of the 2310 away: 64 x 11008 x 4096 fp16 4-bit 20.6 us, now 18.6, 56 rows 18.7 -> 16.6.)
+// 8380 x 10176 bf16 with a zero point); with one and two tiles 1.21 and 1.02 times, three tiles of 8-bit codes
+// with K up to 1024, a phase or two, 1.01 (1037 jobs, 1.19 at worst; from there to 3072 0.95).  (A comparison of
+// expected times, with a tenth to spare, turned 824 of the 2310 away: 64 x 11008 x 4096 fp16 4-bit 20.6 us, now 18.6,
+// 56 rows 18.7 -> 16.6.)
 void gemv_mt_choice(const LinearJob& job, MtChoice* choice) {
   const LinearArgs& a = job.pr[0];
   int64_t total = 0;
