@@ -46,8 +46,8 @@ inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 // for 90 of 100, 64 x 64 tiles within 22 %.  The tile of the least expected time takes 0.8 % longer than the best one in
 // the mean, 0.74 of what rules by ranges of m and block counts chose; 106 of the 15 500 take more than 3 % longer than
 // that (64 x 64 tiles: of some 1000 blocks to 1.24, of some 100 whose weights come from HBM to 1.31, 97 x 3680 x 2688
-// 14.2 us with the slices it had, 18.6 now; a table from weights in HBM alone mends those and makes weights in cache up to
-// 1.5 times slower than this one does).  Without the rounds of four, which long rows of 64 x 64
+// 14.2 us with the slices it had, 18.6 now; a table from weights in HBM alone mends those and makes products on weights in
+// cache up to 1.5 times slower).  Fitted to weights in cache and without the rounds of four, which long rows of 64 x 64
 // tiles show (114 x 13256 x 5824 46.5 us, now 41.2; 321 x 5816 x 2560 21.5, now 17.6; 613 x 3744 x 3456 25.8, now
 // 22.2), it was 275, up to 1.49.
 // 16 bits: fitted to 384 random problems of 1024 to 4096 rows, to 32000 columns and k to 14336; on 2900 others
