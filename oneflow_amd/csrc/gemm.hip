@@ -591,7 +591,7 @@ int launch_gemm_gn(hipStream_t st, const LinearArgs& a, void* workspace) {
 
 using namespace ofq;
 
-// rows of a up to which matmul_quant streams the weights instead of tiling them
+// rows of a up to which the workspace query has no slices for rows of b of less than 8192 elements
 static constexpr int64_t kMatmulQuantRowsMaxM = 64;
 
 namespace ofq {
@@ -608,8 +608,8 @@ int mq_room(int64_t m, int64_t n, int64_t k) {
     if (m <= 768 && t64 >= 128 && t64 <= 768) return 1;
     if (b256 < 192 && b128 >= 192 && b128 <= 512) return 1;
   }
-  // long rows (k >= 8192) already pay for slices from 33 rows of a on: 4096 x 11008 at m = 64
-  // streams in 33 us and runs in 22 us as slices
+  // (33 to 64 rows of k >= 8192 ran as slices once: the query still makes room, the streaming kernel takes them in
+  // 0.55 to 1.0 of the time, 4096 x 11008 at m = 64 26.5 -> 18.6 us)
   if (m <= (k >= 8192 ? kMatmulQuantRowsMaxM / 2 : kMatmulQuantRowsMaxM)) return 1;
   int64_t blocks = m > 128 ? b256 : b128;
   int64_t slots = m > 128 ? 256 : 512;
@@ -635,8 +635,6 @@ struct MqPlan {
   int splits;
 };
 MqPlan mq_plan(int64_t m, int64_t n, int64_t k, int most) {
-  // up to 64 rows (k >= 8192) the rival streams; the slices of the query are the ones that were measured against it
-  if (m <= kMatmulQuantRowsMaxM && most > 1) return MqPlan{kCopy128, most};
   static const TileCost kSliced[2][2] = {{{128, 128, 5.3, 0.0, 0.536, 0.215, 0.0, 0.0, 0.0},
                                           {256, 128, 6.6, 0.0, 0.724, 0.288, 0.0, 0.0, 0.0}},
                                          {{128, 128, 5.6, 0.0, 0.584, 0.327, 0.0, 0.0, 0.0},
@@ -774,6 +772,10 @@ extern "C" int ofq_matmul_quant_ws(void* stream, const void* a, const void* b, c
                 OFQ_ERR_NULL_POINTER);
   OFQ_RETURN_IF(!ofq_aligned16(a) || !ofq_aligned16(b) || !ofq_aligned16(out), OFQ_ERR_MISALIGNED);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  // few rows of a: the weights stream once
+  if (matmul_quant_rows_supported(m, n, k)) {
+    return launch_matmul_quant_rows(st, a, b, a_scale, b_scale, bias, out, out_dtype, m, n, k);
+  }
   BCopyParams bp;
   bp.b = static_cast<const uint8_t*>(b);
   bp.ldb = k;
@@ -803,10 +805,6 @@ extern "C" int ofq_matmul_quant_ws(void* stream, const void* a, const void* b, c
       }
 #undef OFQ_MQS
     }
-  }
-  // few rows of a: the weights stream once
-  if (m <= kMatmulQuantRowsMaxM && matmul_quant_rows_supported(m, n, k)) {
-    return launch_matmul_quant_rows(st, a, b, a_scale, b_scale, bias, out, out_dtype, m, n, k);
   }
   if (k % 128 != 0) {
     switch (out_dtype) {

@@ -1,129 +1,268 @@
-// matmul_quant with few rows of a (m <= 64 per pass): int8 x int8 on v_mfma_i32_16x16x64_i8 with
-// the weights streamed from HBM once.
+// matmul_quant with few rows of a (m <= 64): int8 x int8 on v_mfma_i32_16x16x64_i8 with the weights
+// streamed from HBM once.
 //
-// The tiled GEMM needs 128-row tiles to earn its LDS traffic and leaves most CUs without a block
-// when a has a handful of rows; here a block owns consecutive rows of b (about n / 256, at most
-// 64, walked as 16-row tiles), a wave takes the 64-byte chunks c = wave, wave + NWAVES, ... of K,
-// loads its 16 bytes of every 16-row tile of a straight from L2 and meets each weight tile with
-// one MFMA per tile of a; the codes of the next (tile, chunk) are requested before the current
-// ones are used.  int32 sums stay in registers, are added across the waves through LDS (integer
-// addition: the order cannot matter) and leave through the epilogue of the GEMM path,
+// The tiled GEMM needs 128-row tiles to earn its LDS traffic and leaves most CUs without a block when a has a
+// handful of rows; here a block owns consecutive rows of b (about n / 256, at most 64) and all of K.
+//
+// matmul_quant_stream.  The waves of a block share nothing until the end: a wave takes every eighth 128-byte step
+// of K, and both its columns of a and its columns of the block's rows of b come by asynchronous global -> LDS
+// copies into a ring of its own, D steps ahead, so there is no barrier in the loop and no request waits in a
+// register.  A copy is 8 rows x 128 bytes: whole lines, where an operand request of the matrix instruction
+// (16 rows x 64 bytes) takes half of each; the pieces of a row are XOR-swizzled on the way, so that the operand
+// reads have no conflicts of banks.  Rows come in eights (a: MX, b: WX of them), rows past the end re-read the last
+// one and feed results that are never stored.  int32 sums are added across the waves through LDS (integer addition: the
+// order cannot matter) and leave through the epilogue of the GEMM path,
 //   out = T(float(acc) * (a_scale * b_scale[n]) + bias[n]),
-// so both paths give the same bits.
+// so all paths give the same bits.
+//
+// What bounds it: up to 16 rows of a the stream of b (8 x 11008 x 4096: 9.7 us with weights from HBM, 45 MB at 6.2 TB/s
+// behind 2.4 us of launch, first bytes and fold), beyond that b and the rows of a that every block reads from L2 together
+// (64 x 11008 x 4096: 14.4 us; a CU takes in 50 to 60 bytes per ns).  Two, three or six steps ahead are the same
+// within 3 %.  Codes waiting in registers, one request ahead and a from L2 in 64-byte runs, the kernel that this one
+// took the place of: 12.8 and 21.9 us; 48 x 1024 x 2048 6.6 -> 4.5, 20 x 600 x 8192 11.5 -> 6.4, 24 x 4096 x 11008
+// 18.9 -> 12.8.
 #include <atomic>
+#include "gemm_kernels.h"
 #include "ofq_device.h"
 #include "ofq_internal.h"
 
 namespace ofq {
 namespace {
 
-constexpr int kI8MaxTiles = 4;  // 16-row tiles of b per block
+constexpr int kMqWaves = 8;      // 20 KB of LDS each
+constexpr int kMqMaxRows = 64;   // of b in a block
 
-template<typename T, int NWAVES, int MT>
-__global__ void __launch_bounds__(NWAVES * 64)
-matmul_quant_rows(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
-                  const float* __restrict__ a_scale, const float* __restrict__ b_scale,
-                  const typename TT<T>::storage* __restrict__ bias,
-                  typename TT<T>::storage* __restrict__ out, int M, int N, int K,
-                  int rows_per_block) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  constexpr int NT = NWAVES * 64;
-  const int nchunks = K >> 6;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 15;
-  const int kb = lane >> 4;
-  const int row0 = blockIdx.x * rows_per_block;
-  int rows_blk = N - row0;
-  if (rows_blk > rows_per_block) rows_blk = rows_per_block;
-  if (rows_blk <= 0) return;
-  const int ntiles = (rows_blk + 15) >> 4;
-  int* red = reinterpret_cast<int*>(smem);  // [NWAVES][MT*16 (m)][16 (n)]
+// steps of STEP KB that a wave holds or has requested
+constexpr int mq_depth(int step_kb) { return 20 / step_kb > 3 ? 3 : 20 / step_kb; }
 
-  const uint8_t* bbase = b + (int64_t)row0 * K + kb * 16;
-  auto issue = [&](int tile, int c, bool live) {
-    const int row_l = tile * 16 + r;
-    const bool ok = row_l < rows_blk;
-    const uint8_t* q = bbase + (int64_t)(ok ? row_l : 0) * K + (int64_t)c * 64;
-    return __builtin_nontemporal_load(
-        reinterpret_cast<const i32x4*>(live ? q : b + (int64_t)row0 * K));
-  };
-  int c = wave;
-  i32x4 cur = issue(0, c < nchunks ? c : 0, c < nchunks);
-
-  // this lane's rows of a: row mt*16 + r of every tile (rows >= M feed outputs never stored and
-  // re-read row 0), bytes [16 kb, 16 kb + 16) of each chunk
-  const uint8_t* arow[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int row = mt * 16 + r;
-    arow[mt] = a + (size_t)(row < M ? row : 0) * K + kb * 16;
-  }
-  i32x4 acc[kI8MaxTiles][MT];
-#pragma unroll
-  for (int t = 0; t < kI8MaxTiles; ++t)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[t][mt] = i32x4{0, 0, 0, 0};
-
-  while (c < nchunks) {
-    i32x4 av[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-      av[mt] = *reinterpret_cast<const i32x4*>(arow[mt] + (size_t)c * 64);
-#pragma unroll
-    for (int t = 0; t < kI8MaxTiles; ++t) {
-      if (t < ntiles) {
-        const bool last_t = t + 1 >= ntiles;
-        const int nc = last_t ? c + NWAVES : c;
-        const bool live = nc < nchunks;
-        const i32x4 nxt = issue(last_t ? 0 : t + 1, live ? nc : 0, live);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-          acc[t][mt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[mt], cur, acc[t][mt], 0, 0, 0);
-        cur = nxt;
-      }
-    }
-    c += NWAVES;
-  }
-
-  const float sa = a_scale[0];
-#pragma unroll
-  for (int t = 0; t < kI8MaxTiles; ++t) {
-    if (t < ntiles) {
-      if (t > 0) __syncthreads();  // the previous tile's sums have been read
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int m = mt * 16 + 4 * kb + v;
-          red[(wave * (MT * 16) + m) * 16 + r] = acc[t][mt][v];
-        }
-      __syncthreads();
-      for (int o = tid; o < M * 16; o += NT) {
-        int sum = 0;
-#pragma unroll
-        for (int wv = 0; wv < NWAVES; ++wv) sum += red[wv * (MT * 256) + o];
-        const int m = o >> 4;
-        const int row_l = t * 16 + (o & 15);
-        if (row_l < rows_blk) {
-          const int n = row0 + row_l;
-          float v = (float)sum * (sa * b_scale[n]);
-          if (bias != nullptr) v = v + TT<T>::load(bias + n);
-          TT<T>::store(out + (int64_t)m * N + n, v);
-        }
-      }
-    }
+// all but the youngest n steps of STEP copies have landed
+template<int STEP>
+__device__ __forceinline__ void wait_steps(int n) {
+  switch (n) {
+    case 0: wait_vmem_all(); break;
+    case 1: wait_vmem_le<STEP>(); break;
+    default: wait_vmem_le<2 * STEP>(); break;
   }
 }
 
-// ---- 1 to 4 rows of a: a wave owns whole rows of b -------------------------------------------
-// With so few rows the matrix core adds nothing and its operand layout costs (a request of 16
-// rows x 64 bytes instead of whole rows, a fold across the waves that split K).  Here lane l
-// holds bytes [h * 1024 + 16 l, +16) of every row of a in registers (h < H = ceil(k / 1024)),
-// a wave walks the rows w, w + NW, .. of the block's share of b with the requests of two rows in
-// flight, meets each row with v_dot4_i32_i8 (exact int32) and sums across the lanes; no LDS, no
-// barrier.  Same int32 sums and the same epilogue as the other paths, hence the same bits.
+struct MqStreamArgs {
+  const float* a_scale;
+  const float* b_scale;
+  const void* bias;
+  void* out;
+  int out_dtype;
+  int M, N, K;
+  int rows_per_block;
+};
+
+template<typename T>
+__device__ __forceinline__ void mq_store(const MqStreamArgs& p, int64_t at, float v, bool has_bias, float bias) {
+  if (has_bias) v = v + bias;
+  TT<T>::store(static_cast<typename TT<T>::storage*>(p.out) + at, v);
+}
+
+template<int MX, int WX>
+__global__ void __launch_bounds__(kMqWaves * 64)
+matmul_quant_stream(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, MqStreamArgs p) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  constexpr int STEP = MX + WX, D = mq_depth(STEP);
+  constexpr int MT = (MX + 1) / 2, WT = (WX + 1) / 2;  // 16-row tiles
+  constexpr int R = WT * 16;
+  static_assert(D >= 1 && D * STEP <= 20 && STEP * (D - 1) < 63, "LDS of a wave, vmcnt");
+  const int M = p.M, N = p.N, K = p.K;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row0 = blockIdx.x * p.rows_per_block;
+  int rows_blk = N - row0;
+  if (rows_blk > p.rows_per_block) rows_blk = p.rows_per_block;
+  if (rows_blk <= 0) return;
+  const int steps = (K + 127) >> 7;
+
+  // a thread's outputs are those of one row of b: its scale and the bits of its bias are requested before the
+  // copies, without a branch (the compiler waits at the end of one), and first looked at when the sums are there
+  const int orow = tid % R;
+  const int brow = row0 + (orow < rows_blk ? orow : 0);
+  const float sa = p.a_scale[0];
+  float sb = p.b_scale[brow];
+  const bool has_bias = p.bias != nullptr, wide = p.out_dtype == OFQ_F32;
+  const uint16_t* bias_at = static_cast<const uint16_t*>(has_bias ? p.bias : static_cast<const void*>(p.b_scale))
+                            + (wide ? 2 * (int64_t)brow : brow);
+  uint32_t bias_lo = bias_at[0], bias_hi = bias_at[wide ? 1 : 0];
+
+  // ---- copies -----------------------------------------------------------------------------------
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem
+                        + (uint32_t)wave * (D * STEP * 1024);
+  const int sub = lane >> 3;                    // row of the eight
+  const uint32_t piece = (uint32_t)(((lane & 7) ^ sub) << 4);
+  uint32_t aoff[MX], boff[WX];                  // of this lane's row in every eight; rows past the end: the last one
+#pragma unroll
+  for (int i = 0; i < MX; ++i) aoff[i] = (uint32_t)(i * 8 + sub < M ? i * 8 + sub : M - 1) * (uint32_t)K + piece;
+#pragma unroll
+  for (int i = 0; i < WX; ++i) {
+    boff[i] = (uint32_t)(i * 8 + sub < rows_blk ? i * 8 + sub : rows_blk - 1) * (uint32_t)K + piece;
+  }
+  const uint8_t* const bblk = b + (int64_t)row0 * K;
+  auto copy_step = [&](int s, int slot) {
+    const uint32_t lds = lds0 + (uint32_t)slot * (STEP * 1024);
+    // the second half of the last step of a row of 64 (2 i + 1) bytes re-reads the first
+    const uint32_t back = s * 128 + 64 >= K && piece >= 64 ? 64u : 0u;
+    const uint8_t* as = a + s * 128;
+    const uint8_t* bs = bblk + s * 128;
+#pragma unroll
+    for (int i = 0; i < MX; ++i) {
+      async_copy16_at(as, aoff[i] - back, lds + i * 1024);
+    }
+#pragma unroll
+    for (int i = 0; i < WX; ++i) {
+      async_copy16_once(bs, boff[i] - back, lds + (MX + i) * 1024);
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (wave + d * kMqWaves < steps) copy_step(wave + d * kMqWaves, d);
+
+  // ---- products ---------------------------------------------------------------------------------
+  const int r = lane & 15, kb = lane >> 4;
+  // this lane's piece of row r of a tile, in the two halves of a step; a tile of one eight has its rows twice
+  const int at0 = (r & 7) * 128 + ((kb ^ (r & 7)) << 4), at1 = (r & 7) * 128 + (((4 + kb) ^ (r & 7)) << 4);
+  const int upper = (r >> 3) * 1024;
+  i32x4 acc[WT][MT];
+#pragma unroll
+  for (int t = 0; t < WT; ++t)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[t][mt] = i32x4{0, 0, 0, 0};
+
+  int slot = 0;
+  for (int s = wave; s < steps; s += kMqWaves) {
+    int live = 0;  // later steps under way
+#pragma unroll
+    for (int d = 1; d < D; ++d) live += s + d * kMqWaves < steps ? 1 : 0;
+    wait_steps<STEP>(live);
+    asm volatile("" ::: "memory");
+    const uint8_t* base = smem + wave * (D * STEP * 1024) + slot * (STEP * 1024);
+    i32x4 av[2][MT], bv[2][WT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const uint8_t* q = base + mt * 2048 + (2 * mt + 1 < MX ? upper : 0);
+      av[0][mt] = *reinterpret_cast<const i32x4*>(q + at0);
+      av[1][mt] = *reinterpret_cast<const i32x4*>(q + at1);
+    }
+#pragma unroll
+    for (int t = 0; t < WT; ++t) {
+      const uint8_t* q = base + MX * 1024 + t * 2048 + (2 * t + 1 < WX ? upper : 0);
+      bv[0][t] = *reinterpret_cast<const i32x4*>(q + at0);
+      bv[1][t] = *reinterpret_cast<const i32x4*>(q + at1);
+    }
+    // everything is in registers: the slot is free
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (s + D * kMqWaves < steps) copy_step(s + D * kMqWaves, slot);
+#pragma unroll
+    for (int t = 0; t < WT; ++t)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        acc[t][mt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[0][mt], bv[0][t], acc[t][mt], 0, 0, 0);
+    if (s * 128 + 64 < K) {
+#pragma unroll
+      for (int t = 0; t < WT; ++t)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          acc[t][mt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[1][mt], bv[1][t], acc[t][mt], 0, 0, 0);
+    }
+    slot = slot + 1 == D ? 0 : slot + 1;
+  }
+
+  // ---- sums of the waves, [wave][row of a][row of b + 4] (rings and sums share the memory) -------------
+  __syncthreads();
+  int* red = reinterpret_cast<int*>(smem);
+  constexpr int RP = R + 4;
+  const int waves = steps < kMqWaves ? steps : kMqWaves;  // that have a sum
+  if (wave < waves) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int m = mt * 16 + 4 * kb + v;
+        if (m < M) {
+#pragma unroll
+          for (int t = 0; t < WT; ++t) red[(wave * M + m) * RP + t * 16 + r] = acc[t][mt][v];
+        }
+      }
+  }
+  __syncthreads();
+  asm volatile("" : "+v"(sb), "+v"(bias_lo), "+v"(bias_hi));
+  const float bias = wide ? __builtin_bit_cast(float, bias_lo | bias_hi << 16)
+                     : p.out_dtype == OFQ_F16 ? (float)__builtin_bit_cast(f16, (uint16_t)bias_lo)
+                                              : __builtin_bit_cast(float, bias_lo << 16);
+  constexpr int kRowsAtOnce = kMqWaves * 64 / R;
+  if (tid >= kRowsAtOnce * R || orow >= rows_blk) return;
+  for (int m = tid / R; m < M; m += kRowsAtOnce) {
+    const int* src = red + m * RP + orow;
+    int sum = 0;
+    if (waves == kMqWaves) {
+#pragma unroll
+      for (int w = 0; w < kMqWaves; ++w) sum += src[w * M * RP];
+    } else {
+      for (int w = 0; w < waves; ++w) sum += src[w * M * RP];
+    }
+    const float v = (float)sum * (sa * sb);
+    const int64_t at = (int64_t)m * N + row0 + orow;
+    if (p.out_dtype == OFQ_F16) mq_store<f16>(p, at, v, has_bias, bias);
+    else if (p.out_dtype == OFQ_BF16) mq_store<bf16>(p, at, v, has_bias, bias);
+    else mq_store<float>(p, at, v, has_bias, bias);
+  }
+}
+
+template<int MX, int WX>
+int launch_stream_inst(hipStream_t st, const uint8_t* a, const uint8_t* b, const MqStreamArgs& p) {
+  constexpr int STEP = MX + WX, R = (WX + 1) / 2 * 16;
+  size_t lds = (size_t)kMqWaves * mq_depth(STEP) * STEP * 1024;
+  const size_t red = (size_t)kMqWaves * p.M * (R + 4) * 4;
+  if (red > lds) lds = red;
+  auto kern = matmul_quant_stream<MX, WX>;
+  static std::atomic<uint64_t> lds_allowed{0};  // devices on which the kernel's LDS limit is raised
+  if (!ofq_allow_dynamic_lds(reinterpret_cast<const void*>(kern), 160 * 1024, lds_allowed)) return OFQ_ERR_LAUNCH;
+  kern<<<(unsigned)((p.N + p.rows_per_block - 1) / p.rows_per_block), kMqWaves * 64, lds, st>>>(a, b, p);
+  return ofq_check_launch();
+}
+
+template<int MX>
+int launch_stream_mx(hipStream_t st, const uint8_t* a, const uint8_t* b, const MqStreamArgs& p) {
+  switch ((p.rows_per_block + 7) / 8) {
+    case 1: return launch_stream_inst<MX, 1>(st, a, b, p);
+    case 2: return launch_stream_inst<MX, 2>(st, a, b, p);
+    case 3: return launch_stream_inst<MX, 3>(st, a, b, p);
+    case 4: return launch_stream_inst<MX, 4>(st, a, b, p);
+    case 5: return launch_stream_inst<MX, 5>(st, a, b, p);
+    case 6: return launch_stream_inst<MX, 6>(st, a, b, p);
+    case 7: return launch_stream_inst<MX, 7>(st, a, b, p);
+    case 8: return launch_stream_inst<MX, 8>(st, a, b, p);
+    default: return OFQ_ERR_UNSUPPORTED;
+  }
+}
+
+int launch_stream(hipStream_t st, const uint8_t* a, const uint8_t* b, const MqStreamArgs& args) {
+  MqStreamArgs p = args;
+  constexpr int64_t kCUs = 256;
+  // one block a CU and round, its rows whole: a block of eight rows at least
+  const int64_t rounds = (p.N + kCUs * kMqMaxRows - 1) / (kCUs * kMqMaxRows);
+  p.rows_per_block = (int)((p.N + kCUs * rounds - 1) / (kCUs * rounds));
+  if (p.rows_per_block < 8) p.rows_per_block = 8;
+  if (p.M <= 8) return launch_stream_mx<1>(st, a, b, p);
+  if (p.M <= 16) return launch_stream_mx<2>(st, a, b, p);
+  if (p.M <= 32) return launch_stream_mx<4>(st, a, b, p);
+  if (p.M <= 48) return launch_stream_mx<6>(st, a, b, p);
+  return launch_stream_mx<8>(st, a, b, p);
+}
+
+// ---- one row of a: a wave owns whole rows of b -----------------------------------------------
+// The matrix core has nothing to add, and the ring, its barrier and its fold cost more than they give (11008 x 4096
+// 9.2 us against 9.6).  Here lane l holds bytes [h * 1024 + 16 l, +16) of the row of a in registers (h < H =
+// ceil(k / 1024)), a wave walks the rows w, w + NW, .. of the block's share of b with the requests of two rows in
+// flight, meets each row with v_dot4_i32_i8 (exact int32) and sums across the lanes; no LDS, no barrier.  Same
+// int32 sums and the same epilogue as the other paths, hence the same bits.  Two to four rows of a, which this
+// kernel held in registers too, stream faster (2 rows: 4096 x 4096 5.7 -> 5.2 us, 2048 x 8192 6.2 -> 5.2, 4 rows of
+// 11008 x 4096 12.1 -> 10.0; weights from HBM).
 __device__ __forceinline__ int wave_sum_i32(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
   v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
@@ -133,13 +272,12 @@ __device__ __forceinline__ int wave_sum_i32(int v) {
          + (__builtin_amdgcn_readlane(v, 32) + __builtin_amdgcn_readlane(v, 48));
 }
 
-template<typename T, int NW, int H, int MR>
+template<typename T, int NW, int H>
 __global__ void __launch_bounds__(NW * 64)
 matmul_quant_wave_rows(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                        const float* __restrict__ a_scale, const float* __restrict__ b_scale,
                        const typename TT<T>::storage* __restrict__ bias,
-                       typename TT<T>::storage* __restrict__ out, int M, int N, int K,
-                       int rows_per_block) {
+                       typename TT<T>::storage* __restrict__ out, int N, int K, int rows_per_block) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row0 = blockIdx.x * rows_per_block;
@@ -164,14 +302,10 @@ matmul_quant_wave_rows(const uint8_t* __restrict__ a, const uint8_t* __restrict_
           reinterpret_cast<const i32x4*>(rowp + (live ? voff[h] : 0u)));
     }
   };
-  // the rows of a first (they come from L2 and every row of b needs them), then two rows of b
-  i32x4 av[MR][H];
+  // a first (it comes from L2 and every row of b needs it), then two rows of b
+  i32x4 av[H];
 #pragma unroll
-  for (int m = 0; m < MR; ++m) {
-    const uint8_t* arow = a + (size_t)(m < M ? m : 0) * K;
-#pragma unroll
-    for (int h = 0; h < H; ++h) av[m][h] = *reinterpret_cast<const i32x4*>(arow + voff[h]);
-  }
+  for (int h = 0; h < H; ++h) av[h] = *reinterpret_cast<const i32x4*>(a + voff[h]);
   issue(0, 0);
   issue(1, 1);
   const float sa = a_scale[0];
@@ -180,24 +314,19 @@ matmul_quant_wave_rows(const uint8_t* __restrict__ a, const uint8_t* __restrict_
     const float sb = b_scale[n];
     float bv = 0.f;
     if (bias != nullptr) bv = TT<T>::load(bias + n);
+    int acc = 0;
 #pragma unroll
-    for (int m = 0; m < MR; ++m) {
-      int acc = 0;
+    for (int h = 0; h < H; ++h) {
+      int part = 0;
 #pragma unroll
-      for (int h = 0; h < H; ++h) {
-        int part = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          part = __builtin_amdgcn_sdot4(av[m][h][j], wq[buf][h][j], part, false);
-        }
-        acc += valid[h] ? part : 0;
-      }
-      const int sum = wave_sum_i32(acc);
-      if (lane == 0 && m < M) {
-        float v = (float)sum * (sa * sb);
-        if (bias != nullptr) v = v + bv;
-        TT<T>::store(out + (int64_t)m * N + n, v);
-      }
+      for (int j = 0; j < 4; ++j) part = __builtin_amdgcn_sdot4(av[h][j], wq[buf][h][j], part, false);
+      acc += valid[h] ? part : 0;
+    }
+    const int sum = wave_sum_i32(acc);
+    if (lane == 0) {
+      float v = (float)sum * (sa * sb);
+      if (bias != nullptr) v = v + bv;
+      TT<T>::store(out + n, v);
     }
   };
   for (int i = 0; i < nr; i += 2) {
@@ -208,85 +337,41 @@ matmul_quant_wave_rows(const uint8_t* __restrict__ a, const uint8_t* __restrict_
   }
 }
 
-template<typename T, int H, int MR>
+template<typename T, int H>
 int launch_wave_rows_inst(hipStream_t st, const uint8_t* a, const uint8_t* b, const float* a_scale,
-                          const float* b_scale, const void* bias, void* out, int m, int64_t n,
-                          int64_t k) {
+                          const float* b_scale, const void* bias, void* out, int64_t n, int64_t k) {
   typedef typename TT<T>::storage S;
-  // A lane holds 4 H MR registers of a and 8 H of b: 16 waves (128 registers each) while that
-  // fits, 8 waves (256 each) beyond, where the compiler would otherwise spill to scratch memory
-  // (8192 x 8192, 2 rows).
-  constexpr int NW = H * (4 * MR + 8) <= 100 ? 16 : 8;
+  constexpr int NW = 16;
   // 16 waves per CU, twice as many blocks from 128 rows per block on; a wave then walks its rows
   // two ahead
-  int64_t grid = 256 * (16 / NW);
+  int64_t grid = 256;
   if ((n + grid - 1) / grid >= 128) grid *= 2;
   int rpb = (int)((n + grid - 1) / grid);
   if (rpb < NW) rpb = NW;
   grid = (n + rpb - 1) / rpb;
-  matmul_quant_wave_rows<T, NW, H, MR><<<(unsigned)grid, NW * 64, 0, st>>>(
-      a, b, a_scale, b_scale, static_cast<const S*>(bias), static_cast<S*>(out), m, (int)n, (int)k,
-      rpb);
+  matmul_quant_wave_rows<T, NW, H><<<(unsigned)grid, NW * 64, 0, st>>>(
+      a, b, a_scale, b_scale, static_cast<const S*>(bias), static_cast<S*>(out), (int)n, (int)k, rpb);
   return ofq_check_launch();
 }
 
-// m <= 2 with 16 | k <= 8192, m <= 4 with k <= 4096 (the rows of a are held in registers: 4 H m
-// of them).  Three and four rows of more than 4 KB run faster on the matrix-core kernel below
-// (4096 x 8192, 4 rows: 14.5 us here, 9.4 us there).
+// one row of up to 8192 elements (it is held in registers)
 template<typename T>
 int launch_wave_rows(hipStream_t st, const uint8_t* a, const uint8_t* b, const float* a_scale,
-                     const float* b_scale, const void* bias, void* out, int m, int64_t n,
-                     int64_t k) {
-  const int h = (int)((k + 1023) / 1024);
-#define OFQ_WR(HV)                                                                             \
-  case HV:                                                                                     \
-    if (m == 1) return launch_wave_rows_inst<T, HV, 1>(st, a, b, a_scale, b_scale, bias, out, m, n, k); \
-    if (m == 2) return launch_wave_rows_inst<T, HV, 2>(st, a, b, a_scale, b_scale, bias, out, m, n, k); \
-    if constexpr (HV <= 4) {                                                                   \
-      return launch_wave_rows_inst<T, HV, 4>(st, a, b, a_scale, b_scale, bias, out, m, n, k);  \
-    } else {                                                                                   \
-      return OFQ_ERR_UNSUPPORTED;                                                              \
-    }
-  switch (h) {
+                     const float* b_scale, const void* bias, void* out, int64_t n, int64_t k) {
+#define OFQ_WR(HV) \
+  case HV: return launch_wave_rows_inst<T, HV>(st, a, b, a_scale, b_scale, bias, out, n, k);
+  switch ((k + 1023) / 1024) {
     OFQ_WR(1) OFQ_WR(2) OFQ_WR(3) OFQ_WR(4) OFQ_WR(5) OFQ_WR(6) OFQ_WR(7) OFQ_WR(8)
     default: return OFQ_ERR_UNSUPPORTED;
   }
 #undef OFQ_WR
 }
 
-template<typename T, int NW, int MT>
-int launch_inst(hipStream_t st, const uint8_t* a, const uint8_t* b, const float* a_scale,
-                const float* b_scale, const void* bias, void* out, int m, int64_t n, int64_t k,
-                int grid, int rpb) {
-  typedef typename TT<T>::storage S;
-  const size_t lds = (size_t)NW * MT * 256 * 4;
-  auto kern = matmul_quant_rows<T, NW, MT>;
-  if (lds > 64 * 1024) {
-    static std::atomic<uint64_t> lds_allowed{0};  // devices on which the kernel's LDS limit is raised
-    if (!ofq_allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)lds, lds_allowed)) return OFQ_ERR_LAUNCH;
-  }
-  kern<<<grid, NW * 64, lds, st>>>(a, b, a_scale, b_scale, static_cast<const S*>(bias),
-                                   static_cast<S*>(out), m, (int)n, (int)k, rpb);
-  return ofq_check_launch();
-}
-
 template<typename T>
 int launch_part(hipStream_t st, const uint8_t* a, const uint8_t* b, const float* a_scale,
                 const float* b_scale, const void* bias, void* out, int m, int64_t n, int64_t k) {
-  if (m <= 4 && k <= 8192 && k % 16 == 0) {
-    const int rc = launch_wave_rows<T>(st, a, b, a_scale, b_scale, bias, out, m, n, k);
-    if (rc != OFQ_ERR_UNSUPPORTED) return rc;
-  }
-  constexpr int kCUs = 256;
-  const int64_t max_rows = 16 * kI8MaxTiles;
-  int64_t grid = kCUs;
-  if ((n + grid - 1) / grid > max_rows) grid = (n + max_rows - 1) / max_rows;
-  int rpb = (int)((n + grid - 1) / grid);
-  if (rpb < 16) rpb = 16;
-  grid = (n + rpb - 1) / rpb;
-  if (m <= 16) return launch_inst<T, 16, 1>(st, a, b, a_scale, b_scale, bias, out, m, n, k, (int)grid, rpb);
-  if (m <= 32) return launch_inst<T, 16, 2>(st, a, b, a_scale, b_scale, bias, out, m, n, k, (int)grid, rpb);
-  return launch_inst<T, 16, 4>(st, a, b, a_scale, b_scale, bias, out, m, n, k, (int)grid, rpb);
+  if (m == 1 && k <= 8192) return launch_wave_rows<T>(st, a, b, a_scale, b_scale, bias, out, n, k);
+  return launch_stream(st, a, b, MqStreamArgs{a_scale, b_scale, bias, out, TT<T>::dtype, m, (int)n, (int)k, 0});
 }
 
 }  // namespace
