@@ -15,6 +15,7 @@
 // This file only chooses kernel, tile and slices and fills parameter blocks.
 #include <cmath>
 
+#include "gemm_deep.h"
 #include "gemm_kernels.h"
 #include "ofq_device.h"
 #include "ofq_internal.h"
@@ -40,16 +41,8 @@ inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 // expected time in us of one on m x n outputs and kt k-tiles of 128 bytes,
 //   start + outputs * m n / 10^6 + kt * (alone + share * b/256 + round * ceil(b/256) + pair * ceil(b/512)
 //                                        + four * ceil(b/1024))
-// with b blocks: tiles from 256 rows on run one block a CU (rounds of 256), those of 128 two, those of 64 four.
-// int8: fitted to 15 500 random products of 65 to 8192 rows, 512 to 14336 columns and k from 512 to 8192, half of them with
-// weights from HBM, half with two that take turns in cache, each timed on every tile: within 12 % of the measured time
-// for 90 of 100, 64 x 64 tiles within 22 %.  The tile of the least expected time takes 0.8 % longer than the best one in
-// the mean, 0.74 of what rules by ranges of m and block counts chose; 106 of the 15 500 take more than 3 % longer than
-// that (64 x 64 tiles: of some 1000 blocks to 1.24, of some 100 whose weights come from HBM to 1.31, 97 x 3680 x 2688
-// 14.2 us with the slices it had, 18.6 now; a table from weights in HBM alone mends those and makes products on weights in
-// cache up to 1.5 times slower).  Fitted to weights in cache and without the rounds of four, which long rows of 64 x 64
-// tiles show (114 x 13256 x 5824 46.5 us, now 41.2; 321 x 5816 x 2560 21.5, now 17.6; 613 x 3744 x 3456 25.8, now
-// 22.2), it was 275, up to 1.49.
+// with b blocks: tiles from 256 rows on run one block a CU (rounds of 256), those of 128 two, those of 64 four (of
+// int8's, kCopyCostI8, as many as their stages leave room for).
 // 16 bits: fitted to 384 random problems of 1024 to 4096 rows, to 32000 columns and k to 14336; on 2900 others
 // 0.74 of what the rules chose, 14 more than 3 % longer (1.14 at worst, 1609 x 12072 x 576, where 384 columns are
 // the best tile and 192 the chosen one).
@@ -58,31 +51,54 @@ struct TileCost {
   int bm, bn;
   double start, outputs, alone, share, round, pair, four;
 };
-const TileCost kCopyCost[2][2][kCopyTiles] = {  // [int8][ragged k]
-    {{{64, 64, 5.1, 0.17, 0.088, 0.194, 0.038, 0.0, 0.0},
-      {128, 128, 4.3, 0.73, 0.0, 0.189, 0.013, 0.534, 0.0},
-      {256, 128, 5.8, 0.71, 0.0, 0.203, 0.778, 0.0, 0.0},
-      {256, 192, 8.6, 0.70, 0.0, 0.303, 0.887, 0.0, 0.0},
-      {256, 256, 10.6, 0.75, 0.0, 0.469, 0.952, 0.0, 0.0},
-      {256, 384, 13.9, 0.66, 0.0, 0.617, 1.324, 0.0, 0.0}},
-     {{64, 64, 4.5, 0.37, 0.139, 0.151, 0.115, 0.0, 0.0},
-      {128, 128, 4.4, 0.47, 0.0, 0.174, 0.204, 0.466, 0.0},
-      {256, 128, 4.1, 0.84, 0.0, 0.027, 1.042, 0.0, 0.0},
-      {256, 192, 8.0, 0.54, 0.0, 0.316, 1.100, 0.0, 0.0},
-      {256, 256, 9.9, 0.66, 0.0, 0.382, 1.310, 0.0, 0.0},
-      {256, 384, 14.6, 0.54, 0.0, 0.586, 1.697, 0.0, 0.0}}},
-    {{{64, 64, 2.3, 0.45, 0.0, 0.129, 0.0, 0.0, 0.370},
-      {128, 128, 2.9, 0.60, 0.0, 0.203, 0.078, 0.477, 0.0},
-      {256, 128, 4.8, 0.66, 0.0, 0.323, 0.745, 0.0, 0.0},
-      {256, 192, 9.1, 0.45, 0.0, 0.404, 0.853, 0.0, 0.0},
-      {256, 256, 11.2, 0.36, 0.0, 0.503, 0.976, 0.0, 0.0},
-      {256, 384, 13.5, 0.33, 0.0, 0.606, 1.388, 0.0, 0.0}},
-     {{64, 64, 2.6, 0.43, 0.0, 0.138, 0.019, 0.003, 0.428},
-      {128, 128, 3.2, 0.56, 0.0, 0.228, 0.160, 0.471, 0.0},
-      {256, 128, 5.0, 0.68, 0.0, 0.261, 0.902, 0.0, 0.0},
-      {256, 192, 9.1, 0.44, 0.0, 0.381, 1.075, 0.0, 0.0},
-      {256, 256, 11.3, 0.37, 0.0, 0.402, 1.361, 0.0, 0.0},
-      {256, 384, 14.4, 0.31, 0.0, 0.498, 1.789, 0.0, 0.0}}}};
+const TileCost kCopyCost[2][kCopyTiles] = {  // [ragged k]
+    {{64, 64, 5.1, 0.17, 0.088, 0.194, 0.038, 0.0, 0.0},
+     {128, 128, 4.3, 0.73, 0.0, 0.189, 0.013, 0.534, 0.0},
+     {256, 128, 5.8, 0.71, 0.0, 0.203, 0.778, 0.0, 0.0},
+     {256, 192, 8.6, 0.70, 0.0, 0.303, 0.887, 0.0, 0.0},
+     {256, 256, 10.6, 0.75, 0.0, 0.469, 0.952, 0.0, 0.0},
+     {256, 384, 13.9, 0.66, 0.0, 0.617, 1.324, 0.0, 0.0}},
+    {{64, 64, 4.5, 0.37, 0.139, 0.151, 0.115, 0.0, 0.0},
+     {128, 128, 4.4, 0.47, 0.0, 0.174, 0.204, 0.466, 0.0},
+     {256, 128, 4.1, 0.84, 0.0, 0.027, 1.042, 0.0, 0.0},
+     {256, 192, 8.0, 0.54, 0.0, 0.316, 1.100, 0.0, 0.0},
+     {256, 256, 9.9, 0.66, 0.0, 0.382, 1.310, 0.0, 0.0},
+     {256, 384, 14.6, 0.54, 0.0, 0.586, 1.697, 0.0, 0.0}}};
+// int8: fitted to 9158 random products of 65 to 8192 rows, 512 to 14336 columns and k from 512 to 8192, a third of them
+// with a ragged last k-tile, each timed on every tile with weights from HBM: within 10 to 16 % of the measured time for
+// 90 of 100.  The choice (with the slices of mq_plan and the streaming kernel) takes 1.2 % longer than the best one in
+// the mean.  Of the tiles of gemm_deep the ones of fewer stages leave room for a second and third block, whose
+// products lie under the first one's epilogue: they win where K is short and blocks are many; 128 x 128 does
+// so with two stages of gemm_core2 (1852 x 8323 x 512 19.2 us there, 26.3 with five stages).
+// Time over that of one k-tile under way on every tile (gemm_core2, its own fitted choice, with its slices): 0.72 in the mean at 65 to
+// 128 rows, 0.80 to 256, 0.81 to 512, 0.85 to 1024, 0.88 to 2048, 0.95 to 8192; 256 x 4096 x 4096 26.5 -> 13.0 us,
+// 512 x 4096 x 4096 27.7 -> 17.2, 1024 x 4096 x 4096 33.4 -> 25; 5 of 100 take more than 3 % longer, to 1.35 (rows of
+// 512 elements, 190 x 775 x 2496 10.4 -> 14.0).
+enum MqTile {
+  kMq64, kMq64Short, kMq128x64, kMq128x64Short, kMq128, kMq128Short, kMq256x128, kMq256x192, kMq256x256, kMq256x384,
+  kMqTiles
+};
+const TileCost kCopyCostI8[2][kMqTiles] = {  // [ragged k]
+    {{64, 64, 3.29, 1.088, 0.0, 0.005, 0.187, 0.107, 0.0},
+     {64, 64, 3.22, 0.516, 0.0, 0.121, 0.049, 0.085, 0.136},
+     {128, 64, 3.46, 1.442, 0.0, 0.076, 0.315, 0.0, 0.0},
+     {128, 64, 3.27, 0.607, 0.0, 0.166, 0.123, 0.187, 0.0},
+     {128, 128, 4.49, 1.016, 0.0, 0.117, 0.449, 0.0, 0.0},
+     {128, 128, 3.36, 0.681, 0.0, 0.214, 0.0, 0.684, 0.0},
+     {256, 128, 6.46, 0.754, 0.0, 0.183, 0.649, 0.0, 0.0},
+     {256, 192, 8.86, 0.515, 0.0, 0.314, 1.039, 0.0, 0.0},
+     {256, 256, 10.39, 0.485, 0.0, 0.305, 1.247, 0.0, 0.0},
+     {256, 384, 14.53, 0.423, 0.0, 0.528, 1.506, 0.0, 0.0}},
+    {{64, 64, 3.19, 1.057, 0.0, 0.004, 0.183, 0.244, 0.0},
+     {64, 64, 3.10, 0.681, 0.0, 0.040, 0.114, 0.131, 0.200},
+     {128, 64, 3.36, 1.477, 0.0, 0.038, 0.457, 0.0, 0.0},
+     {128, 64, 3.26, 0.630, 0.0, 0.068, 0.257, 0.204, 0.0},
+     {128, 128, 4.19, 1.048, 0.0, 0.050, 0.610, 0.0, 0.0},
+     {128, 128, 3.19, 0.662, 0.0, 0.213, 0.073, 0.703, 0.0},
+     {256, 128, 6.16, 0.755, 0.0, 0.088, 0.897, 0.0, 0.0},
+     {256, 192, 8.54, 0.422, 0.0, 0.286, 1.299, 0.0, 0.0},
+     {256, 256, 10.32, 0.461, 0.0, 0.253, 1.631, 0.0, 0.0},
+     {256, 384, 14.67, 0.488, 0.0, 0.349, 1.973, 0.0, 0.0}}};
 
 double tile_us(const TileCost& c, int64_t m, int64_t n, int64_t kt, int splits = 1) {
   const double b = (double)((m + c.bm - 1) / c.bm) * (double)((n + c.bn - 1) / c.bn) * splits;
@@ -90,19 +106,21 @@ double tile_us(const TileCost& c, int64_t m, int64_t n, int64_t kt, int splits =
          + kt * (c.alone + c.share * b / 256 + c.round * std::ceil(b / 256) + c.pair * std::ceil(b / 512)
                  + c.four * std::ceil(b / 1024));
 }
-CopyTile pick_copy_tile(bool int8, int64_t m, int64_t n, int64_t row_bytes, double* us) {
-  const TileCost* cost = kCopyCost[int8][row_bytes % 128 != 0];
+int pick_tile(const TileCost* cost, int tiles, int64_t m, int64_t n, int64_t row_bytes, double* us) {
   int best = 0;
   double best_us = 1e300;
-  for (int i = 0; i < kCopyTiles; ++i) {
+  for (int i = 0; i < tiles; ++i) {
     const double t = tile_us(cost[i], m, n, (row_bytes + 127) / 128);
     if (t < best_us) {
       best = i;
       best_us = t;
     }
   }
-  if (us != nullptr) *us = best_us;
-  return (CopyTile)best;
+  *us = best_us;
+  return best;
+}
+CopyTile pick_copy_tile(int64_t m, int64_t n, int64_t row_bytes, double* us) {
+  return (CopyTile)pick_tile(kCopyCost[row_bytes % 128 != 0], kCopyTiles, m, n, row_bytes, us);
 }
 
 }  // namespace
@@ -122,7 +140,8 @@ int launch_plain(hipStream_t st, const LinearArgs& a, const void* wt) {
   ep.bias = static_cast<const S*>(a.bias);
   ep.out = static_cast<S*>(a.out);
   const int64_t kt = (a.k + 63) / 64;
-  const CopyTile tile = pick_copy_tile(false, a.m, a.n, a.k * 2, nullptr);
+  double us;
+  const CopyTile tile = pick_copy_tile(a.m, a.n, a.k * 2, &us);
   switch (tile) {
     case kCopy64:
       return launch_core2<MF, B2Copy<RG, 64, 256>, EP, 64, 64, 2, 2>(st, a.x, a.k * 2, bp, ep, a.m, a.n, kt);
@@ -140,7 +159,7 @@ int launch_plain(hipStream_t st, const LinearArgs& a, const void* wt) {
       return launch_core2<MF, B2Copy<RG, 256, 512>, EP, 256, 256, 4, 2>(st, a.x, a.k * 2, bp, ep, a.m, a.n, kt);
     }
   }
-  const int width = kCopyCost[0][RG][tile].bn;
+  const int width = kCopyCost[RG][tile].bn;
   return std::is_same<T, f16>::value
              ? launch_gemm_pp_f16(st, a.x, wt, a.bias, a.out, a.m, a.n, a.k, width)
              : launch_gemm_pp_bf16(st, a.x, wt, a.bias, a.out, a.m, a.n, a.k, width);
@@ -435,7 +454,7 @@ size_t wr_partial_bytes(const LinearArgs& a, const WrPlan& plan) {
 double two_pass_us(const LinearArgs& a) {
   const double nk = (double)a.n * a.k;
   double us;
-  pick_copy_tile(false, a.m, a.n, a.k * 2, &us);
+  pick_copy_tile(a.m, a.n, a.k * 2, &us);
   return us + 2.2 + nk * (2 + a.bits / 8.0 + (a.symmetric ? 2.0 : 4.0) / a.group_size) / 5.9e6;
 }
 
@@ -591,7 +610,7 @@ int launch_gemm_gn(hipStream_t st, const LinearArgs& a, void* workspace) {
 
 using namespace ofq;
 
-// rows of a up to which the workspace query has no slices for rows of b of less than 8192 elements
+// rows of a up to which matmul_quant streams the weights whatever the shape
 static constexpr int64_t kMatmulQuantRowsMaxM = 64;
 
 namespace ofq {
@@ -627,37 +646,39 @@ int mq_room(int64_t m, int64_t n, int64_t k) {
   return (int)s;
 }
 
-// Tile and slices by the least expected time (kCopyCost), with at most `most` slices (what the workspace that callers
-// know has room for): one slice on any tile, or several of 128 x 128 or 256 x 128 tiles in one resident round,
-// whose int32 sums and second launch cost 2 us and 1.7 to 1.8 us per 10^6 sums.
+// Streaming kernel, tile and slices by the least expected time (kCopyCostI8), with at most `most` slices (what the
+// workspace that callers know has room for): one slice on any tile, or several of 128 x 128 or 256 x 128
+// tiles in one resident round, whose int32 sums and second launch cost 2 us and 1.8 to 2.3 us per 10^6 sums.
 struct MqPlan {
-  CopyTile tile;
+  bool stream;
+  MqTile tile;
   int splits;
 };
 MqPlan mq_plan(int64_t m, int64_t n, int64_t k, int most) {
-  static const TileCost kSliced[2][2] = {{{128, 128, 5.3, 0.0, 0.536, 0.215, 0.0, 0.0, 0.0},
-                                          {256, 128, 6.6, 0.0, 0.724, 0.288, 0.0, 0.0, 0.0}},
-                                         {{128, 128, 5.6, 0.0, 0.584, 0.327, 0.0, 0.0, 0.0},
-                                          {256, 128, 6.9, 0.0, 0.860, 0.286, 0.0, 0.0, 0.0}}};
-  static const double kSums[2][2] = {{1.80, 1.79}, {1.69, 1.79}};  // us per 10^6 of a slice
-  MqPlan plan{kCopy64, 1};
+  static const TileCost kSliced[2][2] = {{{128, 128, 6.47, 0.0, 0.0, 0.111, 0.430, 0.0, 0.0},
+                                          {256, 128, 8.03, 0.0, 0.619, 0.185, 0.0, 0.0, 0.0}},
+                                         {{128, 128, 6.29, 0.0, 0.0, 0.029, 0.614, 0.0, 0.0},
+                                          {256, 128, 7.82, 0.0, 0.0, 0.065, 0.872, 0.0, 0.0}}};
+  static const double kSums[2][2] = {{2.26, 1.78}, {2.22, 1.85}};  // us per 10^6 of a slice
+  MqPlan plan{false, kMq64, 1};
   double best;
-  plan.tile = pick_copy_tile(true, m, n, k, &best);
-  const int64_t kt = (k + 127) / 128;
   const int ragged = k % 128 != 0;
+  plan.tile = (MqTile)pick_tile(kCopyCostI8[ragged], kMqTiles, m, n, k, &best);
+  const int64_t kt = (k + 127) / 128;
   for (int s = 2; s <= most; ++s) {
     const int64_t per = (kt + s - 1) / s;
     if (per < 2 || per * (s - 1) >= kt) continue;
     for (int i = 0; i < 2; ++i) {
       const TileCost& c = kSliced[ragged][i];
-      if ((int64_t)ceil_div(m, c.bm) * ceil_div(n, c.bn) * s > (i == 0 ? 512 : 256)) continue;
+      if ((int64_t)ceil_div(m, c.bm) * ceil_div(n, c.bn) * s > 256) continue;
       const double us = tile_us(c, m, n, per, s) + kSums[ragged][i] * s * 1e-6 * (double)m * n;
       if (us < best) {
         best = us;
-        plan = MqPlan{i == 0 ? kCopy128 : kCopy256x128, s};
+        plan = MqPlan{false, i == 0 ? kMq128 : kMq256x128, s};
       }
     }
   }
+  if (matmul_quant_rows_supported(m, n, k)) plan.stream = matmul_quant_rows_us(m, n, k) < best;
   return plan;
 }
 
@@ -689,12 +710,10 @@ int launch_mq_split(hipStream_t st, const void* a, const BCopyParams& bp, const 
   EpPartialI32::Params pp;
   pp.out = partials;
   int rc;
-  if (plan.tile == kCopy256x128) {
-    rc = launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EpPartialI32, 256, 128, 4, 2>(st, a, k, bp, pp, m,
-                                                                             n, (k + 127) / 128, splits);
+  if (plan.tile == kMq256x128) {
+    rc = launch_deep<MfmaI8, RG, EpPartialI32, 256, 128, 4, 2, 3>(st, a, k, bp, pp, m, n, (k + 127) / 128, splits);
   } else {
-    rc = launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EpPartialI32, 128, 128, 4, 2>(st, a, k, bp, pp, m,
-                                                                             n, (k + 127) / 128, splits);
+    rc = launch_deep<MfmaI8, RG, EpPartialI32, 128, 128, 4, 2, 5>(st, a, k, bp, pp, m, n, (k + 127) / 128, splits);
   }
   if (rc != OFQ_OK) return rc;
   const int64_t mn = m * n;
@@ -709,7 +728,7 @@ int launch_mq_split(hipStream_t st, const void* a, const BCopyParams& bp, const 
 template<bool RG, typename T>
 int launch_mq(hipStream_t st, const void* a, const BCopyParams& bp, const float* a_scale,
               const float* b_scale, const void* bias, void* out, int64_t m, int64_t n, int64_t k,
-              CopyTile tile) {
+              MqTile tile) {
   typedef EpScale<T> EP;
   typename EP::Params ep;
   ep.a_scale = a_scale;
@@ -718,18 +737,21 @@ int launch_mq(hipStream_t st, const void* a, const BCopyParams& bp, const float*
   ep.out = static_cast<typename TT<T>::storage*>(out);
   const int64_t kt = (k + 127) / 128;
   switch (tile) {
-    case kCopy64: return launch_core2<MfmaI8, B2Copy<RG, 64, 256>, EP, 64, 64, 2, 2>(st, a, k, bp, ep, m, n, kt);
-    case kCopy128: return launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EP, 128, 128, 4, 2>(st, a, k, bp, ep, m, n, kt);
-    case kCopy256x128:
-      return launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EP, 256, 128, 4, 2>(st, a, k, bp, ep, m, n, kt);
+    case kMq64: return launch_deep<MfmaI8, RG, EP, 64, 64, 2, 2, 5>(st, a, k, bp, ep, m, n, kt);
+    case kMq64Short: return launch_deep<MfmaI8, RG, EP, 64, 64, 2, 2, 3>(st, a, k, bp, ep, m, n, kt);
+    case kMq128x64: return launch_deep<MfmaI8, RG, EP, 128, 64, 4, 2, 6>(st, a, k, bp, ep, m, n, kt);
+    case kMq128x64Short: return launch_deep<MfmaI8, RG, EP, 128, 64, 4, 2, 3>(st, a, k, bp, ep, m, n, kt);
+    case kMq128: return launch_deep<MfmaI8, RG, EP, 128, 128, 4, 2, 5>(st, a, k, bp, ep, m, n, kt);
+    case kMq128Short: return launch_core2<MfmaI8, B2Copy<RG, 128, 512>, EP, 128, 128, 4, 2>(st, a, k, bp, ep, m, n, kt);
+    case kMq256x128: return launch_deep<MfmaI8, RG, EP, 256, 128, 4, 2, 3>(st, a, k, bp, ep, m, n, kt);
     default: break;
   }
   if constexpr (RG) {  // (why: launch_pp)
-    if (tile == kCopy256x192) {
+    if (tile == kMq256x192) {
       return launch_core2<MfmaI8, B2Copy<RG, 192, 512>, EP, 256, 192, 4, 2>(st, a, k, bp, ep, m, n, kt);
     }
   }
-  const int width = kCopyCost[1][RG][tile].bn;
+  const int width = kCopyCostI8[RG][tile].bn;
   return launch_gemm_pp_i8(st, a, bp.b, a_scale, b_scale, bias, out, TT<T>::dtype, m, n, k, width);
 }
 
@@ -772,39 +794,37 @@ extern "C" int ofq_matmul_quant_ws(void* stream, const void* a, const void* b, c
                 OFQ_ERR_NULL_POINTER);
   OFQ_RETURN_IF(!ofq_aligned16(a) || !ofq_aligned16(b) || !ofq_aligned16(out), OFQ_ERR_MISALIGNED);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // few rows of a: the weights stream once
-  if (matmul_quant_rows_supported(m, n, k)) {
+  auto stream_weights = [&] {
     return launch_matmul_quant_rows(st, a, b, a_scale, b_scale, bias, out, out_dtype, m, n, k);
-  }
+  };
+  // few rows of a: the weights stream once (above 64 rows where that is expected to be faster)
+  if (m <= kMatmulQuantRowsMaxM && matmul_quant_rows_supported(m, n, k)) return stream_weights();
   BCopyParams bp;
   bp.b = static_cast<const uint8_t*>(b);
   bp.ldb = k;
   bp.N = (int)n;
-  MqPlan plan = mq_plan(m, n, k, 1);
-  {
-    const int room = mq_room(m, n, k);
-    const size_t need = (size_t)room * (size_t)m * (size_t)n * 4;
-    if (room > 1 && workspace != nullptr && workspace_bytes >= need && ofq_aligned16(workspace)) {
-      plan = mq_plan(m, n, k, room);
-    }
-    if (plan.splits > 1) {
-      float* part = static_cast<float*>(workspace);
+  const int room = mq_room(m, n, k);
+  const size_t need = (size_t)room * (size_t)m * (size_t)n * 4;
+  const bool slices = room > 1 && workspace != nullptr && workspace_bytes >= need && ofq_aligned16(workspace);
+  const MqPlan plan = mq_plan(m, n, k, slices ? room : 1);
+  if (plan.stream) return stream_weights();
+  if (plan.splits > 1) {
+    float* part = static_cast<float*>(workspace);
 #define OFQ_MQS(RG, T)                                                                           \
   return launch_mq_split<RG, T>(st, a, bp, a_scale, b_scale, bias, out, m, n, k, part, plan)
-      if (k % 128 != 0) {
-        switch (out_dtype) {
-          case OFQ_F16: OFQ_MQS(true, f16);
-          case OFQ_BF16: OFQ_MQS(true, bf16);
-          default: OFQ_MQS(true, float);
-        }
-      }
+    if (k % 128 != 0) {
       switch (out_dtype) {
-        case OFQ_F16: OFQ_MQS(false, f16);
-        case OFQ_BF16: OFQ_MQS(false, bf16);
-        default: OFQ_MQS(false, float);
+        case OFQ_F16: OFQ_MQS(true, f16);
+        case OFQ_BF16: OFQ_MQS(true, bf16);
+        default: OFQ_MQS(true, float);
       }
-#undef OFQ_MQS
     }
+    switch (out_dtype) {
+      case OFQ_F16: OFQ_MQS(false, f16);
+      case OFQ_BF16: OFQ_MQS(false, bf16);
+      default: OFQ_MQS(false, float);
+    }
+#undef OFQ_MQS
   }
   if (k % 128 != 0) {
     switch (out_dtype) {

@@ -147,8 +147,9 @@ int launch_gemv_ring_mt_f16_b8(hipStream_t st, const LinearJob& job, const RingM
 int launch_gemv_ring_mt_bf16_b4(hipStream_t st, const LinearJob& job, const RingMtPlan& plan);
 int launch_gemv_ring_mt_bf16_b8(hipStream_t st, const LinearJob& job, const RingMtPlan& plan);
 
-// matmul_quant with few rows of a (m <= 64; k a multiple of 64): int8 MFMA with the weights
-// streamed once.
+// matmul_quant with few rows of a (m <= 96; k a multiple of 64): int8 MFMA with the weights
+// streamed once; its expected time (m > 64).
+double matmul_quant_rows_us(int64_t m, int64_t n, int64_t k);
 bool matmul_quant_rows_supported(int64_t m, int64_t n, int64_t k);
 int launch_matmul_quant_rows(hipStream_t st, const void* a, const void* b, const float* a_scale,
                              const float* b_scale, const void* bias, void* out, int out_dtype,
