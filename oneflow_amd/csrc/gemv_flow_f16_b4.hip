@@ -1,0 +1,10 @@
+// gemv_flow (gemv_flow.h) for fp16 activations and 4-bit codes.
+#include "gemv_flow_launch.h"
+
+namespace ofq {
+
+int launch_gemv_flow_f16_b4(hipStream_t st, const LinearJob& job, const FlowPlan& plan) {
+  return launch_flow_t<f16, 4>(st, job, plan);
+}
+
+}  // namespace ofq

@@ -30,6 +30,7 @@
 //     to T.
 #include <atomic>
 #include "gemv_kernels.h"
+#include "gemv_flow.h"
 #include "gemv_ring.h"
 #include "gemv_rows.h"
 #include "ofq_device.h"
@@ -390,6 +391,109 @@ bool ring_plan(const LinearJob& job, RingPlan* plan) {
     return true;
   }
   return false;
+}
+
+}  // namespace
+
+namespace {
+
+// The split of gemv_flow for a job, or false where more than a block per CU or LDS would be needed: eight waves, or
+// six where eight leave no room.
+bool flow_plan(const LinearJob& job, FlowPlan* plan) {
+  const LinearArgs& a = job.pr[0];
+  const int lists = job.glu ? 1 : job.count, matrices = job.glu ? 2 : 1;
+  const int G = (int)(a.k / a.group_size);
+  const int regions = matrices * (a.symmetric ? 1 : 2);
+  const int mx = a.m <= 8 ? 1 : 2;
+  const int max_rows = job.glu ? 48 : (mx == 1 ? 96 : 80);
+  int64_t total = 0;
+  for (int i = 0; i < lists; ++i) total += job.pr[i].n;
+  auto blocks_at = [&](int rpb) {
+    int64_t b = 0;
+    for (int i = 0; i < lists; ++i) b += (job.pr[i].n + rpb - 1) / rpb;
+    return b;
+  };
+  int rpb = total > 256 * max_rows ? max_rows + 1 : (int)((total + 255) / 256);
+  if (rpb < 16) rpb = 16;
+  while (rpb <= max_rows && blocks_at(rpb) > 256) ++rpb;
+  if (rpb <= max_rows) {
+    const int tl = (rpb + 15) / 16;
+    const size_t scales = (size_t)(regions * ring_scale_bytes(rpb, G) + 1023) & ~(size_t)1023;
+    const int step = (a.bits == 4 ? 4 : 2) * mx + 2 * tl * matrices;
+    for (int nw = 8; nw >= 6; nw -= 2) {
+      size_t lds = scales + (size_t)nw * step * 1024;
+      const size_t red = (size_t)nw * (size_t)a.m * (tl * matrices * 16 + 4) * 4;
+      if (red > lds) lds = red;
+      if (lds > 160 * 1024) continue;
+      plan->grid = (int)blocks_at(rpb);
+      plan->rows_per_block = rpb;
+      plan->mx = mx;
+      plan->tl = tl;
+      plan->nw = nw;
+      plan->lds = lds;
+      return true;
+    }
+  }
+  return false;
+}
+
+}  // namespace
+
+// Whether gemv_flow takes a job, and how; asked after the row-per-wave kernels of one row of x.  Time over that of the
+// kernels which would run instead, on 260 random jobs (m 1 .. 16, n 512 .. 32000, k 512 .. 14336, all types, widths and
+// groups of 32, 64, 128, weights from HBM):
+//   several linears                                       0.88 (one row of x and more than 48 rows a block: 1.05)
+//   one linear of 9 to 16 rows of x                       0.88
+//   one linear of up to 8, more than 8 rows a block       0.93 (0.78 to 1.08)
+//   gated units of 9 to 16 rows of x                      0.94 (0.57 where x has to pass gemv_w4p_f16_glu in parts)
+//   gated units of up to 8 on one tile, or two that are   0.90 (0.71 to 1.02)
+//   filled to three quarters
+// and where it is not the faster one:
+//   more than one round of blocks                         1.0 to 1.25
+//   blocks of up to 8 rows, up to 8 rows of x             1.0 to 1.28 (half of every tile is nobody's)
+//   other gated units of up to 8 rows of x                1.03 (to 1.13; gemv_ring's 8-row tiles), on fp16 4-bit groups
+//                                                         of whole chunks and up to 4 rows 1.02 (gemv_w4p_f16_glu)
+//   one linear of up to 4 rows of x on fp16 4-bit groups  1.06 to 1.14 (gemv_w4s_f16)
+//   of whole chunks, up to 16 rows a block
+//   bf16 4-bit, more than 64 rows a block                 1.02: bound by the expansion either way
+// On 149 other jobs: 0.94, 6 more than 3 % longer, 1.13 at worst (8 x 2 x 3584 x 1280 fp16 4-bit with a zero point).
+bool gemv_flow_choice(const LinearJob& job, FlowPlan* plan) {
+  const LinearArgs& a = job.pr[0];
+  for (int i = 0; i < job.count; ++i) {
+    const LinearArgs& b = job.pr[i];
+    if (!rows_supported(b) || b.t_dtype != a.t_dtype || b.bits != a.bits || b.w_signed != a.w_signed
+        || b.symmetric != a.symmetric || b.group_size != a.group_size || b.m != a.m || b.k != a.k) {
+      return false;
+    }
+  }
+  int64_t rows = 0;  // of a block
+  for (int i = 0; i < (job.glu ? 1 : job.count); ++i) rows += job.pr[i].n;
+  rows = (rows + 255) / 256;
+  const bool bf16_4 = a.t_dtype == OFQ_BF16 && a.bits == 4;
+  const bool late = a.t_dtype == OFQ_F16 && a.bits == 4 && a.symmetric && a.w_signed && a.group_size % 128 == 0;
+  if (job.glu) {
+    if (rows > 48) return false;
+    if (a.m <= 8 && !(rows <= 16 || (rows >= 25 && rows <= 32) || (rows >= 44 && a.bits == 8))) return false;
+    if (a.m <= 4 && late) return false;
+  } else if (job.count > 1) {
+    if (rows > 80 || (rows > 48 && a.m == 1)) return false;
+  } else {
+    if (rows > (a.m > 8 || bf16_4 ? 64 : 96) || (a.m <= 8 && rows <= 8)) return false;
+    if (late && a.m <= 4 && rows <= 16) return false;
+  }
+  return flow_plan(job, plan);
+}
+
+namespace {
+
+int launch_flow(hipStream_t st, const LinearJob& job) {
+  FlowPlan plan;
+  if (!gemv_flow_choice(job, &plan)) return OFQ_ERR_UNSUPPORTED;
+  const bool four = job.pr[0].bits == 4;
+  if (job.pr[0].t_dtype == OFQ_BF16) {
+    return four ? launch_gemv_flow_bf16_b4(st, job, plan) : launch_gemv_flow_bf16_b8(st, job, plan);
+  }
+  return four ? launch_gemv_flow_f16_b4(st, job, plan) : launch_gemv_flow_f16_b8(st, job, plan);
 }
 
 }  // namespace
@@ -947,9 +1051,13 @@ int launch_gemv_glu(hipStream_t st, const LinearArgs& a, const LinearArgs& g, vo
   int rc = launch_gemv_m1_glu(st, a, g, y, act);
   if (rc != OFQ_ERR_UNSUPPORTED) return rc;
   if (g.n != a.n || g.k != a.k || g.m != a.m || g.x != a.x) return OFQ_ERR_UNSUPPORTED;
+  const LinearArgs both[2] = {a, g};
+  {
+    const int rc = launch_flow(st, LinearJob{both, 2, true, y, act});
+    if (rc != OFQ_ERR_UNSUPPORTED) return rc;
+  }
   rc = launch_w4p_glu(st, a, g, y, act);
   if (rc != OFQ_ERR_UNSUPPORTED) return rc;
-  const LinearArgs both[2] = {a, g};
   return launch_ring(st, LinearJob{both, 2, true, y, act});
 }
 
@@ -970,6 +1078,10 @@ int launch_gemv_grouped(hipStream_t st, const LinearArgs* pr, int count) {
       return OFQ_ERR_UNSUPPORTED;
     }
     all_w4p = all_w4p && w4p_supported(b);
+  }
+  {
+    const int rc = launch_flow(st, LinearJob{pr, count, false, nullptr, 0});
+    if (rc != OFQ_ERR_UNSUPPORTED) return rc;
   }
   if (all_w4p) {
     const int rc = launch_w4p_grouped(st, pr, count);
@@ -1153,6 +1265,10 @@ int launch_gemv_wq(hipStream_t st, const LinearArgs& a) {
   }
   if (gemv_m1_any_supported(a)) {
     const int rc = launch_gemv_m1_any(st, a);
+    if (rc != OFQ_ERR_UNSUPPORTED) return rc;
+  }
+  {
+    const int rc = launch_flow(st, LinearJob{&a, 1, false, nullptr, 0});
     if (rc != OFQ_ERR_UNSUPPORTED) return rc;
   }
   if (w4s_supported(a)) {

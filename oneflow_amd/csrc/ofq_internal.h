@@ -123,6 +123,16 @@ struct RingPlan {
 bool gemv_ring_choice(const LinearJob& job, RingPlan* plan);
 int launch_gemv_ring_f16(hipStream_t st, const LinearJob& job, const RingPlan& plan);
 int launch_gemv_ring_bf16(hipStream_t st, const LinearJob& job, const RingPlan& plan);
+// The kernel whose waves share nothing (gemv_flow.h), up to 16 rows of x
+struct FlowPlan {
+  int grid, rows_per_block, mx, tl, nw;
+  size_t lds;
+};
+bool gemv_flow_choice(const LinearJob& job, FlowPlan* plan);
+int launch_gemv_flow_f16_b4(hipStream_t st, const LinearJob& job, const FlowPlan& plan);
+int launch_gemv_flow_f16_b8(hipStream_t st, const LinearJob& job, const FlowPlan& plan);
+int launch_gemv_flow_bf16_b4(hipStream_t st, const LinearJob& job, const FlowPlan& plan);
+int launch_gemv_flow_bf16_b8(hipStream_t st, const LinearJob& job, const FlowPlan& plan);
 // gemv_rows_mt (gemv_rows.h), 17 to 64 rows of x
 struct RowsMtPlan {
   int grid, rows_per_block, panel_chunks, panel_groups;
