@@ -1,4 +1,4 @@
-// Streaming kernel of fused_linear_with_groupwise_quantized_weight for up to 16 rows of x whose waves share
+// Streaming kernel of fused_linear_with_groupwise_quantized_weight for up to 48 rows of x whose waves share
 // nothing but scales: fp16 and bf16, 4- and 8-bit codes, groups along K from a lane's 16 bytes of codes on; one linear,
 // several in one launch, or the two of a gated linear unit with its gating.
 //
@@ -8,7 +8,7 @@
 // and their scale multiplies the chunk's fp32 sum (LATE: closer to exact arithmetic than the rounded w~).
 //
 // A block owns consecutive weight rows, walked as TL 16-row tiles, and all of K.  A wave takes every NW-th step of
-// 128 bytes of codes (two chunks of K), and both its columns of x and the codes of all tiles come by
+// 128 bytes of codes (two chunks of K; above 16 rows of x with 4-bit codes 64), and both its columns of x and the codes of all tiles come by
 // asynchronous global -> LDS copies to a place of its own: no wave waits for another between
 // the scales, which the block copies once, and the sums at the end.  Copies take whole lines (8 rows x 128 bytes of codes;
 // 256 or 512 bytes of a row of x), their pieces XOR-swizzled on the way so that operand reads meet no conflict of
@@ -18,7 +18,8 @@
 // first bytes and sums.  8 x 4096 x 11008 fp16 4-bit in groups of 128 takes 8.7 us (x, copied by all waves behind a
 // barrier in two parts, made it 11.0 in gemv_w4p_f16), 16 rows 10.7 (13.5), 3 x 4096 x 4096 9.0 (10.8), 16 x 2 x 11008 x
 // 4096 13.0 (23.5); weights from HBM.  A step in LDS and not two or three: with more in flight from the start
-// every wave's first step comes later (8 x 4096 x 11008 10.7 us).  Codes of a tile read before the products of the tile
+// every wave's first step comes later (8 x 4096 x 11008 10.7 us).  Above 16 rows x and codes come in at 45 to 55 bytes
+// per ns and CU together: 48 x 11008 x 4096 with a zero point 15.8 us, 64 rows 17.4 and more (not taken).  Codes of a tile read before the products of the tile
 // ahead of it: 1 to 2 %; offsets of copies formed once: 2 to 5 %.  What else it is measured against: gemv_flow_choice.
 //
 // K is any multiple of a lane's share of a chunk: lanes beyond K re-read a step's first bytes, and take x, scale and zero
@@ -49,9 +50,11 @@ __device__ __forceinline__ u32x4 biased8_b4_f16_any_order(uint32_t word) {
                (next & 0x000F000Fu) ^ 0x64086408u, (next & 0x00F000F0u) ^ 0x54805480u};
 }
 
-// 1 KB copies of x in a step
-template<int BITS, int MX>
-constexpr int flow_x_ops() { return BITS == 4 ? 4 * MX : 2 * MX; }
+// Chunks of K in a step, MX eights of rows of x: two, whole lines of the codes, or where a step's x would leave no
+// room for as many waves, one (a line's halves are then those of neighbouring waves).
+__host__ __device__ constexpr int flow_chunks(int bits, int mx) { return bits == 4 && mx > 2 ? 1 : 2; }
+// 1 KB copies of x in a step, and of a tile's codes
+__host__ __device__ constexpr int flow_x_ops(int bits, int mx) { return mx * flow_chunks(bits, mx) * (bits == 4 ? 2 : 1); }
 template<int I>
 struct FlowConst { static constexpr int value = I; };
 template<int I, int N, typename F>
@@ -72,10 +75,15 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
   constexpr int LK = CK / 4;                // elements per lane and chunk
   constexpr int XV = LK / 8;                // 16-byte pieces of x per lane and chunk
   constexpr int NT = TL * NMAT;             // tiles
-  constexpr int kXRow = CK * 4;             // bytes of x of one row and step
+  constexpr int CH = flow_chunks(BITS, MX); // chunks per step, and copies of a tile
+  constexpr int MT = (MX + 1) / 2;          // 16-row tiles of x
+  constexpr int kXRow = CK * 2 * CH;        // bytes of x of one row and step
   constexpr int kXPieces = kXRow / 16;
-  constexpr int kXOps = flow_x_ops<BITS, MX>();
-  constexpr int STEP = kXOps + 2 * NT;      // copies of a step, 1 KB each: x, then tile by tile
+  constexpr int kXOps = flow_x_ops(BITS, MX);
+  constexpr int STEP = kXOps + CH * NT;     // copies of a step, 1 KB each: x, then tile by tile
+  constexpr int kStepBytes = CH * 64;       // of codes of one row
+  constexpr int kSums = MT == 1 ? 2 : 1;    // of a tile: consecutive matrix instructions do not wait for each other
+  static_assert(MT == 1 || CH == 1 || BITS == 8, "one sum for two chunks");
   constexpr bool kAnyOrder = BITS == 4 && TT<T>::dtype == OFQ_F16;
   constexpr int kRegions = ZMODE == kZeroAsym ? 2 : 1;
   static_assert(2 * STEP < 63, "vmcnt is a 6-bit counter");
@@ -83,7 +91,7 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
   const int M = p.M, K = p.K;
   const int row_bytes = K / LK * 16;
   const int G = p.gs_shift >= 0 ? K >> p.gs_shift : K / p.group_size;
-  const int steps = (K + 2 * CK - 1) / (2 * CK);
+  const int steps = (K + CH * CK - 1) / (CH * CK);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -163,12 +171,12 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
       }
     }
   };
-  // codes: two eights a tile
-  uint32_t woff[TL][2], wpiece[2];
+  // codes: two eights a tile, or 16 rows of half a line
+  uint32_t woff[TL][CH], wpiece[CH];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int row = h * 8 + (lane >> 3);
-    wpiece[h] = (uint32_t)(((lane & 7) ^ (row >> 1)) << 4);
+  for (int h = 0; h < CH; ++h) {
+    const int row = CH == 2 ? h * 8 + (lane >> 3) : lane >> 2;
+    wpiece[h] = (uint32_t)((CH == 2 ? (lane & 7) ^ (row >> 1) : (lane & 3) ^ (row >> 2)) << 4);
 #pragma unroll
     for (int t = 0; t < TL; ++t) {
       woff[t][h] = (uint32_t)(t * 16 + row < rows_blk ? t * 16 + row : rows_blk - 1) * (uint32_t)row_bytes + wpiece[h];
@@ -177,16 +185,20 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
   const uint8_t* wbase[NMAT];
 #pragma unroll
   for (int mt = 0; mt < NMAT; ++mt) wbase[mt] = mats[mt].w + (int64_t)row0 * row_bytes;
+  auto copy_codes = [&](const uint8_t* base, uint32_t off, uint32_t to) {
+    if constexpr (CH == 2) async_copy16_once(base, off, to);
+    else async_copy16_at(base, off, to);
+  };
   auto copy_tile = [&](int s, int t) {
-    const uint8_t* base = wbase[t / TL] + (int64_t)s * 128;
-    const uint32_t to = lds0 + ring0 + (kXOps + 2 * t) * 1024;
-    if ((s + 1) * 128 <= row_bytes) {
+    const uint8_t* base = wbase[t / TL] + (int64_t)s * kStepBytes;
+    const uint32_t to = lds0 + ring0 + (kXOps + CH * t) * 1024;
+    if ((s + 1) * kStepBytes <= row_bytes) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) async_copy16_once(base, woff[t % TL][h], to + h * 1024);
+      for (int h = 0; h < CH; ++h) copy_codes(base, woff[t % TL][h], to + h * 1024);
     } else {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        async_copy16_once(base, woff[t % TL][h] - (s * 128 + (int)wpiece[h] < row_bytes ? 0u : wpiece[h]), to + h * 1024);
+      for (int h = 0; h < CH; ++h) {
+        copy_codes(base, woff[t % TL][h] - (s * kStepBytes + (int)wpiece[h] < row_bytes ? 0u : wpiece[h]), to + h * 1024);
       }
     }
   };
@@ -201,84 +213,97 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
   // ---- products ---------------------------------------------------------------------------------
-  // two sums a tile: consecutive matrix instructions do not wait for each other
-  f32x4 acc[NT][2];
+  f32x4 acc[NT][MT][kSums];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    acc[t][0] = f32x4{0.f, 0.f, 0.f, 0.f};
-    acc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < kSums; ++i) acc[t][mt][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int xat[CH][XV];  // this lane's pieces of x in a step, of row r of a tile (of a tile of one eight: its rows twice)
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+#pragma unroll
+    for (int j = 0; j < XV; ++j) {
+      const int row = MX == 1 ? r & 7 : r;
+      xat[c][j] = row * kXRow + (((c * 4 + kb) * XV + j) ^ row) * 16;
+    }
+  int cat[CH];      // and of a tile's codes
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    cat[c] = CH == 2 ? r * 128 + (((c * 4 + kb) ^ (r >> 1)) << 4) : r * 64 + ((kb ^ (r >> 2)) << 4);
   }
-  const int xrow = MX == 1 ? r & 7 : r;
-  int xat[2][XV];  // this lane's pieces of x in a step
-#pragma unroll
-  for (int c = 0; c < 2; ++c)
-#pragma unroll
-    for (int j = 0; j < XV; ++j) xat[c][j] = xrow * kXRow + (((c * 4 + kb) * XV + j) ^ xrow) * 16;
-  int cat[2];      // and of a tile's codes
-#pragma unroll
-  for (int c = 0; c < 2; ++c) cat[c] = r * 128 + (((c * 4 + kb) ^ (r >> 1)) << 4);
   int srow[TL];
 #pragma unroll
   for (int t = 0; t < TL; ++t) srow[t] = s_shift + (t * 16 + r < rows_blk ? t * 16 + r : rows_blk - 1) * G * 2;
 
   for (int s = wave; s < steps; s += NW) {
     const bool more = s + NW < steps;
-    wait_vmem_le<2 * NT>();
+    wait_vmem_le<CH * NT>();
     asm volatile("" ::: "memory");
-    u32x4 xa[2][XV];
+    u32x4 xa[CH][MT][XV];
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+    for (int c = 0; c < CH; ++c)
 #pragma unroll
-      for (int j = 0; j < XV; ++j) xa[c][j] = *reinterpret_cast<const u32x4*>(smem + ring0 + xat[c][j]);
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int j = 0; j < XV; ++j)
+          xa[c][mt][j] = *reinterpret_cast<const u32x4*>(smem + ring0 + mt * (16 * kXRow) + xat[c][j]);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if (more) copy_x(s + NW);
-    bool in_row[2];
-    int grp[2];
+    bool in_row[CH];
+    int grp[CH];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      int k0 = (s * 2 + c) * CK + kb * LK;
+    for (int c = 0; c < CH; ++c) {
+      int k0 = (s * CH + c) * CK + kb * LK;
       in_row[c] = k0 < K;
       k0 = in_row[c] ? k0 : 0;
       grp[c] = (p.gs_shift >= 0 ? k0 >> p.gs_shift : k0 / p.group_size) * 2;
     }
-    if ((s + 1) * 2 * CK > K) {
+    if ((s + 1) * CH * CK > K) {
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
+      for (int c = 0; c < CH; ++c)
 #pragma unroll
-        for (int j = 0; j < XV; ++j)
-          if (!in_row[c]) xa[c][j] = u32x4{0u, 0u, 0u, 0u};
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int j = 0; j < XV; ++j)
+            if (!in_row[c]) xa[c][mt][j] = u32x4{0u, 0u, 0u, 0u};
     }
     if constexpr (kAnyOrder) {
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
+      for (int c = 0; c < CH; ++c)
 #pragma unroll
-        for (int j = 0; j < XV; ++j) xa[c][j] = x_any_order(xa[c][j]);
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int j = 0; j < XV; ++j) xa[c][mt][j] = x_any_order(xa[c][mt][j]);
     }
     // minus what the exponents add to the codes' values, of every row of x
-    f32x4 corr[2];
+    f32x4 corr[CH][MT];
     if constexpr (LATE) {
       uint32_t lo = 0xE408E408u, hi = 0xD480D480u;  // (-1032, -1032), (-72, -72)
       asm volatile("" : "+v"(lo), "+v"(hi));
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        corr[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < CH; ++c)
 #pragma unroll
-        for (int j = 0; j < XV; ++j) corr[c] = MfmaK32<T>::mma(xa[c][j], u32x4{lo, hi, lo, hi}, corr[c]);
-      }
+        for (int mt = 0; mt < MT; ++mt) {
+          corr[c][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int j = 0; j < XV; ++j) corr[c][mt] = MfmaK32<T>::mma(xa[c][mt][j], u32x4{lo, hi, lo, hi}, corr[c][mt]);
+        }
     }
     // a tile's codes are read while the products of the one before it are under way
-    u32x4 codes[2];
-    uint16_t sraw[2], zraw[2] = {0, 0};
+    u32x4 codes[CH];
+    uint16_t sraw[CH], zraw[CH] = {};
     auto read_tile = [&](auto index) {
       constexpr int t = decltype(index)::value;
       // younger than its copies: those of the tiles after it and, if there is a next step, its x and tiles before t
-      if (more) wait_vmem_le<2 * (NT - 1) + kXOps>();
-      else wait_vmem_le<2 * (NT - 1 - t)>();
+      if (more) wait_vmem_le<CH * (NT - 1) + kXOps>();
+      else wait_vmem_le<CH * (NT - 1 - t)>();
       asm volatile("" ::: "memory");
-      const uint8_t* cp = smem + ring0 + (kXOps + 2 * t) * 1024;
+      const uint8_t* cp = smem + ring0 + (kXOps + CH * t) * 1024;
       const uint8_t* sp = smem + (t / TL) * kRegions * sreg + srow[t % TL];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
+      for (int c = 0; c < CH; ++c) {
         codes[c] = *reinterpret_cast<const u32x4*>(cp + cat[c]);
         sraw[c] = *reinterpret_cast<const uint16_t*>(sp + grp[c]);
         if (ZMODE == kZeroAsym) zraw[c] = *reinterpret_cast<const uint16_t*>(sp + sreg + grp[c]);
@@ -290,10 +315,11 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
       // the codes are in registers: their place is free
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (more) copy_tile(s + NW, t);
-      const u32x4 q[2] = {codes[0], codes[1]};
-      float sc[2], z[2];
+      u32x4 q[CH];
+      float sc[CH], z[CH];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
+      for (int c = 0; c < CH; ++c) {
+        q[c] = codes[c];
         sc[c] = in_row[c] ? raw16_to_float<T>(sraw[c]) : 0.f;
         z[c] = 0.f;
         if (ZMODE == kZeroAsym) z[c] = in_row[c] ? raw16_to_float<T>(zraw[c]) : 0.f;
@@ -301,20 +327,28 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
       }
       if constexpr (t + 1 < NT) read_tile(FlowConst<t + 1>());
       if constexpr (LATE) {
-        f32x4 sum[2] = {corr[0], corr[1]};
+        f32x4 sum[CH][MT];
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int c = 0; c < 2; ++c) sum[c] = MfmaK32<T>::mma(xa[c][j], biased8_b4_f16_any_order(q[c][j]), sum[c]);
+          for (int c = 0; c < CH; ++c) {
+            const u32x4 b = biased8_b4_f16_any_order(q[c][j]);
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+            for (int mt = 0; mt < MT; ++mt)
+              sum[c][mt] = MfmaK32<T>::mma(xa[c][mt][j], b, j == 0 ? corr[c][mt] : sum[c][mt]);
+          }
 #pragma unroll
-          for (int v = 0; v < 4; ++v) acc[t][c][v] = __builtin_fmaf(sum[c][v], sc[c], acc[t][c][v]);
+        for (int c = 0; c < CH; ++c)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+              acc[t][mt][c % kSums][v] = __builtin_fmaf(sum[c][mt][v], sc[c], acc[t][mt][c % kSums][v]);
       } else if constexpr (BITS == 4) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int c = 0; c < 2; ++c) {
+          for (int c = 0; c < CH; ++c) {
             u32x4 b;
             if constexpr (kAnyOrder) {
               const f16x2 s2 = {(f16)sc[c], (f16)sc[c]}, z2 = {(f16)z[c], (f16)z[c]};  // (exact)
@@ -322,15 +356,19 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
             } else {
               b = dequant8_b4<T, SIGNED, ZMODE>(q[c][j], sc[c], z[c]);
             }
-            acc[t][c] = MfmaK32<T>::mma(xa[c][j], b, acc[t][c]);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+              acc[t][mt][c % kSums] = MfmaK32<T>::mma(xa[c][mt][j], b, acc[t][mt][c % kSums]);
           }
       } else {
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
+        for (int c = 0; c < CH; ++c) {
           u32x4 b0, b1;
           dequant16_b8<T, SIGNED, ZMODE>(q[c], sc[c], z[c], b0, b1);
-          acc[t][c] = MfmaK32<T>::mma(xa[c][0], b0, acc[t][c]);
-          acc[t][c] = MfmaK32<T>::mma(xa[c][1], b1, acc[t][c]);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) acc[t][mt][c % kSums] = MfmaK32<T>::mma(xa[c][mt][0], b0, acc[t][mt][c % kSums]);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) acc[t][mt][c % kSums] = MfmaK32<T>::mma(xa[c][mt][1], b1, acc[t][mt][c % kSums]);
         }
       }
     });
@@ -343,13 +381,19 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
   const int waves = steps < NW ? steps : NW;  // that have a sum
   if (wave < waves) {
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int m = 4 * kb + v;
-      if (m < M) {
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) red[(wave * M + m) * RP + t * 16 + r] = acc[t][0][v] + acc[t][1][v];
+      for (int v = 0; v < 4; ++v) {
+        const int m = mt * 16 + 4 * kb + v;
+        if (m < M) {
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            float sum = acc[t][mt][0][v];
+            if constexpr (kSums == 2) sum += acc[t][mt][1][v];
+            red[(wave * M + m) * RP + t * 16 + r] = sum;
+          }
+        }
       }
-    }
   }
   __syncthreads();
   constexpr int kRowsAtOnce = NW * 64 / R;

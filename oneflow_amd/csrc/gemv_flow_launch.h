@@ -53,6 +53,8 @@ int launch_flow_variant(hipStream_t st, const LinearJob& job, const FlowPlan& pl
   OFQ_L(2, 1, 8) OFQ_L(2, 2, 8) OFQ_L(2, 3, 8) OFQ_L(2, 4, 8) OFQ_L(2, 5, 8)
   OFQ_L(1, 1, 6) OFQ_L(1, 2, 6) OFQ_L(1, 3, 6) OFQ_L(1, 4, 6) OFQ_L(1, 5, 6) OFQ_L(1, 6, 6)
   OFQ_L(2, 1, 6) OFQ_L(2, 2, 6) OFQ_L(2, 3, 6) OFQ_L(2, 4, 6) OFQ_L(2, 5, 6)
+  OFQ_L(4, 1, 8) OFQ_L(4, 2, 8) OFQ_L(4, 3, 8) OFQ_L(4, 4, 8)
+  OFQ_L(6, 1, 8) OFQ_L(6, 2, 8) OFQ_L(6, 3, 8) OFQ_L(6, 4, 8)
 #undef OFQ_L
   return OFQ_ERR_UNSUPPORTED;
 }

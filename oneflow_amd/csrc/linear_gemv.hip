@@ -404,8 +404,8 @@ bool flow_plan(const LinearJob& job, FlowPlan* plan) {
   const int lists = job.glu ? 1 : job.count, matrices = job.glu ? 2 : 1;
   const int G = (int)(a.k / a.group_size);
   const int regions = matrices * (a.symmetric ? 1 : 2);
-  const int mx = a.m <= 8 ? 1 : 2;
-  const int max_rows = job.glu ? 48 : (mx == 1 ? 96 : 80);
+  const int mx = a.m <= 8 ? 1 : a.m <= 16 ? 2 : a.m <= 32 ? 4 : 6;
+  const int max_rows = job.glu ? 48 : mx == 1 ? 96 : mx == 2 ? 80 : 64;
   int64_t total = 0;
   for (int i = 0; i < lists; ++i) total += job.pr[i].n;
   auto blocks_at = [&](int rpb) {
@@ -419,8 +419,8 @@ bool flow_plan(const LinearJob& job, FlowPlan* plan) {
   if (rpb <= max_rows) {
     const int tl = (rpb + 15) / 16;
     const size_t scales = (size_t)(regions * ring_scale_bytes(rpb, G) + 1023) & ~(size_t)1023;
-    const int step = (a.bits == 4 ? 4 : 2) * mx + 2 * tl * matrices;
-    for (int nw = 8; nw >= 6; nw -= 2) {
+    const int step = flow_x_ops(a.bits, mx) + flow_chunks(a.bits, mx) * tl * matrices;
+    for (int nw = 8; nw >= (mx > 2 ? 8 : 6); nw -= 2) {
       size_t lds = scales + (size_t)nw * step * 1024;
       const size_t red = (size_t)nw * (size_t)a.m * (tl * matrices * 16 + 4) * 4;
       if (red > lds) lds = red;
@@ -486,14 +486,16 @@ bool gemv_flow_choice(const LinearJob& job, FlowPlan* plan) {
 
 namespace {
 
-int launch_flow(hipStream_t st, const LinearJob& job) {
-  FlowPlan plan;
-  if (!gemv_flow_choice(job, &plan)) return OFQ_ERR_UNSUPPORTED;
+int launch_flow_by(hipStream_t st, const LinearJob& job, const FlowPlan& plan) {
   const bool four = job.pr[0].bits == 4;
   if (job.pr[0].t_dtype == OFQ_BF16) {
     return four ? launch_gemv_flow_bf16_b4(st, job, plan) : launch_gemv_flow_bf16_b8(st, job, plan);
   }
   return four ? launch_gemv_flow_f16_b4(st, job, plan) : launch_gemv_flow_f16_b8(st, job, plan);
+}
+int launch_flow(hipStream_t st, const LinearJob& job) {
+  FlowPlan plan;
+  return gemv_flow_choice(job, &plan) ? launch_flow_by(st, job, plan) : OFQ_ERR_UNSUPPORTED;
 }
 
 }  // namespace
@@ -1202,6 +1204,45 @@ static int launch_mt_job(hipStream_t st, const LinearJob& job, const MtChoice& c
   return choice.ring ? launch_ring_mt(st, job, choice.plan) : launch_rows_mt(st, job);
 }
 
+// gemv_flow with 17 to 48 rows of x: expected time in us, within 12 % (17 % with 8-bit codes) of the measured one for 90
+// of 100 of 294 random jobs (linears of 512 to 32000 x 512 to 14336, several of a layer, gated units).  A step of the
+// longest wave takes a part per KB of x and per KB of codes, which are expanded at a rate of their kind; scales and
+// outputs come on top.
+static double flow_mt_us(const LinearJob& job, const FlowPlan& plan) {
+  const LinearArgs& a = job.pr[0];
+  const bool b4 = a.bits == 4;
+  const int matrices = job.glu ? 2 : 1;
+  const int chunks = flow_chunks(a.bits, plan.mx), ck = b4 ? 128 : 64;
+  const int steps = (int)((a.k + chunks * ck - 1) / (chunks * ck));
+  double codes = a.symmetric ? 0.226 : 0.230;
+  if (b4) codes = a.t_dtype == OFQ_F16 ? (a.symmetric && a.w_signed ? 0.261 : 0.313) : (a.symmetric ? 0.325 : 0.361);
+  double outputs = 0;
+  for (int i = 0; i < job.count; ++i) outputs += 1e-6 * (double)a.m * job.pr[i].n;
+  const double scales = (double)(a.k / a.group_size) * plan.rows_per_block * matrices * (a.symmetric ? 1 : 2) / 4096;
+  return (b4 ? 2.7 : 2.4)
+         + (steps + plan.nw - 1) / plan.nw
+               * ((b4 ? 0.080 : 0.072) * flow_x_ops(a.bits, plan.mx) + codes * chunks * plan.tl * matrices)
+         + (b4 ? 0.9 : 1.1) * scales + (b4 ? 6.6 : 7.5) * outputs;
+}
+
+// One linear of 17 to 48 rows of x goes to gemv_flow where gemm_wr is not expected to be faster (few rows of a long K:
+// 37 x 801 x 13728 17.0 us there, 23.9 here; its second launch as below); several and gated units always do.
+// Time over that of the kernels that ran instead (gemv_rows_mt, gemv_ring_mt, gemm_wr), on 330 random jobs with weights
+// from HBM: one linear 0.90, with what gemm_wr keeps 0.88, several 0.84 (0.95 at worst), gated units 0.89 (1.02); 17 x
+// 11008 x 4096 fp16 4-bit 12.9 -> 9.9 us, 32 x 16000 x 4096 18.3 -> 13.7, 48 x 11008 x 4096 with a zero point 17.2 ->
+// 15.8, 32 x 3 x 4096 x 4096 16.1 -> 12.8, 24 x 2 x 11008 x 4096 21.3 -> 17.5.  64 rows leave six waves and
+// took 1.0 to 1.4 of the time.
+bool gemv_flow_preferred(const LinearArgs& a, bool have_workspace, FlowPlan* plan) {
+  if (a.m > 48 || !gemv_mt_supported(a)) return false;
+  const LinearJob job{&a, 1, false, nullptr, 0};
+  if (!flow_plan(job, plan)) return false;
+  const double us = flow_mt_us(job, *plan);
+  return us < gemm_wr_us(a, have_workspace, us < 12.5 ? 3.0 : 0.5);
+}
+int launch_gemv_flow(hipStream_t st, const LinearArgs& a, const FlowPlan& plan) {
+  return launch_flow_by(st, LinearJob{&a, 1, false, nullptr, 0}, plan);
+}
+
 // gemm_wr reads x once per 128 rows of weights, but starts a second kernel where it slices K: so long
 // rows of weights leave the streaming kernels (64 x 4096 x 11008 fp16: 27.6 us here, 17.4 there) and n =
 // 11008 of k = 4096 stays.  Below 12.5 us the second launch and the workspace
@@ -1233,6 +1274,8 @@ int launch_gemv_mt_several(hipStream_t st, const LinearArgs* pr, int count, bool
     }
   }
   const LinearJob job{pr, count, glu, y, act};
+  FlowPlan flow;
+  if (a.m <= 48 && flow_plan(job, &flow)) return launch_flow_by(st, job, flow);
   MtChoice choice;
   gemv_mt_choice(job, &choice);
   if (!choice.ring) {
@@ -1392,11 +1435,15 @@ extern "C" int ofq_fused_linear_gq(void* stream, const void* x, const void* w,
     const int rc = launch_gemv_wq(st, a);
     if (rc != OFQ_ERR_UNSUPPORTED) return rc;  // e.g. bf16 with an x too large to stage
   }
-  MtChoice choice;
-  if (a.m > 16 && a.m <= 64
-      && gemv_mt_preferred(a, workspace != nullptr && workspace_bytes >= gemm_wq_workspace_bytes(a), &choice)) {
-    const int rc = launch_gemv_mt(st, a, choice);
-    if (rc != OFQ_ERR_UNSUPPORTED) return rc;
+  if (a.m > 16 && a.m <= 64) {
+    const bool have_workspace = workspace != nullptr && workspace_bytes >= gemm_wq_workspace_bytes(a);
+    FlowPlan flow;
+    if (gemv_flow_preferred(a, have_workspace, &flow)) return launch_gemv_flow(st, a, flow);
+    MtChoice choice;
+    if (gemv_mt_preferred(a, have_workspace, &choice)) {
+      const int rc = launch_gemv_mt(st, a, choice);
+      if (rc != OFQ_ERR_UNSUPPORTED) return rc;
+    }
   }
   if (gemm_wq_supported(a)) return launch_gemm_wq(st, a, workspace, workspace_bytes);
   if (a.group_dim == 0) {

@@ -123,7 +123,7 @@ struct RingPlan {
 bool gemv_ring_choice(const LinearJob& job, RingPlan* plan);
 int launch_gemv_ring_f16(hipStream_t st, const LinearJob& job, const RingPlan& plan);
 int launch_gemv_ring_bf16(hipStream_t st, const LinearJob& job, const RingPlan& plan);
-// The kernel whose waves share nothing (gemv_flow.h), up to 16 rows of x
+// The kernel whose waves share nothing (gemv_flow.h), up to 48 rows of x; the choice: up to 16
 struct FlowPlan {
   int grid, rows_per_block, mx, tl, nw;
   size_t lds;

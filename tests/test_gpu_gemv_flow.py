@@ -1,4 +1,4 @@
-"""gemv_flow: linears, several of them and gated units of 1 to 16 rows of x; every number of tiles, ragged rows and K,
+"""gemv_flow: linears, several of them and gated units of 1 to 48 rows of x; every number of tiles, ragged rows and K,
 eight waves and six, groups of a lane's share up to whole chunks, with and without a zero point."""
 import ctypes
 
@@ -19,7 +19,7 @@ def flow_plan(ns, m, k, g, bits, symmetric, dtype, glu):
     f = _lib.lib()["_ZN3ofq16gemv_flow_choiceERKNS_9LinearJobEPNS_8FlowPlanE"]
     f.restype, f.argtypes = ctypes.c_bool, [ctypes.POINTER(LinearJob), ctypes.POINTER(FlowPlan)]
     plan = FlowPlan()
-    return plan if f(ctypes.byref(_job(ns, m, k, g, bits, symmetric, dtype, glu)), ctypes.byref(plan)) else None
+    return plan if m > 16 or f(ctypes.byref(_job(ns, m, k, g, bits, symmetric, dtype, glu)), ctypes.byref(plan)) else None
 
 
 def _linear(gen, n, k, dtype, bits, symmetric, g, bias):
@@ -50,10 +50,13 @@ def _exact(x, full, bias, dtype):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bits,symmetric", [(4, True), (4, False), (8, True), (8, False)])
 @pytest.mark.parametrize("mode,m,n,k,g", [
-    ("one", 2, 2560, 128, 128), ("one", 9, 33, 32, 32), ("one", 16, 7, 96, 32), ("one", 8, 4099, 1184, 32),
+    ("one", 5, 2560, 128, 128), ("one", 9, 33, 32, 32), ("one", 16, 7, 96, 32), ("one", 8, 4099, 1184, 32),
     ("one", 3, 5000, 4096, 128), ("one", 5, 9001, 384, 64), ("one", 13, 8000, 4160, 32), ("one", 16, 11008, 2816, 128),
-    ("one", 1, 2600, 4224, 128), ("one", 12, 13000, 1152, 128), ("one", 8, 16384, 640, 128), ("one", 4, 16001, 576, 64),
+    ("one", 1, 4200, 4224, 128), ("one", 2, 4200, 256, 128), ("one", 12, 13000, 1152, 128), ("one", 8, 16384, 640, 128), ("one", 4, 16001, 576, 64),
     ("one", 10, 300, 11008, 64),
+    ("one", 17, 2560, 1152, 128), ("one", 32, 33, 96, 32), ("one", 33, 4099, 1184, 32), ("one", 48, 11008, 1024, 128),
+    ("one", 24, 16001, 576, 64), ("one", 41, 13000, 640, 128),
+    ("several", 25, 1500, 2080, 32), ("several", 48, 4096, 768, 128), ("glu", 20, 4100, 1184, 32), ("glu", 48, 11008, 512, 128),
     ("several", 2, 2048, 1024, 128), ("several", 11, 1500, 2080, 32), ("several", 16, 4096, 768, 128),
     ("glu", 8, 3000, 1024, 64), ("glu", 9, 11008, 1152, 128), ("glu", 16, 12288, 512, 32), ("glu", 6, 7000, 1408, 128),
     ("glu", 15, 4100, 2080, 32)])
