@@ -4,8 +4,9 @@
 //
 // w~ = T(T(q) * s) + z with the reference's roundings
 // (oneflow/user/kernels/groupwise_quantization_kernels.cu:73-117, :582-642), products and sums in fp32 in
-// the matrix core, one rounding of the result; symmetric 4-bit fp16 codes in groups of whole chunks meet x as they are
-// and their scale multiplies the chunk's fp32 sum (LATE: closer to exact arithmetic than the rounded w~).
+// the matrix core, one rounding of the result; up to 16 rows of x of several linears and gated units, symmetric 4-bit
+// fp16 codes in groups of whole chunks meet x as they are and their scale multiplies the chunk's fp32 sum (LATE: closer
+// to exact arithmetic than the rounded w~, and what gemv_w4p_f16 does with them).
 //
 // A block owns consecutive weight rows, walked as TL 16-row tiles, and all of K.  A wave takes every NW-th step of
 // 128 bytes of codes (two chunks of K; above 16 rows of x with 4-bit codes 64), and both its columns of x and the codes of all tiles come by
@@ -15,9 +16,8 @@
 // banks.  The next step's x and tiles are requested one by one, as the present ones have been read into registers.
 //
 // What bounds it: the expansion of the codes and the stream of them, two waves a SIMD, behind about 2.5 us of launch,
-// first bytes and sums.  8 x 4096 x 11008 fp16 4-bit in groups of 128 takes 8.7 us (x, copied by all waves behind a
-// barrier in two parts, made it 11.0 in gemv_w4p_f16), 16 rows 10.7 (13.5), 3 x 4096 x 4096 9.0 (10.8), 16 x 2 x 11008 x
-// 4096 13.0 (23.5); weights from HBM.  A step in LDS and not two or three: with more in flight from the start
+// first bytes and sums.  8 rows of x of 3 x 4096 x 4096 fp16 4-bit in groups of 128 take 9.0 us (10.8 in
+// gemv_w4p_f16_grouped), 16 of 2 x 11008 x 4096 13.0 (23.5); weights from HBM.  A step in LDS and not two or three: with more in flight from the start
 // every wave's first step comes later (8 x 4096 x 11008 10.7 us).  Above 16 rows x and codes come in at 45 to 55 bytes
 // per ns and CU together: 48 x 11008 x 4096 with a zero point 15.8 us, 64 rows 17.4 and more (not taken).  Codes of a tile read before the products of the tile
 // ahead of it: 1 to 2 %; offsets of copies formed once: 2 to 5 %.  What else it is measured against: gemv_flow_choice.
@@ -428,11 +428,11 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
   }
 }
 
-template<typename T, int BITS, bool SIGNED, int ZMODE, bool LATE, int MX, int TL, int NW>
+template<typename T, int BITS, bool SIGNED, int ZMODE, int MX, int TL, int NW>
 __global__ void __launch_bounds__(NW * 64)
 gemv_flow(const uint16_t* __restrict__ x, RowsMat mat, int N, FlowArgs p) {
   const RowsMat mats[1] = {mat};
-  gemv_flow_body<T, BITS, SIGNED, ZMODE, LATE, MX, TL, 1, NW>((int)blockIdx.x, x, mats, N, nullptr, 0, p);
+  gemv_flow_body<T, BITS, SIGNED, ZMODE, false, MX, TL, 1, NW>((int)blockIdx.x, x, mats, N, nullptr, 0, p);
 }
 // Several linears of the same m, k and quantisation: the grid is the concatenation of their blocks.
 template<typename T, int BITS, bool SIGNED, int ZMODE, bool LATE, int MX, int TL, int NW>

@@ -36,8 +36,10 @@ int launch_flow_inst(hipStream_t st, const LinearJob& job, const FlowPlan& plan)
     GemvGroup g{};
     fill_group(g, job.pr, job.count, plan.rows_per_block);
     kern<<<plan.grid, NW * 64, plan.lds, st>>>(g, p);
+  } else if constexpr (LATE) {
+    return OFQ_ERR_UNSUPPORTED;  // (gemv_flow_choice)
   } else {
-    auto kern = gemv_flow<T, BITS, SIGNED, ZMODE, LATE, MX, TL, NW>;
+    auto kern = gemv_flow<T, BITS, SIGNED, ZMODE, MX, TL, NW>;
     if (!ofq_allow_dynamic_lds(reinterpret_cast<const void*>(kern), 160 * 1024, allowed)) return OFQ_ERR_LAUNCH;
     kern<<<plan.grid, NW * 64, plan.lds, st>>>(x, rows_mat(a), (int)a.n, p);
   }
@@ -53,8 +55,10 @@ int launch_flow_variant(hipStream_t st, const LinearJob& job, const FlowPlan& pl
   OFQ_L(2, 1, 8) OFQ_L(2, 2, 8) OFQ_L(2, 3, 8) OFQ_L(2, 4, 8) OFQ_L(2, 5, 8)
   OFQ_L(1, 1, 6) OFQ_L(1, 2, 6) OFQ_L(1, 3, 6) OFQ_L(1, 4, 6) OFQ_L(1, 5, 6) OFQ_L(1, 6, 6)
   OFQ_L(2, 1, 6) OFQ_L(2, 2, 6) OFQ_L(2, 3, 6) OFQ_L(2, 4, 6) OFQ_L(2, 5, 6)
-  OFQ_L(4, 1, 8) OFQ_L(4, 2, 8) OFQ_L(4, 3, 8) OFQ_L(4, 4, 8)
-  OFQ_L(6, 1, 8) OFQ_L(6, 2, 8) OFQ_L(6, 3, 8) OFQ_L(6, 4, 8)
+  if constexpr (!LATE) {
+    OFQ_L(4, 1, 8) OFQ_L(4, 2, 8) OFQ_L(4, 3, 8) OFQ_L(4, 4, 8)
+    OFQ_L(6, 1, 8) OFQ_L(6, 2, 8) OFQ_L(6, 3, 8) OFQ_L(6, 4, 8)
+  }
 #undef OFQ_L
   return OFQ_ERR_UNSUPPORTED;
 }
@@ -64,7 +68,7 @@ int launch_flow_t(hipStream_t st, const LinearJob& job, const FlowPlan& plan) {
   const LinearArgs& a = job.pr[0];
   const int zmode = !a.symmetric ? kZeroAsym : (a.w_signed ? kZeroNone : kZeroSymU);
   if constexpr (BITS == 4 && TT<T>::dtype == OFQ_F16) {
-    if (zmode == kZeroNone && a.group_size % 128 == 0) {
+    if (zmode == kZeroNone && a.group_size % 128 == 0 && a.m <= 16) {
       return launch_flow_variant<T, BITS, true, kZeroNone, true>(st, job, plan);
     }
   }

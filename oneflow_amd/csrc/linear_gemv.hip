@@ -453,10 +453,9 @@ bool flow_plan(const LinearJob& job, FlowPlan* plan) {
 //   blocks of up to 8 rows, up to 8 rows of x             1.0 to 1.28 (half of every tile is nobody's)
 //   other gated units of up to 8 rows of x                1.03 (to 1.13; gemv_ring's 8-row tiles), on fp16 4-bit groups
 //                                                         of whole chunks and up to 4 rows 1.02 (gemv_w4p_f16_glu)
-//   one linear of up to 4 rows of x on fp16 4-bit groups  1.06 to 1.14 (gemv_w4s_f16)
-//   of whole chunks, up to 16 rows a block
 //   bf16 4-bit, more than 64 rows a block                 1.02: bound by the expansion either way
-// On 149 other jobs: 0.94, 6 more than 3 % longer, 1.13 at worst (8 x 2 x 3584 x 1280 fp16 4-bit with a zero point).
+// One linear of fp16 4-bit groups of whole chunks stays with gemv_w4p_f16 whatever the time (8 x 4096 x 11008 11.0 us
+// there, 8.7 here): a tile-major copy of its weight is read by that kernel, and the two calls give the same bits.
 bool gemv_flow_choice(const LinearJob& job, FlowPlan* plan) {
   const LinearArgs& a = job.pr[0];
   for (int i = 0; i < job.count; ++i) {
@@ -478,8 +477,7 @@ bool gemv_flow_choice(const LinearJob& job, FlowPlan* plan) {
   } else if (job.count > 1) {
     if (rows > 80 || (rows > 48 && a.m == 1)) return false;
   } else {
-    if (rows > (a.m > 8 || bf16_4 ? 64 : 96) || (a.m <= 8 && rows <= 8)) return false;
-    if (late && a.m <= 4 && rows <= 16) return false;
+    if (w4p_supported(a) || rows > (a.m > 8 || bf16_4 ? 64 : 96) || (a.m <= 8 && rows <= 8)) return false;
   }
   return flow_plan(job, plan);
 }
@@ -1228,9 +1226,8 @@ static double flow_mt_us(const LinearJob& job, const FlowPlan& plan) {
 // One linear of 17 to 48 rows of x goes to gemv_flow where gemm_wr is not expected to be faster (few rows of a long K:
 // 37 x 801 x 13728 17.0 us there, 23.9 here; its second launch as below); several and gated units always do.
 // Time over that of the kernels that ran instead (gemv_rows_mt, gemv_ring_mt, gemm_wr), on 330 random jobs with weights
-// from HBM: one linear 0.90, with what gemm_wr keeps 0.88, several 0.84 (0.95 at worst), gated units 0.89 (1.02); 17 x
-// 11008 x 4096 fp16 4-bit 12.9 -> 9.9 us, 32 x 16000 x 4096 18.3 -> 13.7, 48 x 11008 x 4096 with a zero point 17.2 ->
-// 15.8, 32 x 3 x 4096 x 4096 16.1 -> 12.8, 24 x 2 x 11008 x 4096 21.3 -> 17.5.  64 rows leave six waves and
+// from HBM: one linear 0.90, with what gemm_wr keeps 0.88, several 0.84 (0.95 at worst), gated units 0.89 (1.02); 24 x
+// 11008 x 4096 fp16 4-bit in groups of 32 16.6 -> 13.6 us, 48 x 11008 x 4096 with a zero point 17.2 -> 15.8.  64 rows leave six waves and
 // took 1.0 to 1.4 of the time.
 bool gemv_flow_preferred(const LinearArgs& a, bool have_workspace, FlowPlan* plan) {
   if (a.m > 48 || !gemv_mt_supported(a)) return false;
