@@ -4,7 +4,7 @@
 //
 // w~ = T(T(q) * s) + z with the reference's roundings
 // (oneflow/user/kernels/groupwise_quantization_kernels.cu:73-117, :582-642), products and sums in fp32 in
-// the matrix core, one rounding of the result; up to 16 rows of x of several linears and gated units, symmetric 4-bit
+// the matrix core, one rounding of the result; up to 16 rows of x, symmetric 4-bit
 // fp16 codes in groups of whole chunks meet x as they are and their scale multiplies the chunk's fp32 sum (LATE: closer
 // to exact arithmetic than the rounded w~, and what gemv_w4p_f16 does with them).
 //
@@ -16,7 +16,8 @@
 // banks.  The next step's x and tiles are requested one by one, as the present ones have been read into registers.
 //
 // What bounds it: the expansion of the codes and the stream of them, two waves a SIMD, behind about 2.5 us of launch,
-// first bytes and sums.  8 rows of x of 3 x 4096 x 4096 fp16 4-bit in groups of 128 take 9.0 us (10.8 in
+// first bytes and sums.  8 x 4096 x 11008 fp16 4-bit in groups of 128 takes 8.7 us (x, copied by all waves behind a
+// barrier in two parts, made it 11.0 in gemv_w4p_f16), 16 rows 10.7 (13.5); 8 rows of x of 3 x 4096 x 4096 fp16 4-bit in groups of 128 take 9.0 us (10.8 in
 // gemv_w4p_f16_grouped), 16 of 2 x 11008 x 4096 13.0 (23.5); weights from HBM.  A step in LDS and not two or three: with more in flight from the start
 // every wave's first step comes later (8 x 4096 x 11008 10.7 us).  Above 16 rows x and codes come in at 45 to 55 bytes
 // per ns and CU together: 48 x 11008 x 4096 with a zero point 15.8 us, 64 rows 17.4 and more (not taken).  Codes of a tile read before the products of the tile
@@ -65,7 +66,7 @@ __device__ __forceinline__ void flow_for(F&& f) {
   }
 }
 
-template<typename T, int BITS, bool SIGNED, int ZMODE, bool LATE, int MX, int TL, int NMAT, int NW>
+template<typename T, int BITS, bool SIGNED, int ZMODE, bool LATE, bool TILED, int MX, int TL, int NMAT, int NW>
 __device__ __forceinline__ void
 gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[NMAT], int N,
                uint16_t* __restrict__ y, int act, const FlowArgs& p) {
@@ -87,6 +88,7 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
   constexpr bool kAnyOrder = BITS == 4 && TT<T>::dtype == OFQ_F16;
   constexpr int kRegions = ZMODE == kZeroAsym ? 2 : 1;
   static_assert(2 * STEP < 63, "vmcnt is a 6-bit counter");
+  static_assert(!TILED || (CH == 2 && NMAT == 1 && BITS == 4), "a tile-major copy has 1 KB per tile and chunk");
   static_assert(!LATE || (kAnyOrder && SIGNED && ZMODE == kZeroNone), "one scale a chunk and nothing to add");
   const int M = p.M, K = p.K;
   const int row_bytes = K / LK * 16;
@@ -190,6 +192,15 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
     else async_copy16_at(base, off, to);
   };
   auto copy_tile = [&](int s, int t) {
+    if constexpr (TILED) {
+      const int chunks = K / CK;
+      const uint8_t* base = mats[0].w + (((int64_t)block * TL + t) * chunks + s * CH) * 1024;
+#pragma unroll
+      for (int h = 0; h < CH; ++h) {
+        copy_codes(base, (s * CH + h < chunks ? h * 1024u : 0u) + lane * 16u, lds0 + ring0 + (kXOps + CH * t + h) * 1024);
+      }
+      return;
+    }
     const uint8_t* base = wbase[t / TL] + (int64_t)s * kStepBytes;
     const uint32_t to = lds0 + ring0 + (kXOps + CH * t) * 1024;
     if ((s + 1) * kStepBytes <= row_bytes) {
@@ -231,7 +242,8 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
   int cat[CH];      // and of a tile's codes
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    cat[c] = CH == 2 ? r * 128 + (((c * 4 + kb) ^ (r >> 1)) << 4) : r * 64 + ((kb ^ (r >> 2)) << 4);
+    if constexpr (TILED) cat[c] = c * 1024 + lane * 16;  // (as the copy has them)
+    else cat[c] = CH == 2 ? r * 128 + (((c * 4 + kb) ^ (r >> 1)) << 4) : r * 64 + ((kb ^ (r >> 2)) << 4);
   }
   int srow[TL];
 #pragma unroll
@@ -428,11 +440,12 @@ gemv_flow_body(int block, const uint16_t* __restrict__ x, const RowsMat (&mats)[
   }
 }
 
-template<typename T, int BITS, bool SIGNED, int ZMODE, int MX, int TL, int NW>
+// TILED: the codes as the tile-major copy of the weight has them, rows_per_block of its split.
+template<typename T, int BITS, bool SIGNED, int ZMODE, bool LATE, bool TILED, int MX, int TL, int NW>
 __global__ void __launch_bounds__(NW * 64)
 gemv_flow(const uint16_t* __restrict__ x, RowsMat mat, int N, FlowArgs p) {
   const RowsMat mats[1] = {mat};
-  gemv_flow_body<T, BITS, SIGNED, ZMODE, false, MX, TL, 1, NW>((int)blockIdx.x, x, mats, N, nullptr, 0, p);
+  gemv_flow_body<T, BITS, SIGNED, ZMODE, LATE, TILED, MX, TL, 1, NW>((int)blockIdx.x, x, mats, N, nullptr, 0, p);
 }
 // Several linears of the same m, k and quantisation: the grid is the concatenation of their blocks.
 template<typename T, int BITS, bool SIGNED, int ZMODE, bool LATE, int MX, int TL, int NW>
@@ -441,7 +454,7 @@ gemv_flow_grouped(GemvGroup g, FlowArgs p) {
   const GemvProblem pr = select_problem(g, (int)blockIdx.x);
   const RowsMat mats[1] = {{pr.w, static_cast<const uint16_t*>(pr.scale), static_cast<const uint16_t*>(pr.zero),
                             static_cast<const uint16_t*>(pr.bias), static_cast<uint16_t*>(pr.out)}};
-  gemv_flow_body<T, BITS, SIGNED, ZMODE, LATE, MX, TL, 1, NW>((int)blockIdx.x - pr.first_block,
+  gemv_flow_body<T, BITS, SIGNED, ZMODE, LATE, false, MX, TL, 1, NW>((int)blockIdx.x - pr.first_block,
                                                               static_cast<const uint16_t*>(pr.x), mats, pr.N, nullptr,
                                                               0, p);
 }
@@ -452,7 +465,7 @@ __global__ void __launch_bounds__(NW * 64)
 gemv_flow_glu(const uint16_t* __restrict__ x, RowsMat hidden, RowsMat gate, int N, uint16_t* __restrict__ y, int act,
               FlowArgs p) {
   const RowsMat mats[2] = {hidden, gate};
-  gemv_flow_body<T, BITS, SIGNED, ZMODE, LATE, MX, TL, 2, NW>((int)blockIdx.x, x, mats, N, y, act, p);
+  gemv_flow_body<T, BITS, SIGNED, ZMODE, LATE, false, MX, TL, 2, NW>((int)blockIdx.x, x, mats, N, y, act, p);
 }
 
 }  // namespace

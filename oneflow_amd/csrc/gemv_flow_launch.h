@@ -36,10 +36,19 @@ int launch_flow_inst(hipStream_t st, const LinearJob& job, const FlowPlan& plan)
     GemvGroup g{};
     fill_group(g, job.pr, job.count, plan.rows_per_block);
     kern<<<plan.grid, NW * 64, plan.lds, st>>>(g, p);
-  } else if constexpr (LATE) {
-    return OFQ_ERR_UNSUPPORTED;  // (gemv_flow_choice)
   } else {
-    auto kern = gemv_flow<T, BITS, SIGNED, ZMODE, MX, TL, NW>;
+    // (a tile-major copy has groups of whole chunks and up to 64 rows a block)
+    if constexpr (BITS == 4 && TT<T>::dtype == OFQ_F16 && MX <= 2 && TL <= 4 && (LATE || ZMODE != kZeroNone)) {
+      if (plan.tiled) {
+        auto kern = gemv_flow<T, BITS, SIGNED, ZMODE, LATE, true, MX, TL, NW>;
+        static std::atomic<uint64_t> allowed_tiled{0};
+        if (!ofq_allow_dynamic_lds(reinterpret_cast<const void*>(kern), 160 * 1024, allowed_tiled)) return OFQ_ERR_LAUNCH;
+        kern<<<plan.grid, NW * 64, plan.lds, st>>>(x, rows_mat(a), (int)a.n, p);
+        return ofq_check_launch();
+      }
+    }
+    if (plan.tiled) return OFQ_ERR_UNSUPPORTED;
+    auto kern = gemv_flow<T, BITS, SIGNED, ZMODE, LATE, false, MX, TL, NW>;
     if (!ofq_allow_dynamic_lds(reinterpret_cast<const void*>(kern), 160 * 1024, allowed)) return OFQ_ERR_LAUNCH;
     kern<<<plan.grid, NW * 64, plan.lds, st>>>(x, rows_mat(a), (int)a.n, p);
   }

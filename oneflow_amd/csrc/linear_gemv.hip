@@ -430,6 +430,7 @@ bool flow_plan(const LinearJob& job, FlowPlan* plan) {
       plan->mx = mx;
       plan->tl = tl;
       plan->nw = nw;
+      plan->tiled = 0;
       plan->lds = lds;
       return true;
     }
@@ -454,8 +455,11 @@ bool flow_plan(const LinearJob& job, FlowPlan* plan) {
 //   other gated units of up to 8 rows of x                1.03 (to 1.13; gemv_ring's 8-row tiles), on fp16 4-bit groups
 //                                                         of whole chunks and up to 4 rows 1.02 (gemv_w4p_f16_glu)
 //   bf16 4-bit, more than 64 rows a block                 1.02: bound by the expansion either way
-// One linear of fp16 4-bit groups of whole chunks stays with gemv_w4p_f16 whatever the time (8 x 4096 x 11008 11.0 us
-// there, 8.7 here): a tile-major copy of its weight is read by that kernel, and the two calls give the same bits.
+//   one linear of up to 4 rows of x on fp16 4-bit groups  1.06 to 1.14 (gemv_w4s_f16)
+//   of whole chunks, up to 16 rows a block
+// On 149 other jobs: 0.94, 6 more than 3 % longer, 1.13 at worst (8 x 2 x 3584 x 1280 fp16 4-bit with a zero point).
+// A tile-major copy of a weight (fp16, 4 bits, groups of whole chunks) is asked by the same rule, so that the two calls
+// give the same bits; its blocks have up to 64 rows, as many as here.
 bool gemv_flow_choice(const LinearJob& job, FlowPlan* plan) {
   const LinearArgs& a = job.pr[0];
   for (int i = 0; i < job.count; ++i) {
@@ -477,7 +481,8 @@ bool gemv_flow_choice(const LinearJob& job, FlowPlan* plan) {
   } else if (job.count > 1) {
     if (rows > 80 || (rows > 48 && a.m == 1)) return false;
   } else {
-    if (w4p_supported(a) || rows > (a.m > 8 || bf16_4 ? 64 : 96) || (a.m <= 8 && rows <= 8)) return false;
+    if (rows > (a.m > 8 || bf16_4 || w4p_supported(a) ? 64 : 96) || (a.m <= 8 && rows <= 8)) return false;
+    if (late && a.m <= 4 && rows <= 16) return false;
   }
   return flow_plan(job, plan);
 }
@@ -1236,6 +1241,9 @@ bool gemv_flow_preferred(const LinearArgs& a, bool have_workspace, FlowPlan* pla
   const double us = flow_mt_us(job, *plan);
   return us < gemm_wr_us(a, have_workspace, us < 12.5 ? 3.0 : 0.5);
 }
+int launch_flow_tiled(hipStream_t st, const LinearArgs& a, const FlowPlan& plan) {
+  return launch_gemv_flow_f16_b4(st, LinearJob{&a, 1, false, nullptr, 0}, plan);
+}
 int launch_gemv_flow(hipStream_t st, const LinearArgs& a, const FlowPlan& plan) {
   return launch_flow_by(st, LinearJob{&a, 1, false, nullptr, 0}, plan);
 }
@@ -1564,5 +1572,11 @@ extern "C" int ofq_fused_linear_gq_tiled(void* stream, const void* x, const void
   // what the row-balanced kernel takes: fp16, 4 bits, groups of a multiple of 128 along K, at
   // most 16 rows of x whose m * k halves fit LDS
   if (!w4p_supported(a) || !tiled_shape_ok(num_bits, n, k)) return OFQ_ERR_UNSUPPORTED;
-  return launch_w4p(static_cast<hipStream_t>(stream), a, ilog2_exact(a.group_size / 128), true);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  FlowPlan flow;
+  if (a.m > 1 && gemv_flow_choice(LinearJob{&a, 1, false, nullptr, 0}, &flow)) {
+    flow.tiled = 1;
+    return launch_flow_tiled(st, a, flow);
+  }
+  return launch_w4p(st, a, ilog2_exact(a.group_size / 128), true);
 }

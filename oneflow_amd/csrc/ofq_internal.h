@@ -126,6 +126,7 @@ int launch_gemv_ring_bf16(hipStream_t st, const LinearJob& job, const RingPlan& 
 // The kernel whose waves share nothing (gemv_flow.h), up to 48 rows of x; the choice: up to 16
 struct FlowPlan {
   int grid, rows_per_block, mx, tl, nw;
+  int tiled;  // the weight is its tile-major copy
   size_t lds;
 };
 bool gemv_flow_choice(const LinearJob& job, FlowPlan* plan);
